@@ -141,12 +141,13 @@ def _train(ctl):
     if "trained" in _kept:
         return
     cb.predictor_reset(ctl, seed=1)
-    for scale, factor, seed in ((12, 16, 2), (13, 16, 3), (14, 8, 4), (14, 16, 5)):
+    for scale, factor, seed in ((14, 16, 2), (16, 16, 3)):
         m = cb.matrix_dcsr_from_cpu(ctl, *gen.to_dcsr(*gen.rmat(scale, factor, seed)), 1 << scale)
         cb.predictor_harvest(ctl, m, m)
-    m = cb.matrix_dcsr_from_cpu(ctl, *gen.to_dcsr(*gen.hypersparse_zipf(6, log_n=20)), 1 << 20)
-    cb.predictor_harvest(ctl, m, m)
-    cb.predictor_train(ctl, epochs=30, batch=1024, lr=3e-3, seed=1)
+    for log_n, seed in ((21, 4), (22, 5), (22, 6)):
+        m = cb.matrix_dcsr_from_cpu(ctl, *gen.to_dcsr(*gen.hypersparse_zipf(seed, log_n=log_n)), 1 << log_n)
+        cb.predictor_harvest(ctl, m, m)
+    cb.predictor_train(ctl, epochs=60, batch=1024, lr=2e-3, seed=1)
     _kept["trained"] = True
 
 
