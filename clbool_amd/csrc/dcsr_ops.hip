@@ -165,14 +165,14 @@ clb_status clb_dcsr_transpose(clb_controls ctl, const clb_dcsr *a, clb_dcsr *out
         const u64 n = a->nnz;
         DevArray<u32> arow(ctl, n);
         dcsr_expand_rows(ctl, u32p(a->rpt), u32p(a->rows), a->nzr, a->nnz, arow.ptr);
-        DevArray<u64> keys(ctl, n);
-        // key = col << 32 | row: sorted, it is the transposed row-major order
-        pack_pairs(ctl, u32p(a->cols), arow.ptr, n, keys.ptr);
-        sort_pair_keys(ctl, keys.ptr, n, a->ncols ? a->ncols - 1 : 0, a->nrows ? a->nrows - 1 : 0);
         clb_buffer_s *rows = buffer_new(ctl, 4 * n);
         try {
             r.cols = buffer_new(ctl, 4 * n);
-            unpack_pairs(ctl, keys.ptr, n, u32p(rows), u32p(r.cols));
+            // the rows ascend already, so a stable sort by column alone gives
+            // the transposed row-major order: passes over the bits of ncols
+            // only (at 2^20 x 2^20, 3 instead of 6)
+            sort_pairs(ctl, u32p(a->cols), arow.ptr, n, a->ncols ? a->ncols - 1 : 0, a->nrows ? a->nrows - 1 : 0,
+                       true, u32p(rows), u32p(r.cols));
             rows_to_dcsr(ctl, u32p(rows), a->nnz, &r.rpt, &r.rows, &r.nzr);
             r.nnz = a->nnz;
             buffer_release(rows);

@@ -6,13 +6,17 @@
 
 namespace clb {
 
-// Stable LSD radix sort of 64-bit keys row << 32 | col, over the low
-// col_bits of the column half and the low row_bits of the row half.
+// Stable sorts of pairs (row, col), over only the bits that the largest row
+// and column need.  radix_sort_keys: 64-bit keys row << 32 | col in place.
+// sort_pairs_to_keys: two arrays to sorted keys.  sort_pairs: two arrays to
+// two arrays (which may be the same), by_row_only: stable by row alone.
 void radix_sort_keys(clb_controls_s *ctl, u64 *keys, u64 n, int col_bits, int row_bits);
-void sort_pair_keys(clb_controls_s *ctl, u64 *keys, u64 n, u32 max_row, u32 max_col);
+void sort_pairs_to_keys(clb_controls_s *ctl, const u32 *rows, const u32 *cols, u64 n, u32 max_row, u32 max_col,
+                        u64 *keys);
+void sort_pairs(clb_controls_s *ctl, const u32 *rows, const u32 *cols, u64 n, u32 max_row, u32 max_col,
+                bool by_row_only, u32 *out_rows, u32 *out_cols);
 void pack_pairs(clb_controls_s *ctl, const u32 *rows, const u32 *cols, u64 n, u64 *keys);
-void unpack_pairs(clb_controls_s *ctl, const u64 *keys, u64 n, u32 *rows, u32 *cols);
-void key_bounds(clb_controls_s *ctl, const u64 *keys, u64 n, u32 *max_row, u32 *max_col);
+void pair_bounds(clb_controls_s *ctl, const u32 *rows, const u32 *cols, u64 n, u32 *max_row, u32 *max_col);
 // Sorted keys -> new deduplicated (rows, cols) buffers; returns their length.
 u32 unique_keys_to_pairs(clb_controls_s *ctl, const u64 *keys, u64 n, clb_buffer_s **rows_out,
                          clb_buffer_s **cols_out);
