@@ -13,9 +13,9 @@
 // with no per-row load imbalance; the CSR row pointer is rebuilt by one
 // lower-bound search per row.  The DCSR union (the X += T step of a closure)
 // reuses the same engine.
-#include "sort.hpp"
-
 #include "device_utils.hpp"
+#include "expand.hpp"
+#include "sort.hpp"
 
 namespace clb {
 
@@ -79,25 +79,6 @@ __global__ __launch_bounds__(MG_WG) void k_merge_tiles(const u64 *__restrict__ A
         if (k0 + k < n) s[k0 + k] = v[k];
     __syncthreads();
     for (u32 t = threadIdx.x; t < n; t += MG_WG) out[d0 + t] = s[t];
-}
-
-// Keys of a CSR matrix, one wave per row.
-__global__ __launch_bounds__(256) void k_csr_keys(const u32 *__restrict__ rpt, const u32 *__restrict__ cols,
-                                                  u32 nrows, u32 limit, u64 *__restrict__ keys) {
-    const u32 r = blockIdx.x * 4 + dev::wave_id();
-    if (r >= nrows) return;
-    const u32 e = rpt[r + 1] < limit ? rpt[r + 1] : limit;
-    for (u32 j = rpt[r] + dev::lane(); j < e; j += 64) keys[j] = ((u64)r << 32) | cols[j];
-}
-
-// Keys of a DCSR matrix, one wave per stored row.
-__global__ __launch_bounds__(256) void k_dcsr_keys(const u32 *__restrict__ rpt, const u32 *__restrict__ rows,
-                                                   const u32 *__restrict__ cols, u32 nzr, u64 *__restrict__ keys) {
-    const u32 r = blockIdx.x * 4 + dev::wave_id();
-    if (r >= nzr) return;
-    const u64 hi = (u64)rows[r] << 32;
-    const u32 e = rpt[r + 1];
-    for (u32 j = rpt[r] + dev::lane(); j < e; j += 64) keys[j] = hi | cols[j];
 }
 
 // CSR row pointer of sorted rows: rpt[r] = lower_bound(rows, r), r <= nrows.
@@ -222,9 +203,10 @@ clb_status clb_csr_addition(clb_controls ctl, const clb_csr *a, const clb_csr *b
         na = na < a->nnz ? na : a->nnz;
         nb = nb < b->nnz ? nb : b->nnz;
         DevArray<u64> ka(ctl, na ? na : 1), kb(ctl, nb ? nb : 1);
-        k_csr_keys<<<div_up(a->nrows, 4), 256, 0, ctl->stream>>>(u32p(a->rpt), u32p(a->cols), a->nrows, na, ka.ptr);
-        k_csr_keys<<<div_up(b->nrows, 4), 256, 0, ctl->stream>>>(u32p(b->rpt), u32p(b->cols), b->nrows, nb, kb.ptr);
-        CLB_LAUNCHED("csr_keys");
+        expand_rows(ctl, u32p(a->rpt), nullptr, 0, a->nrows, 0, na,
+                    KeyOfNonzero{u32p(a->cols), 0, 0, ka.ptr});
+        expand_rows(ctl, u32p(b->rpt), nullptr, 0, b->nrows, 0, nb,
+                    KeyOfNonzero{u32p(b->cols), 0, 0, kb.ptr});
         clb_buffer_s *rows = nullptr;
         const u32 m = union_keys(ctl, ka.ptr, na, kb.ptr, nb, &rows, &r.cols);
         try {
@@ -271,11 +253,10 @@ clb_status clb_dcsr_addition(clb_controls ctl, const clb_dcsr *a, const clb_dcsr
             return;
         }
         DevArray<u64> ka(ctl, a->nnz), kb(ctl, b->nnz);
-        k_dcsr_keys<<<div_up(a->nzr, 4), 256, 0, ctl->stream>>>(u32p(a->rpt), u32p(a->rows), u32p(a->cols), a->nzr,
-                                                                 ka.ptr);
-        k_dcsr_keys<<<div_up(b->nzr, 4), 256, 0, ctl->stream>>>(u32p(b->rpt), u32p(b->rows), u32p(b->cols), b->nzr,
-                                                                 kb.ptr);
-        CLB_LAUNCHED("dcsr_keys");
+        expand_rows(ctl, u32p(a->rpt), u32p(a->rows), 0, a->nzr, 0, a->nnz,
+                    KeyOfNonzero{u32p(a->cols), 0, 0, ka.ptr});
+        expand_rows(ctl, u32p(b->rpt), u32p(b->rows), 0, b->nzr, 0, b->nnz,
+                    KeyOfNonzero{u32p(b->cols), 0, 0, kb.ptr});
         DevArray<u64> merged(ctl, (u64)a->nnz + b->nnz);
         merge_keys(ctl, ka.ptr, a->nnz, kb.ptr, b->nnz, merged.ptr);
         keys_to_dcsr(ctl, merged.ptr, (u64)a->nnz + b->nnz, r);

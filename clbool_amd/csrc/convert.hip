@@ -1,73 +1,122 @@
 // convert.hip -- format conversions between COO, CSR and DCSR.
 //
 // Restates src/common/matrices_conversions.cpp: coo_to_dcsr_shallow (:78-91,
-// rows compressed by flag/scan/scatter, cols shared), dcsr_to_coo_shallow /
+// rows
+// compressed by counting row starts per tile, cols shared), dcsr_to_coo_shallow /
 // _deep (:43-76), dcsr_to_csr (:247-271, cols shared, nnz checked) and
 // csr_to_dcsr (:211-244, empty rows dropped, cols shared).
-#include "sort.hpp"
-
 #include "device_utils.hpp"
+#include "expand.hpp"
+#include "sort.hpp"
 
 namespace clb {
 
-// prepare_array_for_rows_positions (prepare_positions.cl:29-44), with a
-// trailing 0 so that an exclusive scan of n+1 entries yields nzr at [n].
-__global__ void k_row_start_flags(const u32 *__restrict__ rows, u32 n, u32 *__restrict__ flags) {
-    const u32 i = blockIdx.x * blockDim.x + threadIdx.x;
-    if (i < n) flags[i] = (i == 0 || rows[i] != rows[i - 1]) ? 1u : 0u;
-    if (i == n) flags[n] = 0;
+// Rows of a COO matrix -> the DCSR row pointer and rows
+// (prepare_array_for_rows_positions, prepare_positions.cl:29-44, and
+// set_positions_rows, set_positions.cl:89-113).  A row starts where rows[i]
+// differs from rows[i - 1].  The starts are counted per tile of RP_TILE
+// entries, the tiles' counts are scanned, and a second pass places each start
+// by its rank in the tile.  Both passes read the rows once, 16 bytes per lane;
+// nothing of the size of nnz is written or scanned (flags and their scan over
+// 16.1 million entries took 195 us).
+constexpr u32 RP_WG = 256, RP_ROUNDS = 4, RP_TILE = RP_WG * RP_ROUNDS * 4;
+
+// The flags (bit k: entry i + k starts a row) of the four entries at i.
+__device__ __forceinline__ u32 row_start_bits(const u32 *__restrict__ rows, u32 n, u64 i, u32 (&v)[4]) {
+    u32 prev = i && i < n ? rows[i - 1] : 0u;
+    if (i + 4 <= n) {
+        const uint4 x = *reinterpret_cast<const uint4 *>(rows + i);  // i is a multiple of 4
+        v[0] = x.x;
+        v[1] = x.y;
+        v[2] = x.z;
+        v[3] = x.w;
+    } else {
+#pragma unroll
+        for (u32 k = 0; k < 4; ++k) v[k] = i + k < n ? rows[i + k] : 0u;
+    }
+    u32 f = 0;
+#pragma unroll
+    for (u32 k = 0; k < 4; ++k) {
+        if (i + k < n && (i + k == 0 || v[k] != prev)) f |= 1u << k;
+        prev = v[k];
+    }
+    return f;
 }
 
-// set_positions_rows (set_positions.cl:89-113)
-__global__ void k_set_rows(const u32 *__restrict__ rows, const u32 *__restrict__ pos, u32 n, u32 nzr,
-                           u32 *__restrict__ rpt, u32 *__restrict__ crows) {
-    const u32 i = blockIdx.x * blockDim.x + threadIdx.x;
-    if (i == 0) rpt[nzr] = n;
-    if (i < n && pos[i] != pos[i + 1]) {
-        rpt[pos[i]] = i;
-        crows[pos[i]] = rows[i];
+__global__ __launch_bounds__(RP_WG) void k_row_starts_count(const u32 *__restrict__ rows, u32 n,
+                                                            u32 *__restrict__ counts) {
+    __shared__ u32 red[RP_WG / dev::WAVE + 1];
+    const u64 base = (u64)blockIdx.x * RP_TILE;
+    u32 c = 0;
+#pragma unroll
+    for (u32 q = 0; q < RP_ROUNDS; ++q) {
+        u32 v[4];
+        c += (u32)__popc(row_start_bits(rows, n, base + (q * RP_WG + threadIdx.x) * 4, v));
     }
+    const u32 t = dev::block_sum<u32, RP_WG>(c, red);
+    if (threadIdx.x == 0) counts[blockIdx.x] = t;
+}
+
+__global__ __launch_bounds__(RP_WG) void k_row_starts_place(const u32 *__restrict__ rows, u32 n,
+                                                            const u32 *__restrict__ offs,
+                                                            const u32 *__restrict__ total, u32 *__restrict__ rpt,
+                                                            u32 *__restrict__ crows) {
+    __shared__ u32 red[RP_WG / dev::WAVE + 1];
+    const u64 base = (u64)blockIdx.x * RP_TILE;
+    u32 at = offs[blockIdx.x];
+    for (u32 q = 0; q < RP_ROUNDS; ++q) {
+        const u64 i = base + (q * RP_WG + threadIdx.x) * 4;
+        u32 v[4];
+        const u32 f = row_start_bits(rows, n, i, v);
+        u32 all;
+        u32 p = at + dev::block_excl_scan<u32, RP_WG>((u32)__popc(f), red, all);
+#pragma unroll
+        for (u32 k = 0; k < 4; ++k)
+            if ((f >> k) & 1u) {
+                rpt[p] = (u32)i + k;
+                crows[p] = v[k];
+                ++p;
+            }
+        at += all;
+    }
+    if (blockIdx.x == 0 && threadIdx.x == 0) rpt[*total] = n;
 }
 
 void rows_to_dcsr(clb_controls_s *ctl, const u32 *rows, u32 nnz, clb_buffer_s **rpt_out, clb_buffer_s **rows_out,
                   u32 *nzr_out) {
-    DevArray<u32> pos(ctl, (u64)nnz + 1);
-    k_row_start_flags<<<div_up((u64)nnz + 1, 256), 256, 0, ctl->stream>>>(rows, nnz, pos.ptr);
+    const u32 tiles = div_up(nnz, RP_TILE);
+    DevArray<u32> offs(ctl, (u64)tiles + 1);  // [tiles]: the number of rows
+    k_row_starts_count<<<tiles, RP_WG, 0, ctl->stream>>>(rows, nnz, offs.ptr);
     CLB_LAUNCHED("prepare_array_for_rows_positions");
-    DevArray<u32> tot(ctl, 1);
-    exclusive_scan_u32(ctl, pos.ptr, pos.ptr, (u64)nnz + 1, tot.ptr);
+    exclusive_scan_u32(ctl, offs.ptr, offs.ptr, tiles, offs.ptr + tiles);
     u32 nzr = 0;
-    readback(ctl, &nzr, tot.ptr, 4);
+    readback(ctl, &nzr, offs.ptr + tiles, 4);
     clb_buffer_s *rpt = buffer_new(ctl, 4ull * (nzr + 1ull));
     clb_buffer_s *cr = nullptr;
     try {
         cr = buffer_new(ctl, 4ull * (nzr ? nzr : 1));
+        k_row_starts_place<<<tiles, RP_WG, 0, ctl->stream>>>(rows, nnz, offs.ptr, offs.ptr + tiles, u32p(rpt),
+                                                             u32p(cr));
+        CLB_LAUNCHED("set_positions_rows");
+        sync(ctl);
     } catch (...) {
         buffer_release(rpt);
+        buffer_release(cr);
         throw;
     }
-    k_set_rows<<<div_up(nnz, 256), 256, 0, ctl->stream>>>(rows, pos.ptr, nnz, nzr, u32p(rpt), u32p(cr));
-    CLB_LAUNCHED("set_positions_rows");
-    sync(ctl);
     *rpt_out = rpt;
     *rows_out = cr;
     *nzr_out = nzr;
 }
 
-// dscr_to_coo (dscr_to_coo.cl:8-23): one wave per stored row.
-__global__ __launch_bounds__(256) void k_expand_rows(const u32 *__restrict__ rpt, const u32 *__restrict__ rows,
-                                                     u32 nzr, u32 *__restrict__ out) {
-    const u32 r = blockIdx.x * 4 + dev::wave_id();
-    if (r >= nzr) return;
-    const u32 v = rows[r], e = rpt[r + 1];
-    for (u32 j = rpt[r] + dev::lane(); j < e; j += 64) out[j] = v;
-}
+// dscr_to_coo (dscr_to_coo.cl:8-23)
+struct RowOfNonzero {
+    u32 *out;
+    __device__ __forceinline__ void operator()(u32 e, u32, u32 id) const { out[e] = id; }
+};
 
 void dcsr_expand_rows(clb_controls_s *ctl, const u32 *rpt, const u32 *rows, u32 nzr, u32 nnz, u32 *out_rows) {
-    (void)nnz;
-    if (!nzr) return;
-    k_expand_rows<<<div_up(nzr, 4), 256, 0, ctl->stream>>>(rpt, rows, nzr, out_rows);
-    CLB_LAUNCHED("dscr_to_coo");
+    expand_rows(ctl, rpt, rows, 0, nzr, 0, nnz, RowOfNonzero{out_rows});
 }
 
 // dcsr_to_csr_set_size (conversions.cl:8-18)
