@@ -271,19 +271,15 @@ __global__ void k_failed_keys(const u32 *__restrict__ nnz_row, const u32 *__rest
     key2[i] = nnz_row[i] == FAILED ? (P < ncols ? P : ncols) : 0u;
 }
 
-// Copy each row from the temporary buffers to its exact place and accumulate
-// the prediction error |log2(1+pred) - log2(1+n)|.  A workgroup takes
-// CR_ROWS consecutive rows: each wave copies one of them, except rows of at
-// least CR_LONG columns, which the whole workgroup copies in turn; the error
-// is reduced in LDS and added with one atomic per workgroup.
+// Copy each row from the temporary buffers to its exact place.  A workgroup
+// takes CR_ROWS consecutive rows: each wave copies one of them, except rows of
+// at least CR_LONG columns, which the whole workgroup copies in turn.
 constexpr u32 CR_WG = 256, CR_ROWS = CR_WG / 64, CR_LONG = 2048;
 __global__ __launch_bounds__(CR_WG) void k_compact_rows(const u32 *__restrict__ nnz_row, const u64 *__restrict__ off,
                                                         u32 nrows, const u32 *__restrict__ temp,
                                                         const u64 *__restrict__ toff, const u32 *__restrict__ side,
                                                         const u64 *__restrict__ soff, const u32 *__restrict__ key2,
-                                                        const u32 *__restrict__ isdense, const float *__restrict__ pred,
-                                                        u32 *__restrict__ cols, double *__restrict__ err) {
-    __shared__ double red[CR_ROWS];
+                                                        const u32 *__restrict__ isdense, u32 *__restrict__ cols) {
     const u32 wv = dev::wave_id(), l = (u32)dev::lane();
     const u32 r0 = blockIdx.x * CR_ROWS;
     auto copy = [&](const u32 *src, u32 *dst, u32 n, u32 t, u32 step) {
@@ -305,21 +301,6 @@ __global__ __launch_bounds__(CR_WG) void k_compact_rows(const u32 *__restrict__ 
         u32 *dst = cols + off[r];
         if (n >= CR_LONG) copy(src, dst, n, threadIdx.x, CR_WG);
         else if (wv == j) copy(src, dst, n, l, 64u);
-    }
-    if (pred && err) {
-        double e = 0.0;
-        const u32 r = r0 + wv;
-        if (l == 0 && r < nrows) {
-            const u32 n = nnz_row[r];
-            if (n) e = fabs(log2(1.0 + (double)pred[r]) - log2(1.0 + (double)n));
-        }
-        if (l == 0) red[wv] = e;
-        __syncthreads();
-        if (threadIdx.x == 0) {
-            double t = 0.0;
-            for (u32 k = 0; k < CR_ROWS; ++k) t += red[k];
-            if (t != 0.0) atomicAdd(err, t);
-        }
     }
 }
 
@@ -397,16 +378,19 @@ __global__ __launch_bounds__(CC_WG) void k_compact_tiles(const u32 *__restrict__
     }
 }
 
-// Mean-error numerator sum over rows of |log2(1 + pred) - log2(1 + n)|
-// (rows with output), one atomic per workgroup.
+// Mean-error numerator: sum over rows with output of |log2(1 + pred) -
+// log2(1 + n)|.  Grid-stride with at most PE_GRID workgroups, one atomic each:
+// all of them add to one double, which takes about 11 ns an addition (one per
+// four rows, as part of the compaction, made that kernel 1.65 ms on 582
+// thousand rows).
+constexpr u32 PE_GRID = 256;
 __global__ __launch_bounds__(256) void k_pred_error(const u32 *__restrict__ nnz_row, const float *__restrict__ pred,
                                                     u32 nrows, double *__restrict__ err) {
     __shared__ double red[256 / 64 + 1];
-    const u32 r = blockIdx.x * 256 + threadIdx.x;
     double e = 0.0;
-    if (r < nrows) {
+    for (u64 r = (u64)blockIdx.x * 256 + threadIdx.x; r < nrows; r += (u64)gridDim.x * 256) {
         const u32 n = nnz_row[r];
-        if (n) e = fabs(log2(1.0 + (double)pred[r]) - log2(1.0 + (double)n));
+        if (n) e += fabs(log2(1.0 + (double)pred[r]) - log2(1.0 + (double)n));
     }
     const double s = dev::block_sum<double, 256>(e, red);
     if (threadIdx.x == 0 && s != 0.0) atomicAdd(err, s);
@@ -416,15 +400,16 @@ void compact_rows(hipStream_t st, u32 nrows, u64 nnz, const u32 *nnz_row, const 
                   const u64 *toff, const u32 *side, const u64 *soff, const u32 *key2, const u32 *isdense,
                   const float *pred, u32 *cols, double *err, bool by_tiles) {
     if (!nrows) return;
+    if (pred && err) {
+        const u32 grid = div_up(nrows, 256) < PE_GRID ? div_up(nrows, 256) : PE_GRID;
+        k_pred_error<<<grid, 256, 0, st>>>(nnz_row, pred, nrows, err);
+        CLB_LAUNCHED("pred_error");
+    }
     if (!by_tiles) {
         k_compact_rows<<<div_up(nrows, CR_ROWS), CR_WG, 0, st>>>(nnz_row, off, nrows, temp, toff, side, soff, key2,
-                                                                  isdense, pred, cols, err);
+                                                                  isdense, cols);
         CLB_LAUNCHED("compact_rows");
         return;
-    }
-    if (pred && err) {
-        k_pred_error<<<div_up(nrows, 256), 256, 0, st>>>(nnz_row, pred, nrows, err);
-        CLB_LAUNCHED("pred_error");
     }
     if (nnz) {
         k_compact_tiles<<<div_up(nnz, CC_TILE), CC_WG, 0, st>>>(nnz_row, off, nrows, temp, toff, side, soff, key2,
