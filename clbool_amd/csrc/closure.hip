@@ -16,6 +16,7 @@
 // canonical DCSR) -- and drops duplicates.  Every step of both modes is
 // bit-exact: the products
 // and unions are exact set operations, only the launch structure differs.
+#include "expand.hpp"
 #include "sort.hpp"
 #include "spgemm.hpp"
 
@@ -67,27 +68,65 @@ __global__ void k_stack_cols(const Seg *__restrict__ segs, u32 nseg, u32 total_n
     cols[e] = s.cols[e - s.nnz_off] + s.col_shift;
 }
 
-// Keys (row << 32 | col) of a DCSR matrix with rows shifted, one wave per row.
-__global__ __launch_bounds__(256) void k_keys_shifted(const u32 *__restrict__ rpt, const u32 *__restrict__ rows,
-                                                      const u32 *__restrict__ cols, u32 nzr, u32 row_shift,
-                                                      u64 *__restrict__ keys) {
-    const u32 r = blockIdx.x * 4 + dev::wave_id();
-    if (r >= nzr) return;
-    const u64 hi = (u64)(rows[r] + row_shift) << 32;
-    const u32 e = rpt[r + 1];
-    for (u32 j = rpt[r] + dev::lane(); j < e; j += 64) keys[j] = hi | cols[j];
-}
+// Keys (row << 32 | col) of many pieces of DCSR matrices in one launch.
+struct KeySeg {
+    const u32 *rpt, *rows, *cols;
+    u32 r_lo, r_hi;    // the piece's stored rows: nonzeros [rpt[r_lo], rpt[r_hi])
+    u32 e_lo, e_hi;
+    u32 row_shift;     // added to row ids (modulo 2^32)
+    u32 tile0;         // its first tile of the launch
+    u64 *keys;         // the piece's first key
+};
 
-// Keys (row << 32 | col) of stored rows [r0, r1) of a DCSR matrix, rows
-// shifted (modulo 2^32), written from keys[rpt[r] - nnz_base]; one wave per row.
-__global__ __launch_bounds__(256) void k_keys_range(const u32 *__restrict__ rpt, const u32 *__restrict__ rows,
-                                                    const u32 *__restrict__ cols, u32 r0, u32 r1, u32 row_shift,
-                                                    u32 nnz_base, u64 *__restrict__ keys) {
-    const u32 r = r0 + blockIdx.x * 4 + dev::wave_id();
-    if (r >= r1) return;
-    const u64 hi = (u64)(rows[r] + row_shift) << 32;
-    const u32 e = rpt[r + 1];
-    for (u32 j = rpt[r] + dev::lane(); j < e; j += 64) keys[j - nnz_base] = hi | cols[j];
+// One tile of EX_TILE nonzeros per workgroup.  The piece is found by one
+// probe per thread, the tile's first and last rows by rounds of a 256-way
+// split: dependent loads, but no launch of its own per piece, and a closure's
+// pieces are many and mostly small.
+__global__ __launch_bounds__(EX_WG) void k_keys_segs(const KeySeg *__restrict__ segs, u32 nseg) {
+    __shared__ u32 srpt[EX_TILE], srow[EX_TILE];
+    u32 s = 0;  // last piece with tile0 <= this tile (pieces are not empty)
+    for (u32 b = 0; b < nseg; b += EX_WG) {
+        const u32 k = b + threadIdx.x;
+        s += (u32)__syncthreads_count(k < nseg && segs[k].tile0 <= blockIdx.x);
+    }
+    const KeySeg g = segs[s - 1];
+    const u64 e0 = (u64)g.e_lo + (u64)(blockIdx.x - g.tile0) * EX_TILE;
+    const u64 e1 = e0 + EX_TILE < g.e_hi ? e0 + EX_TILE : g.e_hi;
+    // last row in [lo, hi) that starts at or before e
+    auto row_of = [&](u32 lo, u32 hi, u64 e) {
+        while (hi - lo > 1) {
+            const u32 step = (hi - lo + EX_WG - 1) / EX_WG;
+            const u64 c = (u64)lo + (u64)threadIdx.x * step;
+            const u32 cnt = (u32)__syncthreads_count(c < hi && g.rpt[c] <= e);
+            lo += (cnt - 1) * step;
+            hi = hi - lo < step ? hi : lo + step;
+        }
+        return lo;
+    };
+    const u32 r0 = row_of(g.r_lo, g.r_hi, e0);
+    // at most EX_TILE rows, unless some stored rows are empty
+    const bool near = g.r_hi - r0 > EX_TILE && g.rpt[r0 + EX_TILE] >= e1;
+    const u32 nr = row_of(r0, near ? r0 + EX_TILE : g.r_hi, e1 - 1) - r0 + 1;
+    const bool staged = nr <= EX_TILE;
+    if (staged)
+        for (u32 j = threadIdx.x; j < nr; j += EX_WG) {
+            srpt[j] = g.rpt[r0 + j];
+            srow[j] = g.rows[r0 + j];
+        }
+    __syncthreads();
+#pragma unroll
+    for (u32 q = 0; q < EX_ITEMS; ++q) {
+        const u64 e = e0 + q * EX_WG + threadIdx.x;
+        if (e >= e1) break;
+        u32 a = 0, b = nr;
+        while (b - a > 1) {
+            const u32 m = (a + b) >> 1;
+            if ((staged ? srpt[m] : g.rpt[r0 + m]) <= e) a = m;
+            else b = m;
+        }
+        const u32 id = staged ? srow[a] : g.rows[r0 + a];
+        g.keys[e - g.e_lo] = ((u64)(id + g.row_shift) << 32) | g.cols[e];
+    }
 }
 
 // zlen[row id] = stored length of that row of Z' (zlen pre-filled with 0).
@@ -201,6 +240,119 @@ static Seg seg_of(const clb_dcsr &m, u32 row_shift, u32 col_shift) {
     return Seg{u32p(m.rpt), u32p(m.rows), u32p(m.cols), m.nzr, m.nnz, row_shift, col_shift, 0, 0};
 }
 
+// X |= its products for every distinct X of the step.  A batch of X
+// matrices is united at once: their keys are stacked (matrix x in rows
+// [x * n, (x + 1) * n)) into one sorted list, and so are, for r = 0, 1, ..., the
+// products of each one's r-th triple (a product's parts in consecutive row
+// blocks follow each other in row order).  The products' lists are merged
+// pairwise into one, which the union then meets the matrices' list with.  A
+// batch holds at most UNITE_KEYS keys (or one matrix), which bounds its
+// memory; united one by one, the 17 matrices of a 32-rule step took 4.0 ms,
+// mostly launches and read-backs, for 6.1 million keys.
+constexpr u64 UNITE_KEYS = 1ull << 27;
+
+static void unite_products(clb_controls_s *ctl, clb_dcsr *mats, const std::vector<u32> &xs, const u32 *triples,
+                           u32 ntriples, u32 n, const std::vector<clb_dcsr> &prods,
+                           const std::vector<std::vector<u32>> &splits) {
+    auto part = [&](size_t q, u32 t) -> u64 { return splits[q][2 * t + 3] - splits[q][2 * t + 1]; };
+    std::vector<std::vector<u32>> of(xs.size());  // each X's triples with products
+    std::vector<u64> add(xs.size(), 0);           // their nonzeros
+    for (u32 t = 0; t < ntriples; ++t) {
+        u64 len = 0;
+        for (size_t q = 0; q < prods.size(); ++q) len += part(q, t);
+        if (!len) continue;
+        const size_t k = std::lower_bound(xs.begin(), xs.end(), triples[3 * t]) - xs.begin();
+        of[k].push_back(t);
+        add[k] += len;
+    }
+    size_t k0 = 0;
+    while (k0 < xs.size()) {
+        if (of[k0].empty()) {
+            ++k0;
+            continue;
+        }
+        std::vector<size_t> batch;
+        u64 total = 0, base = 0;  // keys in all, and of the matrices themselves
+        size_t k1 = k0;
+        for (; k1 < xs.size(); ++k1) {
+            if (of[k1].empty()) continue;
+            const u64 mine = mats[xs[k1]].nnz + add[k1];
+            if (mine >= 0xFFFFFFFFull) raise(INVALID_VALUE, "a closure union exceeds uint32 nonzeros");
+            if (!batch.empty() && total + mine > UNITE_KEYS) break;
+            batch.push_back(k1);
+            total += mine;
+            base += mats[xs[k1]].nnz;
+        }
+        k0 = k1;
+        DevArray<u64> keys(ctl, total), tmp(ctl, total - base);  // matrices | products; tmp: products
+        std::vector<KeySeg> segs;
+        u32 tiles = 0;
+        auto piece = [&](const clb_dcsr &m, u32 r_lo, u32 r_hi, u32 e_lo, u32 e_hi, u32 shift, u64 at) {
+            if (e_hi == e_lo) return;
+            segs.push_back(KeySeg{u32p(m.rpt), u32p(m.rows), u32p(m.cols), r_lo, r_hi, e_lo, e_hi, shift, tiles,
+                                  keys.ptr + at});
+            tiles += div_up((u64)e_hi - e_lo, EX_TILE);
+        };
+        u64 pos = 0;
+        size_t rounds = 0;
+        for (size_t i = 0; i < batch.size(); ++i) {
+            const clb_dcsr &x = mats[xs[batch[i]]];
+            piece(x, 0, x.nzr, 0, x.nnz, (u32)i * n, pos);
+            pos += x.nnz;
+            rounds = std::max(rounds, of[batch[i]].size());
+        }
+        std::vector<std::pair<u64, u64>> lists;  // (start, length) after the matrices' keys
+        for (size_t r = 0; r < rounds; ++r) {
+            const u64 start = pos;
+            for (size_t i = 0; i < batch.size(); ++i) {
+                if (r >= of[batch[i]].size()) continue;
+                const u32 t = of[batch[i]][r];
+                for (size_t q = 0; q < prods.size(); ++q) {
+                    const std::vector<u32> &hs = splits[q];
+                    // rows t * n + row -> i * n + row
+                    piece(prods[q], hs[2 * t], hs[2 * t + 2], hs[2 * t + 1], hs[2 * t + 3], ((u32)i - t) * n, pos);
+                    pos += part(q, t);
+                }
+            }
+            lists.push_back({start - base, pos - start});
+        }
+        DevArray<KeySeg> dsegs(ctl, segs.size());
+        CLB_HIP(hipMemcpyAsync(dsegs.ptr, segs.data(), segs.size() * sizeof(KeySeg), hipMemcpyHostToDevice,
+                               ctl->stream),
+                WRITE_BUFFER_ERROR);
+        k_keys_segs<<<tiles, EX_WG, 0, ctl->stream>>>(dsegs.ptr, (u32)segs.size());
+        CLB_LAUNCHED("keys");
+        u64 *cur = keys.ptr + base, *nxt = tmp.ptr;
+        while (lists.size() > 1) {
+            std::vector<std::pair<u64, u64>> next;
+            for (size_t i = 0; i < lists.size(); i += 2) {
+                const auto &la = lists[i];
+                if (i + 1 == lists.size()) {  // odd one out: copied to the other buffer
+                    CLB_HIP(hipMemcpyAsync(nxt + la.first, cur + la.first, 8 * la.second, hipMemcpyDeviceToDevice,
+                                           ctl->stream),
+                            COPY_BUFFER_ERROR);
+                    next.push_back(la);
+                    continue;
+                }
+                const auto &lb = lists[i + 1];  // adjacent
+                merge_keys(ctl, cur + la.first, la.second, cur + lb.first, lb.second, nxt + la.first);
+                next.push_back({la.first, la.second + lb.second});
+            }
+            lists.swap(next);
+            std::swap(cur, nxt);
+        }
+        std::vector<clb_dcsr> united;
+        for (size_t i : batch) united.push_back(mats[xs[i]]);
+        union_keys_to_matrices(ctl, keys.ptr, base, cur, total - base, n, united);
+        for (size_t i = 0; i < batch.size(); ++i) {
+            clb_dcsr &x = mats[xs[batch[i]]];
+            if (united[i].cols == x.cols) continue;  // unchanged
+            clb_dcsr_release(&x);
+            x = united[i];
+        }
+    }
+}
+
 }  // namespace clb
 
 using namespace clb;
@@ -228,7 +380,6 @@ clb_status clb_closure_step(clb_controls ctl, clb_dcsr *mats, uint32_t nmats, co
         for (u32 t = 0; t < ntriples; ++t) xs.push_back(triples[3 * t]);
         std::sort(xs.begin(), xs.end());
         xs.erase(std::unique(xs.begin(), xs.end()), xs.end());
-        auto xid = [&](u32 m) { return (u32)(std::lower_bound(xs.begin(), xs.end(), m) - xs.begin()); };
         clb_spgemm_opts so{};
         so.mode = o.spgemm_mode;
         auto t_prod = t0;  // end of the products phase
@@ -401,78 +552,7 @@ clb_status clb_closure_step(clb_controls ctl, clb_dcsr *mats, uint32_t nmats, co
             sync(ctl);
             t_prod = std::chrono::steady_clock::now();
             try {
-                // one union per distinct X.  Its keys and, per triple that
-                // targets it, the keys of that triple's product rows (its
-                // parts in consecutive row blocks concatenate in row order)
-                // form sorted segments; rounds of pairwise merges turn them
-                // into one sorted list, whose duplicates are then dropped.
-                for (u32 k = 0; k < (u32)xs.size(); ++k) {
-                    clb_dcsr &x = mats[xs[k]];
-                    u64 seg = x.nnz;
-                    for (size_t q = 0; q < prods.size(); ++q)
-                        for (u32 t = 0; t < ntriples; ++t)
-                            if (triples[3 * t] == xs[k]) seg += splits[q][2 * t + 3] - splits[q][2 * t + 1];
-                    if (seg == x.nnz) continue;
-                    if (seg >= 0xFFFFFFFFull)
-                        raise(INVALID_VALUE, "a closure union exceeds uint32 nonzeros");
-                    DevArray<u64> keys(ctl, seg), tmp(ctl, seg);
-                    std::vector<std::pair<u64, u64>> segs;  // (start, length) in keys
-                    u64 pos = 0;
-                    if (x.nnz) {
-                        k_keys_shifted<<<div_up(x.nzr, 4), 256, 0, ctl->stream>>>(u32p(x.rpt), u32p(x.rows),
-                                                                                   u32p(x.cols), x.nzr, 0, keys.ptr);
-                        CLB_LAUNCHED("keys");
-                        segs.push_back({0, x.nnz});
-                        pos = x.nnz;
-                    }
-                    for (u32 t = 0; t < ntriples; ++t) {
-                        if (triples[3 * t] != xs[k]) continue;
-                        const u64 start = pos;
-                        for (size_t q = 0; q < prods.size(); ++q) {
-                            const clb_dcsr &T = prods[q];
-                            const std::vector<u32> &hs = splits[q];
-                            const u32 r0 = hs[2 * t], r1 = hs[2 * t + 2];
-                            const u32 e0 = hs[2 * t + 1], e1 = hs[2 * t + 3];
-                            if (e1 == e0) continue;
-                            // rows t*n + i -> i
-                            k_keys_range<<<div_up(r1 - r0, 4), 256, 0, ctl->stream>>>(
-                                u32p(T.rpt), u32p(T.rows), u32p(T.cols), r0, r1, 0u - t * n,
-                                (u32)(e0 - (u32)pos), keys.ptr);
-                            CLB_LAUNCHED("keys_range");
-                            pos += e1 - e0;
-                        }
-                        if (pos > start) segs.push_back({start, pos - start});
-                    }
-                    u64 *cur = keys.ptr, *nxt = tmp.ptr;
-                    while (segs.size() > 1) {
-                        std::vector<std::pair<u64, u64>> next;
-                        for (size_t i = 0; i < segs.size(); i += 2) {
-                            const auto &sa = segs[i];
-                            if (i + 1 == segs.size()) {  // odd one out: copied to the other buffer
-                                CLB_HIP(hipMemcpyAsync(nxt + sa.first, cur + sa.first, 8 * sa.second,
-                                                       hipMemcpyDeviceToDevice, ctl->stream),
-                                        COPY_BUFFER_ERROR);
-                                next.push_back(sa);
-                                continue;
-                            }
-                            const auto &sb = segs[i + 1];  // adjacent: sb.first == sa.first + sa.second
-                            merge_keys(ctl, cur + sa.first, sa.second, cur + sb.first, sb.second, nxt + sa.first);
-                            next.push_back({sa.first, sa.second + sb.second});
-                        }
-                        segs.swap(next);
-                        std::swap(cur, nxt);
-                    }
-                    clb_dcsr nx{};
-                    nx.nrows = n;
-                    nx.ncols = n;
-                    keys_to_dcsr(ctl, cur, pos, nx);
-                    if (nx.nnz == x.nnz) {  // unions only add: equal size means unchanged
-                        clb_dcsr_release(&nx);
-                        continue;
-                    }
-                    clb_dcsr_release(&x);
-                    x = nx;
-                }
+                unite_products(ctl, mats, xs, triples, ntriples, n, prods, splits);
                 sync(ctl);
             } catch (...) {
                 release_all();

@@ -23,6 +23,13 @@ u32 unique_keys_to_pairs(clb_controls_s *ctl, const u64 *keys, u64 n, clb_buffer
 // Merge of two ascending key lists into out[0, na + nb) (merge path, kept
 // duplicates).
 void merge_keys(clb_controls_s *ctl, const u64 *a, u64 na, const u64 *b, u64 nb, u64 *out);
+// Union of two ascending key lists that hold the rows of mats.size() n x n
+// matrices, matrix x in rows [x * n, (x + 1) * n): mats[x] (what the first
+// list was made from; only its nnz is read) is replaced by a new matrix when
+// the union has more nonzeros, and left alone otherwise.  The caller releases
+// what was replaced.
+void union_keys_to_matrices(clb_controls_s *ctl, const u64 *ka, u64 na, const u64 *kb, u64 nb, u32 n,
+                            std::vector<clb_dcsr> &mats);
 // Sorted keys (row << 32 | col, duplicates allowed) -> a new canonical DCSR
 // of their distinct pairs; out.nrows/ncols are kept as given.
 void keys_to_dcsr(clb_controls_s *ctl, const u64 *keys, u64 n, clb_dcsr &out);
