@@ -255,67 +255,100 @@ __device__ __forceinline__ uint32_t emit_step(uint32_t word, uint32_t cb, uint64
     return st;
 }
 
-// Staged emission: each lane writes its words' columns into the wave's
-// staging area `sg` (STAGE_WORDS words), then the wave copies them out in
-// order, 64 consecutive columns per store instruction.  Scattered per-lane
-// stores would each touch their own cache line; the staged copy writes whole
-// lines.  When the columns average more than four per lane, lanes write
-// about 16 apart, which would put all 64 lanes on a few LDS banks, so column
-// t then sits at sg[t + t / 32] (one padding word per 32); sparser rounds
-// stage unpadded.
-constexpr uint32_t STAGE_WORDS = 2048 + 64;
-// Lane l copies columns l, l + 64, ... of n: column 64k + l sits at src[KS * k]
-// (src = the lane's first slot; KS = 66 padded, 64 unpadded) and goes to byte
-// 4 * (64k + l) of dst (a uniform pointer, so stores use a 32-bit offset).
-template <uint32_t KS>
-__device__ __forceinline__ void staged_copy_out(const uint32_t *src, char *dst, uint32_t l, uint32_t n) {
-    const uint32_t full = n / WAVE;
-    uint32_t k = 0, b = 4u * l;
-    for (; k + 4 <= full; k += 4, b += 4u * 4u * WAVE) {
-        const uint32_t v0 = src[KS * k], v1 = src[KS * (k + 1)], v2 = src[KS * (k + 2)], v3 = src[KS * (k + 3)];
-        *reinterpret_cast<uint32_t *>(dst + b) = v0;
-        *reinterpret_cast<uint32_t *>(dst + b + 4u * WAVE) = v1;
-        *reinterpret_cast<uint32_t *>(dst + b + 8u * WAVE) = v2;
-        *reinterpret_cast<uint32_t *>(dst + b + 12u * WAVE) = v3;
+// Ranked emission of bitmap words as columns: a lane per column.  Every
+// nonzero word leaves an entry (its bits, the rank of its first column and its
+// index) in a list in LDS and a mark at that rank; the wave then takes 64
+// columns at a time: the marks up to a lane's rank number its word, and the
+// column is the word's t-th set bit, t = rank - the word's first rank.  The
+// work follows the number of columns, however they are spread over the words,
+// and every store is a run of 64 columns.  (Each lane walking its own words'
+// bits, 16 per lane at the median and 128 at most in one round, took about
+// twice the instructions on skewed rows.)
+//
+// LDS of one wave: list[256] and marks[RANK_MARKS]; of the workgroup: the
+// table of select8 (rank_table).
+constexpr uint32_t RANK_MARKS = 256;  // 64-bit marks of 8192 ranks, as words
+
+struct RankLds {
+    uint2 list[256];
+    uint32_t marks[RANK_MARKS];
+};
+
+// tab[8 * byte + t] = position of the byte's t-th set bit; 256 threads.
+__device__ __forceinline__ void rank_table(uint8_t *tab) {
+    for (uint32_t b = threadIdx.x; b < 256; b += blockDim.x) {
+        uint32_t v = b, lo = 0, hi = 0;
+        for (uint32_t t = 0; t < 8; ++t) {
+            const uint32_t p = v ? (uint32_t)__builtin_ctz(v) : 0u;
+            if (t < 4) lo |= p << (8 * t);
+            else hi |= p << (8 * (t - 4));
+            v &= v - 1u;
+        }
+        reinterpret_cast<uint2 *>(tab)[b] = make_uint2(lo, hi);
     }
-    for (; k < full; ++k, b += 4u * WAVE) *reinterpret_cast<uint32_t *>(dst + b) = src[KS * k];
-    if (WAVE * k + l < n) *reinterpret_cast<uint32_t *>(dst + b) = src[KS * k];
 }
 
-// Writes the set bits of 256 bitmap words as columns at out[pos ...] (never
-// at or past lim): lane l holds four words x[0..3], bit b of x[e] being
-// column cw[e] + b; the words are in column order by (lane, e).  One wave
-// scan per round; a round whose columns fit the staging area goes through
-// it, a denser one is written two words at a time with a lane per bit (64
-// consecutive columns per ballot, stores in order).  Returns the round's set
-// bits.
-__device__ __forceinline__ uint32_t emit_round4_staged(const uint32_t (&x)[4], const uint32_t (&cw)[4], uint64_t pos,
-                                                       uint32_t *out, uint64_t lim, uint32_t *sg) {
+// Position of the t-th set bit of m (t < popcount).
+__device__ __forceinline__ uint32_t select_bit(uint32_t m, uint32_t t, const uint8_t *tab) {
+    const uint32_t c0 = (uint32_t)__popc(m << 24), c1 = (uint32_t)__popc(m << 16), c2 = (uint32_t)__popc(m << 8);
+    const uint32_t b = (t >= c0) + (t >= c1) + (t >= c2);
+    const uint32_t sh = b * 8u;
+    const uint32_t before = (uint32_t)__popc(__builtin_amdgcn_ubfe(m, 0u, sh));
+    const uint32_t byte = __builtin_amdgcn_ubfe(m, sh, 8u);
+    return sh + tab[byte * 8u + (t - before)];
+}
+
+// Writes the set bits of 256 words as columns at out[pos ...], never at or
+// past lim: lane l holds four words x[0..3], wi[e] < 2^16 being word x[e]'s
+// index and col0 + 32 * wi[e] the column of its bit 0; the words are in column
+// order by (lane, e).  A round of at least RANK_DENSE columns is written two
+// words at a time with a lane per bit instead.  Returns the round's set bits.
+// All 64 lanes must be active.
+constexpr uint32_t RANK_DENSE = 4096;
+__device__ __forceinline__ uint32_t emit_round4_ranked(const uint32_t (&x)[4], const uint32_t (&wi)[4],
+                                                       uint32_t col0, uint64_t pos, uint32_t *out, uint64_t lim,
+                                                       RankLds *sg, const uint8_t *tab) {
     const uint32_t l = (uint32_t)lane();
     const uint32_t pc = (uint32_t)(__popc(x[0]) + __popc(x[1]) + __popc(x[2]) + __popc(x[3]));
-    const uint32_t inc = wave_incl_sum_dpp(pc);
-    const uint32_t st = (uint32_t)__builtin_amdgcn_readlane((int)inc, 63);
+    const uint32_t nz = (x[0] != 0u) + (x[1] != 0u) + (x[2] != 0u) + (x[3] != 0u);
+    const uint32_t inc = wave_incl_sum_dpp((pc << 16) | nz);  // at most 8192 bits and 256 words
+    const uint32_t tot = (uint32_t)__builtin_amdgcn_readlane((int)inc, 63);
+    const uint32_t st = tot >> 16;
     if (st == 0) return 0;
     const uint64_t up = ((uint64_t)(uint32_t)__builtin_amdgcn_readfirstlane((int)(uint32_t)(pos >> 32)) << 32) |
                         (uint32_t)__builtin_amdgcn_readfirstlane((int)(uint32_t)pos);
     char *dst = reinterpret_cast<char *>(out + up);
-    const uint32_t room = (uint32_t)(lim > up ? lim - up : 0);
+    const uint32_t room = (uint32_t)(lim > up ? (lim - up < 8192u ? lim - up : 8192u) : 0u);
     const uint32_t n = st < room ? st : room;
-    if (st <= STAGE_WORDS - WAVE) {
-        const bool padded = st > 4u * WAVE;  // uniform
-        uint32_t q = inc - pc;
+    if (st < RANK_DENSE) {
+        const uint32_t nblk = (st + 63u) / 64u;
+        for (uint32_t k = l; k < 2u * nblk; k += WAVE) sg->marks[k] = 0;
+        __builtin_amdgcn_wave_barrier();
+        const uint32_t ex = inc - ((pc << 16) | nz);
+        uint32_t q = ex >> 16, k = ex & 0xFFFFu;
 #pragma unroll
-        for (uint32_t e = 0; e < 4; ++e) {
-            uint32_t w = x[e];
-            while (w) {
-                sg[padded ? q + (q >> 5) : q] = cw[e] + (uint32_t)__builtin_ctz(w);
-                ++q;
-                w &= w - 1u;
+        for (uint32_t e = 0; e < 4; ++e)
+            if (x[e]) {
+                sg->list[k] = make_uint2(x[e], (q << 16) | wi[e]);
+                atomicOr(&sg->marks[q >> 5], 1u << (q & 31u));
+                q += (uint32_t)__popc(x[e]);
+                ++k;
+            }
+        __builtin_amdgcn_wave_barrier();
+        uint32_t base = 0xFFFFFFFFu;  // words that begin before the block, minus 1
+        for (uint32_t b = 0; b < nblk; ++b) {
+            const uint32_t lo = sg->marks[2u * b], hi = sg->marks[2u * b + 1u];
+            // marks at ranks up to this lane's
+            const uint32_t slo = (lo >> 1) | (hi << 31), shi = hi >> 1;
+            const uint32_t w = __builtin_amdgcn_mbcnt_hi(shi, __builtin_amdgcn_mbcnt_lo(slo, base + (lo & 1u)));
+            base += (uint32_t)__popc(lo) + (uint32_t)__popc(hi);
+            const uint32_t o = b * 64u + l;
+            if (o < n) {
+                const uint2 v = sg->list[w];
+                const uint32_t bit = select_bit(v.x, o - (v.y >> 16), tab);
+                *reinterpret_cast<uint32_t *>(dst + 4u * o) = col0 + (v.y & 0xFFFFu) * 32u + bit;
             }
         }
-        __builtin_amdgcn_wave_barrier();
-        if (padded) staged_copy_out<66>(sg + l + (l >> 5), dst, l, n);
-        else staged_copy_out<64>(sg + l, dst, l, n);
         __builtin_amdgcn_wave_barrier();
     } else {
         // words (j, 2h) and (j, 2h + 1): lanes 0..31 take the first word's
@@ -328,13 +361,14 @@ __device__ __forceinline__ uint32_t emit_round4_staged(const uint32_t (&x)[4], c
                 const uint32_t w0 = (uint32_t)__builtin_amdgcn_readlane((int)x[2 * h], (int)j);
                 const uint32_t w1 = (uint32_t)__builtin_amdgcn_readlane((int)x[2 * h + 1], (int)j);
                 if ((w0 | w1) == 0) continue;
-                const uint32_t b0 = (uint32_t)__builtin_amdgcn_readlane((int)cw[2 * h], (int)j);
-                const uint32_t b1 = (uint32_t)__builtin_amdgcn_readlane((int)cw[2 * h + 1], (int)j);
+                const uint32_t i0 = (uint32_t)__builtin_amdgcn_readlane((int)wi[2 * h], (int)j);
+                const uint32_t i1 = (uint32_t)__builtin_amdgcn_readlane((int)wi[2 * h + 1], (int)j);
                 const uint32_t v = l < 32 ? w0 : w1;
                 const bool set = (v >> sh) & 1u;
                 const uint64_t m = __ballot(set);
                 const uint32_t at = p + lanes_below(m);
-                if (set && at < n) *reinterpret_cast<uint32_t *>(dst + 4u * at) = (l < 32 ? b0 : b1) + sh;
+                if (set && at < n)
+                    *reinterpret_cast<uint32_t *>(dst + 4u * at) = col0 + (l < 32 ? i0 : i1) * 32u + sh;
                 p += (uint32_t)__popcll(m);
             }
         }

@@ -100,7 +100,7 @@ void spgemm_esc(clb_controls_s *ctl, const clb_dcsr &a, const clb_dcsr &b, clb_d
     BinBuf bb;
     BinHost h;
     bin_rows(ctl, s, nullptr, nnz_row.ptr, perm, bb);
-    read_bins(ctl, bb, h);
+    read_bins(ctl, s, bb, h);
     u64 tot[3];
     readback(ctl, &tot[0], s.scal.ptr, 8);
     readback(ctl, &tot[1], toff.ptr + nrows, 8);

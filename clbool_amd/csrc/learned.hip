@@ -495,6 +495,7 @@ struct OnePass {
     DevArray<u64> toff, soff, offs, gpre;
     DevArray<double> err;
     DumpBufs dump;
+    StoreBufs store;  // windows too narrow for the dump
     BinHost h{};
     clb_dcsr out{};
     clb_spgemm_stats st{};
@@ -568,7 +569,7 @@ OnePassPtr one_pass_launch(clb_controls_s *ctl, const clb_dcsr &a, const clb_dcs
     bin_rows(ctl, s, cap, p.nnz_row.ptr, p.perm, bb);
     p.toff.reset(ctl, (u64)nrows + 1);
     exclusive_scan_u32_to_u64(ctl, cap, p.toff.ptr, nrows, s.scal.ptr + 4);
-    read_bins(ctl, bb, p.h);
+    read_bins(ctl, s, bb, p.h);
     u64 sc[8];
     readback(ctl, sc, s.scal.ptr, sizeof(sc));
     st.products = pr ? pr->products : sc[0];
@@ -584,7 +585,12 @@ OnePassPtr one_pass_launch(clb_controls_s *ctl, const clb_dcsr &a, const clb_dcs
     u32 *fails = reinterpret_cast<u32 *>(s.scal.ptr + 5);
     Out o{p.nnz_row.ptr, p.toff.ptr, p.temp.ptr, cap, fails, Dump{}, ONE_PASS_PROBES};
     setup_dump(ctl, s, p.h, p.dump, o, true, p.perm.ptr, cap);
+    if (s.cfg.bm_bits < 14) {
+        setup_store(ctl, s, p.h, s.cfg.bm_bits, p.store);
+        o.keep = p.store.keep;
+    }
     ensure_splits(ctl, s, p.h);
+    ensure_packed(ctl, s, p.h);
     for (hipEvent_t &e : p.bins) CLB_HIP(hipEventCreateWithFlags(&e, hipEventDisableTiming), EVENT_WAITING_ERROR);
     launch_bins(ctl, s, p.perm.ptr, p.h.off, ONE, o, &p.lt, CLB_KP_ONEPASS, p.bins);
     return P;
@@ -630,7 +636,7 @@ void one_pass_post(OnePass &p) {
         bin_rows(ctl, s, p.key2.ptr, nullptr, p.perm2, bb2);
         p.soff.reset(ctl, (u64)nrows + 1);
         exclusive_scan_u32_to_u64(ctl, p.key2.ptr, p.soff.ptr, nrows, s.scal.ptr + 6);
-        read_bins(ctl, bb2, h2);
+        read_bins(ctl, s, bb2, h2);
         u64 side_total = 0;
         readback(ctl, &side_total, s.scal.ptr + 6, 8);
         p.side.reset(ctl, side_total ? side_total : 1);
@@ -684,10 +690,13 @@ void one_pass_post(OnePass &p) {
     CLB_HIP(hipStreamWaitEvent(t1s, ctl->ev_fork, 0), EVENT_WAITING_ERROR);
     p.lt.begin(t0s);
     compact_rows(t0s, nrows, nnz, p.nnz_row.ptr, p.offs.ptr, p.temp.ptr, p.toff.ptr, p.side.ptr, p.soff.ptr,
-                 nfail ? p.key2.ptr : nullptr, p.dump.on ? p.dump.isdense.ptr : nullptr, pred, u32p(cols),
+                 nfail ? p.key2.ptr : nullptr,
+                 p.dump.on ? p.dump.isdense.ptr : p.store.keep.slot_of, pred, u32p(cols),
                  p.err.ptr, ctl->tuning.reserved[CLB_TUNE_COMPACT_TILES] != 0);
     p.lt.end((int)CLB_KF_COMPACT, t0s);
     emit_launch(t1s, ndense, p.perm.ptr, p.h, p.dump, p.gpre.ptr, p.offs.ptr, u32p(cols), &p.lt, CLB_KP_ONEPASS);
+    if (p.store.keep.slots)
+        emit_stored(t1s, p.perm.ptr + p.h.off[BIN_BITMAP0], p.store.keep.slots, p.store.keep, p.offs.ptr, u32p(cols));
     CLB_HIP(hipEventRecord(p.joined, t0s), EVENT_WAITING_ERROR);
     CLB_HIP(hipStreamWaitEvent(t1s, p.joined, 0), EVENT_WAITING_ERROR);
     CLB_HIP(hipEventRecord(p.done, t1s), EVENT_WAITING_ERROR);
@@ -703,7 +712,7 @@ OnePassPtr one_pass_start(clb_controls_s *ctl, const clb_dcsr &a, const clb_dcsr
 bool one_pass_replan(const OnePass &p) { return p.replan; }
 
 u64 one_pass_bytes(const OnePass &p) {
-    u64 b = p.temp.cap + p.dump.store.cap + p.dump.cnt.cap + p.side.cap + p.toff.cap + p.offs.cap +
+    u64 b = p.temp.cap + p.dump.store.cap + p.dump.cnt.cap + p.store.words.cap + p.store.chunks.cap + p.side.cap + p.toff.cap + p.offs.cap +
             p.soff.cap + p.nnz_row.cap + p.perm.cap + p.pos.cap;
     if (p.out.cols) b += p.out.cols->cap;
     return b;
@@ -822,9 +831,10 @@ clb_status clb_predictor_harvest(clb_controls ctl, const clb_dcsr *a, const clb_
             BinBuf bb;
             BinHost h;
             bin_rows(ctl, s, nullptr, nnz_row.ptr, perm, bb);
-            read_bins(ctl, bb, h);
+            read_bins(ctl, s, bb, h);
             Out o{nnz_row.ptr, nullptr, nullptr, nullptr, reinterpret_cast<u32 *>(s.scal.ptr + 3), Dump{}, 0};
             ensure_splits(ctl, s, h);
+            ensure_packed(ctl, s, h);
             launch_bins(ctl, s, perm.ptr, h.off, SYM, o, nullptr, -1);
             const u32 stride = nrows > max_rows ? div_up(nrows, max_rows) : 1;
             const u32 take = div_up(nrows, stride);

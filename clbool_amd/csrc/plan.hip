@@ -26,6 +26,7 @@ struct clb_spgemm_plan_s {
     clb::u64 bound = 0;
     bool empty = false;
     clb::spg::Setup s;                // over all stored rows of A
+    clb::spg::StoreBufs store;        // plain: bitmaps the symbolic pass kept
     clb::DevArray<clb::u32> size;     // exact sizes (plain) or capacities (one pass)
     clb::DevArray<float> pred;        // learned: predicted sizes
     std::vector<clb::u64> ppre, spre;  // host prefixes of products and sizes
@@ -77,7 +78,7 @@ static void plan_create(clb_controls_s *ctl, const clb_dcsr &a, const clb_dcsr &
         p.size.reset(ctl, n);
         if (mode == CLB_SPGEMM_PLAIN) {
             prepare(ctl, a, b, 0, n, p.s, true);
-            plan_sizes_plain(ctl, p.s, p.size.ptr);
+            plan_sizes_plain(ctl, p.s, p.size.ptr, p.store);
         } else {
             if (mode == CLB_SPGEMM_LEARNED) p.pred.reset(ctl, n);
             p.s.nrows = n;
@@ -99,6 +100,9 @@ static void plan_create(clb_controls_s *ctl, const clb_dcsr &a, const clb_dcsr &
         CLB_HIP(hipMemcpyAsync(p.spre.data(), sp.ptr, 8ull * (n + 1), hipMemcpyDeviceToHost, ctl->stream),
                 READ_BUFFER_ERROR);
         sync(ctl);
+        // B packed once for every block, if the whole product reads it often
+        all.products[BIN_BITMAP0] = p.ppre[n];
+        ensure_packed(ctl, p.s, all);
         cut_rows(p.spre.data(), 0, n, p.bound, p.cuts);
         p.info.products = p.ppre[n];
         p.info.planned_nnz = p.spre[n];
@@ -131,10 +135,12 @@ static void recut(clb_controls_s *ctl, clb_spgemm_plan_s &p, u32 k) {
 
 static PlanRows rows_of(clb_spgemm_plan_s &p, u32 k, bool *replan) {
     const u32 rb = p.cuts[k], re = p.cuts[k + 1];
+    Store keep = p.store.keep;
+    if (keep.words) keep.slot_of += rb;
     return PlanRows{&p.s, p.s.P + rb, p.size.ptr + rb, p.pred.ptr ? p.pred.ptr + rb : nullptr,
                     p.ppre[re] - p.ppre[rb],
                     // a single row is never cut further
-                    re - rb > 1 ? p.bound : 0xFFFFFFFFull, replan};
+                    re - rb > 1 ? p.bound : 0xFFFFFFFFull, replan, keep};
 }
 
 static void check_run(clb_controls_s *ctl, const clb_spgemm_plan_s &p, u32 k) {

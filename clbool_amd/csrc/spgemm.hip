@@ -8,6 +8,7 @@
 // (fill_nnz's prefix_sum, :218), numeric pass (:235-280), drop empty rows
 // (prepare_positions + set_positions, :282-296).  Learned mode lives in
 // learned.hip and shares the kernels.
+#include "expand.hpp"
 #include "spgemm.hpp"
 
 #include <chrono>
@@ -42,6 +43,129 @@ __global__ void k_slice_splits(const u32 *__restrict__ b_rpt, const u32 *__restr
     out[nsl] = end;
 }
 
+// Packed B (Mats::b_pairs): a pair begins at every column that starts a row or
+// a new word.  The count pass gives each tile of EX_TILE columns its pairs;
+// once these are scanned, the thread of a pair's first column ORs the columns
+// of its word (its row goes on past the tile if need be) and writes the pair.
+struct PackTile {
+    u64 e0, e1;
+    u32 r0, nr;
+    __device__ __forceinline__ PackTile(const u32 *__restrict__ first, u32 b_nzr, u32 b_nnz) {
+        e0 = (u64)blockIdx.x * EX_TILE;
+        e1 = e0 + EX_TILE < b_nnz ? e0 + EX_TILE : b_nnz;
+        r0 = first[blockIdx.x];
+        nr = (blockIdx.x + 1 < gridDim.x ? first[blockIdx.x + 1] : b_nzr - 1) - r0 + 1;
+    }
+    // the row (from r0) of position e: rows of the tile in s, or too many of them
+    __device__ __forceinline__ u32 row(const u32 *__restrict__ b_rpt, const u32 *s, u64 e) const {
+        u32 a = 0, b = nr;
+        while (b - a > 1) {
+            const u32 m = (a + b) >> 1;
+            if ((nr <= EX_TILE ? s[m] : b_rpt[r0 + m]) <= e) a = m;
+            else b = m;
+        }
+        return a;
+    }
+    __device__ __forceinline__ void stage(const u32 *__restrict__ b_rpt, u32 *s) const {
+        if (nr <= EX_TILE)
+            for (u32 j = threadIdx.x; j < nr; j += EX_WG) s[j] = b_rpt[r0 + j];
+        __syncthreads();
+    }
+};
+
+__global__ __launch_bounds__(EX_WG) void k_pack_count(const u32 *__restrict__ b_rpt, const u32 *__restrict__ b_cols,
+                                                      u32 b_nzr, u32 b_nnz, const u32 *__restrict__ first,
+                                                      u32 *__restrict__ counts) {
+    __shared__ u32 srpt[EX_TILE];
+    __shared__ u32 red[EX_WG / dev::WAVE + 1];
+    const PackTile t(first, b_nzr, b_nnz);
+    t.stage(b_rpt, srpt);
+    u32 c = 0;
+#pragma unroll
+    for (u32 q = 0; q < EX_ITEMS; ++q) {
+        const u64 e = t.e0 + q * EX_WG + threadIdx.x;
+        if (e >= t.e1) break;
+        const u32 a = t.row(b_rpt, srpt, e);
+        c += b_rpt[t.r0 + a] == e || (b_cols[e] >> 5) != (b_cols[e - 1] >> 5);
+    }
+    const u32 sum = dev::block_sum<u32, EX_WG>(c, red);
+    if (threadIdx.x == 0) counts[blockIdx.x] = sum;
+}
+
+__global__ __launch_bounds__(EX_WG) void k_pack_place(const u32 *__restrict__ b_rpt, const u32 *__restrict__ b_cols,
+                                                      u32 b_nzr, u32 b_nnz, const u32 *__restrict__ first,
+                                                      const u32 *__restrict__ offs, u32 *__restrict__ prpt,
+                                                      uint2 *__restrict__ pairs) {
+    constexpr u32 NW = EX_WG / dev::WAVE;
+    __shared__ u32 srpt[EX_TILE];
+    __shared__ u32 wcnt[NW];
+    const PackTile t(first, b_nzr, b_nnz);
+    t.stage(b_rpt, srpt);
+    u32 at = offs[blockIdx.x];
+    for (u32 q = 0; q < EX_ITEMS; ++q) {
+        const u64 e = t.e0 + q * EX_WG + threadIdx.x;
+        bool starts = false, row_start = false;
+        u32 r = 0, w = 0, mask = 0;
+        if (e < t.e1) {
+            r = t.r0 + t.row(b_rpt, srpt, e);
+            const u32 c = b_cols[e];
+            w = c >> 5;
+            row_start = b_rpt[r] == e;
+            starts = row_start || (b_cols[e - 1] >> 5) != w;
+            if (starts) {
+                mask = 1u << (c & 31u);
+                const u32 end = b_rpt[r + 1];
+                for (u64 k = e + 1; k < end; ++k) {
+                    const u32 x = b_cols[k];
+                    if ((x >> 5) != w) break;
+                    mask |= 1u << (x & 31u);
+                }
+            }
+        }
+        const unsigned long long m = __ballot(starts);
+        if (dev::lane() == 0) wcnt[dev::wave_id()] = (u32)__popcll(m);
+        __syncthreads();
+        u32 before = 0, all = 0;
+#pragma unroll
+        for (u32 v = 0; v < NW; ++v) {
+            before += v < (u32)dev::wave_id() ? wcnt[v] : 0u;
+            all += wcnt[v];
+        }
+        __syncthreads();
+        if (starts) {
+            const u32 p = at + before + dev::lanes_below(m);
+            pairs[p] = make_uint2(w, mask);
+            if (row_start) prpt[r] = p;
+        }
+        at += all;
+    }
+    if (blockIdx.x + 1 == gridDim.x && threadIdx.x == 0) prpt[b_nzr] = at;
+}
+
+// Mats::psplits: as k_slice_splits, over pairs (words, slices of span words).
+__global__ void k_pair_splits(const u32 *__restrict__ prpt, const u32 *__restrict__ b_rows,
+                              const uint2 *__restrict__ pairs, u32 b_nzr, u32 mapn, u32 nsl, u32 span,
+                              u32 *__restrict__ splits) {
+    const u32 i = blockIdx.x * blockDim.x + threadIdx.x;
+    if (i >= b_nzr) return;
+    const u32 k = b_rows[i];
+    if (k >= mapn) return;
+    const u32 beg = prpt[i], end = prpt[i + 1];
+    u32 *out = splits + (u64)k * (nsl + 1);
+    u32 lo = beg;
+    out[0] = beg;
+    for (u32 s = 1; s < nsl; ++s) {
+        u32 hi = end;
+        while (lo < hi) {
+            const u32 mid = lo + (hi - lo) / 2;
+            if (pairs[mid].x < s * span) lo = mid + 1;
+            else hi = mid;
+        }
+        out[s] = lo;
+    }
+    out[nsl] = end;
+}
+
 __global__ void k_brange_set(const u32 *__restrict__ b_rpt, const u32 *__restrict__ b_rows, u32 b_nzr, u32 mapn,
                              uint2 *__restrict__ brange, u32 *__restrict__ bpres) {
     const u32 i = blockIdx.x * blockDim.x + threadIdx.x;
@@ -54,9 +178,10 @@ __global__ void k_brange_set(const u32 *__restrict__ b_rpt, const u32 *__restric
 
 // Histogram of bins.  key == nullptr: key = min(P, ncols) (symbolic sizing).
 // Rows in BIN_EMPTY get nnz_row = 0 when zero_empty is set.
+// A row with a slot (slot_of, may be null) is a BIN_STORED row.
 __global__ __launch_bounds__(256) void k_bin_hist(Mats g, const u32 *__restrict__ P, const u32 *__restrict__ key,
                                                   u32 n, BinCfg c, u32 *__restrict__ hist, u64 *__restrict__ sums,
-                                                  u32 *__restrict__ nnz_row) {
+                                                  u32 *__restrict__ nnz_row, const u32 *__restrict__ slot_of) {
     __shared__ u32 h[NBINS];
     __shared__ unsigned long long hs[3][NBINS];  // products, A nonzeros, key (output nnz)
     if (threadIdx.x < NBINS) {
@@ -68,7 +193,7 @@ __global__ __launch_bounds__(256) void k_bin_hist(Mats g, const u32 *__restrict_
     if (i < n) {
         const u32 p = P[i];
         const u32 k = key ? key[i] : (p < c.ncols ? p : c.ncols);
-        const u32 b = classify(p, k, c);
+        const u32 b = slot_of && slot_of[i] ? BIN_STORED : classify(p, k, c);
         atomicAdd(&h[b], 1u);
         atomicAdd(&hs[0][b], (unsigned long long)p);
         atomicAdd(&hs[1][b], (unsigned long long)(g.a_rpt[g.row0 + i + 1] - g.a_rpt[g.row0 + i]));
@@ -95,7 +220,8 @@ __global__ void k_bin_offsets(const u32 *__restrict__ hist, u32 *__restrict__ cu
 // Rows grouped by bin (order inside a bin is not significant: output
 // positions come from the scan of row sizes, not from the processing order).
 __global__ __launch_bounds__(256) void k_bin_scatter(const u32 *__restrict__ P, const u32 *__restrict__ key, u32 n,
-                                                     BinCfg c, u32 *__restrict__ cursor, u32 *__restrict__ perm) {
+                                                     BinCfg c, u32 *__restrict__ cursor, u32 *__restrict__ perm,
+                                                     const u32 *__restrict__ slot_of) {
     __shared__ u32 h[NBINS];
     __shared__ u32 base[NBINS];
     if (threadIdx.x < NBINS) h[threadIdx.x] = 0;
@@ -105,7 +231,7 @@ __global__ __launch_bounds__(256) void k_bin_scatter(const u32 *__restrict__ P, 
     if (i < n) {
         const u32 p = P[i];
         const u32 k = key ? key[i] : (p < c.ncols ? p : c.ncols);
-        b = classify(p, k, c);
+        b = slot_of && slot_of[i] ? BIN_STORED : classify(p, k, c);
         if (b != BIN_EMPTY) local = atomicAdd(&h[b], 1u);
     }
     __syncthreads();
@@ -139,12 +265,10 @@ __global__ void k_set_positions(const u32 *__restrict__ nnz_row, const u64 *__re
 // words at a time (four rounds of 256, 16 bytes per lane per round),
 // double-buffered (the next 1024 words' loads are in flight while the
 // current ones are expanded); a slice dumped as (word index, word) pairs is
-// read 256 pairs per round.  Either way the words go through the wave's LDS
-// staging area (dev::emit_round4_staged: one wave scan per round), so every
-// store instruction is one contiguous run of columns.  Two-wave workgroups
-// (8.4 KB of staging per wave) let nine rows share a CU, so one row's load
-// latency overlaps another's expansion (at 256 threads, four rows: 11%
-// slower).  gpre = exclusive prefix of chunk_cnt over all slots.
+// read 256 pairs per round.  Either way the words are expanded by rank
+// (dev::emit_round4_ranked), a lane per column, so every store instruction is
+// one contiguous run.  Two-wave workgroups let more rows share a CU, so one
+// row's load latency overlaps another's expansion.  gpre = exclusive prefix of chunk_cnt over all slots.
 constexpr int EMIT_WG = 128;
 __global__ __launch_bounds__(EMIT_WG) void k_bitmap_emit(const uint4 *__restrict__ store, u32 nch,
                                                          const u64 *__restrict__ gpre, const u32 *__restrict__ list,
@@ -152,7 +276,10 @@ __global__ __launch_bounds__(EMIT_WG) void k_bitmap_emit(const uint4 *__restrict
                                                          u32 words_per_row, u32 slice_words,
                                                          const u32 *__restrict__ fmt, u32 *__restrict__ cols) {
     constexpr u32 NW = EMIT_WG / 64, ROUNDS = 4, SPAN = ROUNDS * 256;
-    __shared__ u32 stage[NW][dev::STAGE_WORDS];
+    __shared__ dev::RankLds stage[NW];
+    __shared__ __align__(8) uint8_t tab[2048];
+    dev::rank_table(tab);
+    __syncthreads();
     const u32 slot = blockIdx.x;  // slots are claimed densely from 0
     const u32 r = perm[list[slot]];
     u32 *out = cols + off[r];
@@ -180,9 +307,9 @@ __global__ __launch_bounds__(EMIT_WG) void k_bitmap_emit(const uint4 *__restrict
     auto expand = [&](const u32(&w)[ROUNDS][4], u32 s0) {
 #pragma unroll
         for (u32 k = 0; k < ROUNDS; ++k) {
-            const u32 c0 = (s0 + k * 256 + 4 * l) * 32u;
-            const u32 cw[4] = {c0, c0 + 32u, c0 + 64u, c0 + 96u};
-            p += dev::emit_round4_staged(w[k], cw, p, out, lim, stage[wv]);
+            const u32 i0 = 4 * l;
+            const u32 wi[4] = {i0, i0 + 1, i0 + 2, i0 + 3};
+            p += dev::emit_round4_ranked(w[k], wi, (s0 + k * 256) * 32u, p, out, lim, &stage[wv], tab);
         }
     };
     // the wave's words one slice at a time
@@ -206,20 +333,15 @@ __global__ __launch_bounds__(EMIT_WG) void k_bitmap_emit(const uint4 *__restrict
             const u32 pa = seg == s0w ? 0u : lower(seg - s0w);
             const u32 pb = send == s0w + slice_words ? npairs : lower(send - s0w);
             for (u32 k0 = pa; k0 < pb; k0 += 256) {
-                u32 x[4], cw[4];
+                u32 x[4], wi[4];
 #pragma unroll
                 for (u32 e = 0; e < 4; ++e) {
                     const u32 k = k0 + 4 * l + e;
-                    if (k < pb) {
-                        const uint2 pr = pairs[k];
-                        x[e] = pr.y;
-                        cw[e] = (s0w + pr.x) * 32u;
-                    } else {
-                        x[e] = 0;
-                        cw[e] = 0;
-                    }
+                    const uint2 pr = k < pb ? pairs[k] : make_uint2(0u, 0u);
+                    x[e] = pr.y;
+                    wi[e] = pr.x;  // slice-relative, below 2^15
                 }
-                p += dev::emit_round4_staged(x, cw, p, out, lim, stage[wv]);
+                p += dev::emit_round4_ranked(x, wi, s0w * 32u, p, out, lim, &stage[wv], tab);
             }
         } else {
             u32 wa[ROUNDS][4], wb[ROUNDS][4];
@@ -233,6 +355,121 @@ __global__ __launch_bounds__(EMIT_WG) void k_bitmap_emit(const uint4 *__restrict
         }
         seg = send;
     }
+}
+
+// Writes kept rows (Store) at their final positions: one wave per row and
+// chunk of words, whose place is the row's offset plus the sums of the chunks
+// before it.  What bounds it: HBM, the columns written; every store
+// instruction is one contiguous run (dev::emit_round4_ranked).
+constexpr int ES_WG = 256;
+__global__ __launch_bounds__(ES_WG) void k_emit_stored(const u32 *__restrict__ perm, u32 n, Store k,
+                                                       const u64 *__restrict__ off, u32 *__restrict__ cols) {
+    __shared__ dev::RankLds stage[ES_WG / 64];
+    __shared__ __align__(8) uint8_t tab[2048];
+    dev::rank_table(tab);
+    __syncthreads();
+    const u32 l = (u32)dev::lane(), wv = dev::wave_id();
+    const u64 item = (u64)blockIdx.x * (ES_WG / 64) + wv;
+    const u32 row = (u32)(item / k.nch), c = (u32)(item % k.nch);
+    if (row >= n) return;
+    const u32 r = perm[row];
+    const u32 slot = k.slot_of[r] - 1u;
+    const u32 cw = store_chunk(k.win_words), per_slice = k.win_words / cw;  // chunk words, chunks of a slice
+    const u32 s = c / per_slice, c0 = s * per_slice;                       // the slice and its first chunk
+    const u32 *sums = k.chunks + (u64)slot * k.nch;
+    const u32 own = sums[c];
+    if (!own) return;  // uniform
+    u64 before = 0;
+    u32 nz = 0;
+    for (u32 q = l; q < c; q += 64) {
+        const u32 v = sums[q];
+        before += v >> 12;
+        nz += q >= c0 ? v & 0xFFFu : 0u;
+    }
+    u64 p = dev::wave_sum(before);
+    u32 *out = cols + off[r];
+    const u64 lim = off[r + 1] - off[r];
+    const u32 *slice = reinterpret_cast<const u32 *>(k.words) + (u64)slot * k.row_words + (u64)s * k.win_words;
+    const u32 col0 = s * k.win_words * 32u;
+    if (k.fmt[(u64)slot * (k.row_words / k.win_words) + s]) {
+        const uint2 *pairs = reinterpret_cast<const uint2 *>(slice) + dev::wave_sum(nz);
+        const u32 np = own & 0xFFFu;
+        for (u32 k0 = 0; k0 < np; k0 += 256) {
+            u32 x[4], wi[4];
+#pragma unroll
+            for (u32 e = 0; e < 4; ++e) {
+                const u32 q = k0 + 4 * l + e;
+                const uint2 pr = q < np ? pairs[q] : make_uint2(0u, 0u);
+                x[e] = pr.y;
+                wi[e] = pr.x;
+            }
+            p += dev::emit_round4_ranked(x, wi, col0, p, out, lim, &stage[wv], tab);
+        }
+        return;
+    }
+    const u32 w0 = (c - c0) * cw;
+    uint4 v[4];
+#pragma unroll
+    for (u32 q = 0; q < 4; ++q) {
+        const u32 i = q * 256 + 4 * l;
+        v[q] = i < cw ? *reinterpret_cast<const uint4 *>(slice + w0 + i) : make_uint4(0, 0, 0, 0);
+    }
+#pragma unroll
+    for (u32 q = 0; q < 4; ++q) {
+        const u32 x[4] = {v[q].x, v[q].y, v[q].z, v[q].w};
+        const u32 i0 = w0 + q * 256 + 4 * l;
+        const u32 wi[4] = {i0, i0 + 1, i0 + 2, i0 + 3};
+        p += dev::emit_round4_ranked(x, wi, col0, p, out, lim, &stage[wv], tab);
+    }
+}
+
+void emit_stored(hipStream_t st, const u32 *perm, u32 n, const Store &keep, const u64 *off, u32 *cols) {
+    if (!n) return;
+    k_emit_stored<<<div_up((u64)n * keep.nch, ES_WG / 64), ES_WG, 0, st>>>(perm, n, keep, off, cols);
+    CLB_LAUNCHED("emit_stored");
+}
+
+void setup_store(clb_controls_s *ctl, const Setup &s, const BinHost &h, u32 bits, StoreBufs &b) {
+    b.keep = Store{};
+    // with dump_bits_per_chunk set, the numeric pass gathers its rows and dumps
+    // the dense ones, as asked
+    const u32 knob = ctl->tuning.dump_bits_per_chunk;
+    if (knob && knob < 65536u) return;
+    u64 products = 0;
+    for (u32 q = BIN_BITMAP0; q < NBINS; ++q) products += h.products[q];
+    if (products < KEEP_MIN_PRODUCTS) return;
+    const u32 win = 1u << bits;
+    const u64 nsl = ((u64)s.g.ncols + 32ull * win - 1) / (32ull * win);
+    const u64 words = nsl * win;
+    // worth it for rows with at least half as many products as words: writing
+    // and reading a word costs about what gathering a product does
+    u32 lp = 0;
+    while ((2ull << lp) < words) ++lp;
+    const u32 end = lp <= 13 ? h.off[NBINS] : (lp > 31 ? h.off[BIN_BITMAP0] : h.off[bitmap_bin_below(lp)]);
+    u64 slots = end - h.off[BIN_BITMAP0];
+    if (!slots) return;
+    if (slots * words * 4 > (1ull << 30)) {
+        // large: at most a quarter of the memory at hand
+        size_t free_b = 0, total_b = 0;
+        if (hipMemGetInfo(&free_b, &total_b) != hipSuccess) {
+            (void)hipGetLastError();
+            return;
+        }
+        const u64 most = (free_b + pool_for(ctl->device).cached_bytes()) / 4 / (words * 4);
+        if (slots > most) slots = most;
+        if (!slots) return;
+    }
+    const u64 nch = words / store_chunk(win);
+    try {
+        b.words.reset(ctl, slots * words / 4);
+        b.chunks.reset(ctl, slots * nch);
+        b.fmt.reset(ctl, slots * nsl);
+        b.slot_of.reset(ctl, s.nrows);
+    } catch (const Error &) {
+        return;  // no memory for it: the numeric pass gathers as usual
+    }
+    fill_u32(ctl, b.slot_of.ptr, s.nrows, 0u);
+    b.keep = Store{b.words.ptr, b.chunks.ptr, b.fmt.ptr, b.slot_of.ptr, (u32)slots, (u32)nch, (u32)words, win};
 }
 
 // ---------------------------------------------------------------------------
@@ -253,7 +490,7 @@ void setup_dump(clb_controls_s *ctl, const Setup &s, const BinHost &h, DumpBufs 
     // default: on in the one pass (its in-kernel emission writes a temporary
     // slot that the compaction copies again), off in the numeric pass (which
     // writes the final positions directly)
-    const u32 knob = ctl->tuning.dump_bits_per_chunk ? ctl->tuning.dump_bits_per_chunk : (one_pass ? 1024u : 65536u);
+    const u32 knob = ctl->tuning.dump_bits_per_chunk ? ctl->tuning.dump_bits_per_chunk : (one_pass ? 64u : 65536u);
     if (s.cfg.bm_bits < 14 || knob >= 65536u) return;
     const u64 nslices = ((u64)s.g.ncols + (32ull << s.cfg.bm_bits) - 1) / (32ull << s.cfg.bm_bits);
     d.nbm = h.off[NBINS] - h.off[BIN_BITMAP0];
@@ -393,6 +630,47 @@ void ensure_splits(clb_controls_s *ctl, Setup &s, const BinHost &h) {
     s.g.nsl = (u32)nsl;
 }
 
+// Packs B for the bitmap kernels when their rows will read it often enough.
+void ensure_packed(clb_controls_s *ctl, Setup &s, const BinHost &h) {
+    if (s.g.b_pairs || s.pack_tried || s.g.combine || ctl->tuning.bitmap_persistent) return;
+    u64 products = 0;
+    for (u32 b = BIN_BITMAP0; b < NBINS; ++b) products += h.products[b];
+    const clb_dcsr &b = s.b;
+    if (!b.nzr || !b.nnz || products < (u64)PACK_MIN_READS * b.nnz || products < PACK_MIN_PRODUCTS)
+        return;
+    s.pack_tried = true;
+    const u32 tiles = div_up(b.nnz, EX_TILE);
+    DevArray<u32> first(ctl, tiles), offs(ctl, (u64)tiles + 1);
+    k_tile_rows<<<div_up(b.nzr, EX_WG), EX_WG, 0, ctl->stream>>>(u32p(b.rpt), 0, b.nzr, 0, b.nnz, first.ptr);
+    CLB_LAUNCHED("tile_rows");
+    k_pack_count<<<tiles, EX_WG, 0, ctl->stream>>>(u32p(b.rpt), u32p(b.cols), b.nzr, b.nnz, first.ptr, offs.ptr);
+    CLB_LAUNCHED("pack_count");
+    exclusive_scan_u32(ctl, offs.ptr, offs.ptr, tiles, offs.ptr + tiles);
+    u32 npairs = 0;
+    readback(ctl, &npairs, offs.ptr + tiles, 4);
+    if ((u64)npairs * 100 > (u64)b.nnz * PACK_MAX_PCT) return;
+    s.pairs.reset(ctl, npairs);
+    s.prange.reset(ctl, s.mapn);
+    DevArray<u32> prpt(ctl, (u64)b.nzr + 1);
+    k_pack_place<<<tiles, EX_WG, 0, ctl->stream>>>(u32p(b.rpt), u32p(b.cols), b.nzr, b.nnz, first.ptr, offs.ptr,
+                                                   prpt.ptr, s.pairs.ptr);
+    CLB_LAUNCHED("pack_place");
+    if (!s.g.bpres) fill_u64(ctl, reinterpret_cast<u64 *>(s.prange.ptr), s.mapn, 0ull);
+    k_brange_set<<<div_up(b.nzr, 256), 256, 0, ctl->stream>>>(prpt.ptr, u32p(b.rows), b.nzr, s.mapn, s.prange.ptr,
+                                                              nullptr);
+    CLB_LAUNCHED("brange_set");
+    if (s.g.splits) {
+        s.psplits.reset(ctl, s.splits.n);
+        fill_u32(ctl, s.psplits.ptr, s.psplits.n, 0u);
+        k_pair_splits<<<div_up(b.nzr, 256), 256, 0, ctl->stream>>>(prpt.ptr, u32p(b.rows), s.pairs.ptr, b.nzr, s.mapn,
+                                                                    s.g.nsl, 1u << s.g.split_bits, s.psplits.ptr);
+        CLB_LAUNCHED("pair_splits");
+    }
+    s.g.b_pairs = s.pairs.ptr;
+    s.g.prange = s.prange.ptr;
+    s.g.psplits = s.g.splits ? s.psplits.ptr : nullptr;
+}
+
 void prepare(clb_controls_s *ctl, const clb_dcsr &a, const clb_dcsr &b, u32 row_begin, u32 nrows, Setup &s,
              bool count, const Setup *shared) {
     s.nrows = nrows;
@@ -400,6 +678,7 @@ void prepare(clb_controls_s *ctl, const clb_dcsr &a, const clb_dcsr &b, u32 row_
     if (shared) {
         // a plan's block: B's row map and split table were built once
         s.mapn = shared->mapn;
+        s.pack_tried = shared->pack_tried;
         s.g = shared->g;
         s.cfg = shared->cfg;
         s.b = shared->b;
@@ -435,6 +714,10 @@ void prepare(clb_controls_s *ctl, const clb_dcsr &a, const clb_dcsr &b, u32 row_
         s.g.combine = ctl->tuning.reserved[CLB_TUNE_GATHER_COMBINE];
         s.cfg = make_bincfg(ctl, b.ncols);
         s.g.splits = nullptr;
+        s.g.b_pairs = nullptr;
+        s.g.prange = nullptr;
+        s.g.psplits = nullptr;
+        s.pack_tried = false;
         s.g.nsl = 0;
         s.g.split_bits = s.cfg.bm_bits;
         s.b = b;  // the split table is built by ensure_splits, once bitmap rows exist
@@ -455,21 +738,22 @@ void prepare(clb_controls_s *ctl, const clb_dcsr &a, const clb_dcsr &b, u32 row_
 }
 
 void bin_rows(clb_controls_s *ctl, const Setup &s, const u32 *key, u32 *nnz_row_zero, DevArray<u32> &perm,
-              BinBuf &bb) {
+              BinBuf &bb, const u32 *slot_of) {
     bb.buf.reset(ctl, 2 * NBINS + 2 + 2 * 3 * NBINS);
     fill_u32(ctl, bb.buf.ptr, bb.buf.n, 0u);
     perm.reset(ctl, s.nrows ? s.nrows : 1);
     const u32 grid = div_up(s.nrows, 256);
     k_bin_hist<<<grid, 256, 0, ctl->stream>>>(s.g, s.P, key, s.nrows, s.cfg, bb.hist(), bb.sums(),
-                                              nnz_row_zero);
+                                              nnz_row_zero, slot_of);
     CLB_LAUNCHED("bin_hist");
     k_bin_offsets<<<1, 64, 0, ctl->stream>>>(bb.hist(), bb.cursor());
     CLB_LAUNCHED("bin_offsets");
-    k_bin_scatter<<<grid, 256, 0, ctl->stream>>>(s.P, key, s.nrows, s.cfg, bb.cursor(), perm.ptr);
+    k_bin_scatter<<<grid, 256, 0, ctl->stream>>>(s.P, key, s.nrows, s.cfg, bb.cursor(), perm.ptr,
+                                                 slot_of);
     CLB_LAUNCHED("bin_scatter");
 }
 
-void read_bins(clb_controls_s *ctl, const BinBuf &bb, BinHost &h) {
+void read_bins(clb_controls_s *ctl, Setup &s, const BinBuf &bb, BinHost &h) {
     u32 hist[NBINS];
     readback(ctl, hist, bb.hist(), sizeof(hist));
     h.off[0] = 0;
@@ -480,6 +764,7 @@ void read_bins(clb_controls_s *ctl, const BinBuf &bb, BinHost &h) {
         h.products[b] = sums[b];
         h.a_nnz[b] = sums[NBINS + b];
         h.out_nnz[b] = sums[2 * NBINS + b];
+        s.bin_products[b] = sums[b];
     }
 }
 
@@ -555,35 +840,6 @@ LaunchTimer::~LaunchTimer() {
 
 // Launch the per-bin kernels of one pass.  off[b]..off[b+1] is bin b's range
 // of perm.  numeric == false: write nnz_row; true: write columns.
-// One workgroup per row, or (tuning.bitmap_persistent) a persistent grid
-// that takes rows from a counter.
-template <int WBITS, int WG, int MODE, bool COMB>
-static void launch_bitmap_c(clb_controls_s *ctl, hipStream_t st, const Setup &s, const u32 *perm, u32 n,
-                            const Out &o) {
-    if (!ctl->tuning.bitmap_persistent) {
-        k_bitmap<WBITS, WG, MODE, COMB><<<n, WG, 0, st>>>(s.g, perm, o);
-        return;
-    }
-    int per_cu = 0;
-    if (hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, k_bitmap_persist<WBITS, WG, MODE, COMB>, WG, 0) !=
-            hipSuccess ||
-        per_cu < 1) {
-        (void)hipGetLastError();
-        per_cu = 1;
-    }
-    const u64 fit = (u64)ctl->cu_count * (u64)per_cu;
-    u32 *ctr = s.ctr.ptr + MODE;  // one counter per pass of the SpGEMM
-    fill_u32_on(st, ctr, 1, 0u);
-    k_bitmap_persist<WBITS, WG, MODE, COMB><<<(u32)(n < fit ? n : fit), WG, 0, st>>>(s.g, perm, n, ctr, o);
-}
-
-template <int WBITS, int WG, int MODE>
-static void launch_bitmap(clb_controls_s *ctl, hipStream_t st, const Setup &s, const u32 *perm, u32 n,
-                          const Out &o) {
-    if (s.g.combine) launch_bitmap_c<WBITS, WG, MODE, true>(ctl, st, s, perm, n, o);
-    else launch_bitmap_c<WBITS, WG, MODE, false>(ctl, st, s, perm, n, o);
-}
-
 void join_deferred(clb_controls_s *ctl, const hipEvent_t *defer) {
     for (int k = 0; k < clb_controls_s::NSIDE; ++k)
         CLB_HIP(hipStreamWaitEvent(ctl->stream, defer[k], 0), EVENT_WAITING_ERROR);
@@ -592,13 +848,14 @@ void join_deferred(clb_controls_s *ctl, const hipEvent_t *defer) {
 void launch_bins(clb_controls_s *ctl, const Setup &s, const u32 *perm, const u32 off[NBINS + 1], int mode,
                  const Out &o, LaunchTimer *lt, int family, hipEvent_t *defer, bool one_stream) {
     if (!one_stream) fork_side(ctl);
-    // table kernels alternate over side streams 1.. (the first one takes
-    // stream 0 when no bitmap kernel was launched there)
-    int k = 0;
+    // the bitmap kernels take side streams 0.. (one each), the table kernels
+    // alternate over the others
+    int used = 0, k = 0;
     auto next = [&]() {
         constexpr int NS = clb_controls_s::NSIDE;
         if (one_stream) return ctl->stream;
-        return k == 0 ? side_stream(ctl, k++) : side_stream(ctl, 1 + (k++ - 1) % (NS - 1));
+        const int rest = NS - used > 0 ? NS - used : 1;
+        return side_stream(ctl, (used < NS ? used : NS - 1) + k++ % rest);
     };
     LaunchTimer dummy;
     LaunchTimer &t = lt ? *lt : dummy;
@@ -616,33 +873,42 @@ void launch_bins(clb_controls_s *ctl, const Setup &s, const u32 *perm, const u32
     // pass goes first and on a side stream of its own, so that it never
     // queues behind a table kernel; the table kernels fill the CUs around it.
     if (!s.cfg.esc_only) {
+        const u32 ns = off[BIN_STORED + 1] - off[BIN_STORED];
+        if (ns && mode == NUM && o.keep.words) {
+            hipStream_t st = one_stream ? ctl->stream : side_stream(ctl, used++);
+            t.begin(st);
+            emit_stored(st, perm + off[BIN_STORED], ns, o.keep, o.off, o.cols);
+            t.end(fam(CLB_KK_BITMAP), st);
+        }
         const u32 n = off[NBINS] - off[BIN_BITMAP0];
         if (n) {
             const u32 *pp = perm + off[BIN_BITMAP0];
-            hipStream_t st = one_stream ? ctl->stream : side_stream(ctl, 0);
-            k = 1;
-            t.begin(st);
-#define BITMAP3(WB, WGS)                                                   \
-    do {                                                                   \
-        if (mode == SYM) launch_bitmap<WB, WGS, SYM>(ctl, st, s, pp, n, o); \
-        else if (mode == NUM) launch_bitmap<WB, WGS, NUM>(ctl, st, s, pp, n, o); \
-        else launch_bitmap<WB, WGS, ONE>(ctl, st, s, pp, n, o);          \
-    } while (0)
-            switch (mode == SYM ? s.cfg.sym_bits : s.cfg.bm_bits) {
-                case 6: BITMAP3(6, 64); break;
-                case 7: BITMAP3(7, 64); break;
-                case 8: BITMAP3(8, 64); break;
-                case 9: BITMAP3(9, 256); break;
-                case 10: BITMAP3(10, 256); break;
-                case 11: BITMAP3(11, 256); break;
-                case 12: BITMAP3(12, 512); break;
-                case 13: BITMAP3(13, 512); break;
-                case 14: BITMAP3(14, 512); break;
-                case 15: BITMAP3(15, 1024); break;
+            const u32 bits = mode == SYM ? s.cfg.sym_bits : s.cfg.bm_bits;
+            // rows that a workgroup of the usual size would work on for longer
+            // than half of what an even share of the pass takes run with the
+            // widest workgroup, beside the others (R-MAT 2^16, symbolic: its
+            // CUs were busy for 228 of 583 us, waiting for rows of up to 645
+            // thousand products on 256 threads; 421 us with the 493 largest
+            // rows on 1024)
+            const u32 slots = ctl->cu_count * bitmap_resident(bits);
+            u64 products = 0;
+            for (u32 b = BIN_BITMAP0; b < NBINS; ++b) products += s.bin_products[b];
+            u32 lp = 14;
+            while (lp < 32 && (1ull << lp) * 2 * slots < products) ++lp;
+            u32 heavy = 0;
+            if (bitmap_wide(bits) > bitmap_wg(bits) && !ctl->tuning.bitmap_persistent && lp < 32)
+                heavy = off[bitmap_bin_below(lp)] - off[BIN_BITMAP0];
+            for (int wide = 1; wide >= 0; --wide) {
+                const u32 r0 = wide ? 0 : heavy, nr = wide ? heavy : n - heavy;
+                if (!nr) continue;
+                hipStream_t st = one_stream ? ctl->stream : side_stream(ctl, used < 2 ? used++ : 2);
+                t.begin(st);
+                if (mode == SYM) launch_bitmap_sym(ctl, st, s, pp, r0, nr, bits, wide != 0, o);
+                else if (mode == NUM) launch_bitmap_num(ctl, st, s, pp, r0, nr, bits, wide != 0, o);
+                else launch_bitmap_one(ctl, st, s, pp, r0, nr, bits, wide != 0, o);
+                CLB_LAUNCHED("bitmap");
+                t.end(fam(2), st);
             }
-#undef BITMAP3
-            CLB_LAUNCHED("bitmap");
-            t.end(fam(2), st);
         }
     }
     // TINY
@@ -779,7 +1045,10 @@ void spgemm_plain(clb_controls_s *ctl, const clb_dcsr &a, const clb_dcsr &b, u32
     st.n_bins = NBINS;
     DevArray<u32> nnz_row_own;
     u32 *nnz_row = nullptr;
+    StoreBufs store;
+    Store keep{};  // bitmaps the symbolic pass kept
     if (pr) {
+        keep = pr->keep;
         // planned block: products and exact row sizes come from the plan
         s.P = pr->prod;
         nnz_row = pr->size;
@@ -793,7 +1062,7 @@ void spgemm_plain(clb_controls_s *ctl, const clb_dcsr &a, const clb_dcsr &b, u32
         nnz_row_own.reset(ctl, nrows);
         nnz_row = nnz_row_own.ptr;
         bin_rows(ctl, s, nullptr, nnz_row, perm, bb);
-        read_bins(ctl, bb, h1);
+        read_bins(ctl, s, bb, h1);
         u64 total_products = 0;
         readback(ctl, &total_products, s.scal.ptr, 8);
         st.products = total_products;
@@ -803,8 +1072,11 @@ void spgemm_plain(clb_controls_s *ctl, const clb_dcsr &a, const clb_dcsr &b, u32
             out.ncols = b.ncols;
             return;
         }
-        Out o1{nnz_row, nullptr, nullptr, nullptr, reinterpret_cast<u32 *>(s.scal.ptr + 3), Dump{}, 0};
+        setup_store(ctl, s, h1, s.cfg.sym_bits, store);
+        keep = store.keep;
+        Out o1{nnz_row, nullptr, nullptr, nullptr, reinterpret_cast<u32 *>(s.scal.ptr + 3), Dump{}, 0, keep};
         ensure_splits(ctl, s, h1);
+        ensure_packed(ctl, s, h1);
         launch_bins(ctl, s, perm.ptr, h1.off, SYM, o1, &lt, -1);
         tm.mark();  // 2
     }
@@ -819,8 +1091,8 @@ void spgemm_plain(clb_controls_s *ctl, const clb_dcsr &a, const clb_dcsr &b, u32
     DevArray<u32> perm2;
     BinBuf bb2;
     BinHost h2;
-    bin_rows(ctl, s, nnz_row, nullptr, perm2, bb2);
-    read_bins(ctl, bb2, h2);
+    bin_rows(ctl, s, nnz_row, nullptr, perm2, bb2, keep.words ? keep.slot_of : nullptr);
+    read_bins(ctl, s, bb2, h2);
     for (u32 k = 0; k < NBINS; ++k) {
         st.bin_rows[k] = h2.off[k + 1] - h2.off[k];
         st.bin_products[k] = h2.products[k];
@@ -843,10 +1115,11 @@ void spgemm_plain(clb_controls_s *ctl, const clb_dcsr &a, const clb_dcsr &b, u32
     if (nnz == 0) return;
     clb_buffer_s *cols = buffer_new(ctl, 4ull * nnz);
     try {
-        Out o2{nnz_row, offs.ptr, u32p(cols), nullptr, reinterpret_cast<u32 *>(s.scal.ptr + 3), Dump{}, 0};
+        Out o2{nnz_row, offs.ptr, u32p(cols), nullptr, reinterpret_cast<u32 *>(s.scal.ptr + 3), Dump{}, 0, keep};
         DumpBufs dump;
         setup_dump(ctl, s, h2, dump, o2, false, perm2.ptr, nnz_row);
         ensure_splits(ctl, s, h2);
+        ensure_packed(ctl, s, h2);
         launch_bins(ctl, s, perm2.ptr, h2.off, NUM, o2, &lt, -1);
         emit_dense(ctl, perm2.ptr, h2, dump, offs.ptr, u32p(cols), &lt, CLB_KP_NUMERIC, timing ? &st : nullptr);
         tm.mark();  // 4
@@ -873,15 +1146,17 @@ void spgemm_plain(clb_controls_s *ctl, const clb_dcsr &a, const clb_dcsr &b, u32
     }
 }
 
-void plan_sizes_plain(clb_controls_s *ctl, Setup &s, u32 *size) {
+void plan_sizes_plain(clb_controls_s *ctl, Setup &s, u32 *size, StoreBufs &store) {
     // the symbolic pass of spgemm_plain over every stored row of A
     DevArray<u32> perm;
     BinBuf bb;
     BinHost h;
     bin_rows(ctl, s, nullptr, size, perm, bb);
-    read_bins(ctl, bb, h);
-    Out o{size, nullptr, nullptr, nullptr, reinterpret_cast<u32 *>(s.scal.ptr + 3), Dump{}, 0};
+    read_bins(ctl, s, bb, h);
+    setup_store(ctl, s, h, s.cfg.sym_bits, store);
+    Out o{size, nullptr, nullptr, nullptr, reinterpret_cast<u32 *>(s.scal.ptr + 3), Dump{}, 0, store.keep};
     ensure_splits(ctl, s, h);
+    ensure_packed(ctl, s, h);
     launch_bins(ctl, s, perm.ptr, h.off, SYM, o, nullptr, -1);
     u64 flag = 0;
     readback(ctl, &flag, s.scal.ptr + 3, 8);

@@ -17,9 +17,13 @@ struct Setup {
     DevArray<u64> scal;
     DevArray<u32> ctr;  // row counters of persistent launches (zeroed per launch)
     DevArray<u32> splits;  // per-slice B row ranges (Mats::splits) when ncols spans several windows
+    DevArray<uint2> pairs, prange;  // packed B (Mats::b_pairs)
+    DevArray<u32> psplits;
+    bool pack_tried = false;
     Mats g{};
     BinCfg cfg{};
     clb_dcsr b{};  // the B operand (its buffers stay owned by the caller)
+    u64 bin_products[NBINS] = {};  // of the last binning read back (read_bins)
     u32 *P = nullptr;  // products per row of the block: prod.ptr, or a plan's array
 };
 
@@ -36,6 +40,7 @@ struct PlanRows {
                           // assembled; the exact row sizes are written to
                           // `size` and *replan is set instead
     bool *replan;
+    Store keep;           // plain: bitmaps kept by the plan's symbolic pass, slot_of from the block's first row
 };
 
 // HIP-event timing of individual kernel launches, grouped by family
@@ -72,6 +77,21 @@ struct DumpBufs {
     DevArray<uint4> store;
     DevArray<u32> cnt, list, count, isdense, fmt;
 };
+// Buffers of the bitmaps a symbolic pass keeps (see Store).
+struct StoreBufs {
+    DevArray<uint4> words;
+    DevArray<u32> chunks, fmt, slot_of;
+    Store keep{};
+};
+// Below this many products in the bitmap rows their bitmaps are not kept: the
+// buffers cost more than the second gather (98 thousand products: 343 us
+// kept, 315 not; R-MAT 2^16, 400 million: 1.09 ms kept, 1.60 not).
+constexpr u64 KEEP_MIN_PRODUCTS = 1ull << 20;
+// Room for the bitmaps (windows of 2^bits words) of the bitmap rows of `h`
+// that are worth keeping and fit (keep.words == nullptr: none).
+void setup_store(clb_controls_s *ctl, const Setup &s, const BinHost &h, u32 bits, StoreBufs &b);
+// Expands rows perm[0 .. n) of a store at their offsets.
+void emit_stored(hipStream_t st, const u32 *perm, u32 n, const Store &keep, const u64 *off, u32 *cols);
 // Allocates the dense-bitmap scratch for the bitmap bin of `h` (nothing when
 // the window is below 2^14 words, the knob disables it or it would not fit)
 // and fills o.dump.  With perm and key (the rows' capacities or exact
@@ -90,6 +110,18 @@ void emit_launch(hipStream_t es, u32 count, const u32 *perm, const BinHost &h, c
 
 BinCfg make_bincfg(const clb_controls_s *ctl, u32 ncols);
 void ensure_splits(clb_controls_s *ctl, Setup &s, const BinHost &h);
+// B packed by words (Mats::b_pairs) for the bitmap rows of `h`, after
+// ensure_splits.  Packing costs two passes over B, so it needs rows that read
+// B often; and a pair takes twice a column's bytes, so it needs columns that
+// share words.  Measured packed against not (ms): R-MAT 2^16 x 16, plain 1.10
+// / 1.20; 2^18, plain blocks 6.77 / 7.76; 2^20, one pass 42.9 / 47.7; uniform
+// 100 per row of 10^5 columns (98 pairs per 100) 4.83 / 4.92, 600 per row of
+// 10^6 (99) 3.51 / 3.14; R-MAT 20000 vertices, 160000 edges 0.400 / 0.423;
+// uniform 1024 x 1024 with 98 thousand products 0.37 / 0.32.
+constexpr u64 PACK_MIN_PRODUCTS = 1ull << 22;  // launches and one read-back below it
+constexpr u32 PACK_MIN_READS = 8;  // products of the bitmap rows per nonzero of B
+constexpr u32 PACK_MAX_PCT = 95;   // pairs per 100 nonzeros of B
+void ensure_packed(clb_controls_s *ctl, Setup &s, const BinHost &h);
 // B row map, kernel arguments and (count == true) per-row product counts.
 // With `shared`, the B row map, split table and bin config are taken from
 // it (a plan's Setup) instead of being built.
@@ -97,9 +129,9 @@ void prepare(clb_controls_s *ctl, const clb_dcsr &a, const clb_dcsr &b, u32 row_
              bool count = true, const Setup *shared = nullptr);
 // Bins the rows of the block by (P, key) into perm (device only, no sync).
 void bin_rows(clb_controls_s *ctl, const Setup &s, const u32 *key, u32 *nnz_row_zero, DevArray<u32> &perm,
-              BinBuf &bb);
+              BinBuf &bb, const u32 *slot_of = nullptr);
 // Reads the binning back (synchronises the stream).
-void read_bins(clb_controls_s *ctl, const BinBuf &bb, BinHost &h);
+void read_bins(clb_controls_s *ctl, Setup &s, const BinBuf &bb, BinHost &h);
 // Per-bin sums of nnz_row over the rows of each nonempty bin's range of perm
 // (rows marked FAILED count 0); the result is read back into out[NBINS].
 void sum_by_bin(clb_controls_s *ctl, const u32 *perm, const BinHost &h, u32 nrows, const u32 *nnz_row,
@@ -112,6 +144,22 @@ void sum_by_bin(clb_controls_s *ctl, const u32 *perm, const BinHost &h, u32 nrow
 // on the controls' stream instead (no side streams).
 void launch_bins(clb_controls_s *ctl, const Setup &s, const u32 *perm, const u32 off[NBINS + 1], int mode,
                  const Out &o, LaunchTimer *lt, int family, hipEvent_t *defer = nullptr, bool one_stream = false);
+// Bitmap rows perm[r0 .. r0 + n) with windows of 2^bits words, by the usual or
+// the widest workgroup (bitmap_sym.hip, bitmap_num.hip, bitmap_one.hip).
+void launch_bitmap_sym(clb_controls_s *ctl, hipStream_t st, const Setup &s, const u32 *perm, u32 r0, u32 n, u32 bits,
+                       bool wide, const Out &o);
+void launch_bitmap_num(clb_controls_s *ctl, hipStream_t st, const Setup &s, const u32 *perm, u32 r0, u32 n, u32 bits,
+                       bool wide, const Out &o);
+void launch_bitmap_one(clb_controls_s *ctl, hipStream_t st, const Setup &s, const u32 *perm, u32 r0, u32 n, u32 bits,
+                       bool wide, const Out &o);
+// Threads of the bitmap kernels' workgroups and how many of the usual ones a
+// CU holds (waves and LDS).
+constexpr u32 bitmap_wg(u32 bits) { return bits <= 8 ? 64 : (bits <= 11 ? 256 : (bits <= 14 ? 512 : 1024)); }
+constexpr u32 bitmap_wide(u32 bits) { return bits >= 10 ? 1024 : (64u << (bits - 6)); }
+constexpr u32 bitmap_resident(u32 bits) {
+    const u32 waves = 2048 / bitmap_wg(bits), lds = (160u << 10) / ((4u << bits) + 16 * bitmap_wg(bits));
+    return waves < lds ? waves : lds;
+}
 // The controls' stream waits for the work recorded by a deferred launch_bins.
 void join_deferred(clb_controls_s *ctl, const hipEvent_t *defer);
 void scan_sizes(clb_controls_s *ctl, Setup &s, const u32 *nnz_row, DevArray<u64> &off, DevArray<u32> &pos);
@@ -125,7 +173,7 @@ void spgemm_plain(clb_controls_s *ctl, const clb_dcsr &a, const clb_dcsr &b, u32
                   bool timing, clb_dcsr &out, clb_spgemm_stats &st, const PlanRows *pr = nullptr);
 // Planning passes over all stored rows of A (s from prepare over all rows):
 // exact row sizes by the symbolic pass (plain) into size.
-void plan_sizes_plain(clb_controls_s *ctl, Setup &s, u32 *size);
+void plan_sizes_plain(clb_controls_s *ctl, Setup &s, u32 *size, StoreBufs &store);
 // learned.hip.  bound_only: capacities min(P, ncols) for every row, no
 // predictor (CLB_SPGEMM_BOUND).
 void spgemm_learned(clb_controls_s *ctl, const clb_dcsr &a, const clb_dcsr &b, u32 row_begin, u32 row_end,

@@ -35,7 +35,10 @@ constexpr u32 HASH_MAX_BITS = 14;
 constexpr u32 BIN_ESC0 = 10;     // 10 + (ceil(log2 P) - ESC_MIN_BITS): LDS expand-sort-compress rows
 constexpr u32 ESC_MIN_BITS = 11;
 constexpr u32 ESC_MAX_BITS = 13;
-constexpr u32 BIN_BITMAP0 = 13;  // 13 + (31 - floor(log2 P)), clamped to 31
+// rows whose bitmap the symbolic pass kept (Store): the numeric pass only
+// expands them
+constexpr u32 BIN_STORED = 13;
+constexpr u32 BIN_BITMAP0 = 14;  // 14 + (30 - floor(log2 P)), clamped to 14..31
 constexpr u32 BIG_ROW = 256;     // B rows at least this long are shared by the workgroup
 constexpr u32 LONG_ROW = 64;     // B rows at least this long are shared by a wave
 
@@ -65,13 +68,20 @@ struct Mats {
     // and reads brange only for stored rows; brange is written only there.
     // nullptr: brange is complete.
     const u32 *bpres;
+    // Packed B (bitmap kernels only; nullptr: not built): each stored row as
+    // (word, mask) pairs, word = column / 32 ascending and mask = the row's
+    // columns in that word; prange and psplits are brange and splits in pairs.
+    const uint2 *b_pairs;
+    const uint2 *prange;
+    const u32 *psplits;
 };
 
-// [begin, end) of B row k in b_cols ({0, 0} for absent rows).
+// [begin, end) of B row k in b_cols (PACK: in b_pairs), {0, 0} for absent rows.
+template <bool PACK = false>
 __device__ __forceinline__ uint2 b_range(const Mats &g, u32 k) {
     if (k >= g.mapn) return make_uint2(0, 0);
     if (g.bpres && !((g.bpres[k >> 5] >> (k & 31)) & 1u)) return make_uint2(0, 0);
-    return g.brange[k];
+    return PACK ? g.prange[k] : g.brange[k];
 }
 constexpr u32 NOSLICE = 0xFFFFFFFFu;
 
@@ -80,13 +90,14 @@ constexpr u32 NOSLICE = 0xFFFFFFFFu;
 // [slice * sstep, (slice + 1) * sstep) through the split table, which is
 // zero for rows B does not store, so that path needs no brange lookup.
 // k == EMPTY gives {0, 0}.
+template <bool PACK = false>
 __device__ __forceinline__ uint2 b_part(const Mats &g, u32 k, u32 slice, u32 sstep) {
     if (slice == NOSLICE) {
-        const uint2 rr = b_range(g, k);
+        const uint2 rr = b_range<PACK>(g, k);
         return make_uint2(rr.x, rr.y - rr.x);
     }
     if (k >= g.mapn) return make_uint2(0, 0);
-    const u32 *sp = g.splits + (u64)k * (g.nsl + 1);
+    const u32 *sp = (PACK ? g.psplits : g.splits) + (u64)k * (g.nsl + 1);
     const u32 f0 = slice * sstep, f1 = f0 + sstep < g.nsl ? f0 + sstep : g.nsl;
     const u32 b0 = sp[f0];
     return make_uint2(b0, sp[f1] - b0);
@@ -149,9 +160,12 @@ __device__ __forceinline__ u32 classify(u32 P, u32 key, const BinCfg &c) {
     if (!bitmap) return BIN_HASH0 + (bits - HASH_MIN_BITS);
     if (c.multi_slice && P <= c.esc_max) return esc_bin(P);
     const u32 lp = 31 - __clz(P);
-    const u32 b = BIN_BITMAP0 + (31 - lp);
+    const u32 b = BIN_BITMAP0 + (lp < 30 ? 30 - lp : 0u);
     return b < NBINS ? b : NBINS - 1;
 }
+// First bitmap bin of rows with fewer than 2^lp products (rows of the bins
+// before it have at least 2^lp); lp in [14, 31].
+constexpr u32 bitmap_bin_below(u32 lp) { return BIN_BITMAP0 + (31 - lp); }
 
 // ---------------------------------------------------------------------------
 // Product enumeration of one A row [js, je) by a workgroup of WG threads.
@@ -179,10 +193,29 @@ __device__ __forceinline__ u32 classify(u32 P, u32 key, const BinCfg &c) {
 constexpr int UNROLL = 4;
 __host__ __device__ constexpr int BIG_WORDS(int WG) { return 3 * WG + 2 * (WG / 64 + 2); }
 
-template <int WG, int UB, u32 BIGMIN, bool AHEAD = false, typename F, typename FF>
+// PACK: over the packed B rows instead; f and ff take a (word, mask) pair.
+template <bool PACK>
+struct BElem {
+    using T = u32;
+    static __device__ __forceinline__ const T *base(const Mats &g) { return g.b_cols; }
+    static __device__ __forceinline__ T none() { return EMPTY; }
+    static __device__ __forceinline__ bool some(T v) { return v != EMPTY; }
+};
+template <>
+struct BElem<true> {
+    using T = uint2;
+    static __device__ __forceinline__ const T *base(const Mats &g) { return g.b_pairs; }
+    static __device__ __forceinline__ T none() { return make_uint2(0u, 0u); }
+    static __device__ __forceinline__ bool some(T v) { return v.y != 0u; }  // a pair's mask is not empty
+};
+
+template <int WG, int UB, u32 BIGMIN, bool AHEAD = false, bool PACK = false, typename F, typename FF>
 __device__ __forceinline__ void for_each_product(const Mats &g, u32 js, u32 je, u32 *big, F &&f, FF &&ff,
                                                  u32 slice = NOSLICE, u32 sstep = 1, RowAhead *ah = nullptr,
                                                  u32 next_slice = NOSLICE) {
+    using B = BElem<PACK>;
+    using T = typename B::T;
+    const T *const bsrc = B::base(g);
     const int l = dev::lane();
     constexpr int NW = WG / dev::WAVE;
     constexpr u32 WIN = UB * 64;
@@ -197,7 +230,7 @@ __device__ __forceinline__ void for_each_product(const Mats &g, u32 js, u32 je, 
     uint2 part = make_uint2(0u, 0u);
     u32 knext = EMPTY;
     if constexpr (AHEAD) {
-        part = ah ? ah->part : b_part(g, col_at((u64)js + threadIdx.x), slice, sstep);
+        part = ah ? ah->part : b_part<PACK>(g, col_at((u64)js + threadIdx.x), slice, sstep);
         knext = col_at((u64)js + WG + threadIdx.x);
     }
     for (u32 base = js; base < je; base += WG) {
@@ -205,13 +238,13 @@ __device__ __forceinline__ void for_each_product(const Mats &g, u32 js, u32 je, 
         if constexpr (AHEAD) {
             bx = part.x;
             len = part.y;
-            if (ah && base == js && next_slice != NOSLICE) ah->part = b_part(g, ah->k0, next_slice, sstep);
+            if (ah && base == js && next_slice != NOSLICE) ah->part = b_part<PACK>(g, ah->k0, next_slice, sstep);
             if ((u64)base + WG < je) {
-                part = b_part(g, knext, slice, sstep);
+                part = b_part<PACK>(g, knext, slice, sstep);
                 knext = col_at((u64)base + 2 * WG + threadIdx.x);
             }
         } else {
-            const uint2 p = b_part(g, col_at((u64)base + threadIdx.x), slice, sstep);
+            const uint2 p = b_part<PACK>(g, col_at((u64)base + threadIdx.x), slice, sstep);
             bx = p.x;
             len = p.y;
         }
@@ -244,15 +277,15 @@ __device__ __forceinline__ void for_each_product(const Mats &g, u32 js, u32 je, 
             const u32 sb = __shfl(bx, s, dev::WAVE);
             const u32 sl = __shfl(len, s, dev::WAVE);
             for (u32 q = l; q < sl; q += UNROLL * dev::WAVE) {
-                u32 c[UNROLL];
+                T c[UNROLL];
 #pragma unroll
                 for (int u = 0; u < UNROLL; ++u) {
                     const u32 qq = q + u * dev::WAVE;
-                    c[u] = qq < sl ? g.b_cols[sb + qq] : EMPTY;
+                    c[u] = qq < sl ? bsrc[sb + qq] : B::none();
                 }
 #pragma unroll
                 for (int u = 0; u < UNROLL; ++u)
-                    if (c[u] != EMPTY) f(c[u]);
+                    if (B::some(c[u])) f(c[u]);
             }
         }
         // lane expansion of short rows
@@ -261,7 +294,7 @@ __device__ __forceinline__ void for_each_product(const Mats &g, u32 js, u32 je, 
         const u32 wtot = __shfl(inc, dev::WAVE - 1, dev::WAVE);
         const u32 exc = inc - sl;
         for (u32 p0 = 0; p0 < wtot; p0 += UNROLL * dev::WAVE) {
-            u32 c[UNROLL];
+            T c[UNROLL];
 #pragma unroll
             for (int u = 0; u < UNROLL; ++u) {
                 const u32 p = p0 + u * dev::WAVE + l;
@@ -276,11 +309,11 @@ __device__ __forceinline__ void for_each_product(const Mats &g, u32 js, u32 je, 
                     }
                 }
                 const u32 sb = __shfl(bx, s, dev::WAVE);
-                c[u] = p < wtot ? g.b_cols[sb + (p - es)] : EMPTY;
+                c[u] = p < wtot ? bsrc[sb + (p - es)] : B::none();
             }
 #pragma unroll
             for (int u = 0; u < UNROLL; ++u)
-                if (c[u] != EMPTY) f(c[u]);
+                if (B::some(c[u])) f(c[u]);
         }
         if (NW > 1 && nb) {
             __syncthreads();  // the list is complete
@@ -306,7 +339,7 @@ __device__ __forceinline__ void for_each_product(const Mats &g, u32 js, u32 je, 
             // flight the compiler waits for one buffer only while the other
             // buffer's loads are still outstanding, instead of draining all
             // loads before each apply.
-            auto fetch = [&](u32 k, u32(&c)[UB]) -> u32 {
+            auto fetch = [&](u32 k, T(&c)[UB]) -> u32 {
                 u32 start = eb, n = 0;
                 if (k < nwin) {
                     while (k >= next) {
@@ -321,7 +354,7 @@ __device__ __forceinline__ void for_each_product(const Mats &g, u32 js, u32 je, 
                     start = eb + (k - pre) * WIN;
                     n = ee - start < WIN ? ee - start : WIN;
                 }
-                const u32 *src = g.b_cols + start;
+                const T *src = bsrc + start;
                 const u32 last = n ? n - 1 : 0u;  // entries hold at least one column
 #pragma unroll
                 for (int u = 0; u < UB; ++u) {
@@ -330,7 +363,7 @@ __device__ __forceinline__ void for_each_product(const Mats &g, u32 js, u32 je, 
                 }
                 return n;
             };
-            auto apply = [&](const u32(&c)[UB], u32 n) {
+            auto apply = [&](const T(&c)[UB], u32 n) {
                 if (n == WIN) {
                     // all 64 lanes hold consecutive columns of one B row
 #pragma unroll
@@ -341,7 +374,7 @@ __device__ __forceinline__ void for_each_product(const Mats &g, u32 js, u32 je, 
                         if ((u32)(u * 64 + l) < n) f(c[u]);
                 }
             };
-            u32 ca[UB], cb[UB];
+            T ca[UB], cb[UB];
             u32 na = fetch(w, ca), nb2 = 0;
             for (u32 k = w; k < nwin; k += 2 * NW) {
                 nb2 = fetch(k + NW, cb);
@@ -356,11 +389,11 @@ __device__ __forceinline__ void for_each_product(const Mats &g, u32 js, u32 je, 
 }
 
 // The same with one callable for every product.
-template <int WG, int UB, u32 BIGMIN, bool AHEAD = false, typename F>
+template <int WG, int UB, u32 BIGMIN, bool AHEAD = false, bool PACK = false, typename F>
 __device__ __forceinline__ void for_each_product(const Mats &g, u32 js, u32 je, u32 *big, F &&f,
                                                  u32 slice = NOSLICE, u32 sstep = 1, RowAhead *ah = nullptr,
                                                  u32 next_slice = NOSLICE) {
-    for_each_product<WG, UB, BIGMIN, AHEAD>(g, js, je, big, f, f, slice, sstep, ah, next_slice);
+    for_each_product<WG, UB, BIGMIN, AHEAD, PACK>(g, js, je, big, f, f, slice, sstep, ah, next_slice);
 }
 
 // ---------------------------------------------------------------------------
@@ -510,6 +543,29 @@ struct Dump {
                        // (word index, word) pairs of its nonzero words
 };
 
+// Bitmap rows whose bitmap the symbolic pass, or the one pass, keeps in global
+// memory: the numeric pass only expands it (k_emit_stored) instead of
+// gathering the row's products again, and a row of the one pass needs no
+// temporary slot and no capacity.  Slot = the row's position in the bitmap range of
+// perm, for the first `slots` of them (the bins descend by products).  A slice
+// is kept as its words or, when at most a third of them are nonzero and the
+// window is wide, as (word index, word) pairs.
+struct Store {
+    uint4 *words;   // [slot][words_per_row / 4]; nullptr: nothing is kept
+    u32 *chunks;    // [slot][nch]: set bits << 12 | nonzero words of each chunk
+    u32 *fmt;       // [slot][nslices]: 0 = words, 1 = pairs
+    u32 *slot_of;   // [row of the block]: slot + 1, or 0 (set before the pass)
+    u32 slots;
+    u32 nch;        // chunks of a row
+    u32 row_words;  // words of a row: all its slices
+    u32 win_words;  // words of a slice (the symbolic window)
+};
+// Words of a chunk: one wave expands a chunk.
+__host__ __device__ constexpr u32 store_chunk(u32 win_words) {
+    return win_words < EMIT_CHUNK ? win_words : EMIT_CHUNK;
+}
+constexpr u32 STORE_PAIR_WORDS = 1u << 13;  // narrower windows are kept as words
+
 struct Out {
     u32 *nnz_row;
     const u64 *off;
@@ -523,6 +579,7 @@ struct Out {
     // (the prediction was too small); stopping early keeps a badly sized row
     // from probing a full table once per product.  The row is re-run exactly.
     u32 probe_limit;
+    Store keep;  // SYM, ONE: where bitmaps are kept
 };
 constexpr u32 ONE_PASS_PROBES = 256;
 
@@ -754,7 +811,104 @@ __global__ __launch_bounds__(WG) void k_esc(Mats g, const u32 *__restrict__ perm
 // One row (position idx of the bitmap bins) of the bitmap kernel.
 // COMB: full windows OR their words within the wave first (Mats::combine;
 // a separate instantiation, so the plain gather keeps its register budget).
-template <int WBITS, int WG, int MODE, bool COMB>
+// Writes slice s of a kept row (Store) and its chunk sums; adds the thread's
+// share of its set bits to `mine`.
+template <int WBITS, int WG>
+__device__ __forceinline__ void keep_slice(const Store &k, u32 slot, u32 s, u32 nslices, const u32 *bm, u32 *red,
+                                           u32 *sums, u32 &mine) {
+    constexpr u32 W = 1u << WBITS, NW = WG / dev::WAVE, WPW = W / NW;
+    constexpr u32 E = WPW >= 4 * dev::WAVE ? 4 : (WPW >= 2 * dev::WAVE ? 2 : 1), R = WPW / (E * dev::WAVE);
+    constexpr u32 CW = store_chunk(W), NCH = W / CW;
+    // a round of a wave (64 * E words) never straddles two chunks
+    static_assert(R >= 1 && CW % (E * dev::WAVE) == 0 && W <= (1u << 15), "store layout");
+    const u32 wv = dev::wave_id();
+    const int l = dev::lane();
+    const u32 *wb = bm + wv * WPW;
+    auto words = [&](u32 m, u32(&x)[E]) {
+        const u32 *src = wb + (m * dev::WAVE + (u32)l) * E;
+        if constexpr (E == 4) {
+            const uint4 v = *reinterpret_cast<const uint4 *>(src);
+            x[0] = v.x;
+            x[1] = v.y;
+            x[2] = v.z;
+            x[3] = v.w;
+        } else {
+#pragma unroll
+            for (u32 e = 0; e < E; ++e) x[e] = src[e];
+        }
+    };
+    if (threadIdx.x < NCH) sums[threadIdx.x] = 0;
+    __syncthreads();
+    u32 nzw = 0;
+    // rolled loops: this runs beside the gather, whose registers set how many
+    // waves a CU holds
+#pragma unroll 1
+    for (u32 m = 0; m < R; ++m) {
+        u32 x[E], c = 0, nz = 0;
+        words(m, x);
+#pragma unroll
+        for (u32 e = 0; e < E; ++e) {
+            c += (u32)__popc(x[e]);
+            nz += x[e] != 0u;
+        }
+        mine += c;
+        nzw += nz;
+        // at most 32 * 256 bits and 256 words per round
+        const u32 t = dev::wave_incl_sum_dpp((c << 12) | nz);
+        if (l == 63 && t) atomicAdd(&sums[(wv * WPW + m * dev::WAVE * E) / CW], t);
+    }
+    const u64 sl = (u64)slot * nslices + s;
+    if constexpr (W < STORE_PAIR_WORDS) {
+        uint4 *dst = k.words + sl * (W / 4);
+        const uint4 *src = reinterpret_cast<const uint4 *>(bm);
+        for (u32 t = threadIdx.x; t < W / 4; t += WG) dst[t] = src[t];
+        __syncthreads();
+        if (threadIdx.x == 0) k.fmt[sl] = 0u;
+    } else {
+        const u32 wnz = dev::wave_sum(nzw);
+        if (l == 0) red[wv] = wnz;
+        __syncthreads();
+        u32 nzoff = 0, nztot = 0;
+        for (u32 v = 0; v < NW; ++v) {
+            nzoff += v < wv ? red[v] : 0u;
+            nztot += red[v];
+        }
+        const bool as_pairs = nztot <= W / 3;  // uniform
+        if (as_pairs) {
+            uint2 *pairs = reinterpret_cast<uint2 *>(k.words + sl * (W / 4));
+            u32 q0 = nzoff;
+#pragma unroll 1
+            for (u32 m = 0; m < R; ++m) {
+                u32 x[E], nz = 0;
+                words(m, x);
+#pragma unroll
+                for (u32 e = 0; e < E; ++e) nz += x[e] != 0u;
+                const u32 inc = dev::wave_incl_sum_dpp(nz);
+                const u32 rt = (u32)__builtin_amdgcn_readlane((int)inc, 63);
+                if (rt == 0) continue;  // uniform
+                u32 q = q0 + (inc - nz);
+                const u32 i0 = wv * WPW + (m * dev::WAVE + (u32)l) * E;
+#pragma unroll
+                for (u32 e = 0; e < E; ++e)
+                    if (x[e]) pairs[q++] = make_uint2(i0 + e, x[e]);
+                q0 += rt;
+            }
+        } else {
+            uint4 *dst = k.words + sl * (W / 4) + wv * (WPW / 4);
+            const uint4 *src = reinterpret_cast<const uint4 *>(wb);
+#pragma unroll 2
+            for (u32 t = (u32)l; t < WPW / 4; t += dev::WAVE) dst[t] = src[t];
+        }
+        if (threadIdx.x == 0) k.fmt[sl] = as_pairs ? 1u : 0u;
+        __syncthreads();  // red is reused
+    }
+    if (threadIdx.x < NCH) k.chunks[sl * NCH + threadIdx.x] = sums[threadIdx.x];
+    __syncthreads();  // before the next slice clears the bitmap and the list
+}
+
+// PACK: the gather reads packed B rows (Mats::b_pairs), one LDS atomic per
+// word of a B row.
+template <int WBITS, int WG, int MODE, bool COMB, bool PACK>
 __device__ __forceinline__ void bitmap_row(const Mats &g, const u32 *__restrict__ perm, u32 idx, const Out &o,
                                            u32 *bm, u32 *big, u32 *red) {
     constexpr u32 W = 1u << WBITS;
@@ -764,7 +918,7 @@ __device__ __forceinline__ void bitmap_row(const Mats &g, const u32 *__restrict_
     const u32 js = g.a_rpt[i], je = g.a_rpt[i + 1];
     const u32 nslices = (u32)(((u64)g.ncols + SPAN - 1) / SPAN);
     // the split table's slices are this window or a power-of-two fraction of it
-    const bool use_splits = g.splits && g.nsl > 1 && (u32)WBITS >= g.split_bits;
+    const bool use_splits = (PACK ? g.psplits : g.splits) && g.nsl > 1 && (u32)WBITS >= g.split_bits;
     const u32 sstep = use_splits ? 1u << (WBITS - g.split_bits) : 1u;
     u32 mine = 0;
     u64 written = 0;
@@ -775,10 +929,13 @@ __device__ __forceinline__ void bitmap_row(const Mats &g, const u32 *__restrict_
     // the metadata lookahead costs ~16 VGPRs: only where LDS already holds
     // occupancy to two 512-thread (or one 1024-thread) workgroups per CU
     constexpr bool AH = WBITS >= 14;
+    // the wide windows of the one pass dump their dense rows instead; the code
+    // that keeps rows would cost them registers (R-MAT 2^20: 43 -> 58 ms)
+    constexpr bool KEEP = MODE == SYM || (MODE == ONE && WBITS < 14);
     RowAhead ah{EMPTY, make_uint2(0u, 0u)};
     if (AH && use_splits && nslices > 1) {
         if (threadIdx.x < je - js) ah.k0 = g.a_cols[js + threadIdx.x];
-        ah.part = b_part(g, ah.k0, 0, sstep);
+        ah.part = b_part<PACK>(g, ah.k0, 0, sstep);
     }
     for (u32 s = 0; s < nslices; ++s) {
         const u32 sn = s + 1 < nslices ? s + 1 : NOSLICE;
@@ -798,8 +955,20 @@ __device__ __forceinline__ void bitmap_row(const Mats &g, const u32 *__restrict_
         // no range check (base < 2^32 and a multiple of 32)
         auto setu = [&](u32 col) { atomicOr(&bm[(col - (u32)base) >> 5], 1u << (col & 31)); };
         auto setdw = [&](u32 col) { dev::wave_or_sorted_bits(bm, (u32)((u64)col - base)); };
-        constexpr int UBW = MODE == SYM ? 16 : 8;
-        if (nslices == 1) {
+        // a packed element is two registers: 8 of them in flight per buffer,
+        // and 4 where registers and not LDS limit the waves of a CU
+        constexpr int UBW = PACK && WBITS < 14 ? 4 : 8;
+        if constexpr (PACK) {
+            const u32 w0 = (u32)(base >> 5);
+            auto setp = [&](uint2 p) { atomicOr(&bm[p.x - w0], p.y); };
+            auto setq = [&](uint2 p) {
+                const u32 d = p.x - w0;  // wraps below the window
+                if (d < W) atomicOr(&bm[d], p.y);
+            };
+            if (nslices == 1) for_each_product<WG, UBW, LONG_ROW, AH, true>(g, js, je, big, setp);
+            else if (use_splits) for_each_product<WG, UBW, LONG_ROW, AH, true>(g, js, je, big, setp, s, sstep, &ah, sn);
+            else for_each_product<WG, UBW, LONG_ROW, AH, true>(g, js, je, big, setq, NOSLICE, sstep);
+        } else if (nslices == 1) {
             if constexpr (COMB) for_each_product<WG, UBW, LONG_ROW, AH>(g, js, je, big, set1, setw);
             else for_each_product<WG, UBW, LONG_ROW, AH>(g, js, je, big, set1);
         } else {
@@ -814,7 +983,9 @@ __device__ __forceinline__ void bitmap_row(const Mats &g, const u32 *__restrict_
             }
         }
         __syncthreads();
-        if (MODE == SYM) {
+        if (KEEP && idx < o.keep.slots) {
+            if constexpr (KEEP) keep_slice<WBITS, WG>(o.keep, idx, s, nslices, bm, red, big, mine);
+        } else if (MODE == SYM) {
             const uint4 *bm4 = reinterpret_cast<const uint4 *>(bm);
             for (u32 t = threadIdx.x; t < W / 4; t += WG) {
                 const uint4 v = bm4[t];
@@ -1001,9 +1172,12 @@ __device__ __forceinline__ void bitmap_row(const Mats &g, const u32 *__restrict_
         }
         __syncthreads();
     }
-    if (MODE == SYM) {
+    if (MODE == SYM || (KEEP && idx < o.keep.slots)) {
         const u32 n = dev::block_sum<u32, WG>(mine, red);
-        if (threadIdx.x == 0) o.nnz_row[r] = n;
+        if (threadIdx.x == 0) {
+            o.nnz_row[r] = n;
+            if (idx < o.keep.slots) o.keep.slot_of[r] = idx + 1u;
+        }
     } else if (dumping) {
         // listed for emission: in the one pass always (it is written at its
         // exact offset, its capacity does not matter); in the numeric pass
@@ -1037,12 +1211,12 @@ __device__ __forceinline__ void bitmap_row(const Mats &g, const u32 *__restrict_
 // BITMAP rows: one workgroup per row (a launch of one workgroup per row lets
 // the dispatcher balance rows of very different sizes over the CUs and
 // interleave the concurrent hash launches; a persistent grid did neither).
-template <int WBITS, int WG, int MODE, bool COMB>
-__global__ __launch_bounds__(WG) void k_bitmap(Mats g, const u32 *__restrict__ perm, Out o) {
+template <int WBITS, int WG, int MODE, bool COMB, bool PACK>
+__global__ __launch_bounds__(WG) void k_bitmap(Mats g, const u32 *__restrict__ perm, u32 idx0, Out o) {
     __shared__ __align__(16) u32 bm[1u << WBITS];
     __shared__ __align__(8) u32 big[BIG_WORDS(WG)];
     __shared__ u32 red[WG / 64 + 1];
-    bitmap_row<WBITS, WG, MODE, COMB>(g, perm, blockIdx.x, o, bm, big, red);
+    bitmap_row<WBITS, WG, MODE, COMB, PACK>(g, perm, idx0 + blockIdx.x, o, bm, big, red);
 }
 
 // The same rows, persistent: a grid of the workgroups that fit on the device
@@ -1063,7 +1237,7 @@ __global__ __launch_bounds__(WG) void k_bitmap_persist(Mats g, const u32 *__rest
     __syncthreads();
     while (idx < count) {
         if (threadIdx.x == 0) next = atomicAdd(ctr, 1u);
-        bitmap_row<WBITS, WG, MODE, COMB>(g, perm, idx, o, bm, big, red);
+        bitmap_row<WBITS, WG, MODE, COMB, false>(g, perm, idx, o, bm, big, red);
         __syncthreads();
         idx = next;
         __syncthreads();

@@ -1,0 +1,76 @@
+"""Bitmap rows that are kept by the symbolic or the one pass and expanded
+later, and the packed gather of B, against the oracle: column counts at the
+edges of every window size, rows from empty to full (so that rounds are
+expanded by rank and bit by bit), rows of one heavy workgroup, and B rows that
+share words or never do.  Whole numbers: equality."""
+import numpy as np
+import pytest
+
+import clbool_amd as cb
+import oracle
+from clbool_amd import generators as gen
+from helpers import assert_dcsr_equal, upload
+
+pytestmark = pytest.mark.gpu
+NROWS = 400
+
+
+def _dcsr(rows, cols, nrows, ncols):
+    key = np.unique((rows.astype(np.uint64) << np.uint64(32)) | cols.astype(np.uint64))
+    return oracle.pairs_to_dcsr((key >> np.uint64(32)).astype(np.uint32), key.astype(np.uint32), nrows, ncols)
+
+
+def _operands(ncols, kind, seed=3):
+    """A of NROWS rows over 40 B rows, with over 2^20 products in all but the
+    narrowest; the first A rows read all of B."""
+    rng = np.random.default_rng(seed)
+    inner, nrows = 40, NROWS
+    br, bc = [], []
+    for k in range(inner):
+        n = int(min(ncols, rng.choice([1, 40, 300, 2000, 9000])))
+        if kind == "runs":  # neighbours: many columns per word, some words full
+            start = int(rng.integers(0, max(1, ncols - n)))
+            c = np.arange(start, min(ncols, start + n))
+        else:  # one column per word
+            c = rng.integers(0, (ncols + 31) // 32, n) * 32
+            c = c[c < ncols]
+        br.append(np.full(c.size, k))
+        bc.append(c)
+    ar, ac = [], []
+    for r in range(nrows):
+        n = inner if r < 30 else int(rng.integers(0, 12))
+        ac.append(rng.choice(inner, n, replace=False))
+        ar.append(np.full(n, r))
+    return (_dcsr(np.concatenate(ar), np.concatenate(ac), nrows, inner),
+            _dcsr(np.concatenate(br), np.concatenate(bc), inner, ncols))
+
+
+@pytest.mark.parametrize("ncols", [1, 31, 2047, 2048, 2049, 4097, 8191, 16385, 32769, 65535, 131073, 262145, 524289,
+                                   1048576, 1048577, 3000001])
+@pytest.mark.parametrize("kind", ["runs", "apart"])
+def test_kept_rows(controls, ncols, kind):
+    A, B = _operands(ncols, kind)
+    ref = oracle.spgemm(A, B)
+    a, b = upload(controls, A, NROWS, 40), upload(controls, B, 40, ncols)
+    assert_dcsr_equal(controls, cb.dcsr.matrix_multiplication_hash(controls, a, b), ref, "plain")
+    got, _ = cb.dcsr.spgemm(controls, a, b, mode=cb.SPGEMM_BOUND)
+    assert_dcsr_equal(controls, got, ref, "bound")
+    blocks = []
+    plan = cb.dcsr.plan(controls, a, b, mode=cb.SPGEMM_PLAIN, block_bound=max(ncols, ref.nnz // 3 + 1))
+    plan.run_all(lambda k, m, st: blocks.append(m.to_host(controls)[2] if m.nnz else np.zeros(0, np.uint32)))
+    plan.close()
+    assert np.array_equal(np.concatenate(blocks), ref.cols)
+
+
+@pytest.mark.parametrize("hubs", [1, 5])
+def test_heavy_rows(controls, hubs):
+    """A few rows with most of the products run on the widest workgroups."""
+    rng = np.random.default_rng(hubs)
+    n = 20000
+    r = np.concatenate([np.repeat(np.arange(hubs), 3000), rng.integers(0, n, 60000)])
+    c = np.concatenate([rng.integers(0, n, hubs * 3000), rng.integers(0, n, 60000)])
+    A = _dcsr(r, c, n, n)
+    ref = oracle.spgemm(A, A)
+    a = upload(controls, A, n, n)
+    assert_dcsr_equal(controls, cb.dcsr.matrix_multiplication_hash(controls, a, a), ref, "plain")
+    assert_dcsr_equal(controls, cb.dcsr.spgemm(controls, a, a, mode=cb.SPGEMM_BOUND)[0], ref, "bound")
