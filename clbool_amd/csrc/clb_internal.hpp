@@ -124,7 +124,7 @@ struct clb_controls_s {
     clb::u32 cu_count = 0;
     clb::u32 max_wg_size = 1024;
     clb::u32 lds_bytes = 0;
-    clb::u64 *pinned = nullptr;   // small pinned staging area for readbacks
+    clb::u64 *pinned = nullptr;   // PINNED_BYTES of pinned memory, which kernels may write
     clb_tuning tuning{};          // bin thresholds and kernel shapes
     clb_spgemm_stats last{};      // statistics of the last SpGEMM
     void *learned = nullptr;      // learned row-size predictor state (learned.hip)
@@ -178,6 +178,7 @@ void fork_side(clb_controls_s *ctl);
 void join_side(clb_controls_s *ctl);
 inline hipStream_t side_stream(clb_controls_s *ctl, int k) { return ctl->side[k % clb_controls_s::NSIDE]; }
 
+constexpr u64 PINNED_BYTES = 4096;
 // Small synchronous readback through the pinned staging area.
 void readback(clb_controls_s *ctl, void *host, const void *dev, u64 bytes);
 void sync(clb_controls_s *ctl);

@@ -93,18 +93,14 @@ void spgemm_esc(clb_controls_s *ctl, const clb_dcsr &a, const clb_dcsr &b, clb_d
     DevArray<u64> toff(ctl, (u64)nrows + 1), koff(ctl, (u64)nrows + 1), soff(ctl, nrows);
     k_esc_sizes<<<div_up(nrows, 256), 256, 0, ctl->stream>>>(s.P, nrows, lds_max, tlen.ptr, klen.ptr);
     CLB_LAUNCHED("esc_sizes");
-    exclusive_scan_u32_to_u64(ctl, tlen.ptr, toff.ptr, nrows, toff.ptr + nrows);
-    exclusive_scan_u32_to_u64(ctl, klen.ptr, koff.ptr, nrows, koff.ptr + nrows);
+    exclusive_scan_u32_to_u64(ctl, tlen.ptr, toff.ptr, nrows, s.scal.ptr + 1);
+    exclusive_scan_u32_to_u64(ctl, klen.ptr, koff.ptr, nrows, s.scal.ptr + 2);
     fill_u32(ctl, from_side.ptr, nrows, 0u);
     DevArray<u32> perm;
-    BinBuf bb;
     BinHost h;
-    bin_rows(ctl, s, nullptr, nnz_row.ptr, perm, bb);
-    read_bins(ctl, s, bb, h);
-    u64 tot[3];
-    readback(ctl, &tot[0], s.scal.ptr, 8);
-    readback(ctl, &tot[1], toff.ptr + nrows, 8);
-    readback(ctl, &tot[2], koff.ptr + nrows, 8);
+    bin_rows(ctl, s, nullptr, nnz_row.ptr, perm);
+    read_bins(ctl, s, h);
+    const u64 tot[3] = {h.total, h.scal[1], h.scal[2]};
     st.products = tot[0];
     st.rows = nrows;
     st.n_bins = NBINS;

@@ -24,17 +24,23 @@ namespace clb {
 
 constexpr u32 EX_WG = 256, EX_ITEMS = 8, EX_TILE = EX_WG * EX_ITEMS;
 
-// first[t] = the row of nonzero e_lo + t * EX_TILE, for every tile.
-__global__ __launch_bounds__(EX_WG) inline void k_tile_rows(const u32 *__restrict__ rpt, u32 r_lo, u32 r_hi, u32 e_lo,
-                                                            u32 e_hi, u32 *__restrict__ first) {
+// first[t] = the row of nonzero e_lo + t * TILE, for every tile of [e_lo, e_hi)
+// (e_hi == 0: of the rows' own nonzeros, which only the device knows).
+template <u32 TILE>
+__global__ __launch_bounds__(EX_WG) void k_tile_rows(const u32 *__restrict__ rpt, u32 r_lo, u32 r_hi, u32 e_lo,
+                                                     u32 e_hi, u32 *__restrict__ first) {
     const u64 r = (u64)r_lo + (u64)blockIdx.x * EX_WG + threadIdx.x;
+    if (e_hi == 0) {
+        e_lo = rpt[r_lo];
+        e_hi = rpt[r_hi];
+    }
     u32 t0 = 0, n = 0;  // tiles that begin in row r
     if (r < r_hi) {
         const u32 b = rpt[r] > e_lo ? rpt[r] - e_lo : 0u;
         const u32 end = rpt[r + 1] < e_hi ? rpt[r + 1] : e_hi;
         const u32 e = end > e_lo ? end - e_lo : 0u;
-        t0 = (u32)(((u64)b + EX_TILE - 1) / EX_TILE);
-        const u32 t1 = (u32)(((u64)e + EX_TILE - 1) / EX_TILE);
+        t0 = (u32)(((u64)b + TILE - 1) / TILE);
+        const u32 t1 = (u32)(((u64)e + TILE - 1) / TILE);
         n = e > b && t1 > t0 ? t1 - t0 : 0u;
         if (n <= 4) {
             for (u32 k = 0; k < n; ++k) first[t0 + k] = (u32)r;
@@ -97,7 +103,7 @@ void expand_rows(clb_controls_s *ctl, const u32 *rpt, const u32 *rows, u32 r_lo,
     if (e_lo >= e_hi || r_lo >= r_hi) return;
     const u32 tiles = div_up((u64)e_hi - e_lo, EX_TILE);
     DevArray<u32> first(ctl, tiles);  // reused only by later work on this stream
-    k_tile_rows<<<div_up(r_hi - r_lo, EX_WG), EX_WG, 0, ctl->stream>>>(rpt, r_lo, r_hi, e_lo, e_hi, first.ptr);
+    k_tile_rows<EX_TILE><<<div_up(r_hi - r_lo, EX_WG), EX_WG, 0, ctl->stream>>>(rpt, r_lo, r_hi, e_lo, e_hi, first.ptr);
     CLB_LAUNCHED("tile_rows");
     k_expand<F><<<tiles, EX_WG, 0, ctl->stream>>>(rpt, rows, r_hi, e_lo, e_hi, first.ptr, f);
     CLB_LAUNCHED("expand_rows");

@@ -421,19 +421,11 @@ void compact_rows(hipStream_t st, u32 nrows, u64 nnz, const u32 *nnz_row, const 
 // ---------------------------------------------------------------------------
 static void prepare_features(clb_controls_s *ctl, const clb_dcsr &a, const clb_dcsr &b, u32 rb, u32 nrows, Setup &s,
                              DevArray<float> &feat) {
-    // brange, Mats and cfg as in the plain path, but the count kernel is the
-    // feature kernel (it also writes s.prod and the product total)
-    prepare(ctl, a, b, rb, nrows, s, false);
+    // as in the plain path, with the other row statistics beside the products
     feat.reset(ctl, (u64)nrows * NF);
     DevArray<u32> mn(ctl, nrows), mx(ctl, nrows), fc(ctl, nrows), lc(ctl, nrows);
-    fill_u32(ctl, s.prod.ptr, nrows, 0u);
-    fill_u32(ctl, mn.ptr, nrows, 0xFFFFFFFFu);
-    fill_u32(ctl, mx.ptr, nrows, 0u);
-    fill_u32(ctl, fc.ptr, nrows, 0xFFFFFFFFu);
-    fill_u32(ctl, lc.ptr, nrows, 0u);
-    k_row_stats<true><<<div_up(a.nnz, RS_WG), RS_WG, 0, ctl->stream>>>(s.g, nrows, s.prod.ptr, s.scal.ptr, mn.ptr,
-                                                                       mx.ptr, fc.ptr, lc.ptr);
-    CLB_LAUNCHED("row_stats");
+    const RowFeat f{mn.ptr, mx.ptr, fc.ptr, lc.ptr};
+    prepare(ctl, a, b, rb, nrows, s, true, nullptr, &f);
     k_features<<<div_up(nrows, 256), 256, 0, ctl->stream>>>(s.g, nrows, s.prod.ptr, mn.ptr, mx.ptr, fc.ptr, lc.ptr,
                                                              feat.ptr);
     CLB_LAUNCHED("features");
@@ -565,14 +557,12 @@ OnePassPtr one_pass_launch(clb_controls_s *ctl, const clb_dcsr &a, const clb_dcs
         pred = p.pred_own.ptr;
     }
     s.cfg = learned_bincfg(ctl, b.ncols);
-    BinBuf bb;
-    bin_rows(ctl, s, cap, p.nnz_row.ptr, p.perm, bb);
     p.toff.reset(ctl, (u64)nrows + 1);
     exclusive_scan_u32_to_u64(ctl, cap, p.toff.ptr, nrows, s.scal.ptr + 4);
-    read_bins(ctl, s, bb, p.h);
-    u64 sc[8];
-    readback(ctl, sc, s.scal.ptr, sizeof(sc));
-    st.products = pr ? pr->products : sc[0];
+    bin_rows(ctl, s, cap, p.nnz_row.ptr, p.perm);
+    read_bins(ctl, s, p.h);
+    const u64 *sc = p.h.scal;
+    st.products = p.h.total;
     st.rows = nrows;
     st.n_bins = NBINS;
     st.capacity = sc[4];
@@ -631,14 +621,12 @@ void one_pass_post(OnePass &p) {
         CLB_LAUNCHED("failed_keys");
         const BinCfg keep = s.cfg;
         s.cfg = make_bincfg(ctl, b.ncols);  // exact sizing as in the plain symbolic pass
-        BinBuf bb2;
         BinHost h2;
-        bin_rows(ctl, s, p.key2.ptr, nullptr, p.perm2, bb2);
         p.soff.reset(ctl, (u64)nrows + 1);
         exclusive_scan_u32_to_u64(ctl, p.key2.ptr, p.soff.ptr, nrows, s.scal.ptr + 6);
-        read_bins(ctl, s, bb2, h2);
-        u64 side_total = 0;
-        readback(ctl, &side_total, s.scal.ptr + 6, 8);
+        bin_rows(ctl, s, p.key2.ptr, nullptr, p.perm2);
+        read_bins(ctl, s, h2);
+        const u64 side_total = h2.scal[6];
         p.side.reset(ctl, side_total ? side_total : 1);
         u32 *fails2 = reinterpret_cast<u32 *>(s.scal.ptr + 7);
         Out o2{p.nnz_row.ptr, p.soff.ptr, p.side.ptr, p.key2.ptr, fails2, Dump{}, 0};  // exact: full probing
@@ -828,10 +816,9 @@ clb_status clb_predictor_harvest(clb_controls ctl, const clb_dcsr *a, const clb_
             DevArray<float> feat;
             prepare_features(ctl, *a, *b, 0, nrows, s, feat);
             DevArray<u32> nnz_row(ctl, nrows), perm;
-            BinBuf bb;
             BinHost h;
-            bin_rows(ctl, s, nullptr, nnz_row.ptr, perm, bb);
-            read_bins(ctl, s, bb, h);
+            bin_rows(ctl, s, nullptr, nnz_row.ptr, perm);
+            read_bins(ctl, s, h);
             Out o{nnz_row.ptr, nullptr, nullptr, nullptr, reinterpret_cast<u32 *>(s.scal.ptr + 3), Dump{}, 0};
             ensure_splits(ctl, s, h);
             ensure_packed(ctl, s, h);

@@ -165,7 +165,7 @@ void join_side(clb_controls_s *ctl) {
 }
 
 void readback(clb_controls_s *ctl, void *host, const void *dev, u64 bytes) {
-    if (bytes <= 4096) {
+    if (bytes <= PINNED_BYTES) {
         CLB_HIP(hipMemcpyAsync(ctl->pinned, dev, bytes, hipMemcpyDeviceToHost, ctl->stream), READ_BUFFER_ERROR);
         sync(ctl);
         std::memcpy(host, ctl->pinned, bytes);
@@ -362,7 +362,7 @@ clb_status clb_controls_create(uint32_t platform_id, uint32_t device_id, clb_con
             CLB_HIP(hipEventCreateWithFlags(&c->ev_fork, hipEventDisableTiming), CREATE_CONTROLS_ERROR);
             for (int k = 0; k < clb_controls_s::NTAIL; ++k)
                 CLB_HIP(hipStreamCreateWithFlags(&c->tail[k], hipStreamNonBlocking), CREATE_CONTROLS_ERROR);
-            CLB_HIP(hipHostMalloc(reinterpret_cast<void **>(&c->pinned), 4096, hipHostMallocDefault),
+            CLB_HIP(hipHostMalloc(reinterpret_cast<void **>(&c->pinned), PINNED_BYTES, hipHostMallocDefault),
                     CREATE_CONTROLS_ERROR);
             default_tuning(&c->tuning);
         } catch (...) {

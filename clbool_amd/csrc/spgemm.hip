@@ -13,6 +13,7 @@
 
 #include <chrono>
 #include <sstream>
+#include <type_traits>
 
 namespace clb {
 namespace spg {
@@ -176,73 +177,328 @@ __global__ void k_brange_set(const u32 *__restrict__ b_rpt, const u32 *__restric
     if (bpres) atomicOr(&bpres[r >> 5], 1u << (r & 31));
 }
 
-// Histogram of bins.  key == nullptr: key = min(P, ncols) (symbolic sizing).
-// Rows in BIN_EMPTY get nnz_row = 0 when zero_empty is set.
-// A row with a slot (slot_of, may be null) is a BIN_STORED row.
-__global__ __launch_bounds__(256) void k_bin_hist(Mats g, const u32 *__restrict__ P, const u32 *__restrict__ key,
-                                                  u32 n, BinCfg c, u32 *__restrict__ hist, u64 *__restrict__ sums,
-                                                  u32 *__restrict__ nnz_row, const u32 *__restrict__ slot_of) {
+// Per-row statistics of rows [row0, row0 + nrows) of A over its B rows, cut by
+// nonzeros: a tile of RSTAT_WG * ITEMS of them per workgroup, whose rows come
+// from k_tile_rows.  A thread takes ITEMS consecutive nonzeros, sums them up
+// while the row stays the same, and adds to the row's place in LDS; a row
+// inside the tile is stored, one that crosses its border is merged with global
+// atomics (a row spread over several tiles from each).  Random reads of B's
+// row map bound it.  No total is kept here: the row sums are binned anyway,
+// and one counter for all workgroups took 11 ns for each of them (64 thousand
+// workgroups of 256 nonzeros: 728 us for 16.5 million nonzeros, 124 us now).
+//   prod[r] = products (border rows must start at 0);
+//   FEAT: also mn/mx (min/max B-row length, border rows start at ~0 / 0) and
+//   fc/lc (first column of any of its B rows / last column, ~0 / 0).
+constexpr u32 RSTAT_WG = 256;
+template <bool FEAT>
+constexpr u32 rstat_tile() { return RSTAT_WG * (FEAT ? 4 : 8); }
+template <bool FEAT>
+__global__ __launch_bounds__(RSTAT_WG) void k_row_stats(Mats g, u32 nrows, const u32 *__restrict__ first,
+                                                        u32 *__restrict__ prod, RowFeat o) {
+    constexpr u32 TILE = rstat_tile<FEAT>(), ITEMS = TILE / RSTAT_WG;
+    __shared__ u32 rs[TILE + 1], sp[TILE];
+    __shared__ u32 smn[FEAT ? TILE : 1], smx[FEAT ? TILE : 1], sfc[FEAT ? TILE : 1], slc[FEAT ? TILE : 1];
+    const u32 rend = g.row0 + nrows;
+    const u32 jbase = g.a_rpt[g.row0], jend = g.a_rpt[rend];
+    const u64 j0 = (u64)jbase + (u64)blockIdx.x * TILE;
+    if (j0 >= jend) return;  // uniform: the grid covers all of A's nonzeros
+    const u64 j1 = j0 + TILE < jend ? j0 + TILE : jend;
+    const u32 r0 = first[blockIdx.x];
+    const u32 nr = (j1 < jend ? first[blockIdx.x + 1] : rend - 1) - r0 + 1;
+    const bool staged = nr <= TILE;  // else: some stored rows are empty
+    if (staged) {
+        for (u32 t = threadIdx.x; t <= nr; t += RSTAT_WG) rs[t] = g.a_rpt[r0 + t];
+        for (u32 t = threadIdx.x; t < nr; t += RSTAT_WG) {
+            sp[t] = 0;
+            if (FEAT) {
+                smn[t] = sfc[t] = 0xFFFFFFFFu;
+                smx[t] = slc[t] = 0;
+            }
+        }
+    }
+    __syncthreads();
+    const u64 js = j0 + (u64)threadIdx.x * ITEMS;
+    if (js < j1) {
+        uint2 b[ITEMS];
+        u32 c0[ITEMS], c1[ITEMS];
+#pragma unroll
+        for (u32 k = 0; k < ITEMS; ++k) b[k] = js + k < j1 ? b_range(g, g.a_cols[js + k]) : make_uint2(0u, 0u);
+        if (FEAT) {
+#pragma unroll
+            for (u32 k = 0; k < ITEMS; ++k) {
+                c0[k] = b[k].y > b[k].x ? g.b_cols[b[k].x] : 0xFFFFFFFFu;
+                c1[k] = b[k].y > b[k].x ? g.b_cols[b[k].y - 1] : 0u;
+            }
+        }
+        u32 lo = 0, hi = nr;  // the last row that starts at or before js
+        while (hi - lo > 1) {
+            const u32 mid = lo + (hi - lo) / 2;
+            if ((staged ? rs[mid] : g.a_rpt[r0 + mid]) <= js) lo = mid;
+            else hi = mid;
+        }
+        u32 sum = 0, n0 = 0xFFFFFFFFu, n1 = 0, f0 = 0xFFFFFFFFu, f1 = 0;
+        auto flush = [&]() {
+            if (!sum) return;
+            u32 *pp = staged ? &sp[lo] : &prod[r0 + lo - g.row0];
+            atomicAdd(pp, sum);
+            if (FEAT) {
+                const u32 q = r0 + lo - g.row0;
+                atomicMin(staged ? &smn[lo] : &o.mn[q], n0);
+                atomicMax(staged ? &smx[lo] : &o.mx[q], n1);
+                atomicMin(staged ? &sfc[lo] : &o.fc[q], f0);
+                atomicMax(staged ? &slc[lo] : &o.lc[q], f1);
+            }
+            sum = 0;
+            n0 = f0 = 0xFFFFFFFFu;
+            n1 = f1 = 0;
+        };
+#pragma unroll
+        for (u32 k = 0; k < ITEMS; ++k) {
+            if (js + k >= j1) break;
+            while ((staged ? rs[lo + 1] : g.a_rpt[r0 + lo + 1]) <= js + k) {
+                flush();
+                ++lo;
+            }
+            const u32 len = b[k].y - b[k].x;
+            sum += len;
+            if (FEAT && len) {
+                n0 = len < n0 ? len : n0;
+                n1 = len > n1 ? len : n1;
+                f0 = c0[k] < f0 ? c0[k] : f0;
+                f1 = c1[k] > f1 ? c1[k] : f1;
+            }
+        }
+        flush();
+    }
+    __syncthreads();
+    if (!staged) return;
+    for (u32 t = threadIdx.x; t < nr; t += RSTAT_WG) {
+        const u32 row = r0 + t - g.row0;
+        if (rs[t] >= j0 && rs[t + 1] <= j1) {  // the whole row
+            prod[row] = sp[t];
+            if (FEAT) {
+                o.mn[row] = smn[t];
+                o.mx[row] = smx[t];
+                o.fc[row] = sfc[t];
+                o.lc[row] = slc[t];
+            }
+        } else if (sp[t]) {
+            atomicAdd(&prod[row], sp[t]);
+            if (FEAT) {
+                atomicMin(&o.mn[row], smn[t]);
+                atomicMax(&o.mx[row], smx[t]);
+                atomicMin(&o.fc[row], sfc[t]);
+                atomicMax(&o.lc[row], slc[t]);
+            }
+        }
+    }
+}
+
+// The start values of a product's buffers in one launch: the B row map (or its
+// presence bits), the scalars, the row statistics.
+__global__ void k_init(u64 *__restrict__ map, u64 nmap, u32 *__restrict__ bits, u64 nbits, u64 *__restrict__ scal,
+                       u32 nscal, u32 *__restrict__ prod, u32 nrows, RowFeat o) {
+    const u64 stride = (u64)gridDim.x * blockDim.x;
+    const u64 i0 = (u64)blockIdx.x * blockDim.x + threadIdx.x;
+    for (u64 i = i0; i < nmap; i += stride) map[i] = 0;
+    for (u64 i = i0; i < nbits; i += stride) bits[i] = 0;
+    if (i0 < nscal) scal[i0] = 0;
+    if (!prod) return;
+    for (u64 i = i0; i < nrows; i += stride) {
+        prod[i] = 0;
+        if (o.mn) {
+            o.mn[i] = o.fc[i] = 0xFFFFFFFFu;
+            o.mx[i] = o.lc[i] = 0;
+        }
+    }
+}
+
+// Binning in two launches over the same split of the rows into gridDim.x
+// stretches: k_bin_count leaves each stretch's counts and sums per bin,
+// k_bin_place adds up the stretches before its own, places its rows and (the
+// first workgroup) leaves the totals with the product's scalars in host
+// memory.  Few workgroups and no shared counters: 2276 of them adding to 128
+// words took 35 us, and 28 us to place them, for 582 thousand rows; 16 and 13 now.
+//
+// key == nullptr: key = min(P, ncols) (symbolic sizing).  Rows in BIN_EMPTY
+// get nnz_row = 0 when nnz_row is given.  A row with a slot (slot_of, may be
+// null) is a BIN_STORED row.  The order inside a bin is not significant:
+// output positions come from the scan of row sizes.
+constexpr u32 BIN_WG = 256, BIN_GRID = 128;
+struct BinPart {
+    u32 rows[NBINS];
+    u64 sums[3][NBINS];  // products, A nonzeros, key (output nnz)
+};
+__device__ __forceinline__ u32 bin_of(u32 i, const u32 *P, const u32 *key, const BinCfg &c, const u32 *slot_of,
+                                      u32 &p, u32 &k) {
+    p = P[i];
+    k = key ? key[i] : (p < c.ncols ? p : c.ncols);
+    return slot_of && slot_of[i] ? BIN_STORED : classify(p, k, c);
+}
+
+__global__ __launch_bounds__(BIN_WG) void k_bin_count(Mats g, const u32 *__restrict__ P, const u32 *__restrict__ key,
+                                                      u32 n, u32 per, BinCfg c, BinPart *__restrict__ parts,
+                                                      u32 *__restrict__ nnz_row, const u32 *__restrict__ slot_of) {
     __shared__ u32 h[NBINS];
-    __shared__ unsigned long long hs[3][NBINS];  // products, A nonzeros, key (output nnz)
+    __shared__ unsigned long long hs[3][NBINS];
     if (threadIdx.x < NBINS) {
         h[threadIdx.x] = 0;
         hs[0][threadIdx.x] = hs[1][threadIdx.x] = hs[2][threadIdx.x] = 0;
     }
     __syncthreads();
-    const u32 i = blockIdx.x * 256 + threadIdx.x;
-    if (i < n) {
-        const u32 p = P[i];
-        const u32 k = key ? key[i] : (p < c.ncols ? p : c.ncols);
-        const u32 b = slot_of && slot_of[i] ? BIN_STORED : classify(p, k, c);
+    const u64 i0 = (u64)blockIdx.x * per, i1 = i0 + per < n ? i0 + per : n;
+    for (u64 i = i0 + threadIdx.x; i < i1; i += BIN_WG) {
+        u32 p, k;
+        const u32 b = bin_of((u32)i, P, key, c, slot_of, p, k);
         atomicAdd(&h[b], 1u);
-        atomicAdd(&hs[0][b], (unsigned long long)p);
+        if (p) atomicAdd(&hs[0][b], (unsigned long long)p);
         atomicAdd(&hs[1][b], (unsigned long long)(g.a_rpt[g.row0 + i + 1] - g.a_rpt[g.row0 + i]));
-        if (key) atomicAdd(&hs[2][b], (unsigned long long)k);
+        if (key && k) atomicAdd(&hs[2][b], (unsigned long long)k);
         if (b == BIN_EMPTY && nnz_row) nnz_row[i] = 0;
     }
     __syncthreads();
-    if (threadIdx.x < NBINS && h[threadIdx.x]) {
-        atomicAdd(&hist[threadIdx.x], h[threadIdx.x]);
-        for (int q = 0; q < 3; ++q)
-            atomicAdd(reinterpret_cast<unsigned long long *>(&sums[q * NBINS + threadIdx.x]), hs[q][threadIdx.x]);
+    if (threadIdx.x < NBINS) {
+        parts[blockIdx.x].rows[threadIdx.x] = h[threadIdx.x];
+        for (int q = 0; q < 3; ++q) parts[blockIdx.x].sums[q][threadIdx.x] = hs[q][threadIdx.x];
     }
 }
 
-// Exclusive scan of the bin histogram into cursor[0..NBINS] (one wave).
-__global__ void k_bin_offsets(const u32 *__restrict__ hist, u32 *__restrict__ cursor) {
-    const int l = dev::lane();
-    const u32 v = l < (int)NBINS ? hist[l] : 0u;
-    const u32 inc = dev::wave_incl_scan(v);
-    if (l < (int)NBINS) cursor[l] = inc - v;
-    if (l == (int)NBINS - 1) cursor[NBINS] = inc;
-}
-
-// Rows grouped by bin (order inside a bin is not significant: output
-// positions come from the scan of row sizes, not from the processing order).
-__global__ __launch_bounds__(256) void k_bin_scatter(const u32 *__restrict__ P, const u32 *__restrict__ key, u32 n,
-                                                     BinCfg c, u32 *__restrict__ cursor, u32 *__restrict__ perm,
-                                                     const u32 *__restrict__ slot_of) {
-    __shared__ u32 h[NBINS];
-    __shared__ u32 base[NBINS];
-    if (threadIdx.x < NBINS) h[threadIdx.x] = 0;
+__global__ __launch_bounds__(BIN_WG) void k_bin_place(const u32 *__restrict__ P, const u32 *__restrict__ key, u32 n,
+                                                      u32 per, BinCfg c, const BinPart *__restrict__ parts,
+                                                      u32 *__restrict__ perm, const u32 *__restrict__ slot_of,
+                                                      const u64 *__restrict__ scal, BinTotals *__restrict__ host) {
+    __shared__ u32 cursor[NBINS], total[NBINS];
+    __shared__ unsigned long long hs[3 * NBINS];
+    if (threadIdx.x < NBINS) cursor[threadIdx.x] = total[threadIdx.x] = 0;
     __syncthreads();
-    const u32 i = blockIdx.x * 256 + threadIdx.x;
-    u32 b = BIN_EMPTY, local = 0;
-    if (i < n) {
-        const u32 p = P[i];
-        const u32 k = key ? key[i] : (p < c.ncols ? p : c.ncols);
-        b = slot_of && slot_of[i] ? BIN_STORED : classify(p, k, c);
-        if (b != BIN_EMPTY) local = atomicAdd(&h[b], 1u);
+    const u32 b = threadIdx.x % NBINS;
+    u32 before = 0, all = 0;
+#pragma unroll 4
+    for (u32 w = threadIdx.x / NBINS; w < gridDim.x; w += BIN_WG / NBINS) {
+        const u32 v = parts[w].rows[b];
+        before += w < blockIdx.x ? v : 0u;
+        all += v;
+    }
+    atomicAdd(&cursor[b], before);
+    atomicAdd(&total[b], all);
+    __syncthreads();
+    if (threadIdx.x < dev::WAVE) {  // one wave: the bins' starts
+        const u32 v = threadIdx.x < NBINS ? total[threadIdx.x] : 0u;
+        const u32 start = dev::wave_incl_scan(v) - v;
+        if (threadIdx.x < NBINS) cursor[threadIdx.x] += start;
     }
     __syncthreads();
-    if (threadIdx.x < NBINS && h[threadIdx.x]) base[threadIdx.x] = atomicAdd(&cursor[threadIdx.x], h[threadIdx.x]);
-    __syncthreads();
-    if (i < n && b != BIN_EMPTY) perm[base[b] + local] = i;
+    const u64 i0 = (u64)blockIdx.x * per, i1 = i0 + per < n ? i0 + per : n;
+    for (u64 i = i0 + threadIdx.x; i < i1; i += BIN_WG) {
+        u32 p, k;
+        const u32 q = bin_of((u32)i, P, key, c, slot_of, p, k);
+        if (q != BIN_EMPTY) perm[atomicAdd(&cursor[q], 1u)] = (u32)i;
+    }
+    if (blockIdx.x == 0) {
+        if (threadIdx.x < 3 * NBINS) hs[threadIdx.x] = 0;
+        __syncthreads();
+        for (u32 q = 0; q < 3; ++q) {
+            u64 v = 0;
+#pragma unroll 4
+            for (u32 w = threadIdx.x / NBINS; w < gridDim.x; w += BIN_WG / NBINS) v += parts[w].sums[q][b];
+            if (v) atomicAdd(&hs[q * NBINS + b], (unsigned long long)v);
+        }
+        __syncthreads();
+        if (threadIdx.x < NBINS) host->rows[threadIdx.x] = total[threadIdx.x];
+        if (threadIdx.x < 3 * NBINS) host->sums[threadIdx.x] = hs[threadIdx.x];
+        if (threadIdx.x < SCALARS) host->scal[threadIdx.x] = scal[threadIdx.x];
+    }
 }
 
-__global__ void k_nonzero_flags(const u32 *__restrict__ nnz_row, u32 n, u32 *__restrict__ flags) {
-    const u32 i = blockIdx.x * blockDim.x + threadIdx.x;
-    if (i < n) flags[i] = nnz_row[i] != 0;
+// Offsets (off[i], u64; off[n] the total) and stored-row positions (pos[i]: the
+// nonempty rows before i) of the exact row sizes, in tiles of SZ_TILE rows: sums
+// per tile, their scan by one workgroup, and the tiles again.  scal[1] and
+// scal[2] receive the totals.
+constexpr u32 SZ_WG = 256, SZ_ITEMS = 8, SZ_TILE = SZ_WG * SZ_ITEMS;
+struct SizeSum {
+    u64 nnz;
+    u64 rows;
+};
+__device__ __forceinline__ void load_sizes(const u32 *__restrict__ nnz_row, u32 n, u64 i, u32 (&v)[SZ_ITEMS]) {
+    if (i + SZ_ITEMS <= n && (reinterpret_cast<uintptr_t>(nnz_row) & 15u) == 0) {  // i is a multiple of 8
+        const uint4 a = *reinterpret_cast<const uint4 *>(nnz_row + i);
+        const uint4 b = *reinterpret_cast<const uint4 *>(nnz_row + i + 4);
+        v[0] = a.x; v[1] = a.y; v[2] = a.z; v[3] = a.w;
+        v[4] = b.x; v[5] = b.y; v[6] = b.z; v[7] = b.w;
+    } else {
+#pragma unroll
+        for (u32 k = 0; k < SZ_ITEMS; ++k) v[k] = i + k < n ? nnz_row[i + k] : 0u;
+    }
+}
+
+__global__ __launch_bounds__(SZ_WG) void k_sizes_sum(const u32 *__restrict__ nnz_row, u32 n,
+                                                     SizeSum *__restrict__ sums) {
+    __shared__ u64 red[SZ_WG / dev::WAVE + 1];
+    u32 v[SZ_ITEMS];
+    load_sizes(nnz_row, n, (u64)blockIdx.x * SZ_TILE + (u64)threadIdx.x * SZ_ITEMS, v);
+    u64 s = 0, r = 0;
+#pragma unroll
+    for (u32 k = 0; k < SZ_ITEMS; ++k) {
+        s += v[k];
+        r += v[k] != 0u;
+    }
+    const u64 ts = dev::block_sum<u64, SZ_WG>(s, red), tr = dev::block_sum<u64, SZ_WG>(r, red);
+    if (threadIdx.x == 0) sums[blockIdx.x] = SizeSum{ts, tr};
+}
+
+__global__ __launch_bounds__(SZ_WG) void k_sizes_scan(SizeSum *__restrict__ sums, u32 tiles, u64 *__restrict__ last,
+                                                      u64 *__restrict__ scal) {
+    __shared__ u64 red[SZ_WG / dev::WAVE + 1];
+    u64 cs = 0, cr = 0;
+    for (u32 t0 = 0; t0 < tiles; t0 += SZ_WG) {
+        const u32 t = t0 + threadIdx.x;
+        const SizeSum v = t < tiles ? sums[t] : SizeSum{0, 0};
+        u64 as, ar;
+        const u64 s = dev::block_excl_scan<u64, SZ_WG>(v.nnz, red, as);
+        const u64 r = dev::block_excl_scan<u64, SZ_WG>(v.rows, red, ar);
+        if (t < tiles) sums[t] = SizeSum{cs + s, cr + r};
+        cs += as;
+        cr += ar;
+    }
+    if (threadIdx.x == 0) {
+        *last = scal[1] = cs;
+        scal[2] = cr;
+    }
+}
+
+// sums == nullptr: the only tile, which also leaves the totals.
+__global__ __launch_bounds__(SZ_WG) void k_sizes_place(const u32 *__restrict__ nnz_row, u32 n,
+                                                       const SizeSum *__restrict__ sums, u64 *__restrict__ off,
+                                                       u32 *__restrict__ pos, u64 *__restrict__ scal) {
+    __shared__ u64 red[SZ_WG / dev::WAVE + 1];
+    const u64 i = (u64)blockIdx.x * SZ_TILE + (u64)threadIdx.x * SZ_ITEMS;
+    u32 v[SZ_ITEMS];
+    load_sizes(nnz_row, n, i, v);
+    u64 s = 0, r = 0;
+#pragma unroll
+    for (u32 k = 0; k < SZ_ITEMS; ++k) {
+        s += v[k];
+        r += v[k] != 0u;
+    }
+    u64 as, ar;
+    u64 o = dev::block_excl_scan<u64, SZ_WG>(s, red, as);
+    u64 q = dev::block_excl_scan<u64, SZ_WG>(r, red, ar);
+    if (sums) {
+        o += sums[blockIdx.x].nnz;
+        q += sums[blockIdx.x].rows;
+    } else if (threadIdx.x == 0) {
+        off[n] = scal[1] = as;
+        scal[2] = ar;
+    }
+#pragma unroll
+    for (u32 k = 0; k < SZ_ITEMS; ++k) {
+        if (i + k < n) {
+            off[i + k] = o;
+            pos[i + k] = (u32)q;
+        }
+        o += v[k];
+        q += v[k] != 0u;
+    }
 }
 
 // prepare_for_shift_empty_rows + set_positions_pointers_and_rows
@@ -641,7 +897,7 @@ void ensure_packed(clb_controls_s *ctl, Setup &s, const BinHost &h) {
     s.pack_tried = true;
     const u32 tiles = div_up(b.nnz, EX_TILE);
     DevArray<u32> first(ctl, tiles), offs(ctl, (u64)tiles + 1);
-    k_tile_rows<<<div_up(b.nzr, EX_WG), EX_WG, 0, ctl->stream>>>(u32p(b.rpt), 0, b.nzr, 0, b.nnz, first.ptr);
+    k_tile_rows<EX_TILE><<<div_up(b.nzr, EX_WG), EX_WG, 0, ctl->stream>>>(u32p(b.rpt), 0, b.nzr, 0, b.nnz, first.ptr);
     CLB_LAUNCHED("tile_rows");
     k_pack_count<<<tiles, EX_WG, 0, ctl->stream>>>(u32p(b.rpt), u32p(b.cols), b.nzr, b.nnz, first.ptr, offs.ptr);
     CLB_LAUNCHED("pack_count");
@@ -672,7 +928,7 @@ void ensure_packed(clb_controls_s *ctl, Setup &s, const BinHost &h) {
 }
 
 void prepare(clb_controls_s *ctl, const clb_dcsr &a, const clb_dcsr &b, u32 row_begin, u32 nrows, Setup &s,
-             bool count, const Setup *shared) {
+             bool stats, const Setup *shared, const RowFeat *feat) {
     s.nrows = nrows;
     s.row0 = row_begin;
     if (shared) {
@@ -688,18 +944,7 @@ void prepare(clb_controls_s *ctl, const clb_dcsr &a, const clb_dcsr &b, u32 row_
         // hypersparse B (under one stored row in 16): a presence bit per row id
         // instead of clearing the whole row map
         const bool sparse_map = (u64)b.nzr * 16 < s.mapn;
-        if (sparse_map) {
-            s.bpres.reset(ctl, ((u64)s.mapn + 31) / 32);
-            fill_u32(ctl, s.bpres.ptr, s.bpres.n, 0u);
-        } else {
-            fill_u64(ctl, reinterpret_cast<u64 *>(s.brange.ptr), s.mapn, 0ull);
-        }
-        if (b.nzr) {
-            k_brange_set<<<div_up(b.nzr, 256), 256, 0, ctl->stream>>>(u32p(b.rpt), u32p(b.rows), b.nzr, s.mapn,
-                                                                       s.brange.ptr,
-                                                                       sparse_map ? s.bpres.ptr : nullptr);
-            CLB_LAUNCHED("brange_set");
-        }
+        if (sparse_map) s.bpres.reset(ctl, ((u64)s.mapn + 31) / 32);
         s.g.bpres = sparse_map ? s.bpres.ptr : nullptr;
         s.g.a_rpt = u32p(a.rpt);
         s.g.a_rows = u32p(a.rows);
@@ -723,49 +968,74 @@ void prepare(clb_controls_s *ctl, const clb_dcsr &a, const clb_dcsr &b, u32 row_
         s.b = b;  // the split table is built by ensure_splits, once bitmap rows exist
     }
     s.g.row0 = row_begin;
-    s.prod.reset(ctl, nrows);
-    s.P = s.prod.ptr;
     s.ctr.reset(ctl, 4);
-    s.scal.reset(ctl, 8);  // [0] total products, [1] nnz total, [2] nzr total, [3] overflow flag
-    fill_u64(ctl, s.scal.ptr, 8, 0ull);
-    if (!count) return;
-    // count_workload (count_workload.cl:30-53): products of each A row,
-    // balanced over A's nonzeros (k_row_stats)
-    fill_u32(ctl, s.prod.ptr, nrows, 0u);
-    k_row_stats<false><<<div_up(a.nnz, RS_WG), RS_WG, 0, ctl->stream>>>(s.g, nrows, s.prod.ptr, s.scal.ptr, nullptr,
-                                                                        nullptr, nullptr, nullptr);
-    CLB_LAUNCHED("count_workload");
+    s.scal.reset(ctl, SCALARS);  // [1] nnz total, [2] nzr total, [3] overflow flag, ...
+    if (stats) {
+        s.prod.reset(ctl, nrows);
+        s.P = s.prod.ptr;
+    }
+    const u64 nmap = shared || s.bpres.ptr ? 0 : s.mapn, nbits = shared ? 0 : s.bpres.n;
+    u64 most = nmap > nbits ? nmap : nbits;
+    if (stats && nrows > most) most = nrows;
+    const u32 cap = ctl->cu_count * 16, grid = div_up(most ? most : 1, 256);
+    k_init<<<grid < cap ? grid : cap, 256, 0, ctl->stream>>>(reinterpret_cast<u64 *>(s.brange.ptr), nmap, s.bpres.ptr,
+                                                             nbits, s.scal.ptr, SCALARS, stats ? s.prod.ptr : nullptr,
+                                                             nrows, feat ? *feat : RowFeat{});
+    CLB_LAUNCHED("init");
+    if (!shared && b.nzr) {
+        k_brange_set<<<div_up(b.nzr, 256), 256, 0, ctl->stream>>>(u32p(b.rpt), u32p(b.rows), b.nzr, s.mapn,
+                                                                   s.brange.ptr, s.bpres.ptr);
+        CLB_LAUNCHED("brange_set");
+    }
+    if (!stats) return;
+    // count_workload (count_workload.cl:30-53): products of each A row
+    auto run = [&](auto feat_c) {
+        constexpr bool FEAT = decltype(feat_c)::value;
+        const u32 tiles = div_up(a.nnz, rstat_tile<FEAT>());
+        DevArray<u32> first(ctl, tiles);
+        k_tile_rows<rstat_tile<FEAT>()><<<div_up(nrows, EX_WG), EX_WG, 0, ctl->stream>>>(
+            s.g.a_rpt, row_begin, row_begin + nrows, 0, 0, first.ptr);
+        CLB_LAUNCHED("tile_rows");
+        k_row_stats<FEAT><<<tiles, RSTAT_WG, 0, ctl->stream>>>(s.g, nrows, first.ptr, s.prod.ptr,
+                                                               feat ? *feat : RowFeat{});
+        CLB_LAUNCHED("count_workload");
+    };
+    if (feat) run(std::true_type{});
+    else run(std::false_type{});
 }
 
 void bin_rows(clb_controls_s *ctl, const Setup &s, const u32 *key, u32 *nnz_row_zero, DevArray<u32> &perm,
-              BinBuf &bb, const u32 *slot_of) {
-    bb.buf.reset(ctl, 2 * NBINS + 2 + 2 * 3 * NBINS);
-    fill_u32(ctl, bb.buf.ptr, bb.buf.n, 0u);
+              const u32 *slot_of) {
+    static_assert(sizeof(BinTotals) <= PINNED_BYTES, "pinned staging");
     perm.reset(ctl, s.nrows ? s.nrows : 1);
-    const u32 grid = div_up(s.nrows, 256);
-    k_bin_hist<<<grid, 256, 0, ctl->stream>>>(s.g, s.P, key, s.nrows, s.cfg, bb.hist(), bb.sums(),
-                                              nnz_row_zero, slot_of);
-    CLB_LAUNCHED("bin_hist");
-    k_bin_offsets<<<1, 64, 0, ctl->stream>>>(bb.hist(), bb.cursor());
-    CLB_LAUNCHED("bin_offsets");
-    k_bin_scatter<<<grid, 256, 0, ctl->stream>>>(s.P, key, s.nrows, s.cfg, bb.cursor(), perm.ptr,
-                                                 slot_of);
-    CLB_LAUNCHED("bin_scatter");
+    // stretches of at least four rows per thread
+    u32 grid = div_up(s.nrows ? s.nrows : 1, 4 * BIN_WG);
+    if (grid > BIN_GRID) grid = BIN_GRID;
+    const u32 per = div_up(s.nrows, grid);
+    DevArray<BinPart> parts(ctl, grid);
+    k_bin_count<<<grid, BIN_WG, 0, ctl->stream>>>(s.g, s.P, key, s.nrows, per, s.cfg, parts.ptr, nnz_row_zero,
+                                                  slot_of);
+    CLB_LAUNCHED("bin_count");
+    k_bin_place<<<grid, BIN_WG, 0, ctl->stream>>>(s.P, key, s.nrows, per, s.cfg, parts.ptr, perm.ptr, slot_of,
+                                                  s.scal.ptr, reinterpret_cast<BinTotals *>(ctl->pinned));
+    CLB_LAUNCHED("bin_place");
 }
 
-void read_bins(clb_controls_s *ctl, Setup &s, const BinBuf &bb, BinHost &h) {
-    u32 hist[NBINS];
-    readback(ctl, hist, bb.hist(), sizeof(hist));
+void read_bins(clb_controls_s *ctl, Setup &s, BinHost &h) {
+    sync(ctl);
+    BinTotals t;
+    std::memcpy(&t, ctl->pinned, sizeof(t));
     h.off[0] = 0;
-    for (u32 b = 0; b < NBINS; ++b) h.off[b + 1] = h.off[b] + hist[b];
-    u64 sums[3 * NBINS];
-    readback(ctl, sums, bb.sums(), sizeof(sums));
+    h.total = 0;
     for (u32 b = 0; b < NBINS; ++b) {
-        h.products[b] = sums[b];
-        h.a_nnz[b] = sums[NBINS + b];
-        h.out_nnz[b] = sums[2 * NBINS + b];
-        s.bin_products[b] = sums[b];
+        h.off[b + 1] = h.off[b] + t.rows[b];
+        h.products[b] = t.sums[b];
+        h.a_nnz[b] = t.sums[NBINS + b];
+        h.out_nnz[b] = t.sums[2 * NBINS + b];
+        s.bin_products[b] = t.sums[b];
+        h.total += t.sums[b];
     }
+    std::memcpy(h.scal, t.scal, sizeof(h.scal));
 }
 
 // Sums nnz_row over the rows of bins 1..NBINS-1 (perm[off[1] .. off[NBINS]));
@@ -848,14 +1118,21 @@ void join_deferred(clb_controls_s *ctl, const hipEvent_t *defer) {
 void launch_bins(clb_controls_s *ctl, const Setup &s, const u32 *perm, const u32 off[NBINS + 1], int mode,
                  const Out &o, LaunchTimer *lt, int family, hipEvent_t *defer, bool one_stream) {
     if (!one_stream) fork_side(ctl);
-    // the bitmap kernels take side streams 0.. (one each), the table kernels
-    // alternate over the others
-    int used = 0, k = 0;
+    // the longest kernels have streams of their own: kept rows or the bitmap
+    // rows on side stream 0, heavy bitmap rows on side stream 1 (not behind the
+    // previous block's bitmap rows); the table kernels alternate over the rest
+    bool taken[clb_controls_s::NSIDE] = {};
+    int k = 0;
+    auto on = [&](int w) {
+        taken[w] = true;
+        return one_stream ? ctl->stream : side_stream(ctl, w);
+    };
     auto next = [&]() {
         constexpr int NS = clb_controls_s::NSIDE;
         if (one_stream) return ctl->stream;
-        const int rest = NS - used > 0 ? NS - used : 1;
-        return side_stream(ctl, (used < NS ? used : NS - 1) + k++ % rest);
+        do k = (k + 1) % NS;
+        while (taken[k] && k != NS - 1);
+        return side_stream(ctl, k);
     };
     LaunchTimer dummy;
     LaunchTimer &t = lt ? *lt : dummy;
@@ -875,7 +1152,7 @@ void launch_bins(clb_controls_s *ctl, const Setup &s, const u32 *perm, const u32
     if (!s.cfg.esc_only) {
         const u32 ns = off[BIN_STORED + 1] - off[BIN_STORED];
         if (ns && mode == NUM && o.keep.words) {
-            hipStream_t st = one_stream ? ctl->stream : side_stream(ctl, used++);
+            hipStream_t st = on(0);
             t.begin(st);
             emit_stored(st, perm + off[BIN_STORED], ns, o.keep, o.off, o.cols);
             t.end(fam(CLB_KK_BITMAP), st);
@@ -901,7 +1178,7 @@ void launch_bins(clb_controls_s *ctl, const Setup &s, const u32 *perm, const u32
             for (int wide = 1; wide >= 0; --wide) {
                 const u32 r0 = wide ? 0 : heavy, nr = wide ? heavy : n - heavy;
                 if (!nr) continue;
-                hipStream_t st = one_stream ? ctl->stream : side_stream(ctl, used < 2 ? used++ : 2);
+                hipStream_t st = on(wide || (ns && mode == NUM) ? 1 : 0);
                 t.begin(st);
                 if (mode == SYM) launch_bitmap_sym(ctl, st, s, pp, r0, nr, bits, wide != 0, o);
                 else if (mode == NUM) launch_bitmap_num(ctl, st, s, pp, r0, nr, bits, wide != 0, o);
@@ -1024,12 +1301,19 @@ void scan_sizes(clb_controls_s *ctl, Setup &s, const u32 *nnz_row, DevArray<u64>
     off.reset(ctl, s.nrows + 1);
     pos.reset(ctl, s.nrows + 1);
     // off[nrows] holds the total too (row r's size is off[r + 1] - off[r])
-    exclusive_scan_u32_to_u64(ctl, nnz_row, off.ptr, s.nrows, off.ptr + s.nrows);
-    CLB_HIP(hipMemcpyAsync(s.scal.ptr + 1, off.ptr + s.nrows, 8, hipMemcpyDeviceToDevice, ctl->stream),
-            COPY_BUFFER_ERROR);
-    k_nonzero_flags<<<div_up(s.nrows, 256), 256, 0, ctl->stream>>>(nnz_row, s.nrows, pos.ptr);
-    CLB_LAUNCHED("nonzero_flags");
-    exclusive_scan_u32(ctl, pos.ptr, pos.ptr, s.nrows, reinterpret_cast<u32 *>(s.scal.ptr + 2));
+    const u32 tiles = div_up(s.nrows, SZ_TILE);
+    if (tiles <= 1) {
+        k_sizes_place<<<1, SZ_WG, 0, ctl->stream>>>(nnz_row, s.nrows, nullptr, off.ptr, pos.ptr, s.scal.ptr);
+        CLB_LAUNCHED("sizes");
+        return;
+    }
+    DevArray<SizeSum> sums(ctl, tiles);
+    k_sizes_sum<<<tiles, SZ_WG, 0, ctl->stream>>>(nnz_row, s.nrows, sums.ptr);
+    CLB_LAUNCHED("sizes_sum");
+    k_sizes_scan<<<1, SZ_WG, 0, ctl->stream>>>(sums.ptr, tiles, off.ptr + s.nrows, s.scal.ptr);
+    CLB_LAUNCHED("sizes_scan");
+    k_sizes_place<<<tiles, SZ_WG, 0, ctl->stream>>>(nnz_row, s.nrows, sums.ptr, off.ptr, pos.ptr, s.scal.ptr);
+    CLB_LAUNCHED("sizes_place");
 }
 
 void spgemm_plain(clb_controls_s *ctl, const clb_dcsr &a, const clb_dcsr &b, u32 row_begin, u32 row_end,
@@ -1057,17 +1341,14 @@ void spgemm_plain(clb_controls_s *ctl, const clb_dcsr &a, const clb_dcsr &b, u32
         tm.mark();  // 2
     } else {
         DevArray<u32> perm;
-        BinBuf bb;
         BinHost h1;
         nnz_row_own.reset(ctl, nrows);
         nnz_row = nnz_row_own.ptr;
-        bin_rows(ctl, s, nullptr, nnz_row, perm, bb);
-        read_bins(ctl, s, bb, h1);
-        u64 total_products = 0;
-        readback(ctl, &total_products, s.scal.ptr, 8);
-        st.products = total_products;
+        bin_rows(ctl, s, nullptr, nnz_row, perm);
+        read_bins(ctl, s, h1);
+        st.products = h1.total;
         tm.mark();  // 1
-        if (total_products == 0) {
+        if (h1.total == 0) {
             out.nrows = a.nrows;
             out.ncols = b.ncols;
             return;
@@ -1089,18 +1370,16 @@ void spgemm_plain(clb_controls_s *ctl, const clb_dcsr &a, const clb_dcsr &b, u32
     DevArray<u32> pos;
     scan_sizes(ctl, s, nnz_row, offs, pos);
     DevArray<u32> perm2;
-    BinBuf bb2;
     BinHost h2;
-    bin_rows(ctl, s, nnz_row, nullptr, perm2, bb2, keep.words ? keep.slot_of : nullptr);
-    read_bins(ctl, s, bb2, h2);
+    bin_rows(ctl, s, nnz_row, nullptr, perm2, keep.words ? keep.slot_of : nullptr);
+    read_bins(ctl, s, h2);
     for (u32 k = 0; k < NBINS; ++k) {
         st.bin_rows[k] = h2.off[k + 1] - h2.off[k];
         st.bin_products[k] = h2.products[k];
         st.bin_a_nnz[k] = h2.a_nnz[k];
         st.bin_out_nnz[k] = h2.out_nnz[k];
     }
-    u64 sc[4];
-    readback(ctl, sc, s.scal.ptr, sizeof(sc));
+    const u64 *sc = h2.scal;  // taken with the bins
     tm.mark();  // 3
     if (sc[3]) raise(RUN_KERNEL_FAILURE, "hash table overflow in the symbolic pass");
     const u64 nnz = sc[1];
@@ -1149,10 +1428,9 @@ void spgemm_plain(clb_controls_s *ctl, const clb_dcsr &a, const clb_dcsr &b, u32
 void plan_sizes_plain(clb_controls_s *ctl, Setup &s, u32 *size, StoreBufs &store) {
     // the symbolic pass of spgemm_plain over every stored row of A
     DevArray<u32> perm;
-    BinBuf bb;
     BinHost h;
-    bin_rows(ctl, s, nullptr, size, perm, bb);
-    read_bins(ctl, s, bb, h);
+    bin_rows(ctl, s, nullptr, size, perm);
+    read_bins(ctl, s, h);
     setup_store(ctl, s, h, s.cfg.sym_bits, store);
     Out o{size, nullptr, nullptr, nullptr, reinterpret_cast<u32 *>(s.scal.ptr + 3), Dump{}, 0, store.keep};
     ensure_splits(ctl, s, h);

@@ -8,7 +8,7 @@ namespace clb {
 namespace spg {
 
 // Per-call device state: the B row map, per-row product counts and a few
-// device scalars ([0] products, [1] nnz, [2] nzr, [3] overflow flag, ...).
+// device scalars ([1] nnz, [2] nzr, [3] overflow flag, ...).
 struct Setup {
     u32 nrows = 0, row0 = 0, mapn = 0;
     DevArray<uint2> brange;
@@ -56,18 +56,23 @@ struct LaunchTimer {
     ~LaunchTimer();
 };
 
-// Device layout of the binning scratch: hist[NBINS] | cursor[NBINS+1] | pad |
-// products[NBINS] | a_nnz[NBINS] | out_nnz[NBINS] (the last three as u64).
-struct BinBuf {
-    DevArray<u32> buf;
-    u32 *hist() const { return buf.ptr; }
-    u32 *cursor() const { return buf.ptr + NBINS; }
-    u64 *sums() const { return reinterpret_cast<u64 *>(buf.ptr + 2 * NBINS + 2); }
+constexpr u32 SCALARS = 8;  // Setup::scal
+// What a binning leaves in the controls' pinned memory.
+struct BinTotals {
+    u32 rows[NBINS];
+    u64 sums[3 * NBINS];  // products, A nonzeros, key (output nnz)
+    u64 scal[SCALARS];    // the product's scalars when the rows were placed
+};
+// Per-row statistics besides the products (k_row_stats; null: not wanted).
+struct RowFeat {
+    u32 *mn, *mx, *fc, *lc;
 };
 // Host copy of the binning: off[b]..off[b+1] is bin b's range of perm.
 struct BinHost {
     u32 off[NBINS + 1];
     u64 products[NBINS], a_nnz[NBINS], out_nnz[NBINS];
+    u64 total;          // products of all bins
+    u64 scal[SCALARS];
 };
 
 // Scratch of the dense-bitmap path (see Dump in spgemm_kernels.hpp).
@@ -122,16 +127,17 @@ constexpr u64 PACK_MIN_PRODUCTS = 1ull << 22;  // launches and one read-back bel
 constexpr u32 PACK_MIN_READS = 8;  // products of the bitmap rows per nonzero of B
 constexpr u32 PACK_MAX_PCT = 95;   // pairs per 100 nonzeros of B
 void ensure_packed(clb_controls_s *ctl, Setup &s, const BinHost &h);
-// B row map, kernel arguments and (count == true) per-row product counts.
-// With `shared`, the B row map, split table and bin config are taken from
-// it (a plan's Setup) instead of being built.
+// B row map, kernel arguments and (stats) per-row products, with `feat` also
+// the other statistics.  With `shared`, the B row map, split table and bin
+// config are taken from it (a plan's Setup) instead of being built.
 void prepare(clb_controls_s *ctl, const clb_dcsr &a, const clb_dcsr &b, u32 row_begin, u32 nrows, Setup &s,
-             bool count = true, const Setup *shared = nullptr);
-// Bins the rows of the block by (P, key) into perm (device only, no sync).
+             bool stats = true, const Setup *shared = nullptr, const RowFeat *feat = nullptr);
+// Bins the rows of the block by (P, key) into perm (device only, no sync); the
+// totals and the scalars as they are then go to pinned memory.
 void bin_rows(clb_controls_s *ctl, const Setup &s, const u32 *key, u32 *nnz_row_zero, DevArray<u32> &perm,
-              BinBuf &bb, const u32 *slot_of = nullptr);
-// Reads the binning back (synchronises the stream).
-void read_bins(clb_controls_s *ctl, Setup &s, const BinBuf &bb, BinHost &h);
+              const u32 *slot_of = nullptr);
+// Takes the totals of the last bin_rows (synchronises the stream).
+void read_bins(clb_controls_s *ctl, Setup &s, BinHost &h);
 // Per-bin sums of nnz_row over the rows of each nonempty bin's range of perm
 // (rows marked FAILED count 0); the result is read back into out[NBINS].
 void sum_by_bin(clb_controls_s *ctl, const u32 *perm, const BinHost &h, u32 nrows, const u32 *nnz_row,
