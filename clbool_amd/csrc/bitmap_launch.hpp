@@ -8,6 +8,12 @@
 namespace clb {
 namespace spg {
 
+// Packed B serves a window when its groups tell the window's columns: always
+// up to 2^20 columns, above through slices no wider than the window.
+static bool use_packs(const Mats &g, u32 bits) {
+    return g.b_packs && (g.ncols <= (1u << 20) || (g.psplits && bits >= g.split_bits));
+}
+
 // One workgroup per row, or (tuning.bitmap_persistent) a persistent grid that
 // takes rows from a counter.
 template <int WBITS, int WG, int MODE, bool COMB>
@@ -15,7 +21,7 @@ static void launch_bitmap_c(clb_controls_s *ctl, hipStream_t st, const Setup &s,
                             const Out &o) {
     if (!ctl->tuning.bitmap_persistent) {
         if constexpr (!COMB) {
-            if (s.g.b_pairs) {
+            if (use_packs(s.g, WBITS)) {
                 k_bitmap<WBITS, WG, MODE, false, true><<<n, WG, 0, st>>>(s.g, perm, r0, o);
                 return;
             }
@@ -42,7 +48,7 @@ static void launch_bitmap_w(clb_controls_s *ctl, hipStream_t st, const Setup &s,
     constexpr int WG = (int)bitmap_wg(WBITS), WIDE = (int)bitmap_wide(WBITS);
     if constexpr (WIDE > WG) {
         if (wide) {
-            if (s.g.b_pairs) k_bitmap<WBITS, WIDE, MODE, false, true><<<n, WIDE, 0, st>>>(s.g, perm, r0, o);
+            if (use_packs(s.g, WBITS)) k_bitmap<WBITS, WIDE, MODE, false, true><<<n, WIDE, 0, st>>>(s.g, perm, r0, o);
             else k_bitmap<WBITS, WIDE, MODE, false, false><<<n, WIDE, 0, st>>>(s.g, perm, r0, o);
             return;
         }

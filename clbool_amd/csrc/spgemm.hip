@@ -44,10 +44,11 @@ __global__ void k_slice_splits(const u32 *__restrict__ b_rpt, const u32 *__restr
     out[nsl] = end;
 }
 
-// Packed B (Mats::b_pairs): a pair begins at every column that starts a row or
-// a new word.  The count pass gives each tile of EX_TILE columns its pairs;
-// once these are scanned, the thread of a pair's first column ORs the columns
-// of its word (its row goes on past the tile if need be) and writes the pair.
+// Packed B (Mats::b_packs): a pack begins at every column that starts a row or
+// a new group of 16.  The count pass gives each tile of EX_TILE columns its
+// packs; once these are scanned, the thread of a pack's first column collects
+// the columns of its group (its row goes on past the tile if need be) and
+// writes the pack and where its first column is.
 struct PackTile {
     u64 e0, e1;
     u32 r0, nr;
@@ -87,7 +88,7 @@ __global__ __launch_bounds__(EX_WG) void k_pack_count(const u32 *__restrict__ b_
         const u64 e = t.e0 + q * EX_WG + threadIdx.x;
         if (e >= t.e1) break;
         const u32 a = t.row(b_rpt, srpt, e);
-        c += b_rpt[t.r0 + a] == e || (b_cols[e] >> 5) != (b_cols[e - 1] >> 5);
+        c += b_rpt[t.r0 + a] == e || (b_cols[e] >> 4) != (b_cols[e - 1] >> 4);
     }
     const u32 sum = dev::block_sum<u32, EX_WG>(c, red);
     if (threadIdx.x == 0) counts[blockIdx.x] = sum;
@@ -96,7 +97,7 @@ __global__ __launch_bounds__(EX_WG) void k_pack_count(const u32 *__restrict__ b_
 __global__ __launch_bounds__(EX_WG) void k_pack_place(const u32 *__restrict__ b_rpt, const u32 *__restrict__ b_cols,
                                                       u32 b_nzr, u32 b_nnz, const u32 *__restrict__ first,
                                                       const u32 *__restrict__ offs, u32 *__restrict__ prpt,
-                                                      uint2 *__restrict__ pairs) {
+                                                      u32 *__restrict__ packs, u32 *__restrict__ pfirst) {
     constexpr u32 NW = EX_WG / dev::WAVE;
     __shared__ u32 srpt[EX_TILE];
     __shared__ u32 wcnt[NW];
@@ -110,16 +111,16 @@ __global__ __launch_bounds__(EX_WG) void k_pack_place(const u32 *__restrict__ b_
         if (e < t.e1) {
             r = t.r0 + t.row(b_rpt, srpt, e);
             const u32 c = b_cols[e];
-            w = c >> 5;
+            w = c >> 4;
             row_start = b_rpt[r] == e;
-            starts = row_start || (b_cols[e - 1] >> 5) != w;
+            starts = row_start || (b_cols[e - 1] >> 4) != w;
             if (starts) {
-                mask = 1u << (c & 31u);
+                mask = 1u << (c & 15u);
                 const u32 end = b_rpt[r + 1];
                 for (u64 k = e + 1; k < end; ++k) {
                     const u32 x = b_cols[k];
-                    if ((x >> 5) != w) break;
-                    mask |= 1u << (x & 31u);
+                    if ((x >> 4) != w) break;
+                    mask |= 1u << (x & 15u);
                 }
             }
         }
@@ -135,7 +136,8 @@ __global__ __launch_bounds__(EX_WG) void k_pack_place(const u32 *__restrict__ b_
         __syncthreads();
         if (starts) {
             const u32 p = at + before + dev::lanes_below(m);
-            pairs[p] = make_uint2(w, mask);
+            packs[p] = (w << 16) | mask;
+            if (pfirst) pfirst[p] = (u32)e;
             if (row_start) prpt[r] = p;
         }
         at += all;
@@ -143,28 +145,30 @@ __global__ __launch_bounds__(EX_WG) void k_pack_place(const u32 *__restrict__ b_
     if (blockIdx.x + 1 == gridDim.x && threadIdx.x == 0) prpt[b_nzr] = at;
 }
 
-// Mats::psplits: as k_slice_splits, over pairs (words, slices of span words).
-__global__ void k_pair_splits(const u32 *__restrict__ prpt, const u32 *__restrict__ b_rows,
-                              const uint2 *__restrict__ pairs, u32 b_nzr, u32 mapn, u32 nsl, u32 span,
-                              u32 *__restrict__ splits) {
+// Mats::psplits from Mats::splits: slices begin at multiples of 16 columns, so
+// the pack that a slice begins with has the slice's first column first.
+__global__ void k_pack_splits(const u32 *__restrict__ prpt, const u32 *__restrict__ b_rows,
+                              const u32 *__restrict__ pfirst, const u32 *__restrict__ splits, u32 b_nzr, u32 mapn,
+                              u32 nsl, u32 *__restrict__ psplits) {
     const u32 i = blockIdx.x * blockDim.x + threadIdx.x;
     if (i >= b_nzr) return;
     const u32 k = b_rows[i];
     if (k >= mapn) return;
-    const u32 beg = prpt[i], end = prpt[i + 1];
-    u32 *out = splits + (u64)k * (nsl + 1);
-    u32 lo = beg;
-    out[0] = beg;
+    const u32 end = prpt[i + 1];
+    const u64 at = (u64)k * (nsl + 1);
+    u32 lo = prpt[i];
+    psplits[at] = lo;
     for (u32 s = 1; s < nsl; ++s) {
+        const u32 e = splits[at + s];
         u32 hi = end;
         while (lo < hi) {
             const u32 mid = lo + (hi - lo) / 2;
-            if (pairs[mid].x < s * span) lo = mid + 1;
+            if (pfirst[mid] < e) lo = mid + 1;
             else hi = mid;
         }
-        out[s] = lo;
+        psplits[at + s] = lo;
     }
-    out[nsl] = end;
+    psplits[at + nsl] = end;
 }
 
 __global__ void k_brange_set(const u32 *__restrict__ b_rpt, const u32 *__restrict__ b_rows, u32 b_nzr, u32 mapn,
@@ -888,13 +892,15 @@ void ensure_splits(clb_controls_s *ctl, Setup &s, const BinHost &h) {
 
 // Packs B for the bitmap kernels when their rows will read it often enough.
 void ensure_packed(clb_controls_s *ctl, Setup &s, const BinHost &h) {
-    if (s.g.b_pairs || s.pack_tried || s.g.combine || ctl->tuning.bitmap_persistent) return;
+    if (s.g.b_packs || s.pack_tried || s.g.combine || ctl->tuning.bitmap_persistent) return;
     u64 products = 0;
     for (u32 b = BIN_BITMAP0; b < NBINS; ++b) products += h.products[b];
     const clb_dcsr &b = s.b;
     if (!b.nzr || !b.nnz || products < (u64)PACK_MIN_READS * b.nnz || products < PACK_MIN_PRODUCTS)
         return;
     s.pack_tried = true;
+    // a pack's group is known modulo 2^20 columns: wider matrices need slices
+    if (b.ncols > (1u << 20) && !s.g.splits) return;
     const u32 tiles = div_up(b.nnz, EX_TILE);
     DevArray<u32> first(ctl, tiles), offs(ctl, (u64)tiles + 1);
     k_tile_rows<EX_TILE><<<div_up(b.nzr, EX_WG), EX_WG, 0, ctl->stream>>>(u32p(b.rpt), 0, b.nzr, 0, b.nnz, first.ptr);
@@ -902,14 +908,15 @@ void ensure_packed(clb_controls_s *ctl, Setup &s, const BinHost &h) {
     k_pack_count<<<tiles, EX_WG, 0, ctl->stream>>>(u32p(b.rpt), u32p(b.cols), b.nzr, b.nnz, first.ptr, offs.ptr);
     CLB_LAUNCHED("pack_count");
     exclusive_scan_u32(ctl, offs.ptr, offs.ptr, tiles, offs.ptr + tiles);
-    u32 npairs = 0;
-    readback(ctl, &npairs, offs.ptr + tiles, 4);
-    if ((u64)npairs * 100 > (u64)b.nnz * PACK_MAX_PCT) return;
-    s.pairs.reset(ctl, npairs);
+    u32 npacks = 0;
+    readback(ctl, &npacks, offs.ptr + tiles, 4);
+    if ((u64)npacks * 100 > (u64)b.nnz * PACK_MAX_PCT) return;
+    s.packs.reset(ctl, npacks);
+    DevArray<u32> pfirst(ctl, s.g.splits ? npacks : 0);
     s.prange.reset(ctl, s.mapn);
     DevArray<u32> prpt(ctl, (u64)b.nzr + 1);
     k_pack_place<<<tiles, EX_WG, 0, ctl->stream>>>(u32p(b.rpt), u32p(b.cols), b.nzr, b.nnz, first.ptr, offs.ptr,
-                                                   prpt.ptr, s.pairs.ptr);
+                                                   prpt.ptr, s.packs.ptr, pfirst.ptr);
     CLB_LAUNCHED("pack_place");
     if (!s.g.bpres) fill_u64(ctl, reinterpret_cast<u64 *>(s.prange.ptr), s.mapn, 0ull);
     k_brange_set<<<div_up(b.nzr, 256), 256, 0, ctl->stream>>>(prpt.ptr, u32p(b.rows), b.nzr, s.mapn, s.prange.ptr,
@@ -918,11 +925,11 @@ void ensure_packed(clb_controls_s *ctl, Setup &s, const BinHost &h) {
     if (s.g.splits) {
         s.psplits.reset(ctl, s.splits.n);
         fill_u32(ctl, s.psplits.ptr, s.psplits.n, 0u);
-        k_pair_splits<<<div_up(b.nzr, 256), 256, 0, ctl->stream>>>(prpt.ptr, u32p(b.rows), s.pairs.ptr, b.nzr, s.mapn,
-                                                                    s.g.nsl, 1u << s.g.split_bits, s.psplits.ptr);
-        CLB_LAUNCHED("pair_splits");
+        k_pack_splits<<<div_up(b.nzr, 256), 256, 0, ctl->stream>>>(prpt.ptr, u32p(b.rows), pfirst.ptr, s.g.splits,
+                                                                    b.nzr, s.mapn, s.g.nsl, s.psplits.ptr);
+        CLB_LAUNCHED("pack_splits");
     }
-    s.g.b_pairs = s.pairs.ptr;
+    s.g.b_packs = s.packs.ptr;
     s.g.prange = s.prange.ptr;
     s.g.psplits = s.g.splits ? s.psplits.ptr : nullptr;
 }
@@ -959,7 +966,7 @@ void prepare(clb_controls_s *ctl, const clb_dcsr &a, const clb_dcsr &b, u32 row_
         s.g.combine = ctl->tuning.reserved[CLB_TUNE_GATHER_COMBINE];
         s.cfg = make_bincfg(ctl, b.ncols);
         s.g.splits = nullptr;
-        s.g.b_pairs = nullptr;
+        s.g.b_packs = nullptr;
         s.g.prange = nullptr;
         s.g.psplits = nullptr;
         s.pack_tried = false;

@@ -17,7 +17,8 @@ struct Setup {
     DevArray<u64> scal;
     DevArray<u32> ctr;  // row counters of persistent launches (zeroed per launch)
     DevArray<u32> splits;  // per-slice B row ranges (Mats::splits) when ncols spans several windows
-    DevArray<uint2> pairs, prange;  // packed B (Mats::b_pairs)
+    DevArray<u32> packs;  // packed B (Mats::b_packs)
+    DevArray<uint2> prange;
     DevArray<u32> psplits;
     bool pack_tried = false;
     Mats g{};
@@ -115,17 +116,19 @@ void emit_launch(hipStream_t es, u32 count, const u32 *perm, const BinHost &h, c
 
 BinCfg make_bincfg(const clb_controls_s *ctl, u32 ncols);
 void ensure_splits(clb_controls_s *ctl, Setup &s, const BinHost &h);
-// B packed by words (Mats::b_pairs) for the bitmap rows of `h`, after
-// ensure_splits.  Packing costs two passes over B, so it needs rows that read
-// B often; and a pair takes twice a column's bytes, so it needs columns that
-// share words.  Measured packed against not (ms): R-MAT 2^16 x 16, plain 1.10
-// / 1.20; 2^18, plain blocks 6.77 / 7.76; 2^20, one pass 42.9 / 47.7; uniform
-// 100 per row of 10^5 columns (98 pairs per 100) 4.83 / 4.92, 600 per row of
-// 10^6 (99) 3.51 / 3.14; R-MAT 20000 vertices, 160000 edges 0.400 / 0.423;
-// uniform 1024 x 1024 with 98 thousand products 0.37 / 0.32.
-constexpr u64 PACK_MIN_PRODUCTS = 1ull << 22;  // launches and one read-back below it
+// B packed by groups of 16 columns (Mats::b_packs) for the bitmap rows of `h`,
+// after ensure_splits.  Packing costs two passes over B and a read-back, so it
+// needs rows that read B often, and columns that share groups: a pack is as
+// long as a column index.  Measured packed against not (ms; packs per 100
+// nonzeros where they decide): R-MAT 2^16 x 16, plain 0.97 / 1.07; 2^18, plain
+// blocks 5.89 / 6.75; 2^20, one pass 41.2 / 46.3; uniform 100 per row of 10^5
+// columns (99) 4.30 / 4.43, 600 per row of 10^6 (99) 3.16 / 3.04, 100 per row
+// of 20000 (96) 0.77 / 0.79; below 2^24 products the passes cost more than
+// they save: R-MAT 20000 vertices, 160000 edges 0.328 / 0.318, uniform 60 per
+// row of 3000 0.284 / 0.264.
+constexpr u64 PACK_MIN_PRODUCTS = 1ull << 24;
 constexpr u32 PACK_MIN_READS = 8;  // products of the bitmap rows per nonzero of B
-constexpr u32 PACK_MAX_PCT = 95;   // pairs per 100 nonzeros of B
+constexpr u32 PACK_MAX_PCT = 95;   // packs per 100 nonzeros of B
 void ensure_packed(clb_controls_s *ctl, Setup &s, const BinHost &h);
 // B row map, kernel arguments and (stats) per-row products, with `feat` also
 // the other statistics.  With `shared`, the B row map, split table and bin

@@ -41,6 +41,10 @@ constexpr u32 BIN_STORED = 13;
 constexpr u32 BIN_BITMAP0 = 14;  // 14 + (30 - floor(log2 P)), clamped to 14..31
 constexpr u32 BIG_ROW = 256;     // B rows at least this long are shared by the workgroup
 constexpr u32 LONG_ROW = 64;     // B rows at least this long are shared by a wave
+// Loads per buffer of the packed gather over windows below 2^14 words, where
+// registers decide the waves of a CU: 8 is no faster (5.94 against 5.92 ms for
+// the plain blocks of R-MAT 2^18 x 16).
+constexpr int PACK_UB = 4;
 
 struct Mats {
     const u32 *a_rpt;
@@ -69,14 +73,17 @@ struct Mats {
     // nullptr: brange is complete.
     const u32 *bpres;
     // Packed B (bitmap kernels only; nullptr: not built): each stored row as
-    // (word, mask) pairs, word = column / 32 ascending and mask = the row's
-    // columns in that word; prange and psplits are brange and splits in pairs.
-    const uint2 *b_pairs;
+    // packs, one per 16 columns that hold any of its entries, ascending: the
+    // low half has the entries' bits, the high half the columns' group, column
+    // / 16, modulo 2^16 (a window spans at most 2^16 groups and begins at a
+    // multiple of its width).  prange and psplits are brange and splits in
+    // packs.
+    const u32 *b_packs;
     const uint2 *prange;
     const u32 *psplits;
 };
 
-// [begin, end) of B row k in b_cols (PACK: in b_pairs), {0, 0} for absent rows.
+// [begin, end) of B row k in b_cols (PACK: in b_packs), {0, 0} for absent rows.
 template <bool PACK = false>
 __device__ __forceinline__ uint2 b_range(const Mats &g, u32 k) {
     if (k >= g.mapn) return make_uint2(0, 0);
@@ -193,29 +200,13 @@ constexpr u32 bitmap_bin_below(u32 lp) { return BIN_BITMAP0 + (31 - lp); }
 constexpr int UNROLL = 4;
 __host__ __device__ constexpr int BIG_WORDS(int WG) { return 3 * WG + 2 * (WG / 64 + 2); }
 
-// PACK: over the packed B rows instead; f and ff take a (word, mask) pair.
-template <bool PACK>
-struct BElem {
-    using T = u32;
-    static __device__ __forceinline__ const T *base(const Mats &g) { return g.b_cols; }
-    static __device__ __forceinline__ T none() { return EMPTY; }
-    static __device__ __forceinline__ bool some(T v) { return v != EMPTY; }
-};
-template <>
-struct BElem<true> {
-    using T = uint2;
-    static __device__ __forceinline__ const T *base(const Mats &g) { return g.b_pairs; }
-    static __device__ __forceinline__ T none() { return make_uint2(0u, 0u); }
-    static __device__ __forceinline__ bool some(T v) { return v.y != 0u; }  // a pair's mask is not empty
-};
-
+// PACK: over the packed B rows instead; f and ff take a pack.
 template <int WG, int UB, u32 BIGMIN, bool AHEAD = false, bool PACK = false, typename F, typename FF>
 __device__ __forceinline__ void for_each_product(const Mats &g, u32 js, u32 je, u32 *big, F &&f, FF &&ff,
                                                  u32 slice = NOSLICE, u32 sstep = 1, RowAhead *ah = nullptr,
                                                  u32 next_slice = NOSLICE) {
-    using B = BElem<PACK>;
-    using T = typename B::T;
-    const T *const bsrc = B::base(g);
+    const u32 *const bsrc = PACK ? g.b_packs : g.b_cols;
+    constexpr u32 NONE = PACK ? 0u : EMPTY;  // a pack has some bit set
     const int l = dev::lane();
     constexpr int NW = WG / dev::WAVE;
     constexpr u32 WIN = UB * 64;
@@ -277,15 +268,15 @@ __device__ __forceinline__ void for_each_product(const Mats &g, u32 js, u32 je, 
             const u32 sb = __shfl(bx, s, dev::WAVE);
             const u32 sl = __shfl(len, s, dev::WAVE);
             for (u32 q = l; q < sl; q += UNROLL * dev::WAVE) {
-                T c[UNROLL];
+                u32 c[UNROLL];
 #pragma unroll
                 for (int u = 0; u < UNROLL; ++u) {
                     const u32 qq = q + u * dev::WAVE;
-                    c[u] = qq < sl ? bsrc[sb + qq] : B::none();
+                    c[u] = qq < sl ? bsrc[sb + qq] : NONE;
                 }
 #pragma unroll
                 for (int u = 0; u < UNROLL; ++u)
-                    if (B::some(c[u])) f(c[u]);
+                    if (c[u] != NONE) f(c[u]);
             }
         }
         // lane expansion of short rows
@@ -294,7 +285,7 @@ __device__ __forceinline__ void for_each_product(const Mats &g, u32 js, u32 je, 
         const u32 wtot = __shfl(inc, dev::WAVE - 1, dev::WAVE);
         const u32 exc = inc - sl;
         for (u32 p0 = 0; p0 < wtot; p0 += UNROLL * dev::WAVE) {
-            T c[UNROLL];
+            u32 c[UNROLL];
 #pragma unroll
             for (int u = 0; u < UNROLL; ++u) {
                 const u32 p = p0 + u * dev::WAVE + l;
@@ -309,11 +300,11 @@ __device__ __forceinline__ void for_each_product(const Mats &g, u32 js, u32 je, 
                     }
                 }
                 const u32 sb = __shfl(bx, s, dev::WAVE);
-                c[u] = p < wtot ? bsrc[sb + (p - es)] : B::none();
+                c[u] = p < wtot ? bsrc[sb + (p - es)] : NONE;
             }
 #pragma unroll
             for (int u = 0; u < UNROLL; ++u)
-                if (B::some(c[u])) f(c[u]);
+                if (c[u] != NONE) f(c[u]);
         }
         if (NW > 1 && nb) {
             __syncthreads();  // the list is complete
@@ -339,7 +330,7 @@ __device__ __forceinline__ void for_each_product(const Mats &g, u32 js, u32 je, 
             // flight the compiler waits for one buffer only while the other
             // buffer's loads are still outstanding, instead of draining all
             // loads before each apply.
-            auto fetch = [&](u32 k, T(&c)[UB]) -> u32 {
+            auto fetch = [&](u32 k, u32(&c)[UB]) -> u32 {
                 u32 start = eb, n = 0;
                 if (k < nwin) {
                     while (k >= next) {
@@ -354,7 +345,7 @@ __device__ __forceinline__ void for_each_product(const Mats &g, u32 js, u32 je, 
                     start = eb + (k - pre) * WIN;
                     n = ee - start < WIN ? ee - start : WIN;
                 }
-                const T *src = bsrc + start;
+                const u32 *src = bsrc + start;
                 const u32 last = n ? n - 1 : 0u;  // entries hold at least one column
 #pragma unroll
                 for (int u = 0; u < UB; ++u) {
@@ -363,7 +354,7 @@ __device__ __forceinline__ void for_each_product(const Mats &g, u32 js, u32 je, 
                 }
                 return n;
             };
-            auto apply = [&](const T(&c)[UB], u32 n) {
+            auto apply = [&](const u32(&c)[UB], u32 n) {
                 if (n == WIN) {
                     // all 64 lanes hold consecutive columns of one B row
 #pragma unroll
@@ -374,7 +365,7 @@ __device__ __forceinline__ void for_each_product(const Mats &g, u32 js, u32 je, 
                         if ((u32)(u * 64 + l) < n) f(c[u]);
                 }
             };
-            T ca[UB], cb[UB];
+            u32 ca[UB], cb[UB];
             u32 na = fetch(w, ca), nb2 = 0;
             for (u32 k = w; k < nwin; k += 2 * NW) {
                 nb2 = fetch(k + NW, cb);
@@ -470,7 +461,10 @@ struct Store {
 __host__ __device__ constexpr u32 store_chunk(u32 win_words) {
     return win_words < EMIT_CHUNK ? win_words : EMIT_CHUNK;
 }
-constexpr u32 STORE_PAIR_WORDS = 1u << 13;  // narrower windows are kept as words
+// Narrower windows are kept as words.  The pair path at 2^13 words takes the
+// symbolic kernel from 55 to 81 VGPRs, from 7 to 5 waves a SIMD (2.06 against
+// 2.58 ms for R-MAT 2^18 x 16).
+constexpr u32 STORE_PAIR_WORDS = 1u << 14;
 
 struct Out {
     u32 *nnz_row;
@@ -767,6 +761,7 @@ __device__ __forceinline__ void keep_slice(const Store &k, u32 slot, u32 s, u32 
     if constexpr (W < STORE_PAIR_WORDS) {
         uint4 *dst = k.words + sl * (W / 4);
         const uint4 *src = reinterpret_cast<const uint4 *>(bm);
+#pragma unroll 2
         for (u32 t = threadIdx.x; t < W / 4; t += WG) dst[t] = src[t];
         __syncthreads();
         if (threadIdx.x == 0) k.fmt[sl] = 0u;
@@ -812,8 +807,8 @@ __device__ __forceinline__ void keep_slice(const Store &k, u32 slot, u32 s, u32 
     __syncthreads();  // before the next slice clears the bitmap and the list
 }
 
-// PACK: the gather reads packed B rows (Mats::b_pairs), one LDS atomic per
-// word of a B row.
+// PACK: the gather reads packed B rows (Mats::b_packs), one LDS atomic per 16
+// columns of a B row.
 template <int WBITS, int WG, int MODE, bool COMB, bool PACK>
 __device__ __forceinline__ void bitmap_row(const Mats &g, const u32 *__restrict__ perm, u32 idx, const Out &o,
                                            u32 *bm, u32 *big, u32 *red) {
@@ -861,15 +856,16 @@ __device__ __forceinline__ void bitmap_row(const Mats &g, const u32 *__restrict_
         // no range check (base < 2^32 and a multiple of 32)
         auto setu = [&](u32 col) { atomicOr(&bm[(col - (u32)base) >> 5], 1u << (col & 31)); };
         auto setdw = [&](u32 col) { dev::wave_or_sorted_bits(bm, (u32)((u64)col - base)); };
-        // a packed element is two registers: 8 of them in flight per buffer,
-        // and 4 where registers and not LDS limit the waves of a CU
-        constexpr int UBW = PACK && WBITS < 14 ? 4 : 8;
+        constexpr int UBW = PACK && WBITS < 14 ? PACK_UB : 8;
         if constexpr (PACK) {
-            const u32 w0 = (u32)(base >> 5);
-            auto setp = [&](uint2 p) { atomicOr(&bm[p.x - w0], p.y); };
-            auto setq = [&](uint2 p) {
-                const u32 d = p.x - w0;  // wraps below the window
-                if (d < W) atomicOr(&bm[d], p.y);
+            const u32 g0 = (u32)(base >> 4) & 0xFFFFu;  // the window's first group
+            auto setp = [&](u32 p) {
+                const u32 d = (p >> 16) - g0;
+                atomicOr(&bm[d >> 1], (p & 0xFFFFu) << ((d & 1u) * 16u));
+            };
+            auto setq = [&](u32 p) {
+                const u32 d = (p >> 16) - g0;  // wraps below the window
+                if (d < 2u * W) atomicOr(&bm[d >> 1], (p & 0xFFFFu) << ((d & 1u) * 16u));
             };
             if (nslices == 1) for_each_product<WG, UBW, LONG_ROW, AH, true>(g, js, je, big, setp);
             else if (use_splits) for_each_product<WG, UBW, LONG_ROW, AH, true>(g, js, je, big, setp, s, sstep, &ah, sn);
@@ -893,6 +889,7 @@ __device__ __forceinline__ void bitmap_row(const Mats &g, const u32 *__restrict_
             if constexpr (KEEP) keep_slice<WBITS, WG>(o.keep, idx, s, nslices, bm, red, big, mine);
         } else if (MODE == SYM) {
             const uint4 *bm4 = reinterpret_cast<const uint4 *>(bm);
+#pragma unroll 1
             for (u32 t = threadIdx.x; t < W / 4; t += WG) {
                 const uint4 v = bm4[t];
                 mine += __popc(v.x) + __popc(v.y) + __popc(v.z) + __popc(v.w);

@@ -74,3 +74,24 @@ def test_heavy_rows(controls, hubs):
     a = upload(controls, A, n, n)
     assert_dcsr_equal(controls, cb.dcsr.matrix_multiplication_hash(controls, a, a), ref, "plain")
     assert_dcsr_equal(controls, cb.dcsr.spgemm(controls, a, a, mode=cb.SPGEMM_BOUND)[0], ref, "bound")
+
+
+@pytest.mark.parametrize("ncols", [4097, 16385, 65537, 1048575, 1048577, 1100000])
+def test_packed(controls, ncols):
+    """Enough products for B to be packed: B rows of about every second column
+    of a range, with group 65535 and 0 modulo 65536 where there are so many."""
+    rng = np.random.default_rng(ncols)
+    inner, nrows = 40, 600
+    br, bc = [], []
+    for k in range(inner):
+        n = int(min(ncols, rng.integers(3000, 9000)))
+        start = int(rng.integers(0, ncols - n + 1)) if k % 4 else ncols - n
+        c = start + np.flatnonzero(rng.random(n) < 0.6)
+        br.append(np.full(c.size, k))
+        bc.append(c)
+    A = _dcsr(np.repeat(np.arange(nrows), 20), rng.integers(0, inner, nrows * 20), nrows, inner)
+    B = _dcsr(np.concatenate(br), np.concatenate(bc), inner, ncols)
+    ref = oracle.spgemm(A, B)
+    a, b = upload(controls, A, nrows, inner), upload(controls, B, inner, ncols)
+    assert_dcsr_equal(controls, cb.dcsr.matrix_multiplication_hash(controls, a, b), ref, "plain")
+    assert_dcsr_equal(controls, cb.dcsr.spgemm(controls, a, b, mode=cb.SPGEMM_BOUND)[0], ref, "bound")
