@@ -63,7 +63,7 @@ __global__ void k_features(Mats g, u32 nrows, const u32 *__restrict__ prod, cons
     const u32 span = p ? lc[row] - fc[row] + 1 : 0;
     float *f = feat + (u64)row * NF;
     f[0] = flog(p);
-    f[1] = flog(g.a_rpt[i + 1] - g.a_rpt[i]);
+    f[1] = flog(g.a_all[i + 1] - g.a_all[i]);
     f[2] = flog(p ? mn[row] : 0);
     f[3] = flog(mx[row]);
     f[4] = flog(span);

@@ -19,29 +19,29 @@ namespace clb {
 namespace spg {
 
 // Mats::splits of B: for each stored row, the start of each column slice of
-// SPAN columns (lower bounds in the sorted row) and its end.
+// `span` columns (lower bounds in the sorted row) and its end.  A thread per
+// entry: one per row walked its slices' searches one after the other (150 us
+// for 168 thousand rows of 16 slices, 22 us now).  b_rows == nullptr: the
+// table is by stored row.
 __global__ void k_slice_splits(const u32 *__restrict__ b_rpt, const u32 *__restrict__ b_rows,
                                const u32 *__restrict__ b_cols, u32 b_nzr, u32 mapn, u32 nsl, u64 span,
                                u32 *__restrict__ splits) {
-    const u32 i = blockIdx.x * blockDim.x + threadIdx.x;
-    if (i >= b_nzr) return;
-    const u32 k = b_rows[i];
+    const u64 t = (u64)blockIdx.x * blockDim.x + threadIdx.x;
+    if (t >= (u64)b_nzr * (nsl + 1)) return;  // below 2^32: the table is
+    const u32 i = (u32)t / (nsl + 1), s = (u32)t - i * (nsl + 1);
+    const u32 k = b_rows ? b_rows[i] : i;
     if (k >= mapn) return;
-    const u32 beg = b_rpt[i], end = b_rpt[i + 1];
-    u32 *out = splits + (u64)k * (nsl + 1);
-    u32 lo = beg;
-    out[0] = beg;
-    for (u32 s = 1; s < nsl; ++s) {
-        const u64 bound = (u64)s * span;
-        u32 hi = end;
-        while (lo < hi) {  // first column >= bound, searching on from the previous slice
-            const u32 mid = lo + (hi - lo) / 2;
-            if ((u64)b_cols[mid] < bound) lo = mid + 1;
-            else hi = mid;
-        }
-        out[s] = lo;
+    u32 lo = b_rpt[i];
+    const u32 end = b_rpt[i + 1];
+    const u64 bound = (u64)s * span;
+    u32 hi = s ? end : lo;
+    if (s == nsl) lo = end;
+    while (lo < hi) {  // first column >= bound
+        const u32 mid = lo + (hi - lo) / 2;
+        if ((u64)b_cols[mid] < bound) lo = mid + 1;
+        else hi = mid;
     }
-    out[nsl] = end;
+    splits[(u64)k * (nsl + 1) + s] = lo;
 }
 
 // Packed B (Mats::b_packs): a pack begins at every column that starts a row or
@@ -152,7 +152,7 @@ __global__ void k_pack_splits(const u32 *__restrict__ prpt, const u32 *__restric
                               u32 nsl, u32 *__restrict__ psplits) {
     const u32 i = blockIdx.x * blockDim.x + threadIdx.x;
     if (i >= b_nzr) return;
-    const u32 k = b_rows[i];
+    const u32 k = b_rows ? b_rows[i] : i;
     if (k >= mapn) return;
     const u32 end = prpt[i + 1];
     const u64 at = (u64)k * (nsl + 1);
@@ -171,13 +171,19 @@ __global__ void k_pack_splits(const u32 *__restrict__ prpt, const u32 *__restric
     psplits[at + nsl] = end;
 }
 
+// brange by row id (b_rows == nullptr: by stored row); for a filtered A also
+// the stored row of each id (bidx) and the ranges by stored row (crange).
 __global__ void k_brange_set(const u32 *__restrict__ b_rpt, const u32 *__restrict__ b_rows, u32 b_nzr, u32 mapn,
-                             uint2 *__restrict__ brange, u32 *__restrict__ bpres) {
+                             uint2 *__restrict__ brange, u32 *__restrict__ bpres, u32 *__restrict__ bidx,
+                             uint2 *__restrict__ crange) {
     const u32 i = blockIdx.x * blockDim.x + threadIdx.x;
     if (i >= b_nzr) return;
-    const u32 r = b_rows[i];
+    const uint2 range = make_uint2(b_rpt[i], b_rpt[i + 1]);
+    if (crange) crange[i] = range;
+    const u32 r = b_rows ? b_rows[i] : i;
     if (r >= mapn) return;
-    brange[r] = make_uint2(b_rpt[i], b_rpt[i + 1]);
+    brange[r] = range;
+    if (bidx) bidx[r] = i;
     if (bpres) atomicOr(&bpres[r >> 5], 1u << (r & 31));
 }
 
@@ -193,25 +199,32 @@ __global__ void k_brange_set(const u32 *__restrict__ b_rpt, const u32 *__restric
 //   prod[r] = products (border rows must start at 0);
 //   FEAT: also mn/mx (min/max B-row length, border rows start at ~0 / 0) and
 //   fc/lc (first column of any of its B rows / last column, ~0 / 0).
+// With fmask also a bit per nonzero, set if its B row has entries, and each
+// tile's number of them (for k_filter).
 constexpr u32 RSTAT_WG = 256;
 template <bool FEAT>
 constexpr u32 rstat_tile() { return RSTAT_WG * (FEAT ? 4 : 8); }
 template <bool FEAT>
 __global__ __launch_bounds__(RSTAT_WG) void k_row_stats(Mats g, u32 nrows, const u32 *__restrict__ first,
-                                                        u32 *__restrict__ prod, RowFeat o) {
+                                                        u32 *__restrict__ prod, RowFeat o,
+                                                        u32 *__restrict__ fmask, u32 *__restrict__ fcount) {
     constexpr u32 TILE = rstat_tile<FEAT>(), ITEMS = TILE / RSTAT_WG;
+    __shared__ u32 red[RSTAT_WG / dev::WAVE + 1];
     __shared__ u32 rs[TILE + 1], sp[TILE];
     __shared__ u32 smn[FEAT ? TILE : 1], smx[FEAT ? TILE : 1], sfc[FEAT ? TILE : 1], slc[FEAT ? TILE : 1];
     const u32 rend = g.row0 + nrows;
-    const u32 jbase = g.a_rpt[g.row0], jend = g.a_rpt[rend];
+    const u32 jbase = g.a_all[g.row0], jend = g.a_all[rend];
     const u64 j0 = (u64)jbase + (u64)blockIdx.x * TILE;
-    if (j0 >= jend) return;  // uniform: the grid covers all of A's nonzeros
+    if (j0 >= jend) {  // uniform: the grid covers all of A's nonzeros
+        if (fmask && threadIdx.x == 0) fcount[blockIdx.x] = 0;
+        return;
+    }
     const u64 j1 = j0 + TILE < jend ? j0 + TILE : jend;
     const u32 r0 = first[blockIdx.x];
     const u32 nr = (j1 < jend ? first[blockIdx.x + 1] : rend - 1) - r0 + 1;
     const bool staged = nr <= TILE;  // else: some stored rows are empty
     if (staged) {
-        for (u32 t = threadIdx.x; t <= nr; t += RSTAT_WG) rs[t] = g.a_rpt[r0 + t];
+        for (u32 t = threadIdx.x; t <= nr; t += RSTAT_WG) rs[t] = g.a_all[r0 + t];
         for (u32 t = threadIdx.x; t < nr; t += RSTAT_WG) {
             sp[t] = 0;
             if (FEAT) {
@@ -222,11 +235,14 @@ __global__ __launch_bounds__(RSTAT_WG) void k_row_stats(Mats g, u32 nrows, const
     }
     __syncthreads();
     const u64 js = j0 + (u64)threadIdx.x * ITEMS;
+    u32 bits = 0;  // this thread's nonzeros with a B row
     if (js < j1) {
         uint2 b[ITEMS];
         u32 c0[ITEMS], c1[ITEMS];
 #pragma unroll
         for (u32 k = 0; k < ITEMS; ++k) b[k] = js + k < j1 ? b_range(g, g.a_cols[js + k]) : make_uint2(0u, 0u);
+#pragma unroll
+        for (u32 k = 0; k < ITEMS; ++k) bits |= (b[k].y > b[k].x ? 1u : 0u) << k;
         if (FEAT) {
 #pragma unroll
             for (u32 k = 0; k < ITEMS; ++k) {
@@ -237,7 +253,7 @@ __global__ __launch_bounds__(RSTAT_WG) void k_row_stats(Mats g, u32 nrows, const
         u32 lo = 0, hi = nr;  // the last row that starts at or before js
         while (hi - lo > 1) {
             const u32 mid = lo + (hi - lo) / 2;
-            if ((staged ? rs[mid] : g.a_rpt[r0 + mid]) <= js) lo = mid;
+            if ((staged ? rs[mid] : g.a_all[r0 + mid]) <= js) lo = mid;
             else hi = mid;
         }
         u32 sum = 0, n0 = 0xFFFFFFFFu, n1 = 0, f0 = 0xFFFFFFFFu, f1 = 0;
@@ -259,7 +275,7 @@ __global__ __launch_bounds__(RSTAT_WG) void k_row_stats(Mats g, u32 nrows, const
 #pragma unroll
         for (u32 k = 0; k < ITEMS; ++k) {
             if (js + k >= j1) break;
-            while ((staged ? rs[lo + 1] : g.a_rpt[r0 + lo + 1]) <= js + k) {
+            while ((staged ? rs[lo + 1] : g.a_all[r0 + lo + 1]) <= js + k) {
                 flush();
                 ++lo;
             }
@@ -273,6 +289,15 @@ __global__ __launch_bounds__(RSTAT_WG) void k_row_stats(Mats g, u32 nrows, const
             }
         }
         flush();
+    }
+    if (fmask) {  // uniform
+        constexpr u32 PER = 32 / ITEMS;  // threads of a word
+        u32 w = bits << (threadIdx.x % PER * ITEMS);
+#pragma unroll
+        for (u32 d = 1; d < PER; d <<= 1) w |= __shfl_xor(w, d, dev::WAVE);
+        if (threadIdx.x % PER == 0) fmask[(u64)blockIdx.x * (TILE / 32) + threadIdx.x / PER] = w;
+        const u32 sum = dev::block_sum<u32, RSTAT_WG>((u32)__popc(bits), red);
+        if (threadIdx.x == 0) fcount[blockIdx.x] = sum;
     }
     __syncthreads();
     if (!staged) return;
@@ -295,6 +320,46 @@ __global__ __launch_bounds__(RSTAT_WG) void k_row_stats(Mats g, u32 nrows, const
                 atomicMax(&o.lc[row], slc[t]);
             }
         }
+    }
+}
+
+// A without the nonzeros whose B row is absent or empty, its columns renumbered
+// to B's stored rows: the first `tiles` workgroups place the columns of a tile
+// of k_row_stats each, the others the row pointers.
+template <u32 TILE>
+__global__ __launch_bounds__(256) void k_filter(Mats g, u32 nrows, u32 tiles, const u32 *__restrict__ fmask,
+                                                const u32 *__restrict__ offs, const u32 *__restrict__ bidx,
+                                                u32 *__restrict__ f_rpt, u32 *__restrict__ f_cols) {
+    constexpr u32 W = TILE / 32;
+    static_assert(W <= dev::WAVE, "one wave scans a tile's words");
+    const u32 jbase = g.a_all[g.row0];
+    if (blockIdx.x >= tiles) {
+        const u64 r = (u64)(blockIdx.x - tiles) * 256 + threadIdx.x;
+        if (r > nrows) return;
+        const u32 e = g.a_all[g.row0 + r] - jbase, t = e / TILE;
+        u32 n = offs[t];  // offs[tiles]: all of them
+        const u32 *m = fmask + (u64)t * W;
+        for (u32 q = 0; q < e % TILE / 32; ++q) n += (u32)__popc(m[q]);
+        if (e % 32) n += (u32)__popc(m[e % TILE / 32] & ((1u << e % 32) - 1u));
+        f_rpt[r] = n;
+        return;
+    }
+    const u64 n = (u64)g.a_all[g.row0 + nrows] - jbase, e0 = (u64)blockIdx.x * TILE;
+    if (e0 >= n) return;
+    __shared__ u32 sw[W], sp[W];
+    if (threadIdx.x < dev::WAVE) {
+        const u32 w = threadIdx.x < W ? fmask[(u64)blockIdx.x * W + threadIdx.x] : 0u;
+        const u32 c = (u32)__popc(w), inc = dev::wave_incl_scan(c);
+        if (threadIdx.x < W) {
+            sw[threadIdx.x] = w;
+            sp[threadIdx.x] = offs[blockIdx.x] + inc - c;
+        }
+    }
+    __syncthreads();
+#pragma unroll
+    for (u32 q = 0; q < TILE / 256; ++q) {
+        const u32 e = q * 256 + threadIdx.x, w = sw[e / 32], bit = 1u << e % 32;
+        if (w & bit) f_cols[sp[e / 32] + (u32)__popc(w & (bit - 1u))] = bidx[g.a_cols[(u64)jbase + e0 + e]];
     }
 }
 
@@ -356,7 +421,7 @@ __global__ __launch_bounds__(BIN_WG) void k_bin_count(Mats g, const u32 *__restr
         const u32 b = bin_of((u32)i, P, key, c, slot_of, p, k);
         atomicAdd(&h[b], 1u);
         if (p) atomicAdd(&hs[0][b], (unsigned long long)p);
-        atomicAdd(&hs[1][b], (unsigned long long)(g.a_rpt[g.row0 + i + 1] - g.a_rpt[g.row0 + i]));
+        atomicAdd(&hs[1][b], (unsigned long long)(g.a_all[g.row0 + i + 1] - g.a_all[g.row0 + i]));
         if (key && k) atomicAdd(&hs[2][b], (unsigned long long)k);
         if (b == BIN_EMPTY && nnz_row) nnz_row[i] = 0;
     }
@@ -871,20 +936,52 @@ BinCfg make_bincfg(const clb_controls_s *ctl, u32 ncols) {
     return c;
 }
 
+// Slices of a bitmap row and entries of the split table over B's row ids.
+static u64 split_slices(const Setup &s) {
+    const u64 span = 32ull << s.cfg.bm_bits;
+    return ((u64)s.b.ncols + span - 1) / span;
+}
+static u64 split_entries(const Setup &s) {
+    const u64 nsl = split_slices(s);
+    return nsl > 1 ? (u64)s.mapn * (nsl + 1) : 0;
+}
+
+// From here on the row kernels run over the filtered A (prepare left what of A
+// has a B row).
+static void filter_a(clb_controls_s *ctl, Setup &s) {
+    const u32 tiles = (u32)(s.foffs.n - 1), grid = tiles + div_up((u64)s.nrows + 1, 256);
+    exclusive_scan_u32(ctl, s.foffs.ptr, s.foffs.ptr, tiles, s.foffs.ptr + tiles);
+    s.f_rpt.reset(ctl, (u64)s.nrows + 1);
+    s.f_cols.reset(ctl, s.a_nnz);  // how many stay only the device knows
+    auto run = [&](auto tile) {
+        k_filter<decltype(tile)::value><<<grid, 256, 0, ctl->stream>>>(s.g, s.nrows, tiles, s.fmask.ptr, s.foffs.ptr,
+                                                                       s.bidx.ptr, s.f_rpt.ptr, s.f_cols.ptr);
+    };
+    if (s.ftile == rstat_tile<true>()) run(std::integral_constant<u32, rstat_tile<true>()>{});
+    else run(std::integral_constant<u32, rstat_tile<false>()>{});
+    CLB_LAUNCHED("filter");
+    s.filtered = true;
+    s.g.a_rpt = s.f_rpt.ptr - s.row0;  // by A's stored rows, as a_all
+    s.g.a_cols = s.f_cols.ptr;
+    s.g.brange = s.crange.ptr;
+    s.g.bpres = nullptr;
+    s.g.mapn = s.mapn = s.b.nzr;
+}
+
 // The per-slice split table of B (Mats::splits) for bitmap rows over
 // several column windows: built on the first pass that has bitmap rows.
 void ensure_splits(clb_controls_s *ctl, Setup &s, const BinHost &h) {
     if (s.g.splits || h.off[NBINS] == h.off[BIN_BITMAP0]) return;
     const clb_dcsr &b = s.b;
-    const u64 span = 32ull << s.cfg.bm_bits;
-    const u64 nsl = ((u64)b.ncols + span - 1) / span;
+    const u64 span = 32ull << s.cfg.bm_bits, nsl = split_slices(s);
+    if (nsl > 1 && s.fmask.ptr && !s.filtered) filter_a(ctl, s);
     if (nsl <= 1 || !b.nzr || (u64)s.mapn * (nsl + 1) >= (1ull << 32)) return;
     // zero for the rows B does not store (an empty part in every slice), so
     // the gather reads it without looking the row up in brange
     s.splits.reset(ctl, (u64)s.mapn * (nsl + 1));
-    fill_u32(ctl, s.splits.ptr, s.splits.n, 0u);
-    k_slice_splits<<<div_up(b.nzr, 256), 256, 0, ctl->stream>>>(u32p(b.rpt), u32p(b.rows), u32p(b.cols), b.nzr,
-                                                                 s.mapn, (u32)nsl, span, s.splits.ptr);
+    if (!s.filtered) fill_u32(ctl, s.splits.ptr, s.splits.n, 0u);
+    k_slice_splits<<<div_up((u64)b.nzr * (nsl + 1), 256), 256, 0, ctl->stream>>>(
+        u32p(b.rpt), s.filtered ? nullptr : u32p(b.rows), u32p(b.cols), b.nzr, s.mapn, (u32)nsl, span, s.splits.ptr);
     CLB_LAUNCHED("slice_splits");
     s.g.splits = s.splits.ptr;
     s.g.nsl = (u32)nsl;
@@ -918,15 +1015,16 @@ void ensure_packed(clb_controls_s *ctl, Setup &s, const BinHost &h) {
     k_pack_place<<<tiles, EX_WG, 0, ctl->stream>>>(u32p(b.rpt), u32p(b.cols), b.nzr, b.nnz, first.ptr, offs.ptr,
                                                    prpt.ptr, s.packs.ptr, pfirst.ptr);
     CLB_LAUNCHED("pack_place");
-    if (!s.g.bpres) fill_u64(ctl, reinterpret_cast<u64 *>(s.prange.ptr), s.mapn, 0ull);
-    k_brange_set<<<div_up(b.nzr, 256), 256, 0, ctl->stream>>>(prpt.ptr, u32p(b.rows), b.nzr, s.mapn, s.prange.ptr,
-                                                              nullptr);
+    if (!s.g.bpres && !s.filtered) fill_u64(ctl, reinterpret_cast<u64 *>(s.prange.ptr), s.mapn, 0ull);
+    const u32 *rows = s.filtered ? nullptr : u32p(b.rows);
+    k_brange_set<<<div_up(b.nzr, 256), 256, 0, ctl->stream>>>(prpt.ptr, rows, b.nzr, s.mapn, s.prange.ptr, nullptr,
+                                                              nullptr, nullptr);
     CLB_LAUNCHED("brange_set");
     if (s.g.splits) {
         s.psplits.reset(ctl, s.splits.n);
-        fill_u32(ctl, s.psplits.ptr, s.psplits.n, 0u);
-        k_pack_splits<<<div_up(b.nzr, 256), 256, 0, ctl->stream>>>(prpt.ptr, u32p(b.rows), pfirst.ptr, s.g.splits,
-                                                                    b.nzr, s.mapn, s.g.nsl, s.psplits.ptr);
+        if (!s.filtered) fill_u32(ctl, s.psplits.ptr, s.psplits.n, 0u);
+        k_pack_splits<<<div_up(b.nzr, 256), 256, 0, ctl->stream>>>(prpt.ptr, rows, pfirst.ptr, s.g.splits, b.nzr,
+                                                                    s.mapn, s.g.nsl, s.psplits.ptr);
         CLB_LAUNCHED("pack_splits");
     }
     s.g.b_packs = s.packs.ptr;
@@ -942,6 +1040,7 @@ void prepare(clb_controls_s *ctl, const clb_dcsr &a, const clb_dcsr &b, u32 row_
         // a plan's block: B's row map and split table were built once
         s.mapn = shared->mapn;
         s.pack_tried = shared->pack_tried;
+        s.filtered = shared->filtered;
         s.g = shared->g;
         s.cfg = shared->cfg;
         s.b = shared->b;
@@ -953,7 +1052,7 @@ void prepare(clb_controls_s *ctl, const clb_dcsr &a, const clb_dcsr &b, u32 row_
         const bool sparse_map = (u64)b.nzr * 16 < s.mapn;
         if (sparse_map) s.bpres.reset(ctl, ((u64)s.mapn + 31) / 32);
         s.g.bpres = sparse_map ? s.bpres.ptr : nullptr;
-        s.g.a_rpt = u32p(a.rpt);
+        s.g.a_all = s.g.a_rpt = u32p(a.rpt);
         s.g.a_rows = u32p(a.rows);
         s.g.a_cols = u32p(a.cols);
         s.g.brange = s.brange.ptr;
@@ -970,6 +1069,8 @@ void prepare(clb_controls_s *ctl, const clb_dcsr &a, const clb_dcsr &b, u32 row_
         s.g.prange = nullptr;
         s.g.psplits = nullptr;
         s.pack_tried = false;
+        s.filtered = false;
+        s.a_nnz = a.nnz;
         s.g.nsl = 0;
         s.g.split_bits = s.cfg.bm_bits;
         s.b = b;  // the split table is built by ensure_splits, once bitmap rows exist
@@ -981,6 +1082,7 @@ void prepare(clb_controls_s *ctl, const clb_dcsr &a, const clb_dcsr &b, u32 row_
         s.prod.reset(ctl, nrows);
         s.P = s.prod.ptr;
     }
+    const bool filter = !shared && stats && s.bpres.ptr && b.nzr && split_entries(s) >= FILTER_MIN_ENTRIES;
     const u64 nmap = shared || s.bpres.ptr ? 0 : s.mapn, nbits = shared ? 0 : s.bpres.n;
     u64 most = nmap > nbits ? nmap : nbits;
     if (stats && nrows > most) most = nrows;
@@ -990,8 +1092,12 @@ void prepare(clb_controls_s *ctl, const clb_dcsr &a, const clb_dcsr &b, u32 row_
                                                              nrows, feat ? *feat : RowFeat{});
     CLB_LAUNCHED("init");
     if (!shared && b.nzr) {
+        if (filter) {
+            s.bidx.reset(ctl, s.mapn);
+            s.crange.reset(ctl, b.nzr);
+        }
         k_brange_set<<<div_up(b.nzr, 256), 256, 0, ctl->stream>>>(u32p(b.rpt), u32p(b.rows), b.nzr, s.mapn,
-                                                                   s.brange.ptr, s.bpres.ptr);
+                                                                   s.brange.ptr, s.bpres.ptr, s.bidx.ptr, s.crange.ptr);
         CLB_LAUNCHED("brange_set");
     }
     if (!stats) return;
@@ -1003,8 +1109,13 @@ void prepare(clb_controls_s *ctl, const clb_dcsr &a, const clb_dcsr &b, u32 row_
         k_tile_rows<rstat_tile<FEAT>()><<<div_up(nrows, EX_WG), EX_WG, 0, ctl->stream>>>(
             s.g.a_rpt, row_begin, row_begin + nrows, 0, 0, first.ptr);
         CLB_LAUNCHED("tile_rows");
+        if (filter) {
+            s.ftile = rstat_tile<FEAT>();
+            s.fmask.reset(ctl, (u64)tiles * (s.ftile / 32));
+            s.foffs.reset(ctl, (u64)tiles + 1);
+        }
         k_row_stats<FEAT><<<tiles, RSTAT_WG, 0, ctl->stream>>>(s.g, nrows, first.ptr, s.prod.ptr,
-                                                               feat ? *feat : RowFeat{});
+                                                               feat ? *feat : RowFeat{}, s.fmask.ptr, s.foffs.ptr);
         CLB_LAUNCHED("count_workload");
     };
     if (feat) run(std::true_type{});

@@ -13,6 +13,13 @@ struct Setup {
     u32 nrows = 0, row0 = 0, mapn = 0;
     DevArray<uint2> brange;
     DevArray<u32> bpres;  // presence bits of B rows (hypersparse B only)
+    // A without the nonzeros that have no B row (filter_a): a bit per nonzero
+    // and their number per tile of `ftile`, then the matrix itself with columns
+    // renumbered (bidx) to B's stored rows, whose ranges are crange.
+    DevArray<u32> fmask, foffs, bidx, f_rpt, f_cols;
+    DevArray<uint2> crange;
+    u32 ftile = 0, a_nnz = 0;
+    bool filtered = false;
     DevArray<u32> prod;
     DevArray<u64> scal;
     DevArray<u32> ctr;  // row counters of persistent launches (zeroed per launch)
@@ -115,6 +122,17 @@ void emit_launch(hipStream_t es, u32 count, const u32 *perm, const BinHost &h, c
                  const u64 *off, u32 *cols, LaunchTimer *lt, int pass);
 
 BinCfg make_bincfg(const clb_controls_s *ctl, u32 ncols);
+// Where B stores under one row in 16 and the split table over its row ids would
+// have this many entries, bitmap rows make the product run over a filtered A,
+// whose columns are B's stored rows: the table is then as long as B has rows,
+// and no row kernel meets a nonzero without a B row.  Measured filtered against
+// not (ms), squares with Zipf columns, bound / plain: 2^24 ids of which 1% are
+// stored 1.11 / 1.94 and 1.18 / 2.64, 3% 7.7 / 14.8 and 10.0 / 24.7; 2^22, 1%
+// 0.60 / 0.83 and 0.49 / 0.95; 2^21, 3% (6 million entries) 0.84 / 1.05 and
+// 0.83 / 1.36.  Small tables cost more launches than they save (30 us), and
+// rows of one window gain nothing: 16 million nonzeros, 30 a row, 0.996 /
+// 0.963.
+constexpr u64 FILTER_MIN_ENTRIES = 1ull << 18;
 void ensure_splits(clb_controls_s *ctl, Setup &s, const BinHost &h);
 // B packed by groups of 16 columns (Mats::b_packs) for the bitmap rows of `h`,
 // after ensure_splits.  Packing costs two passes over B and a read-back, so it

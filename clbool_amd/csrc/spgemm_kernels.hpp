@@ -47,7 +47,8 @@ constexpr u32 LONG_ROW = 64;     // B rows at least this long are shared by a wa
 constexpr int PACK_UB = 4;
 
 struct Mats {
-    const u32 *a_rpt;
+    const u32 *a_all;     // A's row pointers
+    const u32 *a_rpt;     // the same, or the filtered A's (with a_cols: its columns)
     const u32 *a_rows;
     const u32 *a_cols;
     const uint2 *brange;  // B row id -> [begin, end) into b_cols
