@@ -8,8 +8,8 @@
 // a_rpt[ia] * b_nnz + |A_ia| * b_rpt[ib]: the row pointer is a closed form,
 // no scan.  The reference finds each output's row by a binary search per
 // nonzero; here the work is cut into tiles of B nonzeros (one workgroup per
-// tile and A row): a partition pass finds each tile's first B row, the tile's
-// slice of b_rpt is staged in LDS, and each thread places its B nonzero once
+// tile and group of A rows): a partition pass finds each tile's first B row, the
+// tile's slice of b_rpt is staged in LDS, and each thread places its B nonzero once
 // per column of the A row -- consecutive threads write consecutive columns.
 // Sizes are checked in 64 bits: the reference computes nnz, nzr and the
 // shape as wrapping uint32 products (:10-13), which this library reports as
@@ -21,6 +21,11 @@
 namespace clb {
 
 constexpr u32 KRON_WG = 256, KRON_ITEMS = 4, KRON_TILE = KRON_WG * KRON_ITEMS;
+// A group of A rows shares the search of a tile's rows.  R-MAT 65536 x 16 and
+// an automaton of 64 states and 200 moves (764 MB) / of 30 and 40: 251 / 95 us
+// with a group per A row; about 6 A nonzeros to a group 220 / 67, 10 229 / 62,
+// 16 235 / 62 (later pieces of a line are stored further apart).
+constexpr u32 KRON_MIN_GRID = 1u << 12, KRON_GROUP = 8;
 
 __global__ void k_kron_rows(const u32 *__restrict__ a_rpt, const u32 *__restrict__ b_rpt,
                             const u32 *__restrict__ a_rows, const u32 *__restrict__ b_rows, u32 c_nzr, u32 b_nzr,
@@ -47,14 +52,19 @@ __global__ void k_kron_tiles(const u32 *__restrict__ b_rpt, u32 b_nzr, u32 ntile
     first[t] = lo;
 }
 
-// Workgroup (tile, ia): B nonzeros [tile * KRON_TILE, +KRON_TILE) times A
-// row ia (blocks cover A rows ia0, ia0 + 1, ...).
-__global__ __launch_bounds__(KRON_WG) void k_kron_fill(const u32 *__restrict__ first, u32 ntiles, u32 ia0,
+// Workgroup (tile, group): B nonzeros [tile * KRON_TILE, +KRON_TILE) times the
+// A rows [group * per, +per).  Stores bound it, in pieces of a B row's length:
+// 3.6 TB/s of a fill's 6.9 at 191 million nonzeros.  Stores of 16 bytes from
+// positions found by a search each, and from a tile put together in LDS, were
+// slower (336 and 417 us against 225 for the kernel alone): what they add to
+// the chain of a workgroup costs more than whole lines save.
+__global__ __launch_bounds__(KRON_WG) void k_kron_fill(const u32 *__restrict__ first, u32 ntiles, u32 per, u32 a_nzr,
                                                        const u32 *__restrict__ a_rpt, const u32 *__restrict__ a_cols,
                                                        const u32 *__restrict__ b_rpt, const u32 *__restrict__ b_cols,
                                                        u32 b_nzr, u32 b_nnz, u32 b_ncols, u32 *__restrict__ c_cols) {
     __shared__ u32 srpt[KRON_TILE + 1];
-    const u32 tile = blockIdx.x % ntiles, ia = ia0 + blockIdx.x / ntiles;
+    const u32 tile = blockIdx.x % ntiles, ia0 = blockIdx.x / ntiles * per;
+    const u32 ia1 = a_nzr - ia0 < per ? a_nzr : ia0 + per;
     const u32 e0 = tile * KRON_TILE;
     const u32 e1 = b_nnz - e0 < KRON_TILE ? b_nnz : e0 + KRON_TILE;
     const u32 ib0 = first[tile];
@@ -63,22 +73,32 @@ __global__ __launch_bounds__(KRON_WG) void k_kron_fill(const u32 *__restrict__ f
     const u32 nr = b_nzr - ib0 < KRON_TILE ? b_nzr - ib0 : KRON_TILE;
     for (u32 j = threadIdx.x; j <= nr; j += KRON_WG) srpt[j] = b_rpt[ib0 + j];
     __syncthreads();
-    const u32 a0 = a_rpt[ia], alen = a_rpt[ia + 1] - a0;
-    const u32 abase = a0 * b_nnz;
+    u32 rs[KRON_ITEMS], blen[KRON_ITEMS], bc[KRON_ITEMS];
 #pragma unroll
     for (u32 i = 0; i < KRON_ITEMS; ++i) {
         const u32 e = e0 + i * KRON_WG + threadIdx.x;
-        if (e >= e1) break;
         u32 lo = 0, hi = nr;  // last j with srpt[j] <= e
         while (hi - lo > 1) {
             const u32 mid = (lo + hi) >> 1;
             if (srpt[mid] <= e) lo = mid;
             else hi = mid;
         }
-        const u32 rs = srpt[lo], blen = srpt[lo + 1] - rs;
-        const u32 bc = b_cols[e];
-        u32 *out = c_cols + abase + alen * rs + (e - rs);
-        for (u32 ka = 0; ka < alen; ++ka) out[ka * blen] = a_cols[a0 + ka] * b_ncols + bc;
+        rs[i] = srpt[lo];
+        blen[i] = srpt[lo + 1] - rs[i];
+        bc[i] = e < e1 ? b_cols[e] : 0u;
+    }
+    u32 a0 = a_rpt[ia0];
+    for (u32 ia = ia0; ia < ia1; ++ia) {
+        const u32 a1 = a_rpt[ia + 1], alen = a1 - a0;
+        const u32 abase = a0 * b_nnz;
+#pragma unroll
+        for (u32 i = 0; i < KRON_ITEMS; ++i) {
+            const u32 e = e0 + i * KRON_WG + threadIdx.x;
+            u32 *out = c_cols + abase + alen * rs[i] + (e - rs[i]);
+            if (e < e1)
+                for (u32 ka = 0; ka < alen; ++ka) out[ka * blen[i]] = a_cols[a0 + ka] * b_ncols + bc[i];
+        }
+        a0 = a1;
     }
 }
 
@@ -117,14 +137,18 @@ clb_status clb_dcsr_kronecker(clb_controls ctl, const clb_dcsr *a, const clb_dcs
             DevArray<u32> first(ctl, ntiles);
             k_kron_tiles<<<div_up(ntiles, 256), 256, 0, ctl->stream>>>(u32p(b->rpt), b->nzr, ntiles, first.ptr);
             CLB_LAUNCHED("kron_tiles");
-            // launches of at most 2^22 workgroups, whole A rows each
-            const u32 rows_per = ntiles >= (1u << 22) ? 1u : (1u << 22) / ntiles;
-            for (u32 ia0 = 0; ia0 < a->nzr; ia0 += rows_per) {
-                const u32 nr = a->nzr - ia0 < rows_per ? a->nzr - ia0 : rows_per;
-                k_kron_fill<<<ntiles * nr, KRON_WG, 0, ctl->stream>>>(first.ptr, ntiles, ia0, u32p(a->rpt),
-                                                                       u32p(a->cols), u32p(b->rpt), u32p(b->cols),
-                                                                       b->nzr, b->nnz, b->ncols, u32p(r.cols));
-            }
+            // whole A rows to a workgroup: about KRON_GROUP of A's nonzeros,
+            // but no fewer than KRON_MIN_GRID workgroups
+            u64 per = ((u64)KRON_GROUP * a->nzr + a->nnz / 2) / a->nnz;
+            const u64 most = (u64)ntiles * a->nzr / KRON_MIN_GRID;
+            if (per > most) per = most;
+            if (per < 1) per = 1;
+            // and no more than 2^23 (2^31 threads)
+            while (ntiles * (((u64)a->nzr + per - 1) / per) > (1u << 23)) per *= 2;
+            const u64 groups = ((u64)a->nzr + per - 1) / per;
+            k_kron_fill<<<(u32)(ntiles * groups), KRON_WG, 0, ctl->stream>>>(
+                first.ptr, ntiles, (u32)per, a->nzr, u32p(a->rpt), u32p(a->cols), u32p(b->rpt), u32p(b->cols), b->nzr,
+                b->nnz, b->ncols, u32p(r.cols));
             CLB_LAUNCHED("calculate_kronecker_product");
             sync(ctl);
         } catch (...) {
