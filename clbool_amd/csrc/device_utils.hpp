@@ -451,5 +451,71 @@ __device__ uint32_t *lds_merge_sort(uint32_t *a, uint32_t *b, uint32_t n) {
     return src;
 }
 
+// Stable radix sort of the n values of a, n <= WG * PER, by their low `bits`
+// bits, 8 or fewer at a time: each wave holds a stretch in registers (64
+// consecutive values per item), ranks it by ballots over the digit's bits and
+// a counter per digit, and the values go back in place.  cnt: (WG / 64) * 256
+// counters; red: WG / 64 + 1 words.  Ends with a barrier.
+template <int WG, int PER>
+__device__ void lds_radix_sort(uint32_t *a, uint16_t *cnt, uint32_t *red, uint32_t n, int bits) {
+    constexpr int NW = WG / WAVE;
+    static_assert(WG >= 256 && WG * PER < 65536, "a thread per digit, 16-bit places");
+    const int l = lane(), w = wave_id();
+    const uint32_t wk = ((n + 63u) / 64u + NW - 1) / NW * 64u;  // values of a wave
+    const uint32_t o0 = (uint32_t)w * wk + (uint32_t)l;
+    const int passes = (bits + 7) / 8, db = passes ? (bits + passes - 1) / passes : 0;
+    const uint32_t mask = (1u << db) - 1u;
+    uint16_t *const mine = cnt + w * 256;
+    for (int p = 0; p < passes; ++p) {
+        const int shift = p * db;
+        uint32_t key[PER], rank[PER];
+        for (uint32_t t = threadIdx.x; t < NW * 128; t += WG) reinterpret_cast<uint32_t *>(cnt)[t] = 0;
+#pragma unroll
+        for (int q = 0; q < PER; ++q) {
+            const uint32_t o = o0 + q * WAVE;
+            key[q] = (uint32_t)q * WAVE < wk && o < n ? a[o] : 0u;
+        }
+        __syncthreads();
+#pragma unroll
+        for (int q = 0; q < PER; ++q) {
+            if ((uint32_t)q * WAVE >= wk) break;
+            const bool valid = o0 + q * WAVE < n;
+            const uint32_t d = (key[q] >> shift) & mask;
+            unsigned long long peers = __ballot(valid);
+            for (int b = 0; b < db; ++b) {
+                const bool bit = (d >> b) & 1u;
+                const unsigned long long m = __ballot(bit);
+                peers &= bit ? m : ~m;
+            }
+            const uint32_t below = lanes_below(peers);
+            const uint32_t before = mine[d];
+            rank[q] = before + below;
+            __builtin_amdgcn_wave_barrier();
+            if (valid && below == 0) mine[d] = (uint16_t)(before + (uint32_t)__popcll(peers));
+            __builtin_amdgcn_wave_barrier();
+        }
+        __syncthreads();
+        uint32_t sum = 0, total;
+        if (threadIdx.x < 256) {
+#pragma unroll 4
+            for (int v = 0; v < NW; ++v) {
+                const uint32_t c = cnt[v * 256 + threadIdx.x];
+                cnt[v * 256 + threadIdx.x] = (uint16_t)sum;
+                sum += c;
+            }
+        }
+        const uint32_t base = block_excl_scan<uint32_t, WG>(sum, red, total);
+        if (threadIdx.x < 256) {
+#pragma unroll 4
+            for (int v = 0; v < NW; ++v) cnt[v * 256 + threadIdx.x] = (uint16_t)(cnt[v * 256 + threadIdx.x] + base);
+        }
+        __syncthreads();
+#pragma unroll
+        for (int q = 0; q < PER; ++q)
+            if ((uint32_t)q * WAVE < wk && o0 + q * WAVE < n) a[mine[(key[q] >> shift) & mask] + rank[q]] = key[q];
+        __syncthreads();
+    }
+}
+
 }  // namespace dev
 }  // namespace clb

@@ -6,9 +6,8 @@
 // as 64-bit keys row << 32 | col by a stable LSD radix sort over only the bits
 // the matrix needs.  Deduplication counts the kept keys per tile, scans the counts and places
 // them.
+#include "radix.hpp"
 #include "sort.hpp"
-
-#include "device_utils.hpp"
 
 namespace clb {
 
@@ -32,12 +31,6 @@ namespace clb {
 // counts (16.1 million keys, 7-bit digits: 121 us a pass; here 24 + 8 + 64,
 // 4.0 TB/s in the last kernel; the sort before this one: 53 + 18 + 63, and six
 // passes where the transpose of a 2^20 x 2^20 matrix needs three).
-constexpr int RX_WG = 256;
-constexpr int RX_ITEMS = 16;
-constexpr u32 RX_TILE = RX_WG * RX_ITEMS;
-constexpr int RX_RADIX = 256;
-constexpr u32 RX_COPIES = 4;
-
 // Keys as an array of 64-bit keys, or as two arrays of halves (keys == nullptr).
 struct KeysIn {
     const u64 *keys;
@@ -72,9 +65,7 @@ __global__ void k_pack_pairs(const u32 *__restrict__ rows, const u32 *__restrict
 
 // Digit counts of tiles [g * per, (g + 1) * per) for workgroup g: before[t][d]
 // = keys of digit d in the group's tiles before t, sums[g][d] = in all of
-// them.  RX_COPIES counters per digit, taken by lane, because equal digits of
-// a wave's lanes (sorted or skewed input) would queue on one word, and a wave
-// whose lanes all hold one digit adds them at once.
+// them.
 __global__ __launch_bounds__(RX_WG) void k_radix_hist(KeysIn in, u64 n, int lo_bits, int shift, int digit_bits,
                                                       u32 per, u32 tiles, u32 *__restrict__ before,
                                                       u32 *__restrict__ sums) {
@@ -100,16 +91,7 @@ __global__ __launch_bounds__(RX_WG) void k_radix_hist(KeysIn in, u64 n, int lo_b
 #pragma unroll
             for (int q = 0; q < RX_ITEMS / 2; ++q) {
                 const u64 i = base + (u64)(half * (RX_ITEMS / 2) + q) * RX_WG;
-                const bool valid = i < n;
-                const unsigned long long all = __ballot(valid);
-                const u32 d = radix_digit(k[q], lo_bits, shift, mask);
-                const u32 f = __builtin_amdgcn_readfirstlane(d);
-                u32 *c = &h[d * RX_COPIES + copy];
-                if (__ballot(valid && d == f) == all) {
-                    if (valid && dev::lanes_below(all) == 0) atomicAdd(c, (u32)__popcll(all));
-                } else if (valid) {
-                    atomicAdd(c, 1u);
-                }
+                radix_count(radix_digit(k[q], lo_bits, shift, mask), i < n, h, copy);
             }
         }
         __syncthreads();
@@ -143,8 +125,8 @@ __global__ __launch_bounds__(RX_WG) void k_radix_pass(KeysIn in, KeysOut out, u6
     constexpr int NW = RX_WG / dev::WAVE;
     constexpr u32 WKEYS = RX_TILE / NW;
     __shared__ u64 skey[RX_TILE];
-    __shared__ u32 wcnt[NW][RX_RADIX];  // keys of each digit so far per wave, then the waves' offsets
-    __shared__ u32 gbase[RX_RADIX];     // the digit's first place in the output minus its first place in the tile
+    __shared__ u32 wcnt[NW][RX_RADIX];
+    __shared__ u32 gbase[RX_RADIX];
     __shared__ u32 red[NW + 1];
     const int l = dev::lane(), w = dev::wave_id();
     const u32 mask = (1u << digit_bits) - 1u;
@@ -168,46 +150,10 @@ __global__ __launch_bounds__(RX_WG) void k_radix_pass(KeysIn in, KeysOut out, u6
     const u32 d = threadIdx.x;
     const u32 of_all = totals[d];
     const u32 prior = sums[(u64)(tile / per) * RX_RADIX + d] + before[(u64)tile * RX_RADIX + d];
-    for (int v = 0; v < NW; ++v) wcnt[v][d] = 0;
     u32 total;
     const u32 place = dev::block_excl_scan<u32, RX_WG>(of_all, red, total) + prior;
-    const unsigned long long lt = (1ull << l) - 1ull;
-    u32 rank[RX_ITEMS];
-#pragma unroll
-    for (int q = 0; q < RX_ITEMS; ++q) {
-        const bool valid = o0 + q * dev::WAVE < cnt;
-        const u32 d = radix_digit(key[q], lo_bits, shift, mask);
-        unsigned long long peers = __ballot(valid);
-        for (int b = 0; b < digit_bits; ++b) {
-            const bool bit = (d >> b) & 1u;
-            const unsigned long long m = __ballot(bit);
-            peers &= bit ? m : ~m;
-        }
-        const u32 below = (u32)__popcll(peers & lt);
-        const u32 before = wcnt[w][d];
-        rank[q] = before + below;
-        __builtin_amdgcn_wave_barrier();
-        if (valid && below == 0) wcnt[w][d] = before + (u32)__popcll(peers);
-        __builtin_amdgcn_wave_barrier();
-    }
-    __syncthreads();
-    // digit d's count in the tile and the waves' offsets, from the tile's start
-    u32 mine = 0;
-#pragma unroll
-    for (int v = 0; v < NW; ++v) {
-        const u32 c = wcnt[v][d];
-        wcnt[v][d] = mine;
-        mine += c;
-    }
-    const u32 ls = dev::block_excl_scan<u32, RX_WG>(mine, red, total);
-#pragma unroll
-    for (int v = 0; v < NW; ++v) wcnt[v][d] += ls;
-    gbase[d] = place - ls;
-    __syncthreads();
-#pragma unroll
-    for (int q = 0; q < RX_ITEMS; ++q)
-        if (o0 + q * dev::WAVE < cnt) skey[wcnt[w][radix_digit(key[q], lo_bits, shift, mask)] + rank[q]] = key[q];
-    __syncthreads();
+    radix_tile(key, cnt, digit_bits, place, skey, wcnt, gbase, red,
+               [&](u64 k) { return radix_digit(k, lo_bits, shift, mask); });
 #pragma unroll
     for (int q = 0; q < RX_ITEMS; ++q) {
         const u32 o = q * RX_WG + threadIdx.x;
@@ -225,8 +171,8 @@ static int bits_for(u64 maxv) {
 }
 
 // Sorts by bits [from_bit, hi_bits + lo_bits) of the value hi << lo_bits | lo.
-// The result goes to the halves of `out`, or to its keys; `in` is only read,
-// and halves may be sorted in place.
+// `in` holds halves and is only read; the result goes to the halves of `out`
+// (which may be the same), or to its keys.
 static void radix_sort(clb_controls_s *ctl, KeysIn in, u64 n, int hi_bits, int lo_bits, int from_bit, KeysOut out) {
     if (!n) return;
     if (n > 0xFFFFFFFFull) raise(INVALID_VALUE, "sort of more than 2^32 - 1 keys");
@@ -239,7 +185,7 @@ static void radix_sort(clb_controls_s *ctl, KeysIn in, u64 n, int hi_bits, int l
     // intermediate passes alternate over two buffers; with keys as the result
     // one of them is the result's, taken in turn so that the last pass ends there
     const bool halves = out.keys == nullptr;
-    const bool alias = in.keys ? in.keys == out.keys : in.hi == out.hi;
+    const bool alias = halves && in.hi == out.hi;
     DevArray<u64> tmp0, tmp1;
     if (passes > 1 || (alias && passes == 1)) tmp0.reset(ctl, n);
     if (halves && passes > 2) tmp1.reset(ctl, n);
@@ -250,17 +196,10 @@ static void radix_sort(clb_controls_s *ctl, KeysIn in, u64 n, int hi_bits, int l
     const u32 groups = div_up(tiles, per);
     DevArray<u32> before(ctl, (u64)tiles * RX_RADIX), sums(ctl, (u64)groups * RX_RADIX), totals(ctl, RX_RADIX);
     KeysIn src = in;
-    if (alias && (passes & 1)) {
-        // an odd number of passes would end where it began: one more copy
-        if (in.keys) {
-            CLB_HIP(hipMemcpyAsync(tmp0.ptr, in.keys, n * 8, hipMemcpyDeviceToDevice, ctl->stream),
-                    COPY_BUFFER_ERROR);
-            src = KeysIn{tmp0.ptr, nullptr, nullptr};
-        } else if (passes == 1) {
-            k_pack_pairs<<<div_up(n, 256), 256, 0, ctl->stream>>>(in.hi, in.lo, n, tmp0.ptr);
-            CLB_LAUNCHED("pack_pairs");
-            src = KeysIn{tmp0.ptr, nullptr, nullptr};
-        }
+    if (alias && passes == 1) {  // the one pass reads a copy
+        k_pack_pairs<<<div_up(n, 256), 256, 0, ctl->stream>>>(in.hi, in.lo, n, tmp0.ptr);
+        CLB_LAUNCHED("pack_pairs");
+        src = KeysIn{tmp0.ptr, nullptr, nullptr};
     }
     for (int p = 0; p < passes; ++p) {
         const bool last = p + 1 == passes;
@@ -278,11 +217,6 @@ static void radix_sort(clb_controls_s *ctl, KeysIn in, u64 n, int hi_bits, int l
         CLB_LAUNCHED("radix_pass");
         src = KeysIn{buf, nullptr, nullptr};
     }
-}
-
-void radix_sort_keys(clb_controls_s *ctl, u64 *keys, u64 n, int col_bits, int row_bits) {
-    if (n < 2) return;
-    radix_sort(ctl, KeysIn{keys, nullptr, nullptr}, n, row_bits, col_bits, 0, KeysOut{keys, nullptr, nullptr});
 }
 
 void sort_pairs_to_keys(clb_controls_s *ctl, const u32 *rows, const u32 *cols, u64 n, u32 max_row, u32 max_col,
@@ -341,152 +275,73 @@ void pair_bounds(clb_controls_s *ctl, const u32 *rows, const u32 *cols, u64 n, u
 }
 
 // Sorted keys -> distinct keys, in tiles of KT_TILE keys.  Key i is kept
-// when it differs from key i - 1, and starts a row among the kept keys when
-// its row also differs (the previous distinct key is key i - 1).  A count
-// pass gives each tile's kept keys and row starts, their scans give each
-// tile's output offsets, and the scatter pass places every kept key by its
-// rank inside the tile (ballots per wave and item, counts exchanged in LDS).
-// Loads are striped (item it of thread t is key it * KT_WG + t of the tile),
-// so every load and every run of stores is coalesced.
+// when it differs from key i - 1.  A count pass gives each tile's kept keys,
+// their scan each tile's output offset, and the scatter pass places every kept
+// key by its rank inside the tile (ballots per wave and item, counts exchanged
+// in LDS).  Loads are striped (item it of thread t is key it * KT_WG + t of
+// the tile), so every load and every run of stores is coalesced.
 constexpr int KT_WG = 256, KT_ITEMS = 16;
 constexpr u64 KT_TILE = (u64)KT_WG * KT_ITEMS;
 
-// bit 0: kept, bit 1: starts a row among the kept keys
-__device__ __forceinline__ u32 key_flags(const u64 *__restrict__ keys, u64 i, u64 k) {
-    if (i == 0) return 3u;
-    const u64 p = keys[i - 1];
-    return k == p ? 0u : ((k >> 32) != (p >> 32) ? 3u : 1u);
+__device__ __forceinline__ bool key_kept(const u64 *__restrict__ keys, u64 i, u64 k) {
+    return i == 0 || keys[i - 1] != k;
 }
 
-__global__ __launch_bounds__(KT_WG) void k_keys_count(const u64 *__restrict__ keys, u64 n, u32 *__restrict__ kept,
-                                                      u32 *__restrict__ starts) {
+__global__ __launch_bounds__(KT_WG) void k_keys_count(const u64 *__restrict__ keys, u64 n, u32 *__restrict__ kept) {
     __shared__ u32 red[KT_WG / dev::WAVE + 1];
     const u64 base = (u64)blockIdx.x * KT_TILE;
-    u32 cu = 0, cs = 0;
+    u32 c = 0;
 #pragma unroll 4
     for (int it = 0; it < KT_ITEMS; ++it) {
         const u64 i = base + (u64)it * KT_WG + threadIdx.x;
-        if (i < n) {
-            const u32 f = key_flags(keys, i, keys[i]);
-            cu += f & 1u;
-            cs += f >> 1;
-        }
+        if (i < n) c += key_kept(keys, i, keys[i]);
     }
-    const u32 tu = dev::block_sum<u32, KT_WG>(cu, red);
-    const u32 ts = dev::block_sum<u32, KT_WG>(cs, red);
-    if (threadIdx.x == 0) {
-        kept[blockIdx.x] = tu;
-        starts[blockIdx.x] = ts;
-    }
+    const u32 sum = dev::block_sum<u32, KT_WG>(c, red);
+    if (threadIdx.x == 0) kept[blockIdx.x] = sum;
 }
 
-// DCSR: cols[p] = column of the p-th kept key; for the q-th row start,
-// rows[q] = its row and rpt[q] = p; rpt[nzr] = m.  Pairs (!DCSR): rows[p] =
-// row of the p-th kept key.
-template <bool DCSR>
+// cols[p], rows[p] = column and row of the p-th kept key.
 __global__ __launch_bounds__(KT_WG) void k_keys_scatter(const u64 *__restrict__ keys, u64 n,
-                                                        const u32 *__restrict__ koff, const u32 *__restrict__ soff,
-                                                        const u32 *__restrict__ totals, u32 *__restrict__ cols,
-                                                        u32 *__restrict__ rows, u32 *__restrict__ rpt) {
+                                                        const u32 *__restrict__ koff, u32 *__restrict__ cols,
+                                                        u32 *__restrict__ rows) {
     constexpr int NW = KT_WG / dev::WAVE;
-    __shared__ u32 cu[KT_ITEMS][NW], cs[KT_ITEMS][NW];
+    __shared__ u32 cu[KT_ITEMS][NW];
     const u64 base = (u64)blockIdx.x * KT_TILE;
     const u64 *kt = keys + base;  // the tile, indexed by 32-bit offsets
     const u32 nt = n - base < KT_TILE ? (u32)(n - base) : (u32)KT_TILE;
     const u32 w = dev::wave_id();
-    const u32 l = (u32)dev::lane();
-    u32 fl = 0;  // bit it: kept, bit 16 + it: row start
+    u32 fl = 0;  // bit it: kept
     // pass 1: flags; per wave and item the counts go to LDS
 #pragma unroll 4
     for (int it = 0; it < KT_ITEMS; ++it) {
         const u32 o = (u32)it * KT_WG + threadIdx.x;
-        const u32 f = o < nt ? key_flags(keys, base + o, kt[o]) : 0u;
-        fl |= (f & 1u) << it;
-        fl |= (f >> 1) << (16 + it);
-        const u64 bu = __ballot(f & 1u), bs = __ballot(f >> 1);
-        if (l == 0) {
-            cu[it][w] = (u32)__popcll(bu);
-            cs[it][w] = (u32)__popcll(bs);
-        }
+        const bool f = o < nt && key_kept(keys, base + o, kt[o]);
+        fl |= (f ? 1u : 0u) << it;
+        const u64 m = __ballot(f);
+        if (dev::lane() == 0) cu[it][w] = (u32)__popcll(m);
     }
     __syncthreads();
     // pass 2: ranks; the kept keys are read again (from cache)
-    u32 au = koff[blockIdx.x], as = soff[blockIdx.x];
+    u32 at = koff[blockIdx.x];
 #pragma unroll 4
     for (int it = 0; it < KT_ITEMS; ++it) {
-        u32 lu = 0, ls = 0, tu = 0, ts = 0;
+        u32 before = 0, all = 0;
 #pragma unroll
         for (int v = 0; v < NW; ++v) {
-            const u32 x = cu[it][v], y = cs[it][v];
-            tu += x;
-            ts += y;
-            lu += (u32)v < w ? x : 0u;
-            ls += (u32)v < w ? y : 0u;
+            const u32 x = cu[it][v];
+            all += x;
+            before += (u32)v < w ? x : 0u;
         }
-        const bool kept = (fl >> it) & 1u, start = (fl >> (16 + it)) & 1u;
-        const u64 bu = __ballot(kept), bs = __ballot(start);
+        const bool kept = (fl >> it) & 1u;
+        const u64 m = __ballot(kept);
         if (kept) {
             const u64 k = kt[(u32)it * KT_WG + threadIdx.x];
-            const u32 p = au + lu + dev::lanes_below(bu);
+            const u32 p = at + before + dev::lanes_below(m);
             cols[p] = (u32)k;
-            if (!DCSR) rows[p] = (u32)(k >> 32);
-            if (DCSR && start) {
-                const u32 q = as + ls + dev::lanes_below(bs);
-                rows[q] = (u32)(k >> 32);
-                rpt[q] = p;
-            }
+            rows[p] = (u32)(k >> 32);
         }
-        au += tu;
-        as += ts;
+        at += all;
     }
-    if (DCSR && blockIdx.x == 0 && threadIdx.x == 0) rpt[totals[1]] = totals[0];
-}
-
-// Counts and offsets of the kept keys and row starts: tot[0] = kept keys,
-// tot[1] = row starts.
-static void keys_offsets(clb_controls_s *ctl, const u64 *keys, u64 n, DevArray<u32> &koff, DevArray<u32> &soff,
-                         DevArray<u32> &tot, u32 &m, u32 &nzr) {
-    if (n >= 0xFFFFFFFFull) raise(INVALID_VALUE, "more keys than uint32 indices allow");
-    const u64 tiles = (n + KT_TILE - 1) / KT_TILE;
-    koff.reset(ctl, tiles);
-    soff.reset(ctl, tiles);
-    tot.reset(ctl, 2);
-    k_keys_count<<<(u32)tiles, KT_WG, 0, ctl->stream>>>(keys, n, koff.ptr, soff.ptr);
-    CLB_LAUNCHED("keys_count");
-    exclusive_scan_u32(ctl, koff.ptr, koff.ptr, tiles, tot.ptr);
-    exclusive_scan_u32(ctl, soff.ptr, soff.ptr, tiles, tot.ptr + 1);
-    u32 h[2];
-    readback(ctl, h, tot.ptr, 8);
-    m = h[0];
-    nzr = h[1];
-}
-
-void keys_to_dcsr(clb_controls_s *ctl, const u64 *keys, u64 n, clb_dcsr &out) {
-    clb_dcsr r{};
-    r.nrows = out.nrows;
-    r.ncols = out.ncols;
-    if (n == 0) {
-        out = r;
-        return;
-    }
-    DevArray<u32> koff, soff, tot;
-    u32 m = 0, nzr = 0;
-    keys_offsets(ctl, keys, n, koff, soff, tot, m, nzr);
-    try {
-        r.cols = buffer_new(ctl, 4ull * m);
-        r.rows = buffer_new(ctl, 4ull * nzr);
-        r.rpt = buffer_new(ctl, 4ull * (nzr + 1ull));
-        k_keys_scatter<true><<<(u32)koff.n, KT_WG, 0, ctl->stream>>>(keys, n, koff.ptr, soff.ptr, tot.ptr,
-                                                                      u32p(r.cols), u32p(r.rows), u32p(r.rpt));
-        CLB_LAUNCHED("keys_scatter");
-        sync(ctl);
-    } catch (...) {
-        clb_dcsr_release(&r);
-        throw;
-    }
-    r.nnz = m;
-    r.nzr = nzr;
-    out = r;
 }
 
 void pack_pairs(clb_controls_s *ctl, const u32 *rows, const u32 *cols, u64 n, u64 *keys) {
@@ -504,9 +359,14 @@ u32 unique_keys_to_pairs(clb_controls_s *ctl, const u64 *keys, u64 n, clb_buffer
         *cols_out = buffer_new(ctl, 4);
         return 0;
     }
-    DevArray<u32> koff, soff, tot;
-    u32 m = 0, nzr = 0;
-    keys_offsets(ctl, keys, n, koff, soff, tot, m, nzr);
+    if (n >= 0xFFFFFFFFull) raise(INVALID_VALUE, "more keys than uint32 indices allow");
+    const u32 tiles = (u32)((n + KT_TILE - 1) / KT_TILE);
+    DevArray<u32> koff(ctl, (u64)tiles + 1);
+    k_keys_count<<<tiles, KT_WG, 0, ctl->stream>>>(keys, n, koff.ptr);
+    CLB_LAUNCHED("keys_count");
+    exclusive_scan_u32(ctl, koff.ptr, koff.ptr, tiles, koff.ptr + tiles);
+    u32 m = 0;
+    readback(ctl, &m, koff.ptr + tiles, 4);
     *rows_out = buffer_new(ctl, 4ull * (m ? m : 1));
     try {
         *cols_out = buffer_new(ctl, 4ull * (m ? m : 1));
@@ -515,8 +375,7 @@ u32 unique_keys_to_pairs(clb_controls_s *ctl, const u64 *keys, u64 n, clb_buffer
         *rows_out = nullptr;
         throw;
     }
-    k_keys_scatter<false><<<(u32)koff.n, KT_WG, 0, ctl->stream>>>(keys, n, koff.ptr, soff.ptr, tot.ptr,
-                                                                   u32p(*cols_out), u32p(*rows_out), nullptr);
+    k_keys_scatter<<<tiles, KT_WG, 0, ctl->stream>>>(keys, n, koff.ptr, u32p(*cols_out), u32p(*rows_out));
     CLB_LAUNCHED("keys_scatter");
     return m;
 }

@@ -7,10 +7,9 @@
 namespace clb {
 
 // Stable sorts of pairs (row, col), over only the bits that the largest row
-// and column need.  radix_sort_keys: 64-bit keys row << 32 | col in place.
-// sort_pairs_to_keys: two arrays to sorted keys.  sort_pairs: two arrays to
-// two arrays (which may be the same), by_row_only: stable by row alone.
-void radix_sort_keys(clb_controls_s *ctl, u64 *keys, u64 n, int col_bits, int row_bits);
+// and column need.  sort_pairs_to_keys: two arrays to sorted keys.
+// sort_pairs: two arrays to two arrays (which may be the same), by_row_only:
+// stable by row alone.
 void sort_pairs_to_keys(clb_controls_s *ctl, const u32 *rows, const u32 *cols, u64 n, u32 max_row, u32 max_col,
                         u64 *keys);
 void sort_pairs(clb_controls_s *ctl, const u32 *rows, const u32 *cols, u64 n, u32 max_row, u32 max_col,
@@ -30,9 +29,6 @@ void merge_keys(clb_controls_s *ctl, const u64 *a, u64 na, const u64 *b, u64 nb,
 // what was replaced.
 void union_keys_to_matrices(clb_controls_s *ctl, const u64 *ka, u64 na, const u64 *kb, u64 nb, u32 n,
                             std::vector<clb_dcsr> &mats);
-// Sorted keys (row << 32 | col, duplicates allowed) -> a new canonical DCSR
-// of their distinct pairs; out.nrows/ncols are kept as given.
-void keys_to_dcsr(clb_controls_s *ctl, const u64 *keys, u64 n, clb_dcsr &out);
 void coo_finish(clb_controls_s *ctl, clb_buffer_s *rows, clb_buffer_s *cols, u32 nrows, u32 ncols, u32 nnz,
                 bool sorted, bool nodup, clb_coo &out);
 

@@ -1234,7 +1234,7 @@ void join_deferred(clb_controls_s *ctl, const hipEvent_t *defer) {
 }
 
 void launch_bins(clb_controls_s *ctl, const Setup &s, const u32 *perm, const u32 off[NBINS + 1], int mode,
-                 const Out &o, LaunchTimer *lt, int family, hipEvent_t *defer, bool one_stream) {
+                 const Out &o, LaunchTimer *lt, int family, hipEvent_t *defer, bool one_stream, bool open) {
     if (!one_stream) fork_side(ctl);
     // the longest kernels have streams of their own: kept rows or the bitmap
     // rows on side stream 0, heavy bitmap rows on side stream 1 (not behind the
@@ -1369,7 +1369,7 @@ void launch_bins(clb_controls_s *ctl, const Setup &s, const u32 *perm, const u32
         t.end(fam(1), st);
     }
 #undef DISPATCH3
-    if (one_stream) return;
+    if (one_stream || open) return;
     if (!defer) {
         join_side(ctl);
         return;

@@ -170,7 +170,8 @@ void sum_by_bin(clb_controls_s *ctl, const u32 *perm, const BinHost &h, u32 nrow
 // events, made by the caller) for join_deferred.  one_stream: every kernel
 // on the controls' stream instead (no side streams).
 void launch_bins(clb_controls_s *ctl, const Setup &s, const u32 *perm, const u32 off[NBINS + 1], int mode,
-                 const Out &o, LaunchTimer *lt, int family, hipEvent_t *defer = nullptr, bool one_stream = false);
+                 const Out &o, LaunchTimer *lt, int family, hipEvent_t *defer = nullptr, bool one_stream = false,
+                 bool open = false);
 // Bitmap rows perm[r0 .. r0 + n) with windows of 2^bits words, by the usual or
 // the widest workgroup (bitmap_sym.hip, bitmap_num.hip, bitmap_one.hip).
 void launch_bitmap_sym(clb_controls_s *ctl, hipStream_t st, const Setup &s, const u32 *perm, u32 r0, u32 n, u32 bits,
