@@ -129,25 +129,26 @@ __global__ __launch_bounds__(EX_WG) void k_keys_segs(const KeySeg *__restrict__ 
     }
 }
 
-// zlen[row id] = stored length of that row of Z' (zlen pre-filled with 0).
-__global__ void k_row_lengths(const u32 *__restrict__ rpt, const u32 *__restrict__ rows, u32 nzr,
-                              u32 *__restrict__ zlen) {
+// The output bound of a stored row of Y': min(its products, n).
+struct RowBound {
+    const u32 *prod;
+    u32 n;
+    __device__ __forceinline__ u64 operator()(u64 r) const { return prod[r] < n ? prod[r] : n; }
+};
+
+__global__ void k_row_bounds(RowBound f, u32 nzr, u64 *__restrict__ bound) {
     const u32 r = blockIdx.x * blockDim.x + threadIdx.x;
-    if (r < nzr) zlen[rows[r]] = rpt[r + 1] - rpt[r];
+    if (r < nzr) bound[r] = f(r);
 }
 
-// bound[r] = min(products of stored row r of Y', n): an upper bound of the
-// row's output size.  One wave per row (rows of Y' reach thousands of
-// nonzeros).
-__global__ __launch_bounds__(256) void k_row_bounds(const u32 *__restrict__ rpt, const u32 *__restrict__ cols,
-                                                    u32 nzr, const u32 *__restrict__ zlen, u32 n,
-                                                    u64 *__restrict__ bound) {
-    const u32 r = blockIdx.x * 4 + dev::wave_id();
-    if (r >= nzr) return;
-    u64 p = 0;
-    for (u32 j = rpt[r] + dev::lane(); j < rpt[r + 1]; j += dev::WAVE) p += zlen[cols[j]];
-    p = dev::wave_sum(p);
-    if (dev::lane() == 0) bound[r] = p < n ? p : n;
+// Their sum; at most RB_GRID workgroups, since each adds to one word.
+constexpr u32 RB_GRID = 128;
+__global__ __launch_bounds__(256) void k_bound_sum(RowBound f, u32 nzr, u64 *__restrict__ sum) {
+    __shared__ u64 red[256 / dev::WAVE + 1];
+    u64 v = 0;
+    for (u64 r = (u64)blockIdx.x * 256 + threadIdx.x; r < nzr; r += (u64)gridDim.x * 256) v += f(r);
+    v = dev::block_sum<u64, 256>(v, red);
+    if (threadIdx.x == 0 && v) atomicAdd(reinterpret_cast<unsigned long long *>(sum), (unsigned long long)v);
 }
 
 // cuts[b] = first stored row whose exclusive bound prefix is >= b * step
@@ -204,9 +205,9 @@ static u64 closure_block_limit(u32 block_bound, u32 n) {
     return lim < 0xFFFFFFFFull ? lim : 0xFFFFFFFFull;
 }
 
-// Builds the stack of the given matrices on the device.
-static clb_dcsr stack(clb_controls_s *ctl, const std::vector<Seg> &segs_in, u32 nrows, u32 ncols) {
-    std::vector<Seg> segs = segs_in;
+// Builds the stack of the given matrices on the device; segs stays as it is
+// until the controls' stream has been waited for.
+static clb_dcsr stack(clb_controls_s *ctl, std::vector<Seg> &segs, u32 nrows, u32 ncols) {
     u64 nzr = 0, nnz = 0;
     for (auto &s : segs) {
         s.nzr_off = (u32)nzr;
@@ -230,7 +231,6 @@ static clb_dcsr stack(clb_controls_s *ctl, const std::vector<Seg> &segs_in, u32 
     CLB_LAUNCHED("stack_rows");
     k_stack_cols<<<div_up(nnz, 256), 256, 0, ctl->stream>>>(dseg.ptr, (u32)segs.size(), (u32)nnz, u32p(m.cols));
     CLB_LAUNCHED("stack_cols");
-    sync(ctl);  // dseg is released on return
     m.nnz = (u32)nnz;
     m.nzr = (u32)nzr;
     return m;
@@ -431,34 +431,42 @@ clb_status clb_closure_step(clb_controls ctl, clb_dcsr *mats, uint32_t nmats, co
             try {
                 Z = stack(ctl, zs, ntriples * n, n);
                 if (Y.nnz && Z.nnz) {
-                    // row blocks of Y' with output bound below 2^32 each
-                    DevArray<u32> zlen(ctl, (u64)ntriples * n);
-                    fill_u32(ctl, zlen.ptr, (u64)ntriples * n, 0u);
-                    k_row_lengths<<<div_up(Z.nzr, 256), 256, 0, ctl->stream>>>(u32p(Z.rpt), u32p(Z.rows), Z.nzr,
-                                                                                zlen.ptr);
-                    CLB_LAUNCHED("row_lengths");
-                    DevArray<u64> pre(ctl, (u64)Y.nzr + 1);
-                    k_row_bounds<<<div_up(Y.nzr, 4), 256, 0, ctl->stream>>>(u32p(Y.rpt), u32p(Y.cols), Y.nzr,
-                                                                               zlen.ptr, n, pre.ptr);
-                    CLB_LAUNCHED("row_bounds");
-                    exclusive_scan_u64(ctl, pre.ptr, pre.ptr, Y.nzr, pre.ptr + Y.nzr);
-                    u64 total = 0;
-                    readback(ctl, &total, pre.ptr + Y.nzr, 8);
+                    // row blocks of Y' with output bound below 2^32 each; one
+                    // block when the sum of its rows' bounds says so
                     const u64 lim = closure_block_limit(o.block_bound, n);
                     const u64 step = lim - n + 1;
-                    const u32 nb = (u32)((total + step - 1) / step);
-                    DevArray<u32> cuts(ctl, (u64)nb + 1);
-                    DevArray<u64> bb(ctl, nb ? nb : 1);
-                    k_cuts<<<div_up(nb + 1, 256), 256, 0, ctl->stream>>>(pre.ptr, Y.nzr, step, nb, cuts.ptr);
-                    CLB_LAUNCHED("cuts");
-                    if (nb) {
-                        k_block_bounds<<<div_up(nb, 256), 256, 0, ctl->stream>>>(pre.ptr, cuts.ptr, nb, bb.ptr);
-                        CLB_LAUNCHED("block_bounds");
+                    std::vector<u32> hc{0, Y.nzr};
+                    std::vector<u64> hb(1);
+                    u32 nb = 0;
+                    {
+                        spg::Setup ps;
+                        spg::prepare(ctl, Y, Z, 0, Y.nzr, ps, true);
+                        const RowBound rb{ps.P, n};
+                        const u32 grid = div_up(Y.nzr, 256) < RB_GRID ? div_up(Y.nzr, 256) : RB_GRID;
+                        k_bound_sum<<<grid, 256, 0, ctl->stream>>>(rb, Y.nzr, ps.scal.ptr);
+                        CLB_LAUNCHED("bound_sum");
+                        u64 total = 0;
+                        readback(ctl, &total, ps.scal.ptr, 8);
+                        nb = (u32)((total + step - 1) / step);
+                        if (nb == 1) {
+                            hb[0] = total;
+                        } else if (nb > 1) {
+                            DevArray<u64> pre(ctl, (u64)Y.nzr + 1);
+                            k_row_bounds<<<div_up(Y.nzr, 256), 256, 0, ctl->stream>>>(rb, Y.nzr, pre.ptr);
+                            CLB_LAUNCHED("row_bounds");
+                            exclusive_scan_u64(ctl, pre.ptr, pre.ptr, Y.nzr, pre.ptr + Y.nzr);
+                            DevArray<u32> cuts(ctl, (u64)nb + 1);
+                            DevArray<u64> bb(ctl, nb);
+                            k_cuts<<<div_up(nb + 1, 256), 256, 0, ctl->stream>>>(pre.ptr, Y.nzr, step, nb, cuts.ptr);
+                            CLB_LAUNCHED("cuts");
+                            k_block_bounds<<<div_up(nb, 256), 256, 0, ctl->stream>>>(pre.ptr, cuts.ptr, nb, bb.ptr);
+                            CLB_LAUNCHED("block_bounds");
+                            hc.resize((size_t)nb + 1);
+                            hb.resize(nb);
+                            readback(ctl, hc.data(), cuts.ptr, 4ull * (nb + 1));
+                            readback(ctl, hb.data(), bb.ptr, 8ull * nb);
+                        }
                     }
-                    std::vector<u32> hc(nb + 1);
-                    std::vector<u64> hb(nb);
-                    readback(ctl, hc.data(), cuts.ptr, 4ull * (nb + 1));
-                    if (nb) readback(ctl, hb.data(), bb.ptr, 8ull * nb);
                     for (u32 k = 0; k < nb; ++k) {
                         if (hb[k] > lim) raise(RUN_KERNEL_FAILURE, "closure row block exceeds its output bound");
                         if (hb[k] > st.max_block_bound) st.max_block_bound = hb[k];
@@ -542,6 +550,7 @@ clb_status clb_closure_step(clb_controls ctl, clb_dcsr *mats, uint32_t nmats, co
                     }
                 }
             } catch (...) {
+                (void)hipStreamSynchronize(ctl->stream);
                 release_all();
                 clb_dcsr_release(&Y);
                 clb_dcsr_release(&Z);

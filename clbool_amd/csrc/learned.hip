@@ -275,6 +275,11 @@ __global__ void k_failed_keys(const u32 *__restrict__ nnz_row, const u32 *__rest
 // takes CR_ROWS consecutive rows: each wave copies one of them, except rows of
 // at least CR_LONG columns, which the whole workgroup copies in turn.
 constexpr u32 CR_WG = 256, CR_ROWS = CR_WG / 64, CR_LONG = 2048;
+// k_compact_short below takes many rows of few columns: 582 thousand rows of a
+// closure's products, 140 us against 223 (145 thousand workgroups of four rows
+// wait on their rows' places one after the other); R-MAT 2^16 x 16, 700 columns
+// a row, 1.01 ms with either.
+constexpr u32 CR_SHORT_ROWS = 1u << 16, CR_SHORT_MEAN = 64;
 __global__ __launch_bounds__(CR_WG) void k_compact_rows(const u32 *__restrict__ nnz_row, const u64 *__restrict__ off,
                                                         u32 nrows, const u32 *__restrict__ temp,
                                                         const u64 *__restrict__ toff, const u32 *__restrict__ side,
@@ -301,6 +306,89 @@ __global__ __launch_bounds__(CR_WG) void k_compact_rows(const u32 *__restrict__ 
         u32 *dst = cols + off[r];
         if (n >= CR_LONG) copy(src, dst, n, threadIdx.x, CR_WG);
         else if (wv == j) copy(src, dst, n, l, 64u);
+    }
+}
+
+// The same copy with 64 rows to a wave: the lanes read the rows' sizes and
+// places together, rows below 64 columns are copied as one run of consecutive
+// outputs (each lane finds its column's row among the wave's), longer ones by
+// the wave in turn, those of CR_LONG by the workgroup.
+__global__ __launch_bounds__(CR_WG) void k_compact_short(const u32 *__restrict__ nnz_row,
+                                                         const u64 *__restrict__ off, u32 nrows,
+                                                         const u32 *__restrict__ temp, const u64 *__restrict__ toff,
+                                                         const u32 *__restrict__ side, const u64 *__restrict__ soff,
+                                                         const u32 *__restrict__ key2,
+                                                         const u32 *__restrict__ isdense, u32 *__restrict__ cols) {
+    constexpr int U = 4;
+    __shared__ u32 srow[CR_WG];
+    __shared__ u32 scnt;
+    const int l = dev::lane();
+    const u64 r = (u64)blockIdx.x * CR_WG + threadIdx.x;
+    if (threadIdx.x == 0) scnt = 0;
+    __syncthreads();
+    u32 n = r < nrows ? nnz_row[r] : 0u;
+    if (n && isdense && isdense[r]) n = 0;  // dense bitmap rows are emitted separately
+    const u32 *src = nullptr;
+    u32 *dst = nullptr;
+    if (n) {
+        src = (key2 && key2[r]) ? side + soff[r] : temp + toff[r];
+        dst = cols + off[r];
+    }
+    if (n >= CR_LONG) {
+        srow[atomicAdd(&scnt, 1u)] = threadIdx.x;
+        n = 0;
+    }
+    auto from = [](u64 p, int s) {  // a pointer of lane s
+        return ((u64)(u32)__shfl((u32)(p >> 32), s, dev::WAVE) << 32) | (u32)__shfl((u32)p, s, dev::WAVE);
+    };
+    const u32 sl = n < 64u ? n : 0u;
+    const u32 inc = dev::wave_incl_scan(sl);
+    const u32 total = __shfl(inc, dev::WAVE - 1, dev::WAVE), exc = inc - sl;
+    for (u32 p0 = 0; p0 < total; p0 += U * dev::WAVE) {
+        u32 v[U];
+        u32 *to[U];
+#pragma unroll
+        for (int u = 0; u < U; ++u) {
+            const u32 p = p0 + u * dev::WAVE + l;
+            int s = 0;
+            u32 es = 0;
+#pragma unroll
+            for (int step = 32; step > 0; step >>= 1) {
+                const u32 e = __shfl(exc, s + step, dev::WAVE);
+                if (e <= p) {
+                    s += step;
+                    es = e;
+                }
+            }
+            const u32 *const a = reinterpret_cast<const u32 *>(from(reinterpret_cast<u64>(src), s));
+            to[u] = reinterpret_cast<u32 *>(from(reinterpret_cast<u64>(dst), s)) + (p - es);
+            v[u] = p < total ? a[p - es] : 0u;
+        }
+#pragma unroll
+        for (int u = 0; u < U; ++u)
+            if (p0 + u * dev::WAVE + l < total) *to[u] = v[u];
+    }
+    auto copy = [&](const u32 *a, u32 *b, u32 m, u32 t, u32 step) {
+        for (; t + 3 * step < m; t += 4 * step) {
+            const u32 x = a[t], y = a[t + step], z = a[t + 2 * step], w = a[t + 3 * step];
+            b[t] = x;
+            b[t + step] = y;
+            b[t + 2 * step] = z;
+            b[t + 3 * step] = w;
+        }
+        for (; t < m; t += step) b[t] = a[t];
+    };
+    unsigned long long lm = __ballot(n >= 64u);
+    while (lm) {
+        const int s = __ffsll(lm) - 1;
+        lm &= lm - 1;
+        copy(reinterpret_cast<const u32 *>(from(reinterpret_cast<u64>(src), s)),
+             reinterpret_cast<u32 *>(from(reinterpret_cast<u64>(dst), s)), __shfl(n, s, dev::WAVE), (u32)l, 64u);
+    }
+    __syncthreads();
+    for (u32 k = 0; k < scnt; ++k) {
+        const u64 q = (u64)blockIdx.x * CR_WG + srow[k];
+        copy((key2 && key2[q]) ? side + soff[q] : temp + toff[q], cols + off[q], nnz_row[q], threadIdx.x, CR_WG);
     }
 }
 
@@ -404,6 +492,12 @@ void compact_rows(hipStream_t st, u32 nrows, u64 nnz, const u32 *nnz_row, const 
         const u32 grid = div_up(nrows, 256) < PE_GRID ? div_up(nrows, 256) : PE_GRID;
         k_pred_error<<<grid, 256, 0, st>>>(nnz_row, pred, nrows, err);
         CLB_LAUNCHED("pred_error");
+    }
+    if (!by_tiles && nrows >= CR_SHORT_ROWS && nnz < (u64)CR_SHORT_MEAN * nrows) {
+        k_compact_short<<<div_up(nrows, CR_WG), CR_WG, 0, st>>>(nnz_row, off, nrows, temp, toff, side, soff, key2,
+                                                                isdense, cols);
+        CLB_LAUNCHED("compact_short");
+        return;
     }
     if (!by_tiles) {
         k_compact_rows<<<div_up(nrows, CR_ROWS), CR_WG, 0, st>>>(nnz_row, off, nrows, temp, toff, side, soff, key2,
