@@ -173,8 +173,7 @@ struct DevArray {
     }
 };
 
-// Fork the side streams off the main stream / join them back.
-void fork_side(clb_controls_s *ctl);
+// The main stream waits for the side streams.
 void join_side(clb_controls_s *ctl);
 inline hipStream_t side_stream(clb_controls_s *ctl, int k) { return ctl->side[k % clb_controls_s::NSIDE]; }
 

@@ -762,14 +762,17 @@ void one_pass_post(OnePass &p) {
     assemble(ctl, s, a, p.nnz_row.ptr, p.offs.ptr, p.pos.ptr, nnz, nzr, cols, p.out);
     // the tail: compaction of the temporary slots and emission of the dumped
     // rows write disjoint rows, side by side on the two tail streams, after
-    // everything above on the controls' stream
+    // everything above on the controls' stream (a small tail: on that stream)
     CLB_HIP(hipEventCreateWithFlags(&p.joined, hipEventDisableTiming), EVENT_WAITING_ERROR);
     CLB_HIP(hipEventCreateWithFlags(&p.done, hipEventDisableTiming), EVENT_WAITING_ERROR);
-    CLB_HIP(hipEventRecord(ctl->ev_fork, ctl->stream), EVENT_WAITING_ERROR);
     p.tail = true;
-    hipStream_t t0s = ctl->tail[0], t1s = ctl->tail[1];
-    CLB_HIP(hipStreamWaitEvent(t0s, ctl->ev_fork, 0), EVENT_WAITING_ERROR);
-    CLB_HIP(hipStreamWaitEvent(t1s, ctl->ev_fork, 0), EVENT_WAITING_ERROR);
+    const bool small = nnz <= ONE_STREAM_WORK;
+    hipStream_t t0s = small ? ctl->stream : ctl->tail[0], t1s = small ? ctl->stream : ctl->tail[1];
+    if (!small) {
+        CLB_HIP(hipEventRecord(ctl->ev_fork, ctl->stream), EVENT_WAITING_ERROR);
+        CLB_HIP(hipStreamWaitEvent(t0s, ctl->ev_fork, 0), EVENT_WAITING_ERROR);
+        CLB_HIP(hipStreamWaitEvent(t1s, ctl->ev_fork, 0), EVENT_WAITING_ERROR);
+    }
     p.lt.begin(t0s);
     compact_rows(t0s, nrows, nnz, p.nnz_row.ptr, p.offs.ptr, p.temp.ptr, p.toff.ptr, p.side.ptr, p.soff.ptr,
                  nfail ? p.key2.ptr : nullptr,
@@ -779,8 +782,10 @@ void one_pass_post(OnePass &p) {
     emit_launch(t1s, ndense, p.perm.ptr, p.h, p.dump, p.gpre.ptr, p.offs.ptr, u32p(cols), &p.lt, CLB_KP_ONEPASS);
     if (p.store.keep.slots)
         emit_stored(t1s, p.perm.ptr + p.h.off[BIN_BITMAP0], p.store.keep.slots, p.store.keep, p.offs.ptr, u32p(cols));
-    CLB_HIP(hipEventRecord(p.joined, t0s), EVENT_WAITING_ERROR);
-    CLB_HIP(hipStreamWaitEvent(t1s, p.joined, 0), EVENT_WAITING_ERROR);
+    if (!small) {
+        CLB_HIP(hipEventRecord(p.joined, t0s), EVENT_WAITING_ERROR);
+        CLB_HIP(hipStreamWaitEvent(t1s, p.joined, 0), EVENT_WAITING_ERROR);
+    }
     CLB_HIP(hipEventRecord(p.done, t1s), EVENT_WAITING_ERROR);
 }
 

@@ -151,12 +151,6 @@ void buffer_release(clb_buffer_s *b) {
 
 void sync(clb_controls_s *ctl) { CLB_HIP(hipStreamSynchronize(ctl->stream), EVENT_WAITING_ERROR); }
 
-void fork_side(clb_controls_s *ctl) {
-    CLB_HIP(hipEventRecord(ctl->ev_fork, ctl->stream), EVENT_WAITING_ERROR);
-    for (int k = 0; k < clb_controls_s::NSIDE; ++k)
-        CLB_HIP(hipStreamWaitEvent(ctl->side[k], ctl->ev_fork, 0), EVENT_WAITING_ERROR);
-}
-
 void join_side(clb_controls_s *ctl) {
     for (int k = 0; k < clb_controls_s::NSIDE; ++k) {
         CLB_HIP(hipEventRecord(ctl->ev_join[k], ctl->side[k]), EVENT_WAITING_ERROR);

@@ -1145,6 +1145,7 @@ void read_bins(clb_controls_s *ctl, Setup &s, BinHost &h) {
     std::memcpy(&t, ctl->pinned, sizeof(t));
     h.off[0] = 0;
     h.total = 0;
+    s.bin_work = 0;
     for (u32 b = 0; b < NBINS; ++b) {
         h.off[b + 1] = h.off[b] + t.rows[b];
         h.products[b] = t.sums[b];
@@ -1152,6 +1153,7 @@ void read_bins(clb_controls_s *ctl, Setup &s, BinHost &h) {
         h.out_nnz[b] = t.sums[2 * NBINS + b];
         s.bin_products[b] = t.sums[b];
         h.total += t.sums[b];
+        s.bin_work += t.sums[b] + 4 * t.sums[NBINS + b];
     }
     std::memcpy(h.scal, t.scal, sizeof(h.scal));
 }
@@ -1235,22 +1237,39 @@ void join_deferred(clb_controls_s *ctl, const hipEvent_t *defer) {
 
 void launch_bins(clb_controls_s *ctl, const Setup &s, const u32 *perm, const u32 off[NBINS + 1], int mode,
                  const Out &o, LaunchTimer *lt, int family, hipEvent_t *defer, bool one_stream, bool open) {
-    if (!one_stream) fork_side(ctl);
-    // the longest kernels have streams of their own: kept rows or the bitmap
-    // rows on side stream 0, heavy bitmap rows on side stream 1 (not behind the
-    // previous block's bitmap rows); the table kernels alternate over the rest
-    bool taken[clb_controls_s::NSIDE] = {};
-    int k = 0;
+    constexpr int NS = clb_controls_s::NSIDE;
+    // A fork and a join cost about 50 us of a small product (186 us with both
+    // passes on three side streams, 102 on the controls' stream alone): a single
+    // kernel, and kernels over little work, run on the controls' stream one
+    // after the other, and only streams that get a kernel are waited for.
+    // Otherwise the longest kernels have slots of their own, kept rows slot 0,
+    // bitmap rows and heavy bitmap rows 0 and 1, and the table kernels alternate
+    // over the rest.  Slot 0 is the controls' stream itself, unless the caller
+    // has other work for it meanwhile: there the heavy rows start first, as
+    // they end last (behind the other bitmap rows R-MAT 2^16 took 979 us, before
+    // them 859); of two overlapping blocks they take slot 1, not behind the
+    // previous block's bitmap rows.
+    u32 kernels = 0;
+    for (u32 b = BIN_TINY; b < BIN_BITMAP0; ++b)
+        kernels += off[b + 1] != off[b] && (b != BIN_STORED || (mode == NUM && o.keep.words));
+    kernels += off[NBINS] != off[BIN_BITMAP0] && !s.cfg.esc_only ? 2 : 0;
+    if (!open && s.bin_work <= ONE_STREAM_WORK) one_stream = true;
+    const bool main0 = !defer && !open;
+    if (main0 && kernels <= 1) one_stream = true;
+    if (!one_stream) CLB_HIP(hipEventRecord(ctl->ev_fork, ctl->stream), EVENT_WAITING_ERROR);
+    bool forked[NS] = {}, taken[NS] = {};
     auto on = [&](int w) {
-        taken[w] = true;
-        return one_stream ? ctl->stream : side_stream(ctl, w);
+        if (one_stream || (main0 && w == 0)) return ctl->stream;
+        if (!forked[w]) CLB_HIP(hipStreamWaitEvent(ctl->side[w], ctl->ev_fork, 0), EVENT_WAITING_ERROR);
+        forked[w] = true;
+        return ctl->side[w];
     };
+    int k = NS - 1;
     auto next = [&]() {
-        constexpr int NS = clb_controls_s::NSIDE;
         if (one_stream) return ctl->stream;
         do k = (k + 1) % NS;
         while (taken[k] && k != NS - 1);
-        return side_stream(ctl, k);
+        return on(k);
     };
     LaunchTimer dummy;
     LaunchTimer &t = lt ? *lt : dummy;
@@ -1271,6 +1290,7 @@ void launch_bins(clb_controls_s *ctl, const Setup &s, const u32 *perm, const u32
         const u32 ns = off[BIN_STORED + 1] - off[BIN_STORED];
         if (ns && mode == NUM && o.keep.words) {
             hipStream_t st = on(0);
+            taken[0] = true;
             t.begin(st);
             emit_stored(st, perm + off[BIN_STORED], ns, o.keep, o.off, o.cols);
             t.end(fam(CLB_KK_BITMAP), st);
@@ -1296,7 +1316,9 @@ void launch_bins(clb_controls_s *ctl, const Setup &s, const u32 *perm, const u32
             for (int wide = 1; wide >= 0; --wide) {
                 const u32 r0 = wide ? 0 : heavy, nr = wide ? heavy : n - heavy;
                 if (!nr) continue;
-                hipStream_t st = on(wide || (ns && mode == NUM) ? 1 : 0);
+                const int slot = (ns && mode == NUM) || (wide != 0) != main0 ? 1 : 0;
+                hipStream_t st = on(slot);
+                taken[slot] = true;
                 t.begin(st);
                 if (mode == SYM) launch_bitmap_sym(ctl, st, s, pp, r0, nr, bits, wide != 0, o);
                 else if (mode == NUM) launch_bitmap_num(ctl, st, s, pp, r0, nr, bits, wide != 0, o);
@@ -1369,13 +1391,17 @@ void launch_bins(clb_controls_s *ctl, const Setup &s, const u32 *perm, const u32
         t.end(fam(1), st);
     }
 #undef DISPATCH3
-    if (one_stream || open) return;
-    if (!defer) {
-        join_side(ctl);
+    if (open) return;
+    if (defer) {
+        for (int j = 0; j < NS; ++j)
+            CLB_HIP(hipEventRecord(defer[j], forked[j] ? ctl->side[j] : ctl->stream), EVENT_WAITING_ERROR);
         return;
     }
-    for (int j = 0; j < clb_controls_s::NSIDE; ++j)
-        CLB_HIP(hipEventRecord(defer[j], ctl->side[j]), EVENT_WAITING_ERROR);
+    for (int j = 0; j < NS; ++j) {
+        if (!forked[j]) continue;
+        CLB_HIP(hipEventRecord(ctl->ev_join[j], ctl->side[j]), EVENT_WAITING_ERROR);
+        CLB_HIP(hipStreamWaitEvent(ctl->stream, ctl->ev_join[j], 0), EVENT_WAITING_ERROR);
+    }
 }
 
 struct Timer {

@@ -32,6 +32,7 @@ struct Setup {
     BinCfg cfg{};
     clb_dcsr b{};  // the B operand (its buffers stay owned by the caller)
     u64 bin_products[NBINS] = {};  // of the last binning read back (read_bins)
+    u64 bin_work = 0;              // its products, and A nonzeros at 4 each
     u32 *P = nullptr;  // products per row of the block: prod.ptr, or a plan's array
 };
 
@@ -164,11 +165,19 @@ void read_bins(clb_controls_s *ctl, Setup &s, BinHost &h);
 void sum_by_bin(clb_controls_s *ctl, const u32 *perm, const BinHost &h, u32 nrows, const u32 *nnz_row,
                 u64 out[NBINS]);
 // Launches the row kernels of every nonempty bin in `mode` (SYM, NUM or ONE)
-// on the side streams.  family < 0 times launches as sym_* / num_* by mode.
+// on several streams.  family < 0 times launches as sym_* / num_* by mode.
 // The controls' stream waits for them at the end, unless `defer` is given:
 // then the end of each side stream's work is recorded in defer[k] (NSIDE
 // events, made by the caller) for join_deferred.  one_stream: every kernel
-// on the controls' stream instead (no side streams).
+// on the controls' stream instead (no side streams).  open: no join, the
+// caller joins later (join_side).
+// Up to ONE_STREAM_WORK products (an A nonzero counts as four: rows of nonzeros
+// without a B row take long without products) the pass is on one stream.
+// Measured on one / on several (us): uniform 1024 x 1024 with 98 thousand
+// products 102 / 170, 3000 x 3000 with 0.3 million 112 / 178, 30000 x 30000 with
+// 0.75 million 161 / 215; at several million products and up there is no
+// difference, and 4194 rows of 98 nonzeros, most without a B row, 365 / 319.
+constexpr u64 ONE_STREAM_WORK = 3u << 19;
 void launch_bins(clb_controls_s *ctl, const Setup &s, const u32 *perm, const u32 off[NBINS + 1], int mode,
                  const Out &o, LaunchTimer *lt, int family, hipEvent_t *defer = nullptr, bool one_stream = false,
                  bool open = false);
