@@ -501,10 +501,9 @@ clb_status clb_csr_addition(clb_controls ctl, const clb_csr *a, const clb_csr *b
         na = na < a->nnz ? na : a->nnz;
         nb = nb < b->nnz ? nb : b->nnz;
         DevArray<u64> ka(ctl, na ? na : 1), kb(ctl, nb ? nb : 1);
-        expand_rows(ctl, u32p(a->rpt), nullptr, 0, a->nrows, 0, na,
-                    KeyOfNonzero{u32p(a->cols), 0, 0, ka.ptr});
-        expand_rows(ctl, u32p(b->rpt), nullptr, 0, b->nrows, 0, nb,
-                    KeyOfNonzero{u32p(b->cols), 0, 0, kb.ptr});
+        expand_rows_two(
+            ctl, Expand<KeyOfNonzero>{u32p(a->rpt), nullptr, 0, a->nrows, 0, na, {u32p(a->cols), 0, 0, ka.ptr}},
+            Expand<KeyOfNonzero>{u32p(b->rpt), nullptr, 0, b->nrows, 0, nb, {u32p(b->cols), 0, 0, kb.ptr}});
         clb_buffer_s *rows = nullptr;
         const u32 m = union_keys(ctl, ka.ptr, na, kb.ptr, nb, &rows, &r.cols);
         try {
@@ -551,10 +550,9 @@ clb_status clb_dcsr_addition(clb_controls ctl, const clb_dcsr *a, const clb_dcsr
             return;
         }
         DevArray<u64> ka(ctl, a->nnz), kb(ctl, b->nnz);
-        expand_rows(ctl, u32p(a->rpt), u32p(a->rows), 0, a->nzr, 0, a->nnz,
-                    KeyOfNonzero{u32p(a->cols), 0, 0, ka.ptr});
-        expand_rows(ctl, u32p(b->rpt), u32p(b->rows), 0, b->nzr, 0, b->nnz,
-                    KeyOfNonzero{u32p(b->cols), 0, 0, kb.ptr});
+        expand_rows_two(
+            ctl, Expand<KeyOfNonzero>{u32p(a->rpt), u32p(a->rows), 0, a->nzr, 0, a->nnz, {u32p(a->cols), 0, 0, ka.ptr}},
+            Expand<KeyOfNonzero>{u32p(b->rpt), u32p(b->rows), 0, b->nzr, 0, b->nnz, {u32p(b->cols), 0, 0, kb.ptr}});
         union_keys_to_dcsr(ctl, ka.ptr, a->nnz, kb.ptr, b->nnz, r);
         *out = r;
     });

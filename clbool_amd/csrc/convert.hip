@@ -116,7 +116,7 @@ struct RowOfNonzero {
 };
 
 void dcsr_expand_rows(clb_controls_s *ctl, const u32 *rpt, const u32 *rows, u32 nzr, u32 nnz, u32 *out_rows) {
-    expand_rows(ctl, rpt, rows, 0, nzr, 0, nnz, RowOfNonzero{out_rows});
+    expand_rows(ctl, Expand<RowOfNonzero>{rpt, rows, 0, nzr, 0, nnz, {out_rows}});
 }
 
 // dcsr_to_csr_set_size (conversions.cl:8-18)

@@ -7,6 +7,8 @@ import numpy as np
 import pytest
 
 import clbool_amd as cb
+import oracle
+from helpers import assert_dcsr_equal
 
 pytestmark = pytest.mark.gpu
 
@@ -57,3 +59,27 @@ def test_csr_addition_over_empty_rows(controls, gap):
                                     (br.astype(np.uint64) << np.uint64(32)) | bc]))
     want = np.concatenate([[0], np.cumsum(np.bincount((key >> np.uint64(32)).astype(np.int64), minlength=n))])
     assert np.array_equal(got_rpt, want) and np.array_equal(got_cols, key.astype(np.uint32))
+
+
+@pytest.mark.parametrize("na", [1, 255, 2047, 2048, 2049, 6145])
+@pytest.mark.parametrize("nb", [1, 257, 2048, 4097])
+def test_two_matrices_in_one_launch(controls, na, nb):
+    """Additions expand both operands by the same launches: sizes about a tile,
+    and one row a nonzero or rows of several."""
+    rng = np.random.default_rng(na * 7 + nb)
+    n = 9000
+    keys = []
+    for m, per in ((na, 1), (nb, 3)):
+        rows = (np.arange(m) // per).astype(np.uint64) * np.uint64(per)
+        cols = np.arange(m, dtype=np.uint64) % np.uint64(per) + rng.integers(0, n - per, m).astype(np.uint64) // 3 * 3
+        keys.append(np.unique((rows << np.uint64(32)) | cols))
+    pair = [((k >> np.uint64(32)).astype(np.uint32), k.astype(np.uint32)) for k in keys]
+    u = np.union1d(*keys)
+    ur, uc = (u >> np.uint64(32)).astype(np.uint32), u.astype(np.uint32)
+    D = [oracle.pairs_to_dcsr(r, c, n, n) for r, c in pair]
+    d = [cb.matrix_dcsr_from_cpu(controls, m.rpt, m.rows, m.cols, n) for m in D]
+    assert_dcsr_equal(controls, cb.dcsr.addition(controls, *d), oracle.pairs_to_dcsr(ur, uc, n, n), "dcsr")
+    s = [cb.csr_from_cpu(controls, *oracle.csr_from_pairs(r, c, n), n, n) for r, c in pair]
+    rpt, cols = cb.csr.matrix_addition(controls, *s).to_host(controls)
+    er, ec = oracle.csr_from_pairs(ur, uc, n)
+    assert np.array_equal(rpt, er) and np.array_equal(cols, ec)
