@@ -49,7 +49,8 @@ __global__ __launch_bounds__(SEG_WG) void k_esc_segs(const u32 *__restrict__ per
         const u32 i = i0 + threadIdx.x;
         const u32 P = i < n ? prod[perm[i]] : 0u;
         u64 all;
-        const u64 x = carry + dev::block_excl_scan<u64, SEG_WG>(((u64)P << 32) | (P / RX_TILE + (P % RX_TILE ? 1u : 0u)), red, all);
+        const u32 nt = P / RX_TILE + (P % RX_TILE ? 1u : 0u);
+        const u64 x = carry + dev::block_excl_scan<u64, SEG_WG>(((u64)P << 32) | nt, red, all);
         if (i < n) segs[i] = make_uint2((u32)(x >> 32), (u32)x);
         carry += all;
     }

@@ -77,8 +77,11 @@ typedef struct clb_tuning {
                                       words) whose first window holds at least
                                       this many set bits per 1024 words are
                                       dumped and expanded by a separate emission
-                                      kernel (>= 65536: off; 0: 1024 in the
-                                      learned one pass, off in the numeric pass) */
+                                      kernel (>= 65536: off; 0: 64 in the
+                                      learned one pass, off in the numeric
+                                      pass, and bitmap rows are kept by the
+                                      pass that finds them where that gathers
+                                      their products once)                    */
     uint32_t bitmap_persistent;    /* nonzero: the bitmap rows run on a persistent
                                       grid that takes rows from a counter
                                       instead of one workgroup per row          */
