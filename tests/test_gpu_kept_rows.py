@@ -95,3 +95,27 @@ def test_packed(controls, ncols):
     a, b = upload(controls, A, nrows, inner), upload(controls, B, inner, ncols)
     assert_dcsr_equal(controls, cb.dcsr.matrix_multiplication_hash(controls, a, b), ref, "plain")
     assert_dcsr_equal(controls, cb.dcsr.spgemm(controls, a, b, mode=cb.SPGEMM_BOUND)[0], ref, "bound")
+
+
+@pytest.mark.parametrize("ncols", [4097, 1100000])
+@pytest.mark.parametrize("lens", [(9000,), (2048,), (512, 1536, 4096, 2047, 2049)])
+def test_packed_with_empty_stored_rows(controls, ncols, lens):
+    """Stored rows of B without entries, before, between and after the others,
+    where rows end at the packing's tiles of 2048 columns and where they don't,
+    against the product without them."""
+    rng = np.random.default_rng(ncols + len(lens))
+    full = 40
+    n = np.minimum(np.resize(lens, full), ncols)
+    ids = np.arange(full) * 4 + 3  # ids 4k .. 4k + 2 may be stored without entries
+    cols = np.concatenate([np.sort(rng.choice(min(ncols, 3 * k), k, replace=False)) for k in n])
+    inner, nrows = 4 * full + 8, 800
+    stored = np.sort(np.concatenate([ids, [0, 1, 2, 40, 41, 81, 82], [inner - 3, inner - 1]]))
+    length = dict(zip(ids, n))
+    rpt = np.concatenate([[0], np.cumsum([length.get(k, 0) for k in stored])]).astype(np.uint32)
+    A = _dcsr(np.repeat(np.arange(nrows), 60), rng.integers(0, inner, nrows * 60), nrows, inner)
+    B = _dcsr(np.repeat(ids, n), cols, inner, ncols)
+    ref = oracle.spgemm(A, B)
+    a = upload(controls, A, nrows, inner)
+    b = cb.matrix_dcsr_from_cpu(controls, rpt, stored.astype(np.uint32), cols.astype(np.uint32), inner, ncols)
+    assert_dcsr_equal(controls, cb.dcsr.spgemm(controls, a, b, mode=cb.SPGEMM_BOUND)[0], ref, "bound")
+    assert_dcsr_equal(controls, cb.dcsr.matrix_multiplication_hash(controls, a, b), ref, "plain")
