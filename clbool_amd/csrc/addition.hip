@@ -437,7 +437,7 @@ using namespace clb;
 extern "C" {
 
 clb_status clb_coo_addition(clb_controls ctl, const clb_coo *a, const clb_coo *b, clb_coo *out) {
-    return run_guarded([&] {
+    return run_guarded(ctl, [&] {
         check_same_shape(a->nrows, a->ncols, b->nrows, b->ncols);
         clb_coo r{};
         r.nrows = a->nrows;
@@ -453,6 +453,7 @@ clb_status clb_coo_addition(clb_controls ctl, const clb_coo *a, const clb_coo *b
                 r.cols = copy_buffer(ctl, f->cols, 4ull * f->nnz);
                 sync(ctl);
             } catch (...) {
+                settle(ctl);
                 clb_coo_release(&r);
                 throw;
             }
@@ -470,7 +471,7 @@ clb_status clb_coo_addition(clb_controls ctl, const clb_coo *a, const clb_coo *b
 }
 
 clb_status clb_csr_addition(clb_controls ctl, const clb_csr *a, const clb_csr *b, clb_csr *out) {
-    return run_guarded([&] {
+    return run_guarded(ctl, [&] {
         check_same_shape(a->nrows, a->ncols, b->nrows, b->ncols);
         clb_csr r{};
         r.nrows = a->nrows;
@@ -486,6 +487,7 @@ clb_status clb_csr_addition(clb_controls ctl, const clb_csr *a, const clb_csr *b
                 r.cols = copy_buffer(ctl, f->cols, 4ull * f->nnz);
                 sync(ctl);
             } catch (...) {
+                settle(ctl);
                 clb_csr_release(&r);
                 throw;
             }
@@ -513,6 +515,7 @@ clb_status clb_csr_addition(clb_controls ctl, const clb_csr *a, const clb_csr *b
             CLB_LAUNCHED("rows_lower_bound");
             sync(ctl);
         } catch (...) {
+            settle(ctl);
             buffer_release(rows);
             clb_csr_release(&r);
             throw;
@@ -524,7 +527,7 @@ clb_status clb_csr_addition(clb_controls ctl, const clb_csr *a, const clb_csr *b
 }
 
 clb_status clb_dcsr_addition(clb_controls ctl, const clb_dcsr *a, const clb_dcsr *b, clb_dcsr *out) {
-    return run_guarded([&] {
+    return run_guarded(ctl, [&] {
         check_same_shape(a->nrows, a->ncols, b->nrows, b->ncols);
         clb_dcsr r{};
         r.nrows = a->nrows;
@@ -541,6 +544,7 @@ clb_status clb_dcsr_addition(clb_controls ctl, const clb_dcsr *a, const clb_dcsr
                 r.cols = copy_buffer(ctl, f->cols, 4ull * f->nnz);
                 sync(ctl);
             } catch (...) {
+                settle(ctl);
                 clb_dcsr_release(&r);
                 throw;
             }

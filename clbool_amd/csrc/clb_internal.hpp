@@ -23,7 +23,7 @@
 #include <vector>
 
 #include "../../include/clbool_c.h"
-#include "block_heap.hpp"
+#include "pool_blocks.hpp"
 
 namespace clb {
 
@@ -77,12 +77,22 @@ class Pool {
     static constexpr u64 SEG_MIN = 1ull << 30;    // smallest segment of the large requests
     explicit Pool(int device) : device_(device) {}
     ~Pool();
-    void *alloc(u64 bytes, u64 *cap_out);
-    void release(void *p, u64 cap);
+    // For work on the Controls' stream, in memory that earlier work there may
+    // still use (`own`), or for anyone.
+    void *alloc(u64 bytes, u64 *cap_out, clb_controls_s *ctl, bool own);
+    // Nothing in flight uses p.
+    void release(void *p);
+    // Work on the Controls' stream may still use p.
+    void retire(void *p, u64 cap, clb_controls_s *ctl);
+    // Waits for the Controls' stream, after which what it retired is anyone's.
+    void wait(clb_controls_s *ctl);
+    // The Controls begins, and ends (its streams have been waited for).
+    void enter(clb_controls_s *ctl);
+    void leave(clb_controls_s *ctl);
     void trim();
     u64 cached_bytes() const {
         std::lock_guard<std::mutex> lk(mu_);
-        return small_.free_bytes() + large_.free_bytes();
+        return blocks_.free_bytes();
     }
     int device() const { return device_; }
     // [0] free bytes inside the pool's segments, [1] hipMalloc calls, [2]
@@ -90,7 +100,7 @@ class Pool {
     // failed hipMalloc
     void stats(u64 out[4]) const {
         std::lock_guard<std::mutex> lk(mu_);
-        out[0] = small_.free_bytes() + large_.free_bytes();
+        out[0] = blocks_.free_bytes();
         out[1] = mallocs_;
         out[2] = malloc_bytes_;
         out[3] = drops_;
@@ -100,9 +110,11 @@ class Pool {
     // hands entirely free segments back to HIP (counted in drops_ after a
     // failed hipMalloc)
     void drop_free_segments(bool after_failure);
+    // gives back what Controls whose streams are idle have retired
+    void give_back_idle();
     int device_;
     mutable std::mutex mu_;
-    BlockHeap small_{256}, large_{2ull << 20};
+    PoolBlocks blocks_{SMALL_MAX, 256, 2ull << 20};
     u64 mallocs_ = 0, malloc_bytes_ = 0, drops_ = 0;
 };
 Pool &pool_for(int device);
@@ -137,6 +149,9 @@ struct clb_controls_s {
     // the next block's passes
     static constexpr int NTAIL = 2;
     hipStream_t tail[NTAIL] = {};
+    clb::Pool *pool = nullptr;    // its device's
+    clb::PoolBlocks::Owner retired;  // released temporaries (under the pool's lock)
+    bool settled = false;         // see Settled
     std::mutex mu;
 };
 
@@ -148,29 +163,50 @@ void buffer_release(clb_buffer_s *b);
 inline u32 *u32p(clb_buffer_s *b) { return b ? static_cast<u32 *>(b->ptr) : nullptr; }
 inline const u32 *u32p(const clb_buffer_s *b) { return b ? static_cast<const u32 *>(b->ptr) : nullptr; }
 
-// RAII temporary device array from the pool.
+// RAII temporary device array from the pool.  Once released it may be reused by
+// later work on the controls' stream, and by others after that stream has been
+// waited for.
 template <typename T>
 struct DevArray {
     T *ptr = nullptr;
     u64 n = 0;
     u64 cap = 0;
-    int device = 0;
+    clb_controls_s *ctl = nullptr;
     DevArray() = default;
-    DevArray(clb_controls_s *ctl, u64 count) { reset(ctl, count); }
-    void reset(clb_controls_s *ctl, u64 count) {
+    DevArray(clb_controls_s *c, u64 count) { reset(c, count); }
+    void reset(clb_controls_s *c, u64 count) {
         free_();
         n = count;
-        device = ctl->device;
-        if (count) ptr = static_cast<T *>(pool_for(device).alloc(count * sizeof(T), &cap));
+        ctl = c;
+        if (count) ptr = static_cast<T *>(ctl->pool->alloc(count * sizeof(T), &cap, ctl, true));
     }
     ~DevArray() { free_(); }
     DevArray(const DevArray &) = delete;
     DevArray &operator=(const DevArray &) = delete;
-    DevArray(DevArray &&o) noexcept : ptr(o.ptr), n(o.n), cap(o.cap), device(o.device) { o.ptr = nullptr; }
+    DevArray(DevArray &&o) noexcept : ptr(o.ptr), n(o.n), cap(o.cap), ctl(o.ctl) { o.ptr = nullptr; }
+    void swap(DevArray &o) {
+        std::swap(ptr, o.ptr);
+        std::swap(n, o.n);
+        std::swap(cap, o.cap);
+        std::swap(ctl, o.ctl);
+    }
     void free_() {
-        if (ptr) pool_for(device).release(ptr, cap);
+        if (ptr) {
+            if (ctl->settled) ctl->pool->release(ptr);
+            else ctl->pool->retire(ptr, cap, ctl);
+        }
         ptr = nullptr;
     }
+};
+
+// While one of these lives, arrays of the controls that are released were
+// waited for: nothing in flight uses them.
+struct Settled {
+    clb_controls_s *ctl;
+    explicit Settled(clb_controls_s *c) : ctl(c) { ctl->settled = true; }
+    ~Settled() { ctl->settled = false; }
+    Settled(const Settled &) = delete;
+    Settled &operator=(const Settled &) = delete;
 };
 
 // The main stream waits for the side streams.
@@ -181,6 +217,9 @@ constexpr u64 PINNED_BYTES = 4096;
 // Small synchronous readback through the pinned staging area.
 void readback(clb_controls_s *ctl, void *host, const void *dev, u64 bytes);
 void sync(clb_controls_s *ctl);
+// Waits for all streams of the controls, errors ignored: before a failed call
+// releases buffers that its kernels may still use.
+void settle(clb_controls_s *ctl) noexcept;
 
 // Launch-size helpers.
 inline u32 div_up(u64 a, u64 b) { return static_cast<u32>((a + b - 1) / b); }
@@ -200,6 +239,8 @@ void exclusive_scan_u32_to_u64(clb_controls_s *ctl, const u32 *in, u64 *out, u64
 
 // Runs body, mapping exceptions to C-ABI status codes (runtime.hip).
 clb_status run_guarded(const std::function<void()> &body);
+// The same; a call that fails leaves nothing in flight on the controls.
+clb_status run_guarded(clb_controls_s *ctl, const std::function<void()> &body);
 
 // Frees the learned predictor's device state of a Controls (learned.hip).
 void learned_destroy_state(clb_controls_s *ctl);

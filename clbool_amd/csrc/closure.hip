@@ -361,7 +361,7 @@ extern "C" {
 
 clb_status clb_closure_step(clb_controls ctl, clb_dcsr *mats, uint32_t nmats, const uint32_t *triples,
                             uint32_t ntriples, const clb_closure_opts *opts, clb_closure_stats *stats) {
-    return run_guarded([&] {
+    return run_guarded(ctl, [&] {
         clb_closure_opts o{};
         if (opts) o = *opts;
         clb_closure_stats st{};
@@ -408,6 +408,7 @@ clb_status clb_closure_step(clb_controls ctl, clb_dcsr *mats, uint32_t nmats, co
                     x = u;
                 }
             } catch (...) {
+                settle(ctl);
                 for (auto &p : prods) clb_dcsr_release(&p);
                 throw;
             }
@@ -550,7 +551,7 @@ clb_status clb_closure_step(clb_controls ctl, clb_dcsr *mats, uint32_t nmats, co
                     }
                 }
             } catch (...) {
-                (void)hipStreamSynchronize(ctl->stream);
+                settle(ctl);
                 release_all();
                 clb_dcsr_release(&Y);
                 clb_dcsr_release(&Z);
@@ -564,6 +565,7 @@ clb_status clb_closure_step(clb_controls ctl, clb_dcsr *mats, uint32_t nmats, co
                 unite_products(ctl, mats, xs, triples, ntriples, n, prods, splits);
                 sync(ctl);
             } catch (...) {
+                settle(ctl);
                 release_all();
                 throw;
             }

@@ -151,7 +151,7 @@ using namespace clb;
 extern "C" {
 
 clb_status clb_coo_to_dcsr_shallow(clb_controls ctl, const clb_coo *a, clb_dcsr *out) {
-    return run_guarded([&] {
+    return run_guarded(ctl, [&] {
         clb_dcsr r{};
         r.nrows = a->nrows;
         r.ncols = a->ncols;
@@ -184,6 +184,7 @@ static void dcsr_to_coo(clb_controls ctl, const clb_dcsr *a, clb_coo *out, bool 
             }
             sync(ctl);
         } catch (...) {
+            settle(ctl);
             clb_coo_release(&r);
             throw;
         }
@@ -193,15 +194,15 @@ static void dcsr_to_coo(clb_controls ctl, const clb_dcsr *a, clb_coo *out, bool 
 }
 
 clb_status clb_dcsr_to_coo_shallow(clb_controls ctl, const clb_dcsr *a, clb_coo *out) {
-    return run_guarded([&] { dcsr_to_coo(ctl, a, out, false); });
+    return run_guarded(ctl, [&] { dcsr_to_coo(ctl, a, out, false); });
 }
 
 clb_status clb_dcsr_to_coo_deep(clb_controls ctl, const clb_dcsr *a, clb_coo *out) {
-    return run_guarded([&] { dcsr_to_coo(ctl, a, out, true); });
+    return run_guarded(ctl, [&] { dcsr_to_coo(ctl, a, out, true); });
 }
 
 clb_status clb_dcsr_to_csr(clb_controls ctl, const clb_dcsr *a, clb_csr *out) {
-    return run_guarded([&] {
+    return run_guarded(ctl, [&] {
         clb_csr r{};
         r.nrows = a->nrows;
         r.ncols = a->ncols;
@@ -223,6 +224,7 @@ clb_status clb_dcsr_to_csr(clb_controls ctl, const clb_dcsr *a, clb_csr *out) {
             // :268
             if (c_nnz != a->nnz) raise(INVALID_VALUE, "nnz in dcsr and csr matrices should be equal!");
         } catch (...) {
+            settle(ctl);
             buffer_release(r.rpt);
             throw;
         }
@@ -234,7 +236,7 @@ clb_status clb_dcsr_to_csr(clb_controls ctl, const clb_dcsr *a, clb_csr *out) {
 }
 
 clb_status clb_csr_to_dcsr(clb_controls ctl, const clb_csr *a, clb_dcsr *out) {
-    return run_guarded([&] {
+    return run_guarded(ctl, [&] {
         clb_dcsr r{};
         r.nrows = a->nrows;
         r.ncols = a->ncols;

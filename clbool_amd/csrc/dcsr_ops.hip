@@ -135,7 +135,7 @@ using namespace clb;
 extern "C" {
 
 clb_status clb_dcsr_digest(clb_controls ctl, const clb_dcsr *a, uint64_t *digest) {
-    return run_guarded([&] {
+    return run_guarded(ctl, [&] {
         if (!a || !digest) raise(INVALID_ARGUMENT, "null argument");
         u64 h[2] = {0, 0};
         if (a->nzr && a->nnz) {
@@ -154,7 +154,7 @@ clb_status clb_dcsr_digest(clb_controls ctl, const clb_dcsr *a, uint64_t *digest
 }
 
 clb_status clb_dcsr_transpose(clb_controls ctl, const clb_dcsr *a, clb_dcsr *out) {
-    return run_guarded([&] {
+    return run_guarded(ctl, [&] {
         clb_dcsr r{};
         r.nrows = a->ncols;
         r.ncols = a->nrows;
@@ -177,6 +177,7 @@ clb_status clb_dcsr_transpose(clb_controls ctl, const clb_dcsr *a, clb_dcsr *out
             r.nnz = a->nnz;
             buffer_release(rows);
         } catch (...) {
+            settle(ctl);
             buffer_release(rows);
             release_dcsr(r);
             throw;
@@ -187,7 +188,7 @@ clb_status clb_dcsr_transpose(clb_controls ctl, const clb_dcsr *a, clb_dcsr *out
 
 clb_status clb_dcsr_submatrix(clb_controls ctl, const clb_dcsr *a, uint32_t i, uint32_t j, uint32_t nrows,
                               uint32_t ncols, clb_dcsr *out) {
-    return run_guarded([&] {
+    return run_guarded(ctl, [&] {
         // every empty outcome is a 0 x 0 matrix, as in the reference
         // (:101-108, :112-115, :125-128)
         clb_dcsr r{};
@@ -244,7 +245,7 @@ clb_status clb_dcsr_submatrix(clb_controls ctl, const clb_dcsr *a, uint32_t i, u
 }
 
 clb_status clb_dcsr_reduce(clb_controls ctl, const clb_dcsr *a, clb_dcsr *out) {
-    return run_guarded([&] {
+    return run_guarded(ctl, [&] {
         clb_dcsr r{};
         if (a->nnz == 0) {  // :7-10
             *out = r;

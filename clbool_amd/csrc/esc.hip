@@ -322,7 +322,7 @@ void spgemm_esc(clb_controls_s *ctl, const clb_dcsr &a, const clb_dcsr &b, clb_d
                 assemble(ctl, s, a, nnz_row.ptr, offs.ptr, pos.ptr, nnz, nzr, cols, out);
                 sync(ctl);
             } catch (...) {
-                (void)hipStreamSynchronize(ctl->stream);
+                settle(ctl);
                 clb_dcsr_release(&out);
                 if (!out.cols) buffer_release(cols);
                 throw;
@@ -331,8 +331,7 @@ void spgemm_esc(clb_controls_s *ctl, const clb_dcsr &a, const clb_dcsr &b, clb_d
         st.nnz = nnz;
         st.nzr = nzr;
     } catch (...) {
-        for (int k = 0; k < clb_controls_s::NSIDE; ++k) (void)hipStreamSynchronize(side_stream(ctl, k));
-        (void)hipStreamSynchronize(ctl->stream);
+        settle(ctl);
         throw;
     }
 }
@@ -345,7 +344,7 @@ using namespace clb;
 extern "C" {
 
 clb_status clb_dcsr_spgemm_esc(clb_controls ctl, const clb_dcsr *a, const clb_dcsr *b, clb_dcsr *out) {
-    return run_guarded([&] {
+    return run_guarded(ctl, [&] {
         if (!a || !b || !out) raise(INVALID_ARGUMENT, "null argument");
         clb_spgemm_stats st;
         clb_dcsr r{};

@@ -123,7 +123,7 @@ template <typename F>
 void expand_rows(clb_controls_s *ctl, const Expand<F> &x) {
     const u32 tiles = x.tiles();
     if (!tiles) return;
-    DevArray<u32> first(ctl, tiles);  // reused only by later work on this stream
+    DevArray<u32> first(ctl, tiles);
     k_tile_rows<EX_TILE>
         <<<div_up(x.r_hi - x.r_lo, EX_WG), EX_WG, 0, ctl->stream>>>(x.rpt, x.r_lo, x.r_hi, x.e_lo, x.e_hi, first.ptr);
     CLB_LAUNCHED("tile_rows");

@@ -109,7 +109,7 @@ using namespace clb;
 extern "C" {
 
 clb_status clb_dcsr_kronecker(clb_controls ctl, const clb_dcsr *a, const clb_dcsr *b, clb_dcsr *out) {
-    return run_guarded([&] {
+    return run_guarded(ctl, [&] {
         const u64 c_nnz = (u64)a->nnz * b->nnz;
         const u64 c_nzr = (u64)a->nzr * b->nzr;
         const u64 c_nrows = (u64)a->nrows * b->nrows;
@@ -152,7 +152,7 @@ clb_status clb_dcsr_kronecker(clb_controls ctl, const clb_dcsr *a, const clb_dcs
             CLB_LAUNCHED("calculate_kronecker_product");
             sync(ctl);
         } catch (...) {
-            (void)hipStreamSynchronize(ctl->stream);
+            settle(ctl);
             clb_dcsr_release(&r);
             throw;
         }

@@ -892,7 +892,7 @@ using namespace clb::spg;
 extern "C" {
 
 clb_status clb_predictor_reset(clb_controls ctl, uint32_t seed) {
-    return run_guarded([&] {
+    return run_guarded(ctl, [&] {
         Learned *L = state(ctl);
         init_params(ctl, L, seed);
         L->n = 0;
@@ -902,7 +902,7 @@ clb_status clb_predictor_reset(clb_controls ctl, uint32_t seed) {
 
 clb_status clb_predictor_harvest(clb_controls ctl, const clb_dcsr *a, const clb_dcsr *b, uint32_t max_rows,
                                  uint64_t *total_samples) {
-    return run_guarded([&] {
+    return run_guarded(ctl, [&] {
         check_dims(*a, *b);
         Learned *L = state(ctl);
         if (!L->ready) {
@@ -934,12 +934,8 @@ clb_status clb_predictor_harvest(clb_controls ctl, const clb_dcsr *a, const clb_
                             COPY_BUFFER_ERROR);
                 }
                 sync(ctl);
-                std::swap(L->X.ptr, X2.ptr);
-                std::swap(L->X.cap, X2.cap);
-                std::swap(L->X.n, X2.n);
-                std::swap(L->Y.ptr, Y2.ptr);
-                std::swap(L->Y.cap, Y2.cap);
-                std::swap(L->Y.n, Y2.n);
+                L->X.swap(X2);
+                L->Y.swap(Y2);
                 L->cap = ncap;
             }
             k_harvest<<<div_up(take, 256), 256, 0, ctl->stream>>>(feat.ptr, s.prod.ptr, nnz_row.ptr, nrows, stride,
@@ -953,7 +949,7 @@ clb_status clb_predictor_harvest(clb_controls ctl, const clb_dcsr *a, const clb_
 }
 
 clb_status clb_predictor_train(clb_controls ctl, const clb_train_opts *opts, clb_train_stats *stats) {
-    return run_guarded([&] {
+    return run_guarded(ctl, [&] {
         Learned *L = state(ctl);
         if (!L->ready || L->n == 0) raise(INVALID_VALUE, "no harvested samples to train on");
         const u32 epochs = opts ? opts->epochs : 20;
@@ -1002,7 +998,7 @@ clb_status clb_predictor_train(clb_controls ctl, const clb_train_opts *opts, clb
 }
 
 clb_status clb_predictor_get_params(clb_controls ctl, float *params, uint32_t n) {
-    return run_guarded([&] {
+    return run_guarded(ctl, [&] {
         ensure_ready(ctl);
         if (n != NPARAM) raise(INVALID_ARGUMENT, "expected CLB_MLP_PARAMS parameters");
         readback(ctl, params, state(ctl)->params.ptr, NPARAM * 4);
@@ -1010,7 +1006,7 @@ clb_status clb_predictor_get_params(clb_controls ctl, float *params, uint32_t n)
 }
 
 clb_status clb_predictor_set_params(clb_controls ctl, const float *params, uint32_t n) {
-    return run_guarded([&] {
+    return run_guarded(ctl, [&] {
         if (n != NPARAM) raise(INVALID_ARGUMENT, "expected CLB_MLP_PARAMS parameters");
         Learned *L = state(ctl);
         if (!L->params.ptr) init_params(ctl, L, 1);
@@ -1025,7 +1021,7 @@ clb_status clb_predictor_set_params(clb_controls ctl, const float *params, uint3
 }
 
 clb_status clb_predictor_predict(clb_controls ctl, const clb_dcsr *a, const clb_dcsr *b, float *pred_nnz) {
-    return run_guarded([&] {
+    return run_guarded(ctl, [&] {
         check_dims(*a, *b);
         ensure_ready(ctl);
         if (!a->nzr) return;
@@ -1046,7 +1042,7 @@ clb_status clb_predictor_predict(clb_controls ctl, const clb_dcsr *a, const clb_
 }
 
 clb_status clb_mlp_forward(clb_controls ctl, const float *params, const float *x, uint32_t n, float *y) {
-    return run_guarded([&] {
+    return run_guarded(ctl, [&] {
         if (!n) return;
         DevArray<float> p(ctl, NPARAM), dx(ctl, (u64)n * NF), dy(ctl, n);
         CLB_HIP(hipMemcpyAsync(p.ptr, params, NPARAM * 4, hipMemcpyHostToDevice, ctl->stream), WRITE_BUFFER_ERROR);
@@ -1059,7 +1055,7 @@ clb_status clb_mlp_forward(clb_controls ctl, const float *params, const float *x
 
 clb_status clb_mlp_loss_grad(clb_controls ctl, const float *params, const float *x, const float *t, uint32_t n,
                              float *grad, float *loss) {
-    return run_guarded([&] {
+    return run_guarded(ctl, [&] {
         if (!n) raise(INVALID_ARGUMENT, "empty batch");
         Learned L;
         L.params.reset(ctl, NPARAM);
@@ -1085,7 +1081,7 @@ clb_status clb_mlp_loss_grad(clb_controls ctl, const float *params, const float 
 
 clb_status clb_mlp_adam(clb_controls ctl, float *params, float *m, float *v, const float *grad, float lr, float b1,
                         float b2, float eps, uint32_t step) {
-    return run_guarded([&] {
+    return run_guarded(ctl, [&] {
         if (!step) raise(INVALID_ARGUMENT, "Adam steps count from 1");
         DevArray<float> p(ctl, NPARAM), dm(ctl, NPARAM), dv(ctl, NPARAM), g(ctl, NPARAM);
         CLB_HIP(hipMemcpyAsync(p.ptr, params, NPARAM * 4, hipMemcpyHostToDevice, ctl->stream), WRITE_BUFFER_ERROR);

@@ -276,7 +276,7 @@ extern "C" {
 
 clb_status clb_spgemm_plan_create(clb_controls ctl, const clb_dcsr *a, const clb_dcsr *b, uint32_t mode,
                                   uint64_t block_bound, clb_spgemm_plan *out) {
-    return run_guarded([&] {
+    return run_guarded(ctl, [&] {
         if (!ctl || !a || !b || !out) raise(INVALID_ARGUMENT, "null argument");
         auto *p = new clb_spgemm_plan_s();
         try {
@@ -307,7 +307,7 @@ clb_status clb_spgemm_plan_block(clb_spgemm_plan plan, uint32_t k, uint32_t *row
 
 clb_status clb_spgemm_plan_run(clb_controls ctl, clb_spgemm_plan plan, uint32_t k, uint32_t timing, clb_dcsr *out,
                                clb_spgemm_stats *stats) {
-    return run_guarded([&] {
+    return run_guarded(ctl, [&] {
         if (!plan || !out) raise(INVALID_ARGUMENT, "null argument");
         clb_spgemm_stats st;
         clb_dcsr r{};
@@ -319,7 +319,7 @@ clb_status clb_spgemm_plan_run(clb_controls ctl, clb_spgemm_plan plan, uint32_t 
 
 clb_status clb_spgemm_plan_run_all(clb_controls ctl, clb_spgemm_plan plan, uint32_t timing, clb_spgemm_block_fn fn,
                                    void *user) {
-    return run_guarded([&] {
+    return run_guarded(ctl, [&] {
         if (!plan || !fn) raise(INVALID_ARGUMENT, "null argument");
         spg::plan_run_all(ctl, *plan, timing != 0, fn, user);
     });
@@ -328,7 +328,8 @@ clb_status clb_spgemm_plan_run_all(clb_controls ctl, clb_spgemm_plan plan, uint3
 clb_status clb_spgemm_plan_release(clb_spgemm_plan plan) {
     return run_guarded([&] {
         if (!plan) return;
-        (void)hipStreamSynchronize(plan->ctl->stream);
+        settle(plan->ctl);
+        Settled idle(plan->ctl);
         clb_dcsr_release(&plan->a);
         clb_dcsr_release(&plan->b);
         delete plan;

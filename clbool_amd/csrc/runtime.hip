@@ -35,16 +35,26 @@ static u64 round_capacity(u64 bytes) {
     return (bytes + g - 1) / g * g;
 }
 
-void *Pool::alloc(u64 bytes, u64 *cap_out) {
+void *Pool::alloc(u64 bytes, u64 *cap_out, clb_controls_s *ctl, bool own) {
     const u64 cap = round_capacity(bytes ? bytes : 1);
     const bool small = cap <= SMALL_MAX;
-    BlockHeap &heap = small ? small_ : large_;
-    {
+    auto take = [&](bool reclaim) -> void * {
         std::lock_guard<std::mutex> lk(mu_);
-        if (BlockHeap::Block *b = heap.take(cap)) {
-            *cap_out = b->size;
-            return b->ptr;
-        }
+        if (reclaim) blocks_.reclaim();
+        const PoolBlocks::Block b = blocks_.take(cap, &ctl->retired, own);
+        *cap_out = b.size;
+        return b.ptr;
+    };
+    if (void *p = take(false)) return p;
+    // what Controls keep after a wait; then, before the pool grows, what they
+    // have retired since if their streams are idle, and for a large request what
+    // its own stream works on
+    if (void *p = take(true)) return p;
+    give_back_idle();
+    if (void *p = take(false)) return p;
+    if (!small) {
+        wait(ctl);
+        if (void *p = take(true)) return p;
     }
     // a new segment: SEG_MIN or the request, whichever is larger (only the
     // request itself when that much is not available)
@@ -68,6 +78,11 @@ void *Pool::alloc(u64 bytes, u64 *cap_out) {
     if (e != hipSuccess) {
         (void)hipGetLastError();
         drop_free_segments(true);
+        // (its wait also freed what was retired in other segments)
+        if (void *q = take(true)) {
+            if (prev != device_) (void)hipSetDevice(prev);
+            return q;
+        }
         e = try_malloc();
     }
     if (prev != device_) (void)hipSetDevice(prev);
@@ -80,31 +95,76 @@ void *Pool::alloc(u64 bytes, u64 *cap_out) {
     std::lock_guard<std::mutex> lk(mu_);
     ++mallocs_;
     malloc_bytes_ += got;
-    heap.add_segment(static_cast<char *>(p), got);
-    BlockHeap::Block *b = heap.take(cap);  // fits: the new segment holds cap bytes
-    *cap_out = b->size;
-    return b->ptr;
+    blocks_.add_segment(static_cast<char *>(p), got, cap);
+    const PoolBlocks::Block b = blocks_.take(cap, nullptr, false);  // fits: the new segment holds cap bytes
+    *cap_out = b.size;
+    return b.ptr;
 }
 
-void Pool::release(void *p, u64) {
+void Pool::release(void *p) {
     if (!p) return;
     std::lock_guard<std::mutex> lk(mu_);
-    if (!small_.give_back(static_cast<char *>(p))) (void)large_.give_back(static_cast<char *>(p));
+    (void)blocks_.give_back(static_cast<char *>(p));
+}
+
+void Pool::retire(void *p, u64 cap, clb_controls_s *ctl) {
+    std::lock_guard<std::mutex> lk(mu_);
+    blocks_.retire({static_cast<char *>(p), cap}, &ctl->retired);
+}
+
+void Pool::wait(clb_controls_s *ctl) {
+    u64 began;
+    {
+        std::lock_guard<std::mutex> lk(mu_);
+        began = blocks_.wait_begins();  // what is retired meanwhile is not covered by it
+    }
+    CLB_HIP(hipStreamSynchronize(ctl->stream), EVENT_WAITING_ERROR);
+    std::lock_guard<std::mutex> lk(mu_);
+    blocks_.waited(&ctl->retired, began);
+}
+
+void Pool::enter(clb_controls_s *ctl) {
+    std::lock_guard<std::mutex> lk(mu_);
+    ctl->retired.tag = ctl;
+    blocks_.enter(&ctl->retired);
+}
+
+void Pool::leave(clb_controls_s *ctl) {
+    std::lock_guard<std::mutex> lk(mu_);
+    blocks_.leave(&ctl->retired);
+}
+
+void Pool::give_back_idle() {
+    // under the lock: no Controls ends, and none retires more, meanwhile
+    std::lock_guard<std::mutex> lk(mu_);
+    for (PoolBlocks::Owner *o : blocks_.owners()) {
+        if (o->list.empty()) continue;
+        if (hipStreamQuery(static_cast<clb_controls_s *>(o->tag)->stream) == hipSuccess)
+            blocks_.reclaim(o, blocks_.wait_begins());
+        else
+            (void)hipGetLastError();  // not ready
+    }
 }
 
 void Pool::drop_free_segments(bool after_failure) {
-    std::vector<std::pair<char *, u64>> drop;
+    u64 began;
     {
         std::lock_guard<std::mutex> lk(mu_);
-        small_.collect_free_segments(drop);
-        large_.collect_free_segments(drop);
+        began = blocks_.wait_begins();
         if (after_failure) ++drops_;
     }
-    if (drop.empty()) return;
     int prev = 0;
     (void)hipGetDevice(&prev);
     (void)hipSetDevice(device_);
-    (void)hipDeviceSynchronize();
+    const hipError_t e = hipDeviceSynchronize();
+    if (e != hipSuccess) (void)hipGetLastError();
+    std::vector<std::pair<char *, u64>> drop;
+    {
+        std::lock_guard<std::mutex> lk(mu_);
+        if (e == hipSuccess)
+            for (PoolBlocks::Owner *o : blocks_.owners()) blocks_.reclaim(o, began);
+        blocks_.collect_free_segments(drop);
+    }
     for (auto &kv : drop) (void)hipFree(kv.first);
     (void)hipSetDevice(prev);
 }
@@ -129,7 +189,8 @@ clb_buffer_s *buffer_new(clb_controls_s *ctl, u64 bytes) {
     b->device = ctl->device;
     b->bytes = bytes;
     try {
-        b->ptr = pool_for(ctl->device).alloc(bytes, &b->cap);
+        // the caller may use it on other streams
+        b->ptr = ctl->pool->alloc(bytes, &b->cap, ctl, false);
     } catch (...) {
         delete b;
         throw;
@@ -144,12 +205,21 @@ void buffer_retain(clb_buffer_s *b) {
 void buffer_release(clb_buffer_s *b) {
     if (!b) return;
     if (b->refs.fetch_sub(1, std::memory_order_acq_rel) == 1) {
-        pool_for(b->device).release(b->ptr, b->cap);
+        pool_for(b->device).release(b->ptr);
         delete b;
     }
 }
 
-void sync(clb_controls_s *ctl) { CLB_HIP(hipStreamSynchronize(ctl->stream), EVENT_WAITING_ERROR); }
+void sync(clb_controls_s *ctl) { ctl->pool->wait(ctl); }
+
+void settle(clb_controls_s *ctl) noexcept {
+    try {
+        ctl->pool->wait(ctl);
+    } catch (...) {
+    }
+    for (hipStream_t st : ctl->side) (void)hipStreamSynchronize(st);
+    for (hipStream_t st : ctl->tail) (void)hipStreamSynchronize(st);
+}
 
 void join_side(clb_controls_s *ctl) {
     for (int k = 0; k < clb_controls_s::NSIDE; ++k) {
@@ -340,6 +410,7 @@ clb_status clb_controls_create(uint32_t platform_id, uint32_t device_id, clb_con
                                             ". Run show_devices() to enumerate available platforms and devices.");
         auto *c = new clb_controls_s();
         c->device = static_cast<int>(device_id);
+        c->pool = &pool_for(c->device);
         try {
             CLB_HIP(hipSetDevice(c->device), CREATE_CONTROLS_ERROR);
             hipDeviceProp_t p;
@@ -371,6 +442,7 @@ clb_status clb_controls_create(uint32_t platform_id, uint32_t device_id, clb_con
             delete c;
             throw;
         }
+        c->pool->enter(c);
         *out = c;
     });
 }
@@ -391,6 +463,7 @@ clb_status clb_controls_destroy(clb_controls ctl) {
             (void)hipStreamSynchronize(ctl->tail[k]);
             (void)hipStreamDestroy(ctl->tail[k]);
         }
+        ctl->pool->leave(ctl);  // before its stream ends
         (void)hipStreamDestroy(ctl->stream);
         delete ctl;
     });
@@ -610,4 +683,14 @@ clb_status clb_kernel_lookup(const char *program, const char *kernel) {
 // Shared by the other translation units: run a body under the same mapping.
 namespace clb {
 clb_status run_guarded(const std::function<void()> &body) { return guarded(body); }
+clb_status run_guarded(clb_controls_s *ctl, const std::function<void()> &body) {
+    return guarded([&] {
+        try {
+            body();
+        } catch (...) {
+            if (ctl) settle(ctl);
+            throw;
+        }
+    });
+}
 }  // namespace clb

@@ -162,7 +162,7 @@ using namespace clb;
 extern "C" {
 
 clb_status clb_prefix_sum_noalloc(clb_controls ctl, clb_buffer buf, uint32_t n, uint32_t *total) {
-    return run_guarded([&] {
+    return run_guarded(ctl, [&] {
         if (!ctl || !total) raise(INVALID_ARGUMENT, "prefix_sum_noalloc: null argument");
         *total = 0;
         if ((u64)n > NOALLOC_MAX_N)

@@ -419,7 +419,7 @@ extern "C" {
 
 clb_status clb_coo_from_host(clb_controls ctl, const uint32_t *rows, const uint32_t *cols, uint32_t nrows,
                              uint32_t ncols, uint32_t nnz, int sorted, int no_duplicates, clb_coo *out) {
-    return run_guarded([&] {
+    return run_guarded(ctl, [&] {
         clb_coo r{};
         r.nrows = nrows;
         r.ncols = ncols;
@@ -447,7 +447,7 @@ clb_status clb_coo_from_host(clb_controls ctl, const uint32_t *rows, const uint3
 
 clb_status clb_coo_from_buffers(clb_controls ctl, uint32_t nrows, uint32_t ncols, uint32_t nnz, clb_buffer rows,
                                 clb_buffer cols, int sorted, int no_duplicates, clb_coo *out) {
-    return run_guarded([&] {
+    return run_guarded(ctl, [&] {
         clb_coo r{};
         if (nnz && (!rows || !cols || rows->bytes < 4ull * nnz || cols->bytes < 4ull * nnz))
             raise(INVALID_ARGUMENT, "matrix_coo: buffers smaller than nnz");
@@ -470,7 +470,7 @@ clb_status clb_coo_from_buffers(clb_controls ctl, uint32_t nrows, uint32_t ncols
 }
 
 clb_status clb_coo_sort_arrays(clb_controls ctl, clb_buffer rows, clb_buffer cols, uint32_t n) {
-    return run_guarded([&] {
+    return run_guarded(ctl, [&] {
         if (n == 0) return;
         if (!rows || !cols || rows->bytes < 4ull * n || cols->bytes < 4ull * n)
             raise(INVALID_ARGUMENT, "sort_arrays: buffers smaller than n");

@@ -1575,7 +1575,7 @@ void spgemm_plain(clb_controls_s *ctl, const clb_dcsr &a, const clb_dcsr &b, u32
         readback(ctl, &flag, s.scal.ptr + 3, 8);
         if (flag) raise(RUN_KERNEL_FAILURE, "numeric pass disagreed with the symbolic row sizes");
     } catch (...) {
-        (void)hipStreamSynchronize(ctl->stream);
+        settle(ctl);
         clb_dcsr_release(&out);
         if (!out.cols) buffer_release(cols);
         throw;
@@ -1653,7 +1653,7 @@ using namespace clb;
 extern "C" {
 
 clb_status clb_dcsr_spgemm_hash(clb_controls ctl, const clb_dcsr *a, const clb_dcsr *b, clb_dcsr *out) {
-    return run_guarded([&] {
+    return run_guarded(ctl, [&] {
         clb_spgemm_opts o{};
         o.mode = CLB_SPGEMM_PLAIN;
         clb_spgemm_stats st;
@@ -1665,7 +1665,7 @@ clb_status clb_dcsr_spgemm_hash(clb_controls ctl, const clb_dcsr *a, const clb_d
 
 clb_status clb_dcsr_spgemm(clb_controls ctl, const clb_dcsr *a, const clb_dcsr *b, const clb_spgemm_opts *opts,
                            clb_dcsr *out, clb_spgemm_stats *stats) {
-    return run_guarded([&] {
+    return run_guarded(ctl, [&] {
         clb_spgemm_opts o{};
         if (opts) o = *opts;
         clb_spgemm_stats st;
