@@ -1044,7 +1044,8 @@ void ensure_packed(clb_controls_s *ctl, Setup &s, const BinHost &h) {
                                                               nullptr, nullptr);
     CLB_LAUNCHED("brange_set");
     if (s.g.splits) {
-        s.psplits.reset(ctl, s.splits.n);
+        // (the split table may be a plan's: s.splits is then empty)
+        s.psplits.reset(ctl, (u64)s.mapn * (s.g.nsl + 1));
         if (!s.filtered) fill_u32(ctl, s.psplits.ptr, s.psplits.n, 0u);
         k_pack_splits<<<div_up(b.nzr, 256), 256, 0, ctl->stream>>>(prpt.ptr, rows, pfirst.ptr, s.g.splits, b.nzr,
                                                                     s.mapn, s.g.nsl, s.psplits.ptr);
