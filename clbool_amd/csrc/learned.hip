@@ -589,28 +589,31 @@ struct OnePass {
     // the end of the block's row kernels on each side stream (launch_bins
     // with a deferred join); post makes the controls' stream wait for them
     hipEvent_t bins[clb_controls_s::NSIDE] = {};
-    bool tail = false, timing = false, replan = false;
+    bool timing = false, replan = false;
     // kept from launch for post
     clb_dcsr a{}, b{};
     PlanRows prc{};
     bool planned = false, posted = false, empty = false;
     const float *pred = nullptr;  // predicted sizes (compaction's error statistic)
     std::chrono::steady_clock::time_point t0;
+    bool finished = false;  // its work was waited for
     ~OnePass() {
         for (hipEvent_t &e : bins)
-            if (e) {
-                (void)hipEventSynchronize(e);
-                (void)hipEventDestroy(e);
-            }
-        if (tail)
-            for (int k = 0; k < clb_controls_s::NTAIL; ++k) (void)hipStreamSynchronize(ctl->tail[k]);
+            if (e) (void)hipEventDestroy(e);
         if (joined) (void)hipEventDestroy(joined);
         if (done) (void)hipEventDestroy(done);
         clb_dcsr_release(&out);  // nothing left when the result was handed over
     }
 };
 
-void OnePassDeleter::operator()(OnePass *p) const { delete p; }
+void OnePassDeleter::operator()(OnePass *p) const {
+    clb_controls_s *ctl = p->ctl;
+    // a block that is dropped, because it or another one failed, may still have
+    // work on any of the streams
+    if (!p->finished) settle(ctl);
+    Settled idle(ctl);
+    delete p;
+}
 
 OnePassPtr one_pass_launch(clb_controls_s *ctl, const clb_dcsr &a, const clb_dcsr &b, u32 rb, u32 re, bool timing,
                            bool bound_only, const PlanRows *pr) {
@@ -765,7 +768,6 @@ void one_pass_post(OnePass &p) {
     // everything above on the controls' stream (a small tail: on that stream)
     CLB_HIP(hipEventCreateWithFlags(&p.joined, hipEventDisableTiming), EVENT_WAITING_ERROR);
     CLB_HIP(hipEventCreateWithFlags(&p.done, hipEventDisableTiming), EVENT_WAITING_ERROR);
-    p.tail = true;
     const bool small = nnz <= ONE_STREAM_WORK;
     hipStream_t t0s = small ? ctl->stream : ctl->tail[0], t1s = small ? ctl->stream : ctl->tail[1];
     if (!small) {
@@ -809,7 +811,7 @@ void one_pass_finish(OnePass &p, clb_dcsr &out, clb_spgemm_stats &st) {
     clb_controls_s *ctl = p.ctl;
     one_pass_post(p);
     if (p.done) CLB_HIP(hipEventSynchronize(p.done), EVENT_WAITING_ERROR);
-    p.tail = false;
+    p.finished = true;
     if (p.err.ptr && p.st.nzr) {
         double e = 0;
         readback(ctl, &e, p.err.ptr, 8);

@@ -25,3 +25,25 @@ def assert_dcsr_equal(ctl, got: "cb.matrix_dcsr", ref: "oracle.Dcsr", what=""):
     if not np.array_equal(cols, ref.cols):
         d = np.flatnonzero(cols != ref.cols)[:5]
         raise AssertionError(f"{what}: cols differ at {d}: {cols[d]} vs {ref.cols[d]}")
+
+
+def hold_memory(ctl, leave):
+    """Buffers that hold all of the device's memory but about `leave` bytes: the
+    free blocks of the pool, then what HIP has."""
+    held = []
+    size = 1 << 30
+    while size >= 2 << 20:
+        before = ctl.pool_stats()["mallocs"]
+        x = cb.Buffer.create(ctl, size)
+        if ctl.pool_stats()["mallocs"] == before:
+            held.append(x)
+            continue
+        del x  # from a new segment: no free block is this large
+        ctl.trim()
+        size //= 2
+    for _ in range(8):  # what HIP reports lags behind
+        n = (ctl.pool_stats()["free_bytes"] - leave) >> 21 << 21
+        if n <= 2 << 20:
+            break
+        held.append(cb.Buffer.create(ctl, n))
+    return held
