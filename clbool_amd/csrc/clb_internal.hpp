@@ -237,6 +237,21 @@ void exclusive_scan_u64(clb_controls_s *ctl, const u64 *in, u64 *out, u64 n, u64
 // Exclusive scan of u32 inputs widened to u64 outputs.
 void exclusive_scan_u32_to_u64(clb_controls_s *ctl, const u32 *in, u64 *out, u64 n, u64 *total);
 
+inline bool no_room(const Error &e) { return e.status == CREATE_BUFFER_ERROR; }
+// body(lean): once as usual and, when device memory did not suffice, again
+// without the scratch that only makes it faster (lean).
+template <typename F>
+void with_room(clb_controls_s *ctl, F &&body) {
+    try {
+        body(false);
+        return;
+    } catch (const Error &e) {
+        if (!no_room(e)) throw;
+    }
+    settle(ctl);
+    body(true);
+}
+
 // Runs body, mapping exceptions to C-ABI status codes (runtime.hip).
 clb_status run_guarded(const std::function<void()> &body);
 // The same; a call that fails leaves nothing in flight on the controls.

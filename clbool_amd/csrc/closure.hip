@@ -247,9 +247,83 @@ static Seg seg_of(const clb_dcsr &m, u32 row_shift, u32 col_shift) {
 // blocks follow each other in row order).  The products' lists are merged
 // pairwise into one, which the union then meets the matrices' list with.  A
 // batch holds at most UNITE_KEYS keys (or one matrix), which bounds its
-// memory; united one by one, the 17 matrices of a 32-rule step took 4.0 ms,
-// mostly launches and read-backs, for 6.1 million keys.
+// memory; where there is no room for that either, it is one matrix.  United
+// one by one, the 17 matrices of a 32-rule step took 4.0 ms, mostly launches and
+// read-backs, for 6.1 million keys.
 constexpr u64 UNITE_KEYS = 1ull << 27;
+
+// One batch: matrices xs[batch[i]], `total` keys in all and `base` their own.
+static void unite_batch(clb_controls_s *ctl, clb_dcsr *mats, const std::vector<u32> &xs,
+                        const std::vector<std::vector<u32>> &of, const std::vector<size_t> &batch, u64 total, u64 base,
+                        u32 n, const std::vector<clb_dcsr> &prods, const std::vector<std::vector<u32>> &splits) {
+    auto part = [&](size_t q, u32 t) -> u64 { return splits[q][2 * t + 3] - splits[q][2 * t + 1]; };
+    DevArray<u64> keys(ctl, total), tmp(ctl, total - base);  // matrices | products; tmp: products
+    std::vector<KeySeg> segs;
+    u32 tiles = 0;
+    auto piece = [&](const clb_dcsr &m, u32 r_lo, u32 r_hi, u32 e_lo, u32 e_hi, u32 shift, u64 at) {
+        if (e_hi == e_lo) return;
+        segs.push_back(KeySeg{u32p(m.rpt), u32p(m.rows), u32p(m.cols), r_lo, r_hi, e_lo, e_hi, shift, tiles,
+                              keys.ptr + at});
+        tiles += div_up((u64)e_hi - e_lo, EX_TILE);
+    };
+    u64 pos = 0;
+    size_t rounds = 0;
+    for (size_t i = 0; i < batch.size(); ++i) {
+        const clb_dcsr &x = mats[xs[batch[i]]];
+        piece(x, 0, x.nzr, 0, x.nnz, (u32)i * n, pos);
+        pos += x.nnz;
+        rounds = std::max(rounds, of[batch[i]].size());
+    }
+    std::vector<std::pair<u64, u64>> lists;  // (start, length) after the matrices' keys
+    for (size_t r = 0; r < rounds; ++r) {
+        const u64 start = pos;
+        for (size_t i = 0; i < batch.size(); ++i) {
+            if (r >= of[batch[i]].size()) continue;
+            const u32 t = of[batch[i]][r];
+            for (size_t q = 0; q < prods.size(); ++q) {
+                const std::vector<u32> &hs = splits[q];
+                // rows t * n + row -> i * n + row
+                piece(prods[q], hs[2 * t], hs[2 * t + 2], hs[2 * t + 1], hs[2 * t + 3], ((u32)i - t) * n, pos);
+                pos += part(q, t);
+            }
+        }
+        lists.push_back({start - base, pos - start});
+    }
+    DevArray<KeySeg> dsegs(ctl, segs.size());
+    CLB_HIP(hipMemcpyAsync(dsegs.ptr, segs.data(), segs.size() * sizeof(KeySeg), hipMemcpyHostToDevice,
+                           ctl->stream),
+            WRITE_BUFFER_ERROR);
+    k_keys_segs<<<tiles, EX_WG, 0, ctl->stream>>>(dsegs.ptr, (u32)segs.size());
+    CLB_LAUNCHED("keys");
+    u64 *cur = keys.ptr + base, *nxt = tmp.ptr;
+    while (lists.size() > 1) {
+        std::vector<std::pair<u64, u64>> next;
+        for (size_t i = 0; i < lists.size(); i += 2) {
+            const auto &la = lists[i];
+            if (i + 1 == lists.size()) {  // odd one out: copied to the other buffer
+                CLB_HIP(hipMemcpyAsync(nxt + la.first, cur + la.first, 8 * la.second, hipMemcpyDeviceToDevice,
+                                       ctl->stream),
+                        COPY_BUFFER_ERROR);
+                next.push_back(la);
+                continue;
+            }
+            const auto &lb = lists[i + 1];  // adjacent
+            merge_keys(ctl, cur + la.first, la.second, cur + lb.first, lb.second, nxt + la.first);
+            next.push_back({la.first, la.second + lb.second});
+        }
+        lists.swap(next);
+        std::swap(cur, nxt);
+    }
+    std::vector<clb_dcsr> united;
+    for (size_t i : batch) united.push_back(mats[xs[i]]);
+    union_keys_to_matrices(ctl, keys.ptr, base, cur, total - base, n, united);
+    for (size_t i = 0; i < batch.size(); ++i) {
+        clb_dcsr &x = mats[xs[batch[i]]];
+        if (united[i].cols == x.cols) continue;  // unchanged
+        clb_dcsr_release(&x);
+        x = united[i];
+    }
+}
 
 static void unite_products(clb_controls_s *ctl, clb_dcsr *mats, const std::vector<u32> &xs, const u32 *triples,
                            u32 ntriples, u32 n, const std::vector<clb_dcsr> &prods,
@@ -266,6 +340,7 @@ static void unite_products(clb_controls_s *ctl, clb_dcsr *mats, const std::vecto
         add[k] += len;
     }
     size_t k0 = 0;
+    u64 most = UNITE_KEYS;
     while (k0 < xs.size()) {
         if (of[k0].empty()) {
             ++k0;
@@ -278,78 +353,20 @@ static void unite_products(clb_controls_s *ctl, clb_dcsr *mats, const std::vecto
             if (of[k1].empty()) continue;
             const u64 mine = mats[xs[k1]].nnz + add[k1];
             if (mine >= 0xFFFFFFFFull) raise(INVALID_VALUE, "a closure union exceeds uint32 nonzeros");
-            if (!batch.empty() && total + mine > UNITE_KEYS) break;
+            if (!batch.empty() && total + mine > most) break;
             batch.push_back(k1);
             total += mine;
             base += mats[xs[k1]].nnz;
         }
+        try {
+            unite_batch(ctl, mats, xs, of, batch, total, base, n, prods, splits);
+        } catch (const Error &e) {
+            if (!no_room(e) || batch.size() == 1) throw;
+            settle(ctl);
+            most = 0;
+            continue;
+        }
         k0 = k1;
-        DevArray<u64> keys(ctl, total), tmp(ctl, total - base);  // matrices | products; tmp: products
-        std::vector<KeySeg> segs;
-        u32 tiles = 0;
-        auto piece = [&](const clb_dcsr &m, u32 r_lo, u32 r_hi, u32 e_lo, u32 e_hi, u32 shift, u64 at) {
-            if (e_hi == e_lo) return;
-            segs.push_back(KeySeg{u32p(m.rpt), u32p(m.rows), u32p(m.cols), r_lo, r_hi, e_lo, e_hi, shift, tiles,
-                                  keys.ptr + at});
-            tiles += div_up((u64)e_hi - e_lo, EX_TILE);
-        };
-        u64 pos = 0;
-        size_t rounds = 0;
-        for (size_t i = 0; i < batch.size(); ++i) {
-            const clb_dcsr &x = mats[xs[batch[i]]];
-            piece(x, 0, x.nzr, 0, x.nnz, (u32)i * n, pos);
-            pos += x.nnz;
-            rounds = std::max(rounds, of[batch[i]].size());
-        }
-        std::vector<std::pair<u64, u64>> lists;  // (start, length) after the matrices' keys
-        for (size_t r = 0; r < rounds; ++r) {
-            const u64 start = pos;
-            for (size_t i = 0; i < batch.size(); ++i) {
-                if (r >= of[batch[i]].size()) continue;
-                const u32 t = of[batch[i]][r];
-                for (size_t q = 0; q < prods.size(); ++q) {
-                    const std::vector<u32> &hs = splits[q];
-                    // rows t * n + row -> i * n + row
-                    piece(prods[q], hs[2 * t], hs[2 * t + 2], hs[2 * t + 1], hs[2 * t + 3], ((u32)i - t) * n, pos);
-                    pos += part(q, t);
-                }
-            }
-            lists.push_back({start - base, pos - start});
-        }
-        DevArray<KeySeg> dsegs(ctl, segs.size());
-        CLB_HIP(hipMemcpyAsync(dsegs.ptr, segs.data(), segs.size() * sizeof(KeySeg), hipMemcpyHostToDevice,
-                               ctl->stream),
-                WRITE_BUFFER_ERROR);
-        k_keys_segs<<<tiles, EX_WG, 0, ctl->stream>>>(dsegs.ptr, (u32)segs.size());
-        CLB_LAUNCHED("keys");
-        u64 *cur = keys.ptr + base, *nxt = tmp.ptr;
-        while (lists.size() > 1) {
-            std::vector<std::pair<u64, u64>> next;
-            for (size_t i = 0; i < lists.size(); i += 2) {
-                const auto &la = lists[i];
-                if (i + 1 == lists.size()) {  // odd one out: copied to the other buffer
-                    CLB_HIP(hipMemcpyAsync(nxt + la.first, cur + la.first, 8 * la.second, hipMemcpyDeviceToDevice,
-                                           ctl->stream),
-                            COPY_BUFFER_ERROR);
-                    next.push_back(la);
-                    continue;
-                }
-                const auto &lb = lists[i + 1];  // adjacent
-                merge_keys(ctl, cur + la.first, la.second, cur + lb.first, lb.second, nxt + la.first);
-                next.push_back({la.first, la.second + lb.second});
-            }
-            lists.swap(next);
-            std::swap(cur, nxt);
-        }
-        std::vector<clb_dcsr> united;
-        for (size_t i : batch) united.push_back(mats[xs[i]]);
-        union_keys_to_matrices(ctl, keys.ptr, base, cur, total - base, n, united);
-        for (size_t i = 0; i < batch.size(); ++i) {
-            clb_dcsr &x = mats[xs[batch[i]]];
-            if (united[i].cols == x.cols) continue;  // unchanged
-            clb_dcsr_release(&x);
-            x = united[i];
-        }
     }
 }
 
@@ -441,6 +458,7 @@ clb_status clb_closure_step(clb_controls ctl, clb_dcsr *mats, uint32_t nmats, co
                     u32 nb = 0;
                     {
                         spg::Setup ps;
+                        ps.lean = true;  // the products per row are all it is for
                         spg::prepare(ctl, Y, Z, 0, Y.nzr, ps, true);
                         const RowBound rb{ps.P, n};
                         const u32 grid = div_up(Y.nzr, 256) < RB_GRID ? div_up(Y.nzr, 256) : RB_GRID;
@@ -522,15 +540,16 @@ clb_status clb_closure_step(clb_controls ctl, clb_dcsr *mats, uint32_t nmats, co
                             if (hipMemGetInfo(&free_b, &total_b) != hipSuccess) (void)hipGetLastError();
                             return free_b + pool_for(ctl->device).cached_bytes();
                         };
+                        bool lean = false;
                         auto launch = [&](u32 k) {
                             const bool bound_only = so.mode == CLB_SPGEMM_BOUND;
-                            return spg::one_pass_launch(ctl, Y, Z, hc[k], hc[k + 1], false, bound_only, nullptr);
+                            return spg::one_pass_launch(ctl, Y, Z, hc[k], hc[k + 1], false, bound_only, nullptr, lean);
                         };
                         auto nonempty = [&](u32 k) {  // the first block from k with rows
                             while (k < nb && hc[k + 1] <= hc[k]) ++k;
                             return k;
                         };
-                        for (u32 k = nonempty(0); k < nb;) {
+                        for (u32 k = nonempty(0); k < nb;) try {
                             if (!cur) {
                                 if (pend && avail() < 3 * spg::one_pass_bytes(*pend)) finish_pending();
                                 cur = launch(k);
@@ -546,6 +565,14 @@ clb_status clb_closure_step(clb_controls ctl, clb_dcsr *mats, uint32_t nmats, co
                             pend = std::move(cur);
                             cur = std::move(nxt);
                             k = k2;
+                        } catch (const Error &e) {
+                            // block k (or the one after it) again, alone and lean
+                            if (!no_room(e) || lean) throw;
+                            nxt.reset();
+                            cur.reset();
+                            if (pend) finish_pending();
+                            settle(ctl);
+                            lean = true;
                         }
                         if (pend) finish_pending();
                     }

@@ -232,6 +232,7 @@ void spgemm_esc(clb_controls_s *ctl, const clb_dcsr &a, const clb_dcsr &b, clb_d
     if (a.nnz == 0 || b.nnz == 0 || a.nzr == 0) return;
     const u32 nrows = a.nzr;
     Setup s;
+    s.lean = true;  // no bitmap rows
     prepare(ctl, a, b, 0, nrows, s, true);
     s.cfg.esc_only = 1;
     s.cfg.tiny_max = 64;
@@ -323,8 +324,8 @@ void spgemm_esc(clb_controls_s *ctl, const clb_dcsr &a, const clb_dcsr &b, clb_d
                 sync(ctl);
             } catch (...) {
                 settle(ctl);
+                if (!out.cols) buffer_release(cols);  // else out's
                 clb_dcsr_release(&out);
-                if (!out.cols) buffer_release(cols);
                 throw;
             }
         }

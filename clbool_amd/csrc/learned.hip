@@ -616,7 +616,7 @@ void OnePassDeleter::operator()(OnePass *p) const {
 }
 
 OnePassPtr one_pass_launch(clb_controls_s *ctl, const clb_dcsr &a, const clb_dcsr &b, u32 rb, u32 re, bool timing,
-                           bool bound_only, const PlanRows *pr) {
+                           bool bound_only, const PlanRows *pr, bool lean) {
     OnePassPtr P(new OnePass());
     OnePass &p = *P;
     p.ctl = ctl;
@@ -633,6 +633,7 @@ OnePassPtr one_pass_launch(clb_controls_s *ctl, const clb_dcsr &a, const clb_dcs
     }
     clb_spgemm_stats &st = p.st;
     Setup &s = p.s;
+    s.lean = lean;
     const u32 nrows = re - rb;
     p.nnz_row.reset(ctl, nrows);
     u32 *cap = nullptr;
@@ -792,8 +793,8 @@ void one_pass_post(OnePass &p) {
 }
 
 OnePassPtr one_pass_start(clb_controls_s *ctl, const clb_dcsr &a, const clb_dcsr &b, u32 rb, u32 re, bool timing,
-                          bool bound_only, const PlanRows *pr) {
-    OnePassPtr p = one_pass_launch(ctl, a, b, rb, re, timing, bound_only, pr);
+                          bool bound_only, const PlanRows *pr, bool lean) {
+    OnePassPtr p = one_pass_launch(ctl, a, b, rb, re, timing, bound_only, pr, lean);
     one_pass_post(*p);
     return p;
 }
@@ -826,8 +827,8 @@ void one_pass_finish(OnePass &p, clb_dcsr &out, clb_spgemm_stats &st) {
 }
 
 void spgemm_learned(clb_controls_s *ctl, const clb_dcsr &a, const clb_dcsr &b, u32 rb, u32 re, bool timing,
-                    clb_dcsr &out, clb_spgemm_stats &st, bool bound_only, const PlanRows *pr) {
-    OnePassPtr p = one_pass_start(ctl, a, b, rb, re, timing, bound_only, pr);
+                    clb_dcsr &out, clb_spgemm_stats &st, bool bound_only, const PlanRows *pr, bool lean) {
+    OnePassPtr p = one_pass_start(ctl, a, b, rb, re, timing, bound_only, pr, lean);
     clb_dcsr r{};
     one_pass_finish(*p, r, st);
     out = r;
@@ -912,39 +913,42 @@ clb_status clb_predictor_harvest(clb_controls ctl, const clb_dcsr *a, const clb_
             L->ready = true;
         }
         if (a->nnz && b->nnz && a->nzr && max_rows) {
-            const u32 nrows = a->nzr;
-            Setup s;
-            DevArray<float> feat;
-            prepare_features(ctl, *a, *b, 0, nrows, s, feat);
-            DevArray<u32> nnz_row(ctl, nrows), perm;
-            BinHost h;
-            bin_rows(ctl, s, nullptr, nnz_row.ptr, perm);
-            read_bins(ctl, s, h);
-            Out o{nnz_row.ptr, nullptr, nullptr, nullptr, reinterpret_cast<u32 *>(s.scal.ptr + 3), Dump{}, 0};
-            ensure_splits(ctl, s, h);
-            ensure_packed(ctl, s, h);
-            launch_bins(ctl, s, perm.ptr, h.off, SYM, o, nullptr, -1);
-            const u32 stride = nrows > max_rows ? div_up(nrows, max_rows) : 1;
-            const u32 take = div_up(nrows, stride);
-            if (L->n + take > L->cap) {  // grow the sample store
-                const u64 ncap = std::max<u64>(L->cap * 2, L->n + take + 4096);
-                DevArray<float> X2(ctl, ncap * NF), Y2(ctl, ncap);
-                if (L->n) {
-                    CLB_HIP(hipMemcpyAsync(X2.ptr, L->X.ptr, L->n * NF * 4, hipMemcpyDeviceToDevice, ctl->stream),
-                            COPY_BUFFER_ERROR);
-                    CLB_HIP(hipMemcpyAsync(Y2.ptr, L->Y.ptr, L->n * 4, hipMemcpyDeviceToDevice, ctl->stream),
-                            COPY_BUFFER_ERROR);
+            with_room(ctl, [&](bool lean) {
+                const u32 nrows = a->nzr;
+                Setup s;
+                s.lean = lean;
+                DevArray<float> feat;
+                prepare_features(ctl, *a, *b, 0, nrows, s, feat);
+                DevArray<u32> nnz_row(ctl, nrows), perm;
+                BinHost h;
+                bin_rows(ctl, s, nullptr, nnz_row.ptr, perm);
+                read_bins(ctl, s, h);
+                Out o{nnz_row.ptr, nullptr, nullptr, nullptr, reinterpret_cast<u32 *>(s.scal.ptr + 3), Dump{}, 0};
+                ensure_splits(ctl, s, h);
+                ensure_packed(ctl, s, h);
+                launch_bins(ctl, s, perm.ptr, h.off, SYM, o, nullptr, -1);
+                const u32 stride = nrows > max_rows ? div_up(nrows, max_rows) : 1;
+                const u32 take = div_up(nrows, stride);
+                if (L->n + take > L->cap) {  // grow the sample store
+                    const u64 ncap = std::max<u64>(L->cap * 2, L->n + take + 4096);
+                    DevArray<float> X2(ctl, ncap * NF), Y2(ctl, ncap);
+                    if (L->n) {
+                        CLB_HIP(hipMemcpyAsync(X2.ptr, L->X.ptr, L->n * NF * 4, hipMemcpyDeviceToDevice, ctl->stream),
+                                COPY_BUFFER_ERROR);
+                        CLB_HIP(hipMemcpyAsync(Y2.ptr, L->Y.ptr, L->n * 4, hipMemcpyDeviceToDevice, ctl->stream),
+                                COPY_BUFFER_ERROR);
+                    }
+                    sync(ctl);
+                    L->X.swap(X2);
+                    L->Y.swap(Y2);
+                    L->cap = ncap;
                 }
+                k_harvest<<<div_up(take, 256), 256, 0, ctl->stream>>>(feat.ptr, s.prod.ptr, nnz_row.ptr, nrows, stride,
+                                                                       L->X.ptr, L->Y.ptr, L->n);
+                CLB_LAUNCHED("harvest");
                 sync(ctl);
-                L->X.swap(X2);
-                L->Y.swap(Y2);
-                L->cap = ncap;
-            }
-            k_harvest<<<div_up(take, 256), 256, 0, ctl->stream>>>(feat.ptr, s.prod.ptr, nnz_row.ptr, nrows, stride,
-                                                                   L->X.ptr, L->Y.ptr, L->n);
-            CLB_LAUNCHED("harvest");
-            sync(ctl);
-            L->n += take;
+                L->n += take;
+            });
         }
         if (total_samples) *total_samples = L->n;
     });
@@ -1032,6 +1036,7 @@ clb_status clb_predictor_predict(clb_controls ctl, const clb_dcsr *a, const clb_
             return;
         }
         Setup s;
+        s.lean = true;  // nothing is multiplied
         DevArray<float> feat, pred(ctl, a->nzr);
         DevArray<u32> cap(ctl, a->nzr);
         prepare_features(ctl, *a, *b, 0, a->nzr, s, feat);

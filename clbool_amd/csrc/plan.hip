@@ -115,6 +115,16 @@ static void plan_create(clb_controls_s *ctl, const clb_dcsr &a, const clb_dcsr &
     p.info.ms_plan = std::chrono::duration<double, std::milli>(std::chrono::steady_clock::now() - t0).count();
 }
 
+// Blocks run without the scratch that only saves time from here on: there was
+// no room for one beside it.  No block may be running.
+static void make_lean(clb_controls_s *ctl, clb_spgemm_plan_s &p) {
+    settle(ctl);
+    Settled idle(ctl);
+    p.store.drop();
+    drop_packed(p.s);
+    p.s.lean = true;
+}
+
 // Block k exceeded the bound: size[cuts[k], cuts[k+1]) holds its exact row
 // sizes now; cut those rows again.
 static void recut(clb_controls_s *ctl, clb_spgemm_plan_s &p, u32 k) {
@@ -166,10 +176,16 @@ static void plan_run(clb_controls_s *ctl, clb_spgemm_plan_s &p, u32 k, bool timi
         PlanRows pr = rows_of(p, k, &replan);
         clb_dcsr r{};
         std::memset(&st, 0, sizeof(st));
-        if (p.mode == CLB_SPGEMM_PLAIN)
-            spgemm_plain(ctl, p.a, p.b, rb, re, timing, r, st, &pr);
-        else
-            spgemm_learned(ctl, p.a, p.b, rb, re, timing, r, st, p.mode == CLB_SPGEMM_BOUND, &pr);
+        try {
+            if (p.mode == CLB_SPGEMM_PLAIN)
+                spgemm_plain(ctl, p.a, p.b, rb, re, timing, r, st, &pr, p.s.lean);
+            else
+                spgemm_learned(ctl, p.a, p.b, rb, re, timing, r, st, p.mode == CLB_SPGEMM_BOUND, &pr, p.s.lean);
+        } catch (const Error &e) {
+            if (!no_room(e) || p.s.lean) throw;
+            make_lean(ctl, p);
+            continue;
+        }
         if (!replan) {
             out = r;
             break;
@@ -223,10 +239,11 @@ static void plan_run_all(clb_controls_s *ctl, clb_spgemm_plan_s &p, bool timing,
     };
     auto launch = [&](u32 k) {
         const PlanRows pr = rows_of(p, k, nullptr);
-        return one_pass_launch(ctl, p.a, p.b, p.cuts[k], p.cuts[k + 1], timing, p.mode == CLB_SPGEMM_BOUND, &pr);
+        return one_pass_launch(ctl, p.a, p.b, p.cuts[k], p.cuts[k + 1], timing, p.mode == CLB_SPGEMM_BOUND, &pr,
+                               p.s.lean);
     };
     u32 k = 0;
-    while (go && k + 1 < p.cuts.size()) {
+    while (go && k + 1 < p.cuts.size()) try {
         if (!cur) {
             // overlap only when there is room for a second block of about
             // the pending one's size beside it (with room to spare for its
@@ -261,6 +278,13 @@ static void plan_run_all(clb_controls_s *ctl, clb_spgemm_plan_s &p, bool timing,
         pend_k = k;
         cur = std::move(nxt);
         ++k;
+    } catch (const Error &e) {
+        // block k (or the one after it) again, alone and lean
+        if (!no_room(e) || p.s.lean) throw;
+        nxt.reset();
+        cur.reset();
+        if (pend) finish_pending();
+        make_lean(ctl, p);
     }
     nxt.reset();
     cur.reset();  // launched after a stop: dropped
@@ -278,14 +302,12 @@ clb_status clb_spgemm_plan_create(clb_controls ctl, const clb_dcsr *a, const clb
                                   uint64_t block_bound, clb_spgemm_plan *out) {
     return run_guarded(ctl, [&] {
         if (!ctl || !a || !b || !out) raise(INVALID_ARGUMENT, "null argument");
-        auto *p = new clb_spgemm_plan_s();
-        try {
+        with_room(ctl, [&](bool lean) {
+            auto p = std::make_unique<clb_spgemm_plan_s>();
+            p->s.lean = lean;
             spg::plan_create(ctl, *a, *b, mode, block_bound, *p);
-        } catch (...) {
-            delete p;
-            throw;
-        }
-        *out = p;
+            *out = p.release();
+        });
     });
 }
 

@@ -779,6 +779,7 @@ void emit_stored(hipStream_t st, const u32 *perm, u32 n, const Store &keep, cons
 
 void setup_store(clb_controls_s *ctl, const Setup &s, const BinHost &h, u32 bits, StoreBufs &b) {
     b.keep = Store{};
+    if (s.lean) return;
     // with dump_bits_per_chunk set, the numeric pass gathers its rows and dumps
     // the dense ones, as asked
     const u32 knob = ctl->tuning.dump_bits_per_chunk;
@@ -813,8 +814,10 @@ void setup_store(clb_controls_s *ctl, const Setup &s, const BinHost &h, u32 bits
         b.chunks.reset(ctl, slots * nch);
         b.fmt.reset(ctl, slots * nsl);
         b.slot_of.reset(ctl, s.nrows);
-    } catch (const Error &) {
-        return;  // no memory for it: the numeric pass gathers as usual
+    } catch (const Error &e) {
+        if (!no_room(e)) throw;
+        b.drop();
+        return;  // the numeric pass gathers as usual
     }
     fill_u32(ctl, b.slot_of.ptr, s.nrows, 0u);
     b.keep = Store{b.words.ptr, b.chunks.ptr, b.fmt.ptr, b.slot_of.ptr, (u32)slots, (u32)nch, (u32)words, win};
@@ -838,7 +841,7 @@ void setup_dump(clb_controls_s *ctl, const Setup &s, const BinHost &h, DumpBufs 
     // default: on in the one pass (its in-kernel emission writes a temporary
     // slot that the compaction copies again), off in the numeric pass (which
     // writes the final positions directly)
-    const u32 knob = ctl->tuning.dump_bits_per_chunk ? ctl->tuning.dump_bits_per_chunk : (one_pass ? 64u : 65536u);
+    const u32 knob = ctl->tuning.dump_bits_per_chunk ? ctl->tuning.dump_bits_per_chunk : (one_pass ? (s.lean ? 1024u : 64u) : 65536u);
     if (s.cfg.bm_bits < 14 || knob >= 65536u) return;
     const u64 nslices = ((u64)s.g.ncols + (32ull << s.cfg.bm_bits) - 1) / (32ull << s.cfg.bm_bits);
     d.nbm = h.off[NBINS] - h.off[BIN_BITMAP0];
@@ -1012,7 +1015,7 @@ void ensure_splits(clb_controls_s *ctl, Setup &s, const BinHost &h) {
 
 // Packs B for the bitmap kernels when their rows will read it often enough.
 void ensure_packed(clb_controls_s *ctl, Setup &s, const BinHost &h) {
-    if (s.g.b_packs || s.pack_tried || s.g.combine || ctl->tuning.bitmap_persistent) return;
+    if (s.lean || s.g.b_packs || s.pack_tried || s.g.combine || ctl->tuning.bitmap_persistent) return;
     u64 products = 0;
     for (u32 b = BIN_BITMAP0; b < NBINS; ++b) products += h.products[b];
     const clb_dcsr &b = s.b;
@@ -1056,6 +1059,16 @@ void ensure_packed(clb_controls_s *ctl, Setup &s, const BinHost &h) {
     s.g.psplits = s.g.splits ? s.psplits.ptr : nullptr;
 }
 
+void drop_packed(Setup &s) {
+    s.packs.free_();
+    s.prange.free_();
+    s.psplits.free_();
+    s.g.b_packs = nullptr;
+    s.g.prange = nullptr;
+    s.g.psplits = nullptr;
+    s.pack_tried = true;
+}
+
 void prepare(clb_controls_s *ctl, const clb_dcsr &a, const clb_dcsr &b, u32 row_begin, u32 nrows, Setup &s,
              bool stats, const Setup *shared, const RowFeat *feat) {
     s.nrows = nrows;
@@ -1065,6 +1078,7 @@ void prepare(clb_controls_s *ctl, const clb_dcsr &a, const clb_dcsr &b, u32 row_
         s.mapn = shared->mapn;
         s.pack_tried = shared->pack_tried;
         s.filtered = shared->filtered;
+        s.lean = shared->lean;
         s.g = shared->g;
         s.cfg = shared->cfg;
         s.b = shared->b;
@@ -1106,7 +1120,7 @@ void prepare(clb_controls_s *ctl, const clb_dcsr &a, const clb_dcsr &b, u32 row_
         s.prod.reset(ctl, nrows);
         s.P = s.prod.ptr;
     }
-    const bool filter = !shared && stats && s.bpres.ptr && b.nzr && split_entries(s) >= FILTER_MIN_ENTRIES;
+    const bool filter = !shared && !s.lean && stats && s.bpres.ptr && b.nzr && split_entries(s) >= FILTER_MIN_ENTRIES;
     const u64 nmap = shared || s.bpres.ptr ? 0 : s.mapn, nbits = shared ? 0 : s.bpres.n;
     u64 most = nmap > nbits ? nmap : nbits;
     if (stats && nrows > most) most = nrows;
@@ -1485,11 +1499,12 @@ void scan_sizes(clb_controls_s *ctl, Setup &s, const u32 *nnz_row, DevArray<u64>
 }
 
 void spgemm_plain(clb_controls_s *ctl, const clb_dcsr &a, const clb_dcsr &b, u32 row_begin, u32 row_end,
-                  bool timing, clb_dcsr &out, clb_spgemm_stats &st, const PlanRows *pr) {
+                  bool timing, clb_dcsr &out, clb_spgemm_stats &st, const PlanRows *pr, bool lean) {
     Timer tm(timing, ctl->stream);
     tm.mark();  // 0
     const u32 nrows = row_end - row_begin;
     Setup s;
+    s.lean = lean;
     prepare(ctl, a, b, row_begin, nrows, s, pr == nullptr, pr ? pr->shared : nullptr);
     LaunchTimer lt;
     lt.on = timing;
@@ -1577,8 +1592,8 @@ void spgemm_plain(clb_controls_s *ctl, const clb_dcsr &a, const clb_dcsr &b, u32
         if (flag) raise(RUN_KERNEL_FAILURE, "numeric pass disagreed with the symbolic row sizes");
     } catch (...) {
         settle(ctl);
+        if (!out.cols) buffer_release(cols);  // else out's
         clb_dcsr_release(&out);
-        if (!out.cols) buffer_release(cols);
         throw;
     }
     st.nnz = nnz;
@@ -1634,12 +1649,15 @@ void spgemm_dispatch(clb_controls_s *ctl, const clb_dcsr &a, const clb_dcsr &b, 
         return;
     }
     auto t0 = std::chrono::steady_clock::now();
-    if (o.mode == CLB_SPGEMM_LEARNED || o.mode == CLB_SPGEMM_BOUND)
-        spgemm_learned(ctl, a, b, rb, re, o.timing != 0, r, st, o.mode == CLB_SPGEMM_BOUND);
-    else if (o.mode == CLB_SPGEMM_PLAIN)
-        spgemm_plain(ctl, a, b, rb, re, o.timing != 0, r, st);
-    else
-        raise(INVALID_ARGUMENT, "unknown SpGEMM mode");
+    const bool one_pass = o.mode == CLB_SPGEMM_LEARNED || o.mode == CLB_SPGEMM_BOUND;
+    if (!one_pass && o.mode != CLB_SPGEMM_PLAIN) raise(INVALID_ARGUMENT, "unknown SpGEMM mode");
+    with_room(ctl, [&](bool lean) {
+        std::memset(&st, 0, sizeof(st));
+        if (one_pass)
+            spgemm_learned(ctl, a, b, rb, re, o.timing != 0, r, st, o.mode == CLB_SPGEMM_BOUND, nullptr, lean);
+        else
+            spgemm_plain(ctl, a, b, rb, re, o.timing != 0, r, st, nullptr, lean);
+    });
     if (!o.timing)
         st.ms_total = std::chrono::duration<double, std::milli>(std::chrono::steady_clock::now() - t0).count();
     ctl->last = st;

@@ -28,6 +28,9 @@ struct Setup {
     DevArray<uint2> prange;
     DevArray<u32> psplits;
     bool pack_tried = false;
+    // no scratch that only saves time (kept bitmaps, packed B, filtered A, slots
+    // of all but the densest dumped rows): there was no room for it
+    bool lean = false;
     Mats g{};
     BinCfg cfg{};
     clb_dcsr b{};  // the B operand (its buffers stay owned by the caller)
@@ -96,6 +99,13 @@ struct StoreBufs {
     DevArray<uint4> words;
     DevArray<u32> chunks, fmt, slot_of;
     Store keep{};
+    void drop() {
+        words.free_();
+        chunks.free_();
+        fmt.free_();
+        slot_of.free_();
+        keep = Store{};
+    }
 };
 // Below this many products in the bitmap rows their bitmaps are not kept: the
 // buffers cost more than the second gather (98 thousand products: 343 us
@@ -149,6 +159,8 @@ constexpr u64 PACK_MIN_PRODUCTS = 1ull << 24;
 constexpr u32 PACK_MIN_READS = 8;  // products of the bitmap rows per nonzero of B
 constexpr u32 PACK_MAX_PCT = 95;   // packs per 100 nonzeros of B
 void ensure_packed(clb_controls_s *ctl, Setup &s, const BinHost &h);
+// Gives packed B back; it is not packed again.
+void drop_packed(Setup &s);
 // B row map, kernel arguments and (stats) per-row products, with `feat` also
 // the other statistics.  With `shared`, the B row map, split table and bin
 // config are taken from it (a plan's Setup) instead of being built.
@@ -207,7 +219,7 @@ void check_dims(const clb_dcsr &a, const clb_dcsr &b);
 // pr != nullptr: the block of a plan (the count and symbolic pass were run
 // over all rows at planning time; pr->size holds the exact row sizes).
 void spgemm_plain(clb_controls_s *ctl, const clb_dcsr &a, const clb_dcsr &b, u32 row_begin, u32 row_end,
-                  bool timing, clb_dcsr &out, clb_spgemm_stats &st, const PlanRows *pr = nullptr);
+                  bool timing, clb_dcsr &out, clb_spgemm_stats &st, const PlanRows *pr = nullptr, bool lean = false);
 // Planning passes over all stored rows of A (s from prepare over all rows):
 // exact row sizes by the symbolic pass (plain) into size.
 void plan_sizes_plain(clb_controls_s *ctl, Setup &s, u32 *size, StoreBufs &store);
@@ -215,7 +227,7 @@ void plan_sizes_plain(clb_controls_s *ctl, Setup &s, u32 *size, StoreBufs &store
 // predictor (CLB_SPGEMM_BOUND).
 void spgemm_learned(clb_controls_s *ctl, const clb_dcsr &a, const clb_dcsr &b, u32 row_begin, u32 row_end,
                     bool timing, clb_dcsr &out, clb_spgemm_stats &st, bool bound_only = false,
-                    const PlanRows *pr = nullptr);
+                    const PlanRows *pr = nullptr, bool lean = false);
 // The one pass of one block in two halves: start runs everything up to the
 // tail (compaction and dense-row emission), which it leaves running on the
 // controls' tail streams; finish waits for it and hands over the result.  A
@@ -231,9 +243,9 @@ struct OnePassDeleter {
 };
 using OnePassPtr = std::unique_ptr<OnePass, OnePassDeleter>;
 OnePassPtr one_pass_start(clb_controls_s *ctl, const clb_dcsr &a, const clb_dcsr &b, u32 row_begin, u32 row_end,
-                          bool timing, bool bound_only, const PlanRows *pr);
+                          bool timing, bool bound_only, const PlanRows *pr, bool lean);
 OnePassPtr one_pass_launch(clb_controls_s *ctl, const clb_dcsr &a, const clb_dcsr &b, u32 row_begin, u32 row_end,
-                           bool timing, bool bound_only, const PlanRows *pr);
+                           bool timing, bool bound_only, const PlanRows *pr, bool lean);
 void one_pass_post(OnePass &p);
 bool one_pass_replan(const OnePass &p);
 u64 one_pass_bytes(const OnePass &p);  // device memory the block holds

@@ -28,22 +28,21 @@ def assert_dcsr_equal(ctl, got: "cb.matrix_dcsr", ref: "oracle.Dcsr", what=""):
 
 
 def hold_memory(ctl, leave):
-    """Buffers that hold all of the device's memory but about `leave` bytes: the
-    free blocks of the pool, then what HIP has."""
+    """Buffers that hold all of the device's memory but about `leave` bytes: most
+    of what HIP says is free (that lags), then pieces until there is no more, of
+    which `leave` bytes are given back."""
+    piece = 16 << 20
+    ctl.trim()
     held = []
-    size = 1 << 30
-    while size >= 2 << 20:
-        before = ctl.pool_stats()["mallocs"]
-        x = cb.Buffer.create(ctl, size)
-        if ctl.pool_stats()["mallocs"] == before:
-            held.append(x)
-            continue
-        del x  # from a new segment: no free block is this large
-        ctl.trim()
-        size //= 2
-    for _ in range(8):  # what HIP reports lags behind
-        n = (ctl.pool_stats()["free_bytes"] - leave) >> 21 << 21
-        if n <= 2 << 20:
-            break
+    n = (ctl.pool_stats()["free_bytes"] - leave - (2 << 30)) // piece * piece
+    if n > 0:
         held.append(cb.Buffer.create(ctl, n))
-    return held
+    pieces = []
+    try:
+        while True:
+            pieces.append(cb.Buffer.create(ctl, piece))
+    except cb.ClboolError:
+        pass
+    del pieces[-(leave // piece):]
+    ctl.trim()
+    return held + pieces
