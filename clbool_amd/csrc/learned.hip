@@ -710,6 +710,16 @@ void one_pass_post(OnePass &p) {
             st.bin_a_nnz[k] = p.h.a_nnz[k];
             st.bin_out_nnz[k] = outs[k];
         }
+        if (const u32 kept = p.store.keep.slots) {  // the first of the bitmap rows; their columns are bin BIN_STORED's
+            BinHost first = p.h;
+            for (u32 k = BIN_BITMAP0 + 1; k <= NBINS; ++k)
+                first.off[k] = std::min(first.off[k], first.off[BIN_BITMAP0] + kept);
+            sum_by_bin(ctl, p.perm.ptr, first, nrows, p.nnz_row.ptr, outs);
+            for (u32 k = BIN_BITMAP0; k < NBINS; ++k) {
+                st.bin_out_nnz[k] -= outs[k];
+                st.bin_out_nnz[BIN_STORED] += outs[k];
+            }
+        }
     }
     // exact re-run of the rows that overflowed their predicted capacity
     if (nfail) {
@@ -783,8 +793,11 @@ void one_pass_post(OnePass &p) {
                  p.err.ptr, ctl->tuning.reserved[CLB_TUNE_COMPACT_TILES] != 0);
     p.lt.end((int)CLB_KF_COMPACT, t0s);
     emit_launch(t1s, ndense, p.perm.ptr, p.h, p.dump, p.gpre.ptr, p.offs.ptr, u32p(cols), &p.lt, CLB_KP_ONEPASS);
-    if (p.store.keep.slots)
+    if (p.store.keep.slots) {
+        p.lt.begin(t1s);
         emit_stored(t1s, p.perm.ptr + p.h.off[BIN_BITMAP0], p.store.keep.slots, p.store.keep, p.offs.ptr, u32p(cols));
+        p.lt.end((int)CLB_KF(CLB_KP_ONEPASS, CLB_KK_EMIT), t1s);
+    }
     if (!small) {
         CLB_HIP(hipEventRecord(p.joined, t0s), EVENT_WAITING_ERROR);
         CLB_HIP(hipStreamWaitEvent(t1s, p.joined, 0), EVENT_WAITING_ERROR);

@@ -169,7 +169,8 @@ typedef struct clb_spgemm_stats {
     uint32_t bin_rows[CLB_MAX_BINS];     /* rows per bin (numeric binning)          */
     uint64_t bin_products[CLB_MAX_BINS]; /* intermediate products per bin           */
     uint64_t bin_a_nnz[CLB_MAX_BINS];    /* A nonzeros of the bin's rows            */
-    uint64_t bin_out_nnz[CLB_MAX_BINS];  /* output nonzeros of the bin's rows       */
+    uint64_t bin_out_nnz[CLB_MAX_BINS];  /* output nonzeros of the bin's rows.  Bin 13: kept bitmap rows,
+                                            which an emission writes (one pass: only their output) */
     double   pred_abs_log2_err; /* learned mode: mean |log2(1+pred)-log2(1+nnz)| */
     double   ms_setup, ms_symbolic, ms_numeric, ms_assemble, ms_total;
     /* with opts.timing: HIP-event durations summed per kernel family, indexed
@@ -189,7 +190,7 @@ typedef struct clb_spgemm_stats {
 #define CLB_KK_TINY     0u
 #define CLB_KK_HASH     1u  /* LDS hash tables and LDS expand-sort-compress rows */
 #define CLB_KK_BITMAP   2u
-#define CLB_KK_EMIT     3u  /* emission of dumped dense bitmap rows    */
+#define CLB_KK_EMIT     3u  /* emission of dumped dense bitmap rows, in the one pass of kept ones too */
 #define CLB_KF(pass, kind) ((pass) * 4u + (kind))
 /* The re-run never dumps rows (it has no emission launch), so its EMIT slot
  * holds the one pass's compaction instead: every row copied from its
