@@ -100,9 +100,14 @@ static void plan_create(clb_controls_s *ctl, const clb_dcsr &a, const clb_dcsr &
         CLB_HIP(hipMemcpyAsync(p.spre.data(), sp.ptr, 8ull * (n + 1), hipMemcpyDeviceToHost, ctl->stream),
                 READ_BUFFER_ERROR);
         sync(ctl);
-        // B packed once for every block, if the whole product reads it often
-        all.products[BIN_BITMAP0] = p.ppre[n];
-        ensure_packed(ctl, p.s, all);
+        // B packed once for every block, if the bitmap rows read it often: the
+        // plain plan's symbolic pass has decided that from its bins
+        if (mode != CLB_SPGEMM_PLAIN && pack_pays(p.ppre[n], b.nnz)) {
+            DevArray<u32> perm;
+            bin_rows(ctl, p.s, p.size.ptr, nullptr, perm);
+            read_bins(ctl, p.s, all);
+            ensure_packed(ctl, p.s, all);
+        }
         cut_rows(p.spre.data(), 0, n, p.bound, p.cuts);
         p.info.products = p.ppre[n];
         p.info.planned_nnz = p.spre[n];

@@ -1019,8 +1019,7 @@ void ensure_packed(clb_controls_s *ctl, Setup &s, const BinHost &h) {
     u64 products = 0;
     for (u32 b = BIN_BITMAP0; b < NBINS; ++b) products += h.products[b];
     const clb_dcsr &b = s.b;
-    if (!b.nzr || !b.nnz || products < (u64)PACK_MIN_READS * b.nnz || products < PACK_MIN_PRODUCTS)
-        return;
+    if (!b.nzr || !b.nnz || !pack_pays(products, b.nnz)) return;
     s.pack_tried = true;
     // a pack's group is known modulo 2^20 columns: wider matrices need slices
     if (b.ncols > (1u << 20) && !s.g.splits) return;

@@ -158,6 +158,9 @@ void ensure_splits(clb_controls_s *ctl, Setup &s, const BinHost &h);
 constexpr u64 PACK_MIN_PRODUCTS = 1ull << 24;
 constexpr u32 PACK_MIN_READS = 8;  // products of the bitmap rows per nonzero of B
 constexpr u32 PACK_MAX_PCT = 95;   // packs per 100 nonzeros of B
+constexpr bool pack_pays(u64 products, u32 b_nnz) {
+    return products >= PACK_MIN_PRODUCTS && products >= (u64)PACK_MIN_READS * b_nnz;
+}
 void ensure_packed(clb_controls_s *ctl, Setup &s, const BinHost &h);
 // Gives packed B back; it is not packed again.
 void drop_packed(Setup &s);
