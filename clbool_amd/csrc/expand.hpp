@@ -25,7 +25,9 @@ namespace clb {
 constexpr u32 EX_WG = 256, EX_ITEMS = 8, EX_TILE = EX_WG * EX_ITEMS;
 
 // first[t] = the row of nonzero e_lo + t * TILE, for every tile of [e_lo, e_hi)
-// (e_hi == 0: of the rows' own nonzeros, which only the device knows).
+// (e_hi == 0: of the rows' own nonzeros, which only the device knows).  Row
+// pointers that cover less than [e_lo, e_hi), as of a CSR matrix with unused
+// columns at its end, leave the rest to the first and the last row.
 template <u32 TILE>
 __device__ __forceinline__ void tile_rows(const u32 *__restrict__ rpt, u32 r_lo, u32 r_hi, u32 e_lo, u32 e_hi,
                                           u32 *__restrict__ first, u32 block) {
@@ -36,8 +38,8 @@ __device__ __forceinline__ void tile_rows(const u32 *__restrict__ rpt, u32 r_lo,
     }
     u32 t0 = 0, n = 0;  // tiles that begin in row r
     if (r < r_hi) {
-        const u32 b = rpt[r] > e_lo ? rpt[r] - e_lo : 0u;
-        const u32 end = rpt[r + 1] < e_hi ? rpt[r + 1] : e_hi;
+        const u32 b = r != r_lo && rpt[r] > e_lo ? rpt[r] - e_lo : 0u;
+        const u32 end = r + 1 != r_hi && rpt[r + 1] < e_hi ? rpt[r + 1] : e_hi;
         const u32 e = end > e_lo ? end - e_lo : 0u;
         t0 = (u32)(((u64)b + TILE - 1) / TILE);
         const u32 t1 = (u32)(((u64)e + TILE - 1) / TILE);

@@ -57,12 +57,19 @@ constexpr u32 PK_WORDS = EX_TILE / 32;
 struct PackTile {
     u64 e0, e1;
     u32 r0, nr;  // rows from the one that holds e0 to the one that holds e1
-    __device__ __forceinline__ PackTile(const u32 *__restrict__ first, u32 b_nzr, u32 b_nnz) {
+    bool last;
+    // (columns past the last row's end are no entries)
+    __device__ __forceinline__ PackTile(const u32 *__restrict__ first, const u32 *__restrict__ b_rpt, u32 b_nzr,
+                                        u32 b_nnz) {
+        const u32 end = b_rpt[b_nzr];
+        const u64 n = end < b_nnz ? end : b_nnz;
         e0 = (u64)blockIdx.x * EX_TILE;
-        e1 = e0 + EX_TILE < b_nnz ? e0 + EX_TILE : b_nnz;
+        e1 = e0 + EX_TILE < n ? e0 + EX_TILE : n;
+        last = e1 == n;
         r0 = first[blockIdx.x];
-        nr = (blockIdx.x + 1 < gridDim.x ? first[blockIdx.x + 1] : b_nzr - 1) - r0 + 1;
+        nr = (last ? b_nzr - 1 : first[blockIdx.x + 1]) - r0 + 1;
     }
+    __device__ __forceinline__ bool empty() const { return e0 >= e1; }
     // c[q] = column e0 + q * EX_WG + threadIdx.x, sb = a bit per column that
     // begins a pack (complete after a barrier).
     __device__ __forceinline__ void starts(const u32 *__restrict__ b_rpt, const u32 *__restrict__ b_cols,
@@ -98,7 +105,11 @@ __global__ __launch_bounds__(EX_WG) void k_pack_count(const u32 *__restrict__ b_
                                                       u32 b_nzr, u32 b_nnz, const u32 *__restrict__ first,
                                                       u32 *__restrict__ counts) {
     __shared__ u32 sb[PK_WORDS];
-    const PackTile t(first, b_nzr, b_nnz);
+    const PackTile t(first, b_rpt, b_nzr, b_nnz);
+    if (t.empty()) {  // uniform
+        if (threadIdx.x == 0) counts[blockIdx.x] = 0;
+        return;
+    }
     u32 c[EX_ITEMS];
     t.starts(b_rpt, b_cols, c, sb);
     __syncthreads();
@@ -113,7 +124,8 @@ __global__ __launch_bounds__(EX_WG) void k_pack_place(const u32 *__restrict__ b_
                                                       const u32 *__restrict__ offs, u32 *__restrict__ prpt,
                                                       u32 *__restrict__ packs, u32 *__restrict__ pfirst) {
     __shared__ u32 sb[PK_WORDS], spre[PK_WORDS + 1];
-    const PackTile t(first, b_nzr, b_nnz);
+    const PackTile t(first, b_rpt, b_nzr, b_nnz);
+    if (t.empty()) return;  // uniform
     u32 c[EX_ITEMS];
     t.starts(b_rpt, b_cols, c, sb);
     __syncthreads();
@@ -129,7 +141,7 @@ __global__ __launch_bounds__(EX_WG) void k_pack_place(const u32 *__restrict__ b_
     };
     // where the row that holds the tile's last column ends
     const u32 rn = t.r0 + t.nr - 1;
-    const u64 limit = blockIdx.x + 1 < gridDim.x && b_rpt[rn] < t.e1 ? b_rpt[rn + 1] : t.e1;
+    const u64 limit = !t.last && b_rpt[rn] < t.e1 ? b_rpt[rn + 1] : t.e1;
     const int l = dev::lane();
 #pragma unroll
     for (u32 q = 0; q < EX_ITEMS; ++q) {
@@ -165,7 +177,7 @@ __global__ __launch_bounds__(EX_WG) void k_pack_place(const u32 *__restrict__ b_
     }
     if (blockIdx.x == 0)
         for (u32 r = threadIdx.x; r < t.r0; r += EX_WG) prpt[r] = 0;  // without entries
-    if (blockIdx.x + 1 == gridDim.x && threadIdx.x == 0) prpt[b_nzr] = spre[PK_WORDS];
+    if (t.last && threadIdx.x == 0) prpt[b_nzr] = spre[PK_WORDS];
 }
 
 // Mats::psplits from Mats::splits: slices begin at multiples of 16 columns, so
