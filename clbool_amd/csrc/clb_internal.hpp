@@ -151,8 +151,12 @@ struct clb_controls_s {
     hipStream_t tail[NTAIL] = {};
     clb::Pool *pool = nullptr;    // its device's
     clb::PoolBlocks::Owner retired;  // released temporaries (under the pool's lock)
-    bool settled = false;         // see Settled
+    std::atomic<bool> settled{false};  // see Settled
+    // Plans hold arrays of the controls: one that is destroyed before its last
+    // plan is released ends with that release.
     std::mutex mu;
+    clb::u32 plans = 0;           // under mu
+    bool destroyed = false;       // under mu
 };
 
 namespace clb {
@@ -208,6 +212,10 @@ struct Settled {
     Settled(const Settled &) = delete;
     Settled &operator=(const Settled &) = delete;
 };
+
+// A plan of the controls begins, and has released its arrays.
+void plan_begins(clb_controls_s *ctl);
+void plan_ends(clb_controls_s *ctl);
 
 // The main stream waits for the side streams.
 void join_side(clb_controls_s *ctl);

@@ -311,6 +311,7 @@ clb_status clb_spgemm_plan_create(clb_controls ctl, const clb_dcsr *a, const clb
             auto p = std::make_unique<clb_spgemm_plan_s>();
             p->s.lean = lean;
             spg::plan_create(ctl, *a, *b, mode, block_bound, *p);
+            plan_begins(ctl);
             *out = p.release();
         });
     });
@@ -355,11 +356,18 @@ clb_status clb_spgemm_plan_run_all(clb_controls ctl, clb_spgemm_plan plan, uint3
 clb_status clb_spgemm_plan_release(clb_spgemm_plan plan) {
     return run_guarded([&] {
         if (!plan) return;
-        settle(plan->ctl);
-        Settled idle(plan->ctl);
+        // possibly on another thread than the one that uses the controls now
+        clb_controls_s *const ctl = plan->ctl;
         clb_dcsr_release(&plan->a);
         clb_dcsr_release(&plan->b);
         delete plan;
+        try {
+            sync(ctl);  // its arrays are anyone's
+        } catch (...) {
+            plan_ends(ctl);
+            throw;
+        }
+        plan_ends(ctl);
     });
 }
 

@@ -221,6 +221,38 @@ void settle(clb_controls_s *ctl) noexcept {
     for (hipStream_t st : ctl->tail) (void)hipStreamSynchronize(st);
 }
 
+static void controls_end(clb_controls_s *ctl) {
+    (void)hipStreamSynchronize(ctl->stream);
+    learned_destroy_state(ctl);
+    (void)hipHostFree(ctl->pinned);
+    for (int k = 0; k < clb_controls_s::NSIDE; ++k) {
+        (void)hipStreamSynchronize(ctl->side[k]);
+        (void)hipStreamDestroy(ctl->side[k]);
+        (void)hipEventDestroy(ctl->ev_join[k]);
+    }
+    (void)hipEventDestroy(ctl->ev_fork);
+    for (int k = 0; k < clb_controls_s::NTAIL; ++k) {
+        (void)hipStreamSynchronize(ctl->tail[k]);
+        (void)hipStreamDestroy(ctl->tail[k]);
+    }
+    ctl->pool->leave(ctl);  // before its stream ends
+    (void)hipStreamDestroy(ctl->stream);
+    delete ctl;
+}
+
+void plan_begins(clb_controls_s *ctl) {
+    std::lock_guard<std::mutex> lk(ctl->mu);
+    ++ctl->plans;
+}
+
+void plan_ends(clb_controls_s *ctl) {
+    {
+        std::lock_guard<std::mutex> lk(ctl->mu);
+        if (--ctl->plans || !ctl->destroyed) return;
+    }
+    controls_end(ctl);
+}
+
 void join_side(clb_controls_s *ctl) {
     for (int k = 0; k < clb_controls_s::NSIDE; ++k) {
         CLB_HIP(hipEventRecord(ctl->ev_join[k], ctl->side[k]), EVENT_WAITING_ERROR);
@@ -450,22 +482,12 @@ clb_status clb_controls_create(uint32_t platform_id, uint32_t device_id, clb_con
 clb_status clb_controls_destroy(clb_controls ctl) {
     return guarded([&] {
         if (!ctl) return;
-        (void)hipStreamSynchronize(ctl->stream);
-        clb::learned_destroy_state(ctl);
-        (void)hipHostFree(ctl->pinned);
-        for (int k = 0; k < clb_controls_s::NSIDE; ++k) {
-            (void)hipStreamSynchronize(ctl->side[k]);
-            (void)hipStreamDestroy(ctl->side[k]);
-            (void)hipEventDestroy(ctl->ev_join[k]);
+        {
+            std::lock_guard<std::mutex> lk(ctl->mu);
+            ctl->destroyed = true;
+            if (ctl->plans) return;  // the last plan ends it
         }
-        (void)hipEventDestroy(ctl->ev_fork);
-        for (int k = 0; k < clb_controls_s::NTAIL; ++k) {
-            (void)hipStreamSynchronize(ctl->tail[k]);
-            (void)hipStreamDestroy(ctl->tail[k]);
-        }
-        ctl->pool->leave(ctl);  // before its stream ends
-        (void)hipStreamDestroy(ctl->stream);
-        delete ctl;
+        controls_end(ctl);
     });
 }
 

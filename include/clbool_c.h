@@ -339,6 +339,7 @@ clb_status clb_spgemm_plan_run(clb_controls ctl, clb_spgemm_plan plan, uint32_t 
 typedef int32_t (*clb_spgemm_block_fn)(void *user, uint32_t k, clb_dcsr *block, const clb_spgemm_stats *stats);
 clb_status clb_spgemm_plan_run_all(clb_controls ctl, clb_spgemm_plan plan, uint32_t timing, clb_spgemm_block_fn fn,
                                    void *user);
+/* On any thread, also after the controls were destroyed. */
 clb_status clb_spgemm_plan_release(clb_spgemm_plan plan);
 
 /* dcsr::kronecker_product (src/dcsr/dcsr_kronecker_product.cpp:6-65) */
