@@ -1353,14 +1353,15 @@ void launch_bins(clb_controls_s *ctl, const Setup &s, const u32 *perm, const u32
             // widest workgroup, beside the others (R-MAT 2^16, symbolic: its
             // CUs were busy for 228 of 583 us, waiting for rows of up to 645
             // thousand products on 256 threads; 421 us with the 493 largest
-            // rows on 1024)
+            // rows on 1024); the widest have no word-combining gather, which is
+            // asked for by a knob
             const u32 slots = ctl->cu_count * bitmap_resident(bits);
             u64 products = 0;
             for (u32 b = BIN_BITMAP0; b < NBINS; ++b) products += s.bin_products[b];
             u32 lp = 14;
             while (lp < 32 && (1ull << lp) * 2 * slots < products) ++lp;
             u32 heavy = 0;
-            if (bitmap_wide(bits) > bitmap_wg(bits) && !ctl->tuning.bitmap_persistent && lp < 32)
+            if (bitmap_wide(bits) > bitmap_wg(bits) && !ctl->tuning.bitmap_persistent && !s.g.combine && lp < 32)
                 heavy = off[bitmap_bin_below(lp)] - off[BIN_BITMAP0];
             for (int wide = 1; wide >= 0; --wide) {
                 const u32 r0 = wide ? 0 : heavy, nr = wide ? heavy : n - heavy;
