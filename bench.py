@@ -17,6 +17,7 @@ also carries the roofline of the dominant kernel (algorithmic bytes per
 launch over its HIP-event duration) and the CPU baseline (the reference test
 suite's host SpGEMM, matrix_multiplication_cpu restated in oracle/, timed on
 a bounded row sample) beside a multi-threaded Gustavson on the host cores.
+The line holds one summary per workload; --details FILE takes the rest.
 Reported beside the main metric as well: the 64-label closure (4 steps; to
 its fixed point with --closure-only), the hypersparse learned-sizing workload
 (2^24 x 2^24, the predictor trained on 200 instances) and the automaton (x)
@@ -484,18 +485,24 @@ def roofline_of(cb, agg, workload):
     # column), not by the bitmap family that found them; the bitmap dump in
     # between is not counted.  The compaction moves 4 B in and 4 B out per
     # column it copies.
+    # Bin 13 holds the rows whose bitmap an earlier kernel kept: the numeric
+    # pass's bitmap family and the one pass's emission only expand them, 4 B per
+    # column (the kept bitmap in between is not counted either).
     pass_, kind = divmod(fam, 4)
-    bins = {0: range(1, 2), 1: range(2, 13), 2: range(13, 32)}.get(kind, range(0))
+    bins = {0: range(1, 2), 1: range(2, 13), 2: range(14, 32)}.get(kind, range(0))
+    if kind == 2 and pass_ == 0:
+        bins = range(13, 32)  # the symbolic pass gathers the rows it keeps
     writes = pass_ != 0
     rows_f = sum(agg["bin_rows"][b] for b in bins)
+    kept_nnz = agg["bin_out_nnz"][13]
     bytes_total = sum(12 * agg["bin_a_nnz"][b] + 4 * agg["bin_products"][b] +
                       (4 * agg["bin_out_nnz"][b] if writes else 0) for b in bins) + 8 * rows_f
     if kind == 2 and writes:
-        bytes_total -= 4 * agg["dense_nnz"]
+        bytes_total += (4 * kept_nnz if pass_ == 1 else 0) - 4 * agg["dense_nnz"]
     if fam_names[fam] == "onepass_compact":
-        bytes_total = 8 * (agg["nnz"] - agg["dense_nnz"])
+        bytes_total = 8 * (agg["nnz"] - agg["dense_nnz"] - kept_nnz)
     elif kind == 3:
-        bytes_total = 4 * agg["dense_nnz"]
+        bytes_total = 4 * (agg["dense_nnz"] + (kept_nnz if pass_ == 2 else 0))
     bytes_per_launch = bytes_total / launches
     achieved = bytes_per_launch / (avg_ms / 1e3) / 1e9
     traffic = None
@@ -586,6 +593,49 @@ def bench_product(cb, gen, ctl, oracle, workload, modes, steps, warmup, tuned, v
     return out, A
 
 
+def rounded(x):
+    """Floats to six significant digits: the line has to stay short."""
+    if isinstance(x, float):
+        return float(f"{x:.6g}")
+    if isinstance(x, dict):
+        return {k: rounded(v) for k, v in x.items()}
+    return [rounded(v) for v in x] if isinstance(x, list) else x
+
+
+def report(workload, steps, warmup, best, details):
+    """The printed line: the metric, and of every workload what sums it up."""
+    res, dev = details["workloads"][workload], details["device"]
+    R = res["modes"][best]
+    out = {
+        "metric": METRIC, "value": R["products_per_s"], "unit": "products/s", "n_gpus": 1, "steps": steps,
+        "warmup": warmup, "ms_per_step": R["ms_per_step"], "higher_is_better": True, "scaling": "weak",
+        "vs_baseline": None, "dtype": "u32", "data": "synthetic",
+        "config": {**res["config"], "nnz_out": res["nnz_out"], "row_blocks": R["row_blocks"],
+                   "mode": best, "device": dev["arch"], "compute_units": dev["compute_units"]},
+        "output_nnz_per_s": R["nnz_per_s"], "roofline": R["roofline"], "fallback_rate": R["fallback_rate"],
+    }
+    for w, r in details["workloads"].items():
+        out[w] = {"ms": {m: v["ms_per_step"] for m, v in r["modes"].items()},
+                  **{k: r[k] for k in ("learned_vs_plain", "bound_vs_plain") if k in r},
+                  "validated_rows": sum(r["validated_rows"].values())}
+    if c := details.get("closure"):
+        out["closure"] = {"ms": {k: 1e3 * v["seconds"] for k, v in c.items() if isinstance(v, dict)},
+                          "products": c["batched_learned"]["products"], "identical": c["identical_results"]}
+    if h := details.get("hypersparse"):
+        t = h["tests"]
+        out["hypersparse"] = {"plain_ms": [x["plain_ms"] for x in t], "learned_ms": [x["learned_ms"] for x in t],
+                              "fallback_rows": sum(x["fallback_rows"] for x in t),
+                              "identical": all(x["identical"] for x in t)}
+    if c := details.get("c5"):
+        out["c5"] = {"kronecker_ms": 1e3 * c["kronecker"]["seconds"], "kronecker_GB_per_s": c["kronecker"]["GB_per_s"],
+                     "kk_ms": {m: 1e3 * c["kk_step"][m]["seconds"] for m in ("plain", "learned")},
+                     "identical": c["kk_step"]["identical_results"]}
+    if "cpu_baseline" in details:
+        out["cpu_baseline"] = details["cpu_baseline"]
+        out["cpu_gustavson"] = {k: details["cpu_gustavson"][k] for k in ("value", "cores")}
+    return json.dumps(rounded(out), separators=(",", ":"))
+
+
 def main():
     ap = argparse.ArgumentParser()
     ap.add_argument("--gpus", type=int, default=1)
@@ -617,6 +667,8 @@ def main():
     ap.add_argument("--closure-cold", action="store_true", help="with --closure-only: no warm-up runs")
     ap.add_argument("--closure-legs", default="per_triple_plain,batched_learned",
                     help="with --closure-only: comma-separated legs (per_triple_plain, batched_plain, batched_learned)")
+    ap.add_argument("--details", metavar="FILE", default=None,
+                    help="also write everything measured (per kernel family, per bin, knobs, closure steps) as JSON")
     ap.add_argument("--no-c5", action="store_true",
                     help="skip the automaton (x) R-MAT 22/32 workload reported beside the main metric")
     ap.add_argument("--c5-only", action="store_true",
@@ -706,54 +758,41 @@ def main():
 
     main_res, A = bench_product(cb, gen, ctl, oracle, args.workload, modes, args.steps, args.warmup, tuned,
                                 not args.no_validate, block_bound, log)
-    best = "learned" if "learned" in main_res["modes"] else modes[0]
-    R = main_res["modes"][best]
-    out = {
-        "metric": METRIC, "value": R["products_per_s"], "unit": "products/s", "n_gpus": 1, "steps": args.steps,
-        "warmup": args.warmup, "ms_per_step": R["ms_per_step"], "higher_is_better": True, "scaling": "weak",
-        "vs_baseline": None, "dtype": "u32", "data": "synthetic",
-        "config": {**main_res["config"], "nnz_out": main_res["nnz_out"], "row_blocks": R["row_blocks"],
-                   "mode": best, "device": dev["arch"], "compute_units": dev["compute_units"]},
-        "output_nnz_per_s": R["nnz_per_s"],
-        "roofline": R["roofline"],
-        "predictor_training": train,
-        "pred_abs_log2_err": R.get("pred_abs_log2_err"),
-        "fallback_rate": R.get("fallback_rate"),
-    }
-    for k in ("learned_vs_plain", "bound_vs_plain", "learned_vs_bound", "modes", "validated_rows"):
-        if k in main_res:
-            out[k] = main_res[k]
+    details = {"device": dev, "workloads": {args.workload: main_res}, "predictor_training": train}
     for w in [w for w in args.also.split(",") if w and w != args.workload]:
         wt = os.path.join(ROOT, "profiles", f"tuning_{w}.json")
         wl = json.load(open(wt)) if os.path.exists(wt) else {}
         tw = {m: {**base_tuning, **wl.get(m, {}), **overrides} for m in modes}
-        res, _ = bench_product(cb, gen, ctl, oracle, w, modes, args.steps, args.warmup, tw, not args.no_validate,
-                               block_bound, log)
-        out[w] = res
+        details["workloads"][w], _ = bench_product(cb, gen, ctl, oracle, w, modes, args.steps, args.warmup, tw,
+                                                   not args.no_validate, block_bound, log)
     if args.closure_iters > 0 and "learned" in modes:
         at.apply(ctl, tuned.get("learned", base_tuning))
-        out["closure"] = bench_closure(cb, gen, ctl, args.closure_iters, log)
+        details["closure"] = bench_closure(cb, gen, ctl, args.closure_iters, log)
     if args.hypersparse > 0:
-        out["hypersparse"] = bench_hypersparse(cb, gen, ctl, args.hypersparse, log)
+        details["hypersparse"] = bench_hypersparse(cb, gen, ctl, args.hypersparse, log)
     if not args.no_c5 and "learned" in modes:
         ctl.trim()
         # each mode's step with that mode's knobs of the main workload (K is
         # 2^22 columns wide, as R-MAT 22)
-        out["c5"] = bench_c5(cb, gen, ctl, log,
-                             tunings={m: tuned.get(m, base_tuning) for m in ("plain", "learned")})
+        details["c5"] = bench_c5(cb, gen, ctl, log,
+                                 tunings={m: tuned.get(m, base_tuning) for m in ("plain", "learned")})
     if not args.no_cpu_baseline:
         log("[bench] timing the CPU baseline")
-        out["cpu_baseline"] = cpu_baseline(oracle, A)
+        details["cpu_baseline"] = cpu_baseline(oracle, A)
         try:
             nproc = len(os.sched_getaffinity(0))
         except AttributeError:
             nproc = os.cpu_count() or 1
         threads = int(os.environ.get("OMP_NUM_THREADS", nproc))
-        out["cpu_gustavson"] = cpu_gustavson(oracle, A, threads)
-        out["host"] = {"nproc": nproc, "os_cpu_count": os.cpu_count(), "omp_num_threads": threads}
-        out["clbool_cpu_opencl"] = ("not run: clBool's create_controls asks only for GPU devices "
-                                    "(src/common/env.cpp:21) and no CPU OpenCL runtime is installed")
-    print(json.dumps(out), flush=True)
+        details["cpu_gustavson"] = cpu_gustavson(oracle, A, threads)
+        details["host"] = {"nproc": nproc, "os_cpu_count": os.cpu_count(), "omp_num_threads": threads}
+        details["clbool_cpu_opencl"] = ("not run: clBool's create_controls asks only for GPU devices "
+                                        "(src/common/env.cpp:21) and no CPU OpenCL runtime is installed")
+    if args.details:
+        with open(args.details, "w") as f:
+            json.dump(details, f, indent=1)
+    best = "learned" if "learned" in main_res["modes"] else modes[0]
+    print(report(args.workload, args.steps, args.warmup, best, details), flush=True)
 
 
 if __name__ == "__main__":
