@@ -94,6 +94,11 @@ class Pool {
         std::lock_guard<std::mutex> lk(mu_);
         return blocks_.free_bytes();
     }
+    // The largest block it can hand out without new memory.
+    u64 largest_free() const {
+        std::lock_guard<std::mutex> lk(mu_);
+        return blocks_.largest_free();
+    }
     int device() const { return device_; }
     // [0] free bytes inside the pool's segments, [1] hipMalloc calls, [2]
     // bytes they allocated, [3] times free segments were handed back after a

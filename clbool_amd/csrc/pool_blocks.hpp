@@ -126,6 +126,8 @@ class PoolBlocks {
         small_.collect_free_segments(out);
         large_.collect_free_segments(out);
     }
+    // The largest free block; retired ones are not among them.
+    u64 largest_free() const { return large_.largest_free(); }
     // Bytes that are not in use, retired ones among them.
     u64 free_bytes() const { return small_.free_bytes() + large_.free_bytes() + retired_bytes_; }
 
