@@ -472,9 +472,11 @@ def cpu_gustavson(oracle, A, threads, target_rows=20000, seed=11):
 MODE_CODES = {"plain": 0, "learned": 1, "bound": 2}
 
 
-def roofline_of(cb, agg, workload):
+def roofline_of(cb, agg, workload, learned=True):
     """Roofline of the dominant kernel family of a timed step: algorithmic
-    bytes of that family's launches over their HIP-event durations."""
+    bytes of that family's launches over their HIP-event durations (launches side
+    by side on several streams each count in full).  The measured traffic is that
+    of the learned step."""
     fam_names = cb._capi.KERNEL_FAMILIES
     fam = int(np.argmax(agg["ms_kernel"]))
     launches = max(agg["launches"][fam], 1)
@@ -507,7 +509,7 @@ def roofline_of(cb, agg, workload):
     achieved = bytes_per_launch / (avg_ms / 1e3) / 1e9
     traffic = None
     tpath = os.path.join(ROOT, "profiles", f"traffic_{workload}.json")
-    if os.path.exists(tpath):
+    if learned and os.path.exists(tpath):
         try:
             traffic = json.load(open(tpath)).get(fam_names[fam])
         except Exception:
@@ -582,7 +584,7 @@ def bench_product(cb, gen, ctl, oracle, workload, modes, steps, warmup, tuned, v
             # per bin (0 empty, 1 tiny, 2-9 hash 2^7..2^14 slots, 10-12 LDS ESC,
             # 13-31 bitmap by product count), last timed step
             "bin_rows": agg["bin_rows"], "bin_products": agg["bin_products"],
-            "roofline": roofline_of(cb, agg, workload),
+            "roofline": roofline_of(cb, agg, workload, m == "learned"),
             "step_hbm_frac": step_algorithmic_bytes(int(rows.size), int(cols.size), total_products,
                                                     int(rows.size), agg["nnz"]) / (v["ms_per_step"] / 1e3) / 1e9
             / HBM_PEAK_GBS}

@@ -31,7 +31,7 @@ KNOBS = {
     "bitmap_pred_caps": [0, 1],   # one pass: bitmap rows sized by the prediction (1) or the bound (0)
     "gather_combine": [0, 1],     # bitmap gather: one LDS atomic per word and wave (1) or per product (0)
     "esc_max_products": [0, 2048, 8192],  # multi-window bitmap rows up to this many products sort in LDS
-    "compact_tiles": [0, 1],      # one pass: compaction by output tiles (1) or one workgroup per row (0)
+    "compact_tiles": [0, 1],      # one pass: compaction by output tiles (1) or by rows (0)
     "onepass_bitmap_min": [0, 8192, 32768, 131072],  # one pass: product count that forces a bitmap (0: never)
     "bitmap_window_bits": [0, 13, 14, 15],  # numeric / one-pass bitmap window, 2^bits words (0: by width)
     "emit_sparse_bits": [0, 64, 1024, 4096],  # bitmap slices below this many bits per 1024 words: lane-own emission

@@ -10,7 +10,7 @@
 // (create_final_matrix, :97-158).  Here, with the same one-pass structure:
 //  * rows of at most 64 products: one wave, register bitonic sort (k_tiny);
 //  * up to 2^13 products: one workgroup expands the products into LDS,
-//    merge-sorts them there and keeps the first of each run (k_esc);
+//    radix-sorts them there and keeps the first of each run (k_esc);
 //  * longer rows: all their products are expanded at once into HBM, a stretch
 //    per row, each stretch is radix-sorted by column and deduplicated, instead
 //    of the reference's pairwise merges of B rows per row; beside the kernels

@@ -1288,13 +1288,13 @@ LaunchTimer::~LaunchTimer() {
     if (pending) (void)hipEventDestroy(pending);
 }
 
-// Launch the per-bin kernels of one pass.  off[b]..off[b+1] is bin b's range
-// of perm.  numeric == false: write nnz_row; true: write columns.
 void join_deferred(clb_controls_s *ctl, const hipEvent_t *defer) {
     for (int k = 0; k < clb_controls_s::NSIDE; ++k)
         CLB_HIP(hipStreamWaitEvent(ctl->stream, defer[k], 0), EVENT_WAITING_ERROR);
 }
 
+// Launch the per-bin kernels of one pass.  off[b]..off[b+1] is bin b's range
+// of perm.  mode SYM writes nnz_row, NUM the columns, ONE both.
 void launch_bins(clb_controls_s *ctl, const Setup &s, const u32 *perm, const u32 off[NBINS + 1], int mode,
                  const Out &o, LaunchTimer *lt, int family, hipEvent_t *defer, bool one_stream, bool open) {
     constexpr int NS = clb_controls_s::NSIDE;

@@ -443,8 +443,9 @@ struct Dump {
 
 // Bitmap rows whose bitmap the symbolic pass, or the one pass, keeps in global
 // memory: the numeric pass only expands it (k_emit_stored) instead of
-// gathering the row's products again, and a row of the one pass needs no
-// temporary slot and no capacity.  Slot = the row's position in the bitmap range of
+// gathering the row's products again, and a row of the one pass is not held to
+// its capacity (its temporary slot, which is given out before the rows to keep
+// are known, stays unused).  Slot = the row's position in the bitmap range of
 // perm, for the first `slots` of them (the bins descend by products).  A slice
 // is kept as its words or, when at most a third of them are nonzero and the
 // window is wide, as (word index, word) pairs.

@@ -81,7 +81,8 @@ typedef struct clb_tuning {
                                       learned one pass, off in the numeric
                                       pass, and bitmap rows are kept by the
                                       pass that finds them where that gathers
-                                      their products once)                    */
+                                      their products once; a value below 65536
+                                      dumps rows instead of keeping them)     */
     uint32_t bitmap_persistent;    /* nonzero: the bitmap rows run on a persistent
                                       grid that takes rows from a counter
                                       instead of one workgroup per row          */
@@ -103,7 +104,7 @@ typedef struct clb_tuning {
                                       reserved[CLB_TUNE_COMPACT_TILES]: nonzero:
                                       the one pass's compaction gives every
                                       workgroup an equal tile of output columns
-                                      (0: one workgroup per row)
+                                      (0: rows to waves, long ones to workgroups)
                                       reserved[CLB_TUNE_HASH_WIDE]: bit b set:
                                       LDS hash tables of 2^(7+b) slots run with
                                       twice the default workgroup (64 threads
