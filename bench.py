@@ -277,7 +277,7 @@ def _dcsr_rows(rpt, rows, cols, keep):
     return np.r_[0, np.cumsum(lens)].astype(np.uint32), rows[keep].astype(np.uint32), cols[idx].astype(np.uint32)
 
 
-def bench_c5(cb, gen, ctl, log, scale=22, ef=32, step_scale=16, seed=1, tunings=None):
+def bench_c5(cb, gen, ctl, log, scale=22, ef=32, step_scale=16, seed=1):
     """The RPQ input of a 64x64 automaton M (200 uniform nonzeros) and an
     R-MAT graph G (scale 22, edge factor 32).  K = M (x) G has about 2.6e10
     nonzeros, more than one uint32 DCSR holds, so it is built in blocks of
@@ -286,8 +286,7 @@ def bench_c5(cb, gen, ctl, log, scale=22, ef=32, step_scale=16, seed=1, tunings=
     about 3e14 products, beyond one GPU; the step itself is measured on the
     same automaton with G at scale `step_scale` (K of width 64 * 2^16 = 2^22),
     whole, in row blocks of output bound below 2^32, plain and learned; both
-    results must agree.  tunings: knobs per mode ("plain", "learned") applied
-    before that mode's step (None: the controls' current knobs for both)."""
+    results must agree."""
     mr, mc = gen.uniform_pairs(200, 64, 64, seed)
     mrpt, mrows, mcols = gen.to_dcsr(mr, mc)
     out = {"automaton": {"n": 64, "nnz": int(mr.size), "seed": seed}}
@@ -341,9 +340,6 @@ def bench_c5(cb, gen, ctl, log, scale=22, ef=32, step_scale=16, seed=1, tunings=
     train = train_predictor(cb, gen, ctl, log)
     prints = {}
     for name, mode in (("plain", cb.SPGEMM_PLAIN), ("learned", cb.SPGEMM_LEARNED)):
-        if tunings and name in tunings:
-            from clbool_amd import autotune as at
-            at.apply(ctl, tunings[name])
         best = None
         for rep in range(3):
             ctl.sync()
@@ -768,16 +764,18 @@ def main():
         details["workloads"][w], _ = bench_product(cb, gen, ctl, oracle, w, modes, args.steps, args.warmup, tw,
                                                    not args.no_validate, block_bound, log)
     if args.closure_iters > 0 and "learned" in modes:
-        at.apply(ctl, tuned.get("learned", base_tuning))
+        # the knobs of A * A are not this workload's: its plain legs are slower
+        # with them (per triple 419 against 291 ms), the learned one too (326 / 306)
+        at.apply(ctl, {**base_tuning, **overrides})
         details["closure"] = bench_closure(cb, gen, ctl, args.closure_iters, log)
     if args.hypersparse > 0:
+        at.apply(ctl, tuned.get("learned", {**base_tuning, **overrides}))
         details["hypersparse"] = bench_hypersparse(cb, gen, ctl, args.hypersparse, log)
     if not args.no_c5 and "learned" in modes:
         ctl.trim()
-        # each mode's step with that mode's knobs of the main workload (K is
-        # 2^22 columns wide, as R-MAT 22)
-        details["c5"] = bench_c5(cb, gen, ctl, log,
-                                 tunings={m: tuned.get(m, base_tuning) for m in ("plain", "learned")})
+        # (K*K learned 1756 ms, 1912 with the knobs of R-MAT 22; plain 2583 / 2522)
+        at.apply(ctl, {**base_tuning, **overrides})
+        details["c5"] = bench_c5(cb, gen, ctl, log)
     if not args.no_cpu_baseline:
         log("[bench] timing the CPU baseline")
         details["cpu_baseline"] = cpu_baseline(oracle, A)
