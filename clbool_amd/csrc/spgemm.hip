@@ -789,6 +789,32 @@ void emit_stored(hipStream_t st, const u32 *perm, u32 n, const Store &keep, cons
     CLB_LAUNCHED("emit_stored");
 }
 
+// Room for `want` bytes of scratch that may be smaller: a share of the memory at
+// hand, so that most of it stays for the operands and the output (what the pool
+// caches counts as free: it hands that back when an allocation fails).  Not new
+// memory where the largest free block nearly does, since HIP takes back and
+// gives out again at some 30 ms a GB:
+//  * the memory at hand is never twice quite the same, so a block limited by it
+//    would be a little larger at every call.  R-MAT 22 planned and run in a loop
+//    took another 77 GB of kept bitmaps three times, then handed 249 GB back:
+//    2.9 s of one call, 1.5 s of each on average, 0.65 now.
+//  * where HIP has not got that much left, a new block costs the pool all it
+//    caches: half is enough then.  The first learned R-MAT 22 product, whose 18
+//    blocks dump more and more rows, took 5.0 s, 0.45 now.
+static u64 scratch_bytes(clb_controls_s *ctl, u64 want, u64 share) {
+    size_t free_b = 0, total_b = 0;
+    if (hipMemGetInfo(&free_b, &total_b) != hipSuccess) {
+        (void)hipGetLastError();
+        return 0;
+    }
+    Pool &pool = pool_for(ctl->device);
+    const u64 budget = (free_b + pool.cached_bytes()) / share, have = pool.largest_free();
+    const u64 bytes = want < budget ? want : budget;
+    if (have >= bytes) return bytes;
+    if (bytes > free_b) return have >= bytes / 2 ? have : bytes;
+    return bytes < want && have >= bytes - bytes / 8 ? have : bytes;
+}
+
 void setup_store(clb_controls_s *ctl, const Setup &s, const BinHost &h, u32 bits, StoreBufs &b) {
     b.keep = Store{};
     if (s.lean) return;
@@ -809,28 +835,8 @@ void setup_store(clb_controls_s *ctl, const Setup &s, const BinHost &h, u32 bits
     const u32 end = lp <= 13 ? h.off[NBINS] : (lp > 31 ? h.off[BIN_BITMAP0] : h.off[bitmap_bin_below(lp)]);
     u64 slots = end - h.off[BIN_BITMAP0];
     if (!slots) return;
-    if (slots * words * 4 > (1ull << 30)) {
-        // large: at most a quarter of the memory at hand
-        size_t free_b = 0, total_b = 0;
-        if (hipMemGetInfo(&free_b, &total_b) != hipSuccess) {
-            (void)hipGetLastError();
-            return;
-        }
-        Pool &pool = pool_for(ctl->device);
-        const u64 budget = (free_b + pool.cached_bytes()) / 4, have = pool.largest_free();
-        u64 most = budget / (words * 4);
-        if (slots > most) {
-            // what is free is never twice quite the same, and a block a little
-            // larger than the last call's is new memory: the block that is there
-            // is taken when it is about as large.  (R-MAT 22 planned and run in a
-            // loop took another 77 GB three times, then gave 249 GB back and
-            // asked for them again: 2.9 s of one call, 1.5 s of each on average,
-            // 0.66 now.)
-            if (have < budget && have >= budget - budget / 8) most = have / (words * 4);
-            slots = most;
-        }
-        if (!slots) return;
-    }
+    if (slots * words * 4 > (1ull << 30)) slots = scratch_bytes(ctl, slots * words * 4, 4) / (words * 4);
+    if (!slots) return;
     const u64 nch = words / store_chunk(win);
     try {
         b.words.reset(ctl, slots * words / 4);
@@ -890,16 +896,8 @@ void setup_dump(clb_controls_s *ctl, const Setup &s, const BinHost &h, DumpBufs 
         const u64 want = (u64)cand + cand / 8 + 256;
         slots = want < d.nbm ? (u32)want : d.nbm;
     }
-    size_t free_b = 0, total_b = 0;
-    if (hipMemGetInfo(&free_b, &total_b) != hipSuccess) {
-        (void)hipGetLastError();
-        return;
-    }
-    // keep most of HBM for the operands and the output; blocks cached by the
-    // pool count as free (the pool hands them back when an allocation fails)
-    const u64 budget = (free_b + pool_for(ctl->device).cached_bytes()) / 3;
     const u64 per_slot = (u64)d.words * 4;
-    if ((u64)slots * per_slot > budget) slots = (u32)(budget / per_slot);
+    slots = (u32)(scratch_bytes(ctl, slots * per_slot, 3) / per_slot);
     if (slots == 0) return;
     d.slots = slots;
     d.store.reset(ctl, (u64)slots * d.words / 4);
