@@ -618,9 +618,9 @@ __global__ void k_set_positions(const u32 *__restrict__ nnz_row, const u64 *__re
     c_rows[q] = a_rows[row0 + i];
 }
 
-// Writes one dumped row (one workgroup per row) into its columns at their
-// final positions.  Each of the 2 waves owns a contiguous half of the row's
-// words; its start position is the prefix of the chunk counts before its
+// Writes one dumped row (`parts` workgroups per row) into its columns at their
+// final positions.  Each of the 2 waves owns a contiguous half of its part of the
+// row's words; its start position is the prefix of the chunk counts before its
 // first chunk, so the waves need no exchange.  A bitmap slice is loaded 1024
 // words at a time (four rounds of 256, 16 bytes per lane per round),
 // double-buffered (the next 1024 words' loads are in flight while the
@@ -629,26 +629,32 @@ __global__ void k_set_positions(const u32 *__restrict__ nnz_row, const u64 *__re
 // (dev::emit_round4_ranked), a lane per column, so every store instruction is
 // one contiguous run.  Two-wave workgroups let more rows share a CU, so one
 // row's load latency overlaps another's expansion.  gpre = exclusive prefix of chunk_cnt over all slots.
+// A wave's expansion is a chain of LDS reads, so few rows with a workgroup each
+// would leave the chip idle: the one pass of 10 rows of 0.9 million products over
+// 2^22 columns takes 2.24 ms so, 0.99 with 32 workgroups a row; of 300 rows of 150
+// thousand products 1.01, 0.70 with 8 (0.73 with 4); of 2000 rows 1.52 either way.
 constexpr int EMIT_WG = 128;
+constexpr u32 EMIT_PART = 2048, EMIT_MIN_GRID = 2048;
 __global__ __launch_bounds__(EMIT_WG) void k_bitmap_emit(const uint4 *__restrict__ store, u32 nch,
                                                          const u64 *__restrict__ gpre, const u32 *__restrict__ list,
                                                          const u32 *__restrict__ perm, const u64 *__restrict__ off,
-                                                         u32 words_per_row, u32 slice_words,
+                                                         u32 words_per_row, u32 slice_words, u32 parts,
                                                          const u32 *__restrict__ fmt, u32 *__restrict__ cols) {
     constexpr u32 NW = EMIT_WG / 64, ROUNDS = 4, SPAN = ROUNDS * 256;
     __shared__ dev::RankLds stage[NW];
     __shared__ __align__(8) uint8_t tab[2048];
     dev::rank_table(tab);
     __syncthreads();
-    const u32 slot = blockIdx.x;  // slots are claimed densely from 0
+    const u32 slot = blockIdx.x / parts;  // slots are claimed densely from 0
     const u32 r = perm[list[slot]];
     u32 *out = cols + off[r];
     const u64 lim = off[r + 1] - off[r];
     const u32 wv = dev::wave_id(), l = (u32)dev::lane();
-    // words_per_row and slice_words are multiples of 2^14, so wpw and every
-    // slice boundary inside it are multiples of 2 * SPAN and of EMIT_CHUNK
-    const u32 wpw = words_per_row / NW;
-    const u32 first = wv * wpw, last = first + wpw;
+    // slice_words is a multiple of 2^14, and so are words_per_row and its parts
+    // or the parts divide a slice (emit_launch), so wpw and every slice boundary
+    // inside it are multiples of 2 * SPAN and of EMIT_CHUNK
+    const u32 wpw = words_per_row / (NW * parts);
+    const u32 first = (blockIdx.x % parts * NW + wv) * wpw, last = first + wpw;
     const u32 nsl = words_per_row / slice_words;
     const u32 *row = reinterpret_cast<const u32 *>(store) + (u64)slot * words_per_row;
     u64 p = gpre[(u64)slot * nch + first / EMIT_CHUNK] - gpre[(u64)slot * nch];
@@ -936,8 +942,12 @@ void emit_launch(hipStream_t es, u32 count, const u32 *perm, const BinHost &h, c
                  const u64 *off, u32 *cols, LaunchTimer *lt, int pass) {
     if (!count) return;
     if (lt) lt->begin(es);
-    k_bitmap_emit<<<count, EMIT_WG, 0, es>>>(d.store.ptr, d.nch, gpre, d.list.ptr, perm + h.off[BIN_BITMAP0], off,
-                                            d.words, d.slice_words, d.fmt.ptr, cols);
+    // few rows: several workgroups to each, until EMIT_MIN_GRID or parts of two
+    // rounds for each wave
+    u32 parts = 1;
+    while (count * parts < EMIT_MIN_GRID && d.words % (2 * parts * EMIT_WG / 64 * EMIT_PART) == 0) parts *= 2;
+    k_bitmap_emit<<<count * parts, EMIT_WG, 0, es>>>(d.store.ptr, d.nch, gpre, d.list.ptr, perm + h.off[BIN_BITMAP0],
+                                                     off, d.words, d.slice_words, parts, d.fmt.ptr, cols);
     CLB_LAUNCHED("bitmap_emit");
     if (lt) lt->end((int)CLB_KF(pass, CLB_KK_EMIT), es);
 }
