@@ -9,9 +9,9 @@
 // Consecutive threads take consecutive nonzeros, so f's reads and writes are
 // coalesced whatever the row lengths.
 //
-// What bounds it: HBM, at the bytes f moves.  One wave per row, which this
-// replaces, is bound by the chain row pointer -> columns and leaves most lanes
-// idle on short rows (keys of 15.3 million nonzeros in 532 thousand rows: 258
+// What bounds it: HBM, at the bytes f moves.  One wave per row, which few rows or
+// long ones still get (k_expand_by_rows), is bound by the chain row pointer ->
+// columns and leaves most lanes idle on short rows (keys of 15.3 million nonzeros in 532 thousand rows: 258
 // us, 68 us now; row ids of 16.1 million nonzeros: 94 us, 39 us now); finding
 // each tile's first row inside its workgroup (a 256-way search, three
 // dependent rounds) took 71 and 57 us.
@@ -121,10 +121,63 @@ __global__ __launch_bounds__(EX_WG) void k_expand(Expand<F> x, const u32 *__rest
     expand_tile(x, first, blockIdx.x, gridDim.x);
 }
 
+// A wave per row instead, for its first ER_LONG nonzeros, and one per ER_LONG
+// nonzeros for what their first one's row has past that.  Rows that begin among
+// them are written that far by their own waves, so nothing else is left to it.
+constexpr u32 ER_LONG = 4096;
+template <typename F>
+__global__ __launch_bounds__(EX_WG) void k_expand_by_rows(Expand<F> x) {
+    const u32 n = x.r_hi - x.r_lo, l = (u32)dev::lane();
+    const u64 w = (u64)blockIdx.x * (EX_WG / dev::WAVE) + __builtin_amdgcn_readfirstlane(threadIdx.x / dev::WAVE);
+    const u32 *__restrict__ rpt = x.rpt;
+    // row r's nonzeros from its `skip`-th on, up to position stop
+    auto fill = [&](u32 r, u32 skip, u64 pos, u64 stop) {
+        u32 b = rpt[r], end = rpt[r + 1];
+        const u32 id = x.rows ? x.rows[r] : r;
+        if (r == x.r_lo || b < x.e_lo) b = x.e_lo;
+        if (r + 1 == x.r_hi || end > x.e_hi) end = x.e_hi;
+        if (b >= end || end - b <= skip) return;
+        b += skip;
+        if (b < pos) b = (u32)pos;
+        if (end > stop) end = (u32)stop;
+        if (b >= end) return;
+        const u32 cnt = skip || end - b <= ER_LONG ? end - b : ER_LONG;
+#pragma unroll 4
+        for (u32 o = l; o < cnt; o += dev::WAVE) x.f(b + o, r, id);
+    };
+    if (w < n) {
+        fill(x.r_lo + (u32)w, 0, 0, x.e_hi);
+        return;
+    }
+    const u64 pos = x.e_lo + (w - n) * ER_LONG;
+    if (pos >= x.e_hi) return;
+    u32 r = x.r_lo, hi = x.r_hi;
+    while (hi - r > 1) {  // the last row that starts at or before pos
+        const u32 step = (hi - r + dev::WAVE - 1) / dev::WAVE;
+        const u64 c = (u64)r + (u64)l * step;
+        const u32 cnt = (u32)__popcll(__ballot(l == 0 || (c < hi && rpt[c] <= pos)));
+        r += (cnt - 1) * step;
+        hi = hi - r < step ? hi : r + step;
+    }
+    fill(r, ER_LONG, pos, pos + ER_LONG);
+}
+
 template <typename F>
 void expand_rows(clb_controls_s *ctl, const Expand<F> &x) {
     const u32 tiles = x.tiles();
     if (!tiles) return;
+    // One launch instead of two, but a wave for every row, however short: where
+    // that takes no longer than the other launch and the search of a tile's rows.
+    // Row ids in a call, by rows / by tiles (us): 1000 rows of 20 14.3 / 22.1, 30
+    // thousand of 500 25.2 / 35.7, 100 thousand of 64 24.8 / 29.8, 200 thousand of
+    // 30 36 / 31, a million of 17 129 / 53.
+    const u32 n = x.r_hi - x.r_lo;
+    if (n <= (1u << 16) + (x.e_hi - x.e_lo) / 64) {
+        const u64 waves = (u64)n + div_up((u64)x.e_hi - x.e_lo, ER_LONG);
+        k_expand_by_rows<F><<<div_up(waves, EX_WG / dev::WAVE), EX_WG, 0, ctl->stream>>>(x);
+        CLB_LAUNCHED("expand_rows");
+        return;
+    }
     DevArray<u32> first(ctl, tiles);
     k_tile_rows<EX_TILE>
         <<<div_up(x.r_hi - x.r_lo, EX_WG), EX_WG, 0, ctl->stream>>>(x.rpt, x.r_lo, x.r_hi, x.e_lo, x.e_hi, first.ptr);
