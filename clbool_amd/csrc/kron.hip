@@ -68,29 +68,44 @@ __global__ __launch_bounds__(KRON_WG) void k_kron_fill(const u32 *__restrict__ f
     const u32 e0 = tile * KRON_TILE;
     const u32 e1 = b_nnz - e0 < KRON_TILE ? b_nnz : e0 + KRON_TILE;
     const u32 ib0 = first[tile];
+    u32 a0 = a_rpt[ia0], a1 = a_rpt[ia0 + 1];  // needed last: on their way meanwhile
     // the tile's rows start at ib0 and number at most KRON_TILE (each holds a
     // nonzero); srpt[j] = b_rpt[ib0 + j], the end row clamped to b_nzr
     const u32 nr = b_nzr - ib0 < KRON_TILE ? b_nzr - ib0 : KRON_TILE;
     for (u32 j = threadIdx.x; j <= nr; j += KRON_WG) srpt[j] = b_rpt[ib0 + j];
     __syncthreads();
-    u32 rs[KRON_ITEMS], blen[KRON_ITEMS], bc[KRON_ITEMS];
-#pragma unroll
-    for (u32 i = 0; i < KRON_ITEMS; ++i) {
-        const u32 e = e0 + i * KRON_WG + threadIdx.x;
-        u32 lo = 0, hi = nr;  // last j with srpt[j] <= e
+    auto row_of = [&](u32 e) {  // last j with srpt[j] <= e
+        u32 lo = 0, hi = nr;
         while (hi - lo > 1) {
             const u32 mid = (lo + hi) >> 1;
             if (srpt[mid] <= e) lo = mid;
             else hi = mid;
         }
-        rs[i] = srpt[lo];
-        blen[i] = srpt[lo + 1] - rs[i];
+        return lo;
+    };
+    if (per == 1) {  // nothing to share: each item's stores behind its own search
+        const u32 alen = a1 - a0, abase = a0 * b_nnz;
+#pragma unroll
+        for (u32 i = 0; i < KRON_ITEMS; ++i) {
+            const u32 e = e0 + i * KRON_WG + threadIdx.x;
+            if (e >= e1) break;
+            const u32 j = row_of(e), rs = srpt[j], blen = srpt[j + 1] - rs, bc = b_cols[e];
+            u32 *out = c_cols + abase + alen * rs + (e - rs);
+            for (u32 ka = 0; ka < alen; ++ka) out[ka * blen] = a_cols[a0 + ka] * b_ncols + bc;
+        }
+        return;
+    }
+    u32 rs[KRON_ITEMS], blen[KRON_ITEMS], bc[KRON_ITEMS];
+#pragma unroll
+    for (u32 i = 0; i < KRON_ITEMS; ++i) {
+        const u32 e = e0 + i * KRON_WG + threadIdx.x, j = row_of(e);
+        rs[i] = srpt[j];
+        blen[i] = srpt[j + 1] - rs[i];
         bc[i] = e < e1 ? b_cols[e] : 0u;
     }
-    u32 a0 = a_rpt[ia0];
     for (u32 ia = ia0; ia < ia1; ++ia) {
-        const u32 a1 = a_rpt[ia + 1], alen = a1 - a0;
-        const u32 abase = a0 * b_nnz;
+        const u32 next = ia + 1 < ia1 ? a_rpt[ia + 2] : 0u;
+        const u32 alen = a1 - a0, abase = a0 * b_nnz;
 #pragma unroll
         for (u32 i = 0; i < KRON_ITEMS; ++i) {
             const u32 e = e0 + i * KRON_WG + threadIdx.x;
@@ -99,6 +114,7 @@ __global__ __launch_bounds__(KRON_WG) void k_kron_fill(const u32 *__restrict__ f
                 for (u32 ka = 0; ka < alen; ++ka) out[ka * blen[i]] = a_cols[a0 + ka] * b_ncols + bc[i];
         }
         a0 = a1;
+        a1 = next;
     }
 }
 
