@@ -63,6 +63,15 @@ __global__ void k_pack_pairs(const u32 *__restrict__ rows, const u32 *__restrict
     if (i < n) keys[i] = ((u64)rows[i] << 32) | cols[i];
 }
 
+__global__ void k_copy_pairs(const u32 *__restrict__ rows, const u32 *__restrict__ cols, u64 n,
+                             u32 *__restrict__ out_rows, u32 *__restrict__ out_cols) {
+    const u64 i = (u64)blockIdx.x * blockDim.x + threadIdx.x;
+    if (i < n) {
+        out_rows[i] = rows[i];
+        out_cols[i] = cols[i];
+    }
+}
+
 // Digit counts of tiles [g * per, (g + 1) * per) for workgroup g: before[t][d]
 // = keys of digit d in the group's tiles before t, sums[g][d] = in all of
 // them.
@@ -177,8 +186,18 @@ static void radix_sort(clb_controls_s *ctl, KeysIn in, u64 n, int hi_bits, int l
     if (!n) return;
     if (n > 0xFFFFFFFFull) raise(INVALID_VALUE, "sort of more than 2^32 - 1 keys");
     const int bits = hi_bits + lo_bits - from_bit;
-    // digits of equal width; every sort takes at least one pass, which also
-    // turns halves into keys or back
+    if (n == 1 || bits <= 0) {  // in order as it is
+        if (out.keys) {
+            k_pack_pairs<<<div_up(n, 256), 256, 0, ctl->stream>>>(in.hi, in.lo, n, out.keys);
+            CLB_LAUNCHED("pack_pairs");
+        } else if (in.hi != out.hi) {
+            k_copy_pairs<<<div_up(n, 256), 256, 0, ctl->stream>>>(in.hi, in.lo, n, out.hi, out.lo);
+            CLB_LAUNCHED("copy_pairs");
+        }
+        return;
+    }
+    // digits of equal width; a sort takes at least one pass, which also turns
+    // halves into keys or back
     const int passes = bits > 8 ? (bits + 7) / 8 : 1;
     const int digit_bits = bits > passes ? (bits + passes - 1) / passes : 1;
     const u32 tiles = div_up(n, RX_TILE);
