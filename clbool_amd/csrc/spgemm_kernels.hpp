@@ -653,7 +653,10 @@ __global__ __launch_bounds__(WG) void k_hash(Mats g, const u32 *__restrict__ per
 // each wave keeps the values of its stretch that differ from their predecessor.
 // Merge rounds through a second array, which this replaces, took 162 / 268 us
 // for 1565 rows of up to 4096 and 878 of up to 8192 products (89 / 162 now), in
-// twice the LDS.  64 VGPRs: eight waves a SIMD, as LDS allows.
+// twice the LDS.  Two radix passes or more over at most 128 products take longer
+// than one merge round, though: 100 thousand rows of 120 products over 60 thousand
+// columns 692 us, 579 with it, over 3 million 776 and 575 (of 200 products 571,
+// and 634 with merges).  64 VGPRs: eight waves a SIMD, as LDS allows.
 template <int CAPB, int WG, int MODE>
 __global__ __launch_bounds__(WG, 8) void k_esc(Mats g, const u32 *__restrict__ perm, Out o) {
     constexpr u32 CAP = 1u << CAPB;
@@ -680,8 +683,10 @@ __global__ __launch_bounds__(WG, 8) void k_esc(Mats g, const u32 *__restrict__ p
     for_each_product<WG, 8, BIG_ROW>(g, js, je, big, append);
     __syncthreads();
     const u32 n = cnt < CAP ? cnt : CAP;  // the bin holds rows of at most CAP products
-    dev::lds_radix_sort<WG, PER>(keys, reinterpret_cast<uint16_t *>(big), red, n,
-                                 g.ncols > 1 ? 32 - __clz((int)(g.ncols - 1)) : 0);
+    const int bits = g.ncols > 1 ? 32 - __clz((int)(g.ncols - 1)) : 0;
+    const u32 *sorted = keys;
+    if (CAPB == ESC_MIN_BITS && n <= 128 && bits > 8) sorted = dev::lds_merge_sort<WG>(keys, keys + CAP / 2, n);
+    else dev::lds_radix_sort<WG, PER>(keys, reinterpret_cast<uint16_t *>(big), red, n, bits);
     const u32 wk = ((n + 63) / 64 + NW - 1) / NW * 64;
     const u32 t0 = dev::wave_id() * wk + dev::lane();
     u32 v[PER], c = 0, flags = 0;
@@ -689,8 +694,8 @@ __global__ __launch_bounds__(WG, 8) void k_esc(Mats g, const u32 *__restrict__ p
     for (int q = 0; q < PER; ++q) {
         const u32 t = t0 + q * 64;
         const bool in = (u32)q * 64 < wk && t < n;
-        v[q] = in ? keys[t] : 0u;
-        const bool keep = in && (t == 0 || keys[t - 1] != v[q]);
+        v[q] = in ? sorted[t] : 0u;
+        const bool keep = in && (t == 0 || sorted[t - 1] != v[q]);
         flags |= (keep ? 1u : 0u) << q;
         c += (u32)__popcll(__ballot(keep));
     }
