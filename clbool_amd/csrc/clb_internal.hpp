@@ -233,6 +233,9 @@ void sync(clb_controls_s *ctl);
 // Waits for all streams of the controls, errors ignored: before a failed call
 // releases buffers that its kernels may still use.
 void settle(clb_controls_s *ctl) noexcept;
+// The same before a call that found no room is tried again; whole segments go back
+// to HIP, or what is tried first would take a piece of each.
+void make_room(clb_controls_s *ctl) noexcept;
 
 // Launch-size helpers.
 inline u32 div_up(u64 a, u64 b) { return static_cast<u32>((a + b - 1) / b); }
@@ -261,7 +264,7 @@ void with_room(clb_controls_s *ctl, F &&body) {
     } catch (const Error &e) {
         if (!no_room(e)) throw;
     }
-    settle(ctl);
+    make_room(ctl);
     body(true);
 }
 

@@ -362,7 +362,7 @@ static void unite_products(clb_controls_s *ctl, clb_dcsr *mats, const std::vecto
             unite_batch(ctl, mats, xs, of, batch, total, base, n, prods, splits);
         } catch (const Error &e) {
             if (!no_room(e) || batch.size() == 1) throw;
-            settle(ctl);
+            make_room(ctl);
             most = 0;
             continue;
         }
@@ -571,7 +571,7 @@ clb_status clb_closure_step(clb_controls ctl, clb_dcsr *mats, uint32_t nmats, co
                             nxt.reset();
                             cur.reset();
                             if (pend) finish_pending();
-                            settle(ctl);
+                            make_room(ctl);
                             lean = true;
                         }
                         if (pend) finish_pending();

@@ -124,9 +124,12 @@ static void plan_create(clb_controls_s *ctl, const clb_dcsr &a, const clb_dcsr &
 // no room for one beside it.  No block may be running.
 static void make_lean(clb_controls_s *ctl, clb_spgemm_plan_s &p) {
     settle(ctl);
-    Settled idle(ctl);
-    p.store.drop();
-    drop_packed(p.s);
+    {
+        Settled idle(ctl);
+        p.store.drop();
+        drop_packed(p.s);
+    }
+    make_room(ctl);
     p.s.lean = true;
 }
 

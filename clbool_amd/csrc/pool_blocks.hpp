@@ -36,7 +36,7 @@ class PoolBlocks {
     static constexpr std::size_t KEEP = 64;  // small blocks that stay with an owner after a wait
 
     PoolBlocks(u64 small_max, u64 small_unit, u64 large_unit)
-        : small_max_(small_max), small_(small_unit), large_(large_unit) {}
+        : small_max_(small_max), large_unit_(large_unit), small_(small_unit), large_(large_unit) {}
 
     // A block of at least cap bytes (ptr == nullptr: none): the owner's smallest
     // retired one of at most a quarter more (in_flight: also of those that its
@@ -57,6 +57,12 @@ class PoolBlocks {
             }
         }
         const BlockHeap::Block *b = heap(cap).take(cap);
+        return b ? Block{b->ptr, b->size} : Block{};
+    }
+    // For a small request where there is no memory for a small segment: a large
+    // block, which give_back and retire know by its size.
+    Block take_large(u64 cap) {
+        const BlockHeap::Block *b = large_.take(cap > large_unit_ ? cap : large_unit_);
         return b ? Block{b->ptr, b->size} : Block{};
     }
     void add_segment(char *base, u64 size, u64 cap) { heap(cap).add_segment(base, size); }
@@ -137,7 +143,7 @@ class PoolBlocks {
         retired_bytes_ -= r.size;
         (void)heap(r.size).give_back(r.ptr);
     }
-    u64 small_max_;
+    u64 small_max_, large_unit_;
     BlockHeap small_, large_;
     std::vector<Owner *> owners_;
     u64 retired_bytes_ = 0, clock_ = 1;

@@ -88,6 +88,12 @@ void *Pool::alloc(u64 bytes, u64 *cap_out, clb_controls_s *ctl, bool own) {
     if (prev != device_) (void)hipSetDevice(prev);
     if (e != hipSuccess) {
         (void)hipGetLastError();
+        if (small) {
+            std::lock_guard<std::mutex> lk(mu_);
+            const PoolBlocks::Block b = blocks_.take_large(cap);
+            *cap_out = b.size;
+            if (b.ptr) return b.ptr;
+        }
         std::ostringstream os;
         os << "device allocation of " << cap << " bytes failed: " << hipGetErrorString(e);
         raise(CREATE_BUFFER_ERROR, os.str());
@@ -251,6 +257,14 @@ void plan_ends(clb_controls_s *ctl) {
         if (--ctl->plans || !ctl->destroyed) return;
     }
     controls_end(ctl);
+}
+
+void make_room(clb_controls_s *ctl) noexcept {
+    settle(ctl);
+    try {
+        ctl->pool->trim();
+    } catch (...) {
+    }
 }
 
 void join_side(clb_controls_s *ctl) {
