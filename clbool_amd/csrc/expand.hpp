@@ -11,10 +11,10 @@
 //
 // What bounds it: HBM, at the bytes f moves.  One wave per row, which few rows or
 // long ones still get (k_expand_by_rows), is bound by the chain row pointer ->
-// columns and leaves most lanes idle on short rows (keys of 15.3 million nonzeros in 532 thousand rows: 258
-// us, 68 us now; row ids of 16.1 million nonzeros: 94 us, 39 us now); finding
-// each tile's first row inside its workgroup (a 256-way search, three
-// dependent rounds) took 71 and 57 us.
+// columns and leaves most lanes idle on short rows (keys of 15.3 million nonzeros
+// in 532 thousand rows: 258 us, 68 us now; row ids of 16.1 million nonzeros: 94
+// us, 39 us now); finding each tile's first row inside its workgroup (a 256-way
+// search, three dependent rounds) took 71 and 57 us.
 #pragma once
 
 #include "clb_internal.hpp"
